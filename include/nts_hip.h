@@ -210,7 +210,8 @@ int nts_spmm_gather_static_scratch(const float *in, float *out, const float *w, 
 /* Degree-bucketed schedule for a fixed offsets array (full-graph chunks: CSC_segment_pinned,
  * core/GraphSegment.h:54-133).  Rows are ordered by descending degree class; rows longer than
  * `chunk_edges` are split into chunks whose partial sums are combined by a second kernel in a
- * fixed order (deterministic).  chunk_edges = 0 selects the default.  The call reads `offsets`
+ * fixed order (deterministic).  chunk_edges = 0 selects the default: about 1/8,192 of the edges, a power
+ * of two between 32 and 4,096.  The call reads `offsets`
  * back to the host once and synchronises `stream`. */
 typedef struct nts_spmm_plan nts_spmm_plan_t;
 int nts_spmm_plan_create(nts_spmm_plan_t **plan, const uint32_t *offsets, uint32_t rows,

@@ -1403,6 +1403,21 @@ struct Piece {
   uint32_t slab, row, e0, e1, slot;
 };
 
+// Piece length of a schedule without source ranges when the caller names none.  A piece is one serial
+// chain of row reads, so a launch lasts at least as long as its longest piece: with 4,096-edge pieces
+// whatever the graph, the two widths of an Arxiv-shaped pass (2.48 M edges, F = 128) took 340 us, all of
+// it the tail of a few hub rows.  The chip holds 8,192 wavefronts, so pieces of E / 8,192 edges keep the
+// longest chain at the average share of a wavefront; shorter ones only add partial sums.  Measured, us
+// per pass, 4,096-edge pieces -> the power of two below E / 8,192: 10,556 edges F = 1,433 163 -> 31, F = 16
+// 44 -> 11; 200 K edges F = 128 206 -> 19; 2.48 M edges F = 128 340 -> 107, F = 16 809 -> 70, F = 602 1,187 -> 747;
+// 6 M edges F = 128 326 -> 135.  From 33 M edges up it is 4,096, the better one there (50 M edges F = 128: 512
+// 1,746, 4,096 1,406 us: long pieces of ascending rows keep neighbouring wavefronts on the same sources).
+uint32_t default_chunk(uint32_t edges) {
+  uint32_t chunk = 32;
+  while (chunk < 4096u && 2u * chunk <= edges / 8192u) chunk *= 2;
+  return chunk;
+}
+
 // Builds the work-item list.  Rows with more than `chunk` edges are split into pieces that write
 // partial sums (slots numbered in ascending edge order inside a row, so the second-stage sum has
 // a fixed order).  With n_slabs > 1 and a host copy of the gather indices, pieces of rows whose
@@ -1787,7 +1802,7 @@ int nts_spmm_plan_create(nts_spmm_plan_t **plan_out, const uint32_t *offsets, ui
   if (rows != 0 && !offsets) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_create: null offsets");
   std::vector<uint32_t> off;
   if (int rc = read_offsets(off, offsets, rows, edges, stream)) return rc;
-  return build_plan(plan_out, offsets, off, nullptr, rows, edges, chunk_edges ? chunk_edges : 4096u, 1u, 0u);
+  return build_plan(plan_out, offsets, off, nullptr, rows, edges, chunk_edges ? chunk_edges : default_chunk(edges), 1u, 0u);
 }
 
 int nts_spmm_plan_create_slabs(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const uint32_t *indices,
@@ -1837,7 +1852,9 @@ int nts_spmm_plan_schedule_host(const uint32_t *offsets_host, const uint32_t *in
     return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_schedule_host: null indices");
   Schedule sched;
   const bool with_ranges = indices_host != nullptr;
-  make_schedule(sched, offsets_host, indices_host, rows, chunk_edges ? chunk_edges : (with_ranges ? 512u : 4096u),
+  const uint32_t edges = rows ? offsets_host[rows] : 0u;
+  make_schedule(sched, offsets_host, indices_host, rows,
+                chunk_edges ? chunk_edges : (with_ranges ? 512u : default_chunk(edges)),
                 with_ranges ? (n_slabs ? n_slabs : 32u) : 1u, n_index);
   if (n_items) *n_items = static_cast<uint32_t>(sched.items.size());
   if (n_split_rows) *n_split_rows = static_cast<uint32_t>(sched.splits.size());
