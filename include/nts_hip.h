@@ -407,6 +407,19 @@ int nts_spmm_gather_heads_planned(nts_spmm_plan_t *plan, const float *in, float 
 int nts_sddmm_heads(float *galpha, const float *in, const float *gout, const uint32_t *co,
                     const uint32_t *ri, uint32_t Vd, uint32_t H, uint32_t Fh, nts_stream_t stream);
 
+/* Backward of the attention-weighted aggregation, both gradients in one pass over the gathered rows
+ * (DistAggregateDstFuseWeight::backward and get_additional_grad, core/ntsDistCPUGraphOp.hpp:442-502):
+ *   gx[s, h*Fh + f] (+)= sum_{k in CSR(s)} alpha[perm[k], h] * gout[ci[k], h*Fh + f]
+ *   galpha[perm[k], h] = < x[s, h*Fh : (h+1)*Fh], gout[ci[k], h*Fh : (h+1)*Fh] >
+ * i.e. nts_spmm_gather_heads over the CSR and nts_sddmm_heads over the CSC, which the call falls back to
+ * for heads of more than 64 vectors (256 floats; 64 floats where Fh or an array is off a 16-byte boundary)
+ * and when perm is NULL (alpha and galpha then as those two calls take them; co and ri are only read there).
+ * Scratch as nts_spmm_gather.  accumulate applies to gx. */
+int nts_gat_aggregate_bwd(float *gx, float *galpha, const float *x, const float *gout, const float *alpha,
+                          const uint32_t *perm, const uint32_t *ro, const uint32_t *ci, const uint32_t *co,
+                          const uint32_t *ri, uint32_t Vd, uint32_t Vs, uint32_t edges, uint32_t H, uint32_t Fh,
+                          int accumulate, nts_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Mini-batch assembly
  * ------------------------------------------------------------------------------------------- */

@@ -104,6 +104,10 @@ __device__ __forceinline__ void vfma(float4 &a, float4 x, float w) {
   a.z = fmaf(x.z, w, a.z);
   a.w = fmaf(x.w, w, a.w);
 }
+__device__ __forceinline__ float vdot(float a, float b) { return a * b; }
+__device__ __forceinline__ float vdot(float4 a, float4 b) {
+  return fmaf(a.w, b.w, fmaf(a.z, b.z, fmaf(a.y, b.y, a.x * b.x)));
+}
 __device__ __forceinline__ void vadd(float &a, float x) { a += x; }
 __device__ __forceinline__ void vadd(float2 &a, float2 x) {
   a.x += x.x;
@@ -496,6 +500,142 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
   }
 }
 
+// Backward of the attention-weighted aggregation over the transposed structure, both gradients from one
+// pass over the gathered rows: for source row s and its edges k (destination d = indices[k], edge id
+// e = perm[k] in alpha's order)
+//   out[s, h, :]  = sum_k alpha[e, h] * gout[d, h, :]          (the aggregation, in edge order)
+//   galpha[e, h]  = < x[s, h, :], gout[d, h, :] >
+// The row gout[d] is what either gradient gathers, so the second costs the products and a 4 * H byte
+// store per edge instead of a pass of its own over E rows (DESIGN has the figures).
+// A group of G lanes owns a row (or a piece of one) and G / LH heads of it: LH lanes per head, each with
+// NJ vectors of VEC floats at (sub + LH * j) * VEC of the head's slice, so that a head never shares a lane
+// with another whatever its width (41 or 47 floats: 16 lanes with three floats each).  x[s] stays in
+// registers.  The products of U edges are added over a head's lanes together: each butterfly step
+// halves the edges a lane still holds (U - 1 exchanges for U edges instead of U log2 LH), which leaves
+// lane `sub` with edge sub's sum and spreads the stores over the lanes.
+template <int G, int LH, int NJ, int VEC>
+__global__ __launch_bounds__(256) void attention_grad_kernel(const float *__restrict__ gout, float *__restrict__ out,
+                                                             const float *__restrict__ alpha,
+                                                             const uint32_t *__restrict__ offsets,
+                                                             const uint32_t *__restrict__ indices, uint32_t n_items,
+                                                             uint32_t n_list, uint32_t F,
+                                                             const Item *__restrict__ items,
+                                                             float *__restrict__ partial, int accumulate,
+                                                             HeadArgs heads, uint32_t row_edge_limit,
+                                                             const float *__restrict__ x, float *__restrict__ galpha) {
+  using V = typename Vec<VEC>::type;
+  constexpr int U = NJ * VEC >= 8 ? 4 : 8;   // edges per step
+  constexpr int S = LH < U ? LH : U;         // lanes of a head that end up with a sum to store
+  const uint32_t gl = threadIdx.x & (G - 1), sub = gl & (LH - 1);
+  const uint32_t item = (blockIdx.x * blockDim.x + threadIdx.x) / G;
+  if (item >= n_items) return;  // whole groups leave together; shuffles stay inside a group
+  uint32_t row, e0, e1, slot;
+  if (item < n_list) {
+    const Item it = items[item];
+    row = it.x;
+    e0 = it.y;
+    e1 = it.z;
+    slot = it.w;
+  } else {
+    row = item - n_list;
+    e0 = offsets[row];
+    e1 = offsets[row + 1];
+    slot = kNoSlot;
+    if (e1 - e0 > row_edge_limit) return;  // a long row: its pieces are separate work items
+  }
+  const uint32_t H = heads.H, Fh = heads.Fh;
+  const uint32_t my_head = blockIdx.y * (G / LH) + gl / LH;
+  const bool head_live = my_head < H;
+  const uint32_t head = head_live ? my_head : H - 1;
+  uint32_t col[NJ];
+  bool live[NJ];
+  V acc[NJ], xr[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const uint32_t c = (sub + LH * j) * VEC;
+    live[j] = head_live && c < Fh;
+    col[j] = head * Fh + (c < Fh ? c : 0u);  // idle lanes re-read the head's first columns
+    acc[j] = vzero<VEC>();
+    xr[j] = *reinterpret_cast<const V *>(x + static_cast<size_t>(row) * F + col[j]);
+  }
+  auto fetch_pair = [&](uint32_t e, uint32_t &pi, uint32_t &ps) {
+    pi = ps = 0;
+    if (e < e1) {
+      pi = indices[e];
+      ps = heads.perm[e];
+    }
+  };
+  uint32_t nxt_i, nxt_s;
+  fetch_pair(e0 + gl, nxt_i, nxt_s);
+  for (uint32_t eb = e0; eb < e1; eb += G) {
+    const uint32_t n = min(static_cast<uint32_t>(G), e1 - eb);
+    const uint32_t my_i = nxt_i, my_s = nxt_s;
+    fetch_pair(eb + G + gl, nxt_i, nxt_s);
+    for (uint32_t j0 = 0; j0 < n; j0 += U) {
+      const uint32_t left = n - j0;
+      V v[U][NJ];
+      float wv[U], p[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t si = __shfl(my_i, (j0 + u) & (G - 1), G);
+        const uint32_t ss = __shfl(my_s, (j0 + u) & (G - 1), G);
+        wv[u] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) v[u][j] = vzero<VEC>();
+        if (static_cast<uint32_t>(u) < left) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) v[u][j] = *reinterpret_cast<const V *>(gout + static_cast<size_t>(si) * F + col[j]);
+          wv[u] = alpha[static_cast<size_t>(ss) * H + head];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        p[u] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          if (static_cast<uint32_t>(u) < left) vfma(acc[j], v[u][j], wv[u]);
+          const float q = vdot(v[u][j], xr[j]);
+          p[u] += live[j] ? q : 0.f;
+        }
+      }
+      int cnt = U;
+#pragma unroll
+      for (int m = 1; m < LH; m <<= 1) {
+        if (cnt > 1) {
+          const bool upper = sub & m;
+#pragma unroll
+          for (int i = 0; i < U / 2; ++i) {
+            if (i < cnt / 2) {
+              const float keep = upper ? p[2 * i + 1] : p[2 * i];
+              const float send = upper ? p[2 * i] : p[2 * i + 1];
+              p[i] = keep + __shfl_xor(send, m, kWave);
+            }
+          }
+          cnt /= 2;
+        } else {
+          p[0] += __shfl_xor(p[0], m, kWave);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < U / S; ++i) {
+        const uint32_t u = S * i + (sub & (S - 1));
+        const uint32_t id = __shfl(my_s, (j0 + u) & (G - 1), G);
+        if (head_live && sub < S && u < left) galpha[static_cast<size_t>(id) * H + head] = p[i];
+      }
+    }
+  }
+  float *dst = (slot == kNoSlot) ? out + static_cast<size_t>(row) * F : partial + static_cast<size_t>(slot) * F;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    if (live[j]) {
+      V *q = reinterpret_cast<V *>(dst + col[j]);
+      V r = acc[j];
+      if (accumulate && slot == kNoSlot) vadd(r, *q);
+      *q = r;
+    }
+  }
+}
+
 // Second stage for split rows: out[row,:] (+)= partial[first,:] + partial[first+1,:] + ... in slot
 // order.  Block (x, y) owns 256 columns (tile y) of split row x; `splits[i]` = (row, first slot,
 // slot count, unused).  Eight slots are loaded at a time and then added one after the other, so the
@@ -636,7 +776,50 @@ struct LaunchArgs {
   uint32_t partial_ld = 0;                     // row stride of `partial` in floats (0 = F)
   bool dup_runs = false;                       // rows hold runs of equal indices worth loading once per run
   uint32_t rows_after_items = 0;               // with items: this many whole rows follow the listed items in the launch
+  const float *dot_rows = nullptr;             // with dot_out: the rows whose products with the gathered ones
+  float *dot_out = nullptr;                    // are the gradient of alpha (attention_grad_kernel)
 };
+
+// Lanes per head and vectors per lane of attention_grad_kernel for heads of `vecs` vectors; 16 lanes with up to
+// four vectors each cover 64 vectors, wider heads are not its business.
+constexpr uint32_t kGradMaxVecs = 64;
+bool attention_grad_takes(const LaunchArgs &a, int *vec) {
+  const bool a16 = aligned_to(a.in, 16) && aligned_to(a.out, 16) && aligned_to(a.dot_rows, 16);
+  *vec = a.heads.Fh % 4 == 0 && a16 ? 4 : 1;
+  return a.heads.Fh / *vec <= kGradMaxVecs;
+}
+
+template <int G, int LH, int NJ, int VEC>
+void launch_attention_grad_as(const LaunchArgs &a) {
+  const uint32_t n_list = a.items ? a.n_items : 0u, n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
+  const dim3 grid(ceil_div(n_total, 256 / G), ceil_div(a.heads.H, G / LH));
+  hipLaunchKernelGGL((attention_grad_kernel<G, LH, NJ, VEC>), grid, dim3(256), 0, a.stream, a.in, a.out, a.w, a.offsets,
+                     a.indices, n_total, n_list, a.F, a.items, a.partial, a.accumulate, a.heads, a.row_edge_limit,
+                     a.dot_rows, a.dot_out);
+}
+
+template <int LH, int NJ, int VEC>
+void launch_attention_grad_lanes(const LaunchArgs &a) {
+  // As many heads side by side as there are, in groups of 8 (a tile of edge pairs is one per lane) to 64 lanes.
+  const uint32_t H = a.heads.H;
+  if constexpr (LH <= 8) {
+    if (H * LH <= 8) return launch_attention_grad_as<8, LH, NJ, VEC>(a);
+  }
+  if (H * LH <= 16) return launch_attention_grad_as<16, LH, NJ, VEC>(a);
+  if (H * LH <= 32) return launch_attention_grad_as<32, LH, NJ, VEC>(a);
+  return launch_attention_grad_as<64, LH, NJ, VEC>(a);
+}
+
+template <int VEC>
+void launch_attention_grad(const LaunchArgs &a) {
+  const uint32_t vecs = ceil_div(a.heads.Fh, VEC);
+  if (vecs <= 4) return launch_attention_grad_lanes<4, 1, VEC>(a);
+  if (vecs <= 8) return launch_attention_grad_lanes<8, 1, VEC>(a);
+  if (vecs <= 16) return launch_attention_grad_lanes<16, 1, VEC>(a);
+  if (vecs <= 32) return launch_attention_grad_lanes<16, 2, VEC>(a);
+  if (vecs <= 48) return launch_attention_grad_lanes<16, 3, VEC>(a);
+  return launch_attention_grad_lanes<16, 4, VEC>(a);
+}
 
 template <int VEC, int NACC>
 void launch_wave(const LaunchArgs &a, uint32_t col_base) {
@@ -739,6 +922,11 @@ int pick_vec(const LaunchArgs &a) {
 
 void launch_spmm(const LaunchArgs &a) {
   if (a.n_items == 0) return;
+  if (a.dot_out) {
+    int dot_vec = 1;
+    attention_grad_takes(a, &dot_vec);
+    return dot_vec == 4 ? launch_attention_grad<4>(a) : launch_attention_grad<1>(a);
+  }
   const int vec = pick_vec(a);
   const uint32_t F = a.F;
   // Narrow rows: sub-wavefront groups so that lanes are not left idle.
@@ -2058,6 +2246,34 @@ int nts_spmm_gather_heads_bounded(const float *in, float *out, const float *alph
     return rc;
   }
   NTS_LAUNCH_CHECK("nts_spmm_gather_heads_bounded");
+  return NTS_OK;
+}
+
+int nts_gat_aggregate_bwd(float *gx, float *galpha, const float *x, const float *gout, const float *alpha,
+                          const uint32_t *perm, const uint32_t *ro, const uint32_t *ci, const uint32_t *co,
+                          const uint32_t *ri, uint32_t Vd, uint32_t Vs, uint32_t edges, uint32_t H, uint32_t Fh,
+                          int accumulate, nts_stream_t stream) {
+  NTS_TRACE_RANGE("nts_gat_aggregate_bwd");
+  if (H == 0 || Fh == 0) return nts::fail(NTS_ERR_INVALID, "nts_gat_aggregate_bwd: H or Fh is 0");
+  if (static_cast<uint64_t>(H) * Fh > 0xFFFFFFFFull) return nts::fail(NTS_ERR_INVALID, "nts_gat_aggregate_bwd: H*Fh overflows");
+  if (Vs == 0) return NTS_OK;
+  if (!gx || !ro || (edges && (!galpha || !x || !gout || !alpha || !ci)))
+    return nts::fail(NTS_ERR_INVALID, "nts_gat_aggregate_bwd: null pointer");
+  nts::LaunchArgs a{gout, gx, alpha, ro, ci, 0u, Vs, H * Fh, nullptr, nullptr, accumulate, stream};
+  a.heads = nts::HeadArgs{perm, H, Fh};
+  a.dot_rows = x;
+  a.dot_out = galpha;
+  int vec = 1;
+  if (!edges || !perm || !nts::attention_grad_takes(a, &vec)) {
+    // Heads wider than the fused kernel's lanes, or a structure without its edge permutation: one
+    // pass per gradient.
+    if (edges)
+      if (int rc = nts_sddmm_heads(galpha, x, gout, co, ri, Vd, H, Fh, stream)) return rc;
+    a.dot_rows = nullptr;
+    a.dot_out = nullptr;
+  }
+  if (int rc = nts::launch_spmm_balanced(a, edges)) return rc;
+  NTS_LAUNCH_CHECK("nts_gat_aggregate_bwd");
   return NTS_OK;
 }
 

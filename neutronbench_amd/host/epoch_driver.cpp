@@ -9,8 +9,8 @@
 // (sources can be hubs: nts_spmm_gather cuts long rows on the device).  Outputs are written, not added
 // to, so no buffer is cleared first.  With --heads H every
 // layer is a GAT layer instead: fused attention (nts_gat_attention_fwd) and attention-weighted
-// aggregation (nts_spmm_gather_heads) forward; backward the aggregation over the CSR, the per-edge
-// gradient of alpha (nts_sddmm_heads), the fused attention backward and the sum of the edge
+// aggregation (nts_spmm_gather_heads) forward; backward the aggregation over the CSR with the per-edge
+// gradient of alpha (nts_gat_aggregate_bwd), the fused attention backward and the sum of the edge
 // gradients per source (nts_gather_edge_to_src).  Inputs of the layers after the first, the attention
 // terms and the incoming gradients stand in for the dense layers' results: constant buffers of the
 // right shape, filled once with pseudo-random values.
@@ -368,9 +368,8 @@ int main(int argc, char **argv) {
     for (uint32_t k = hops; k-- > 0;) {
       const nts_sampled_layer_t &L = s.layers[k];
       const float *x = d_ones, *el = d_ones + 8, *g_out = d_ones + 4;  // g_out: [v_size, H * Fh]
-      NTS(nts_spmm_gather_heads(g_out, d_gin, d_alpha[k], L.csr_to_csc, L.row_offset, L.column_indices, L.src_size,
-                                L.e_size, H, Fh, 0, stream));
-      NTS(nts_sddmm_heads(d_galpha, x, g_out, L.column_offset, L.row_indices, L.v_size, H, Fh, stream));
+      NTS(nts_gat_aggregate_bwd(d_gin, d_galpha, x, g_out, d_alpha[k], L.csr_to_csc, L.row_offset, L.column_indices,
+                                L.column_offset, L.row_indices, L.v_size, L.src_size, L.e_size, H, Fh, 0, stream));
       NTS(nts_gat_attention_bwd_bounded(d_gs, d_ger, d_galpha, d_alpha[k], el, d_er, L.column_offset, L.row_indices,
                                         L.v_size, H, slope, L.max_in_degree, stream));
       NTS(nts_gather_edge_to_src(d_gel, d_gs, L.row_offset, L.csr_to_csc, L.src_size, H, 0, stream));

@@ -237,11 +237,10 @@ class GATAggregateOp:
         dev = g_out.device
         stream = torch.cuda.current_stream(dev).cuda_stream
         gx = torch.empty(sg.src_size, g_out.shape[1], dtype=torch.float32, device=dev)
-        call("nts_spmm_gather_heads", ptr(g_out), ptr(gx), ptr(self.alpha), ptr(sg.dev_csr_to_csc), ptr(sg.dev_r_o()),
-             ptr(sg.dev_c_i()), sg.src_size, sg.e_size, self.H, Fh, 0, stream)
         self.galpha = torch.empty(sg.e_size, self.H, dtype=torch.float32, device=dev)
-        call("nts_sddmm_heads", ptr(self.galpha), ptr(self.x), ptr(g_out), ptr(sg.dev_c_o()), ptr(sg.dev_r_i()),
-             sg.v_size, self.H, Fh, stream)
+        call("nts_gat_aggregate_bwd", ptr(gx), ptr(self.galpha), ptr(self.x), ptr(g_out), ptr(self.alpha),
+             ptr(sg.dev_csr_to_csc), ptr(sg.dev_r_o()), ptr(sg.dev_c_i()), ptr(sg.dev_c_o()), ptr(sg.dev_r_i()),
+             sg.v_size, sg.src_size, sg.e_size, self.H, Fh, 0, stream)
         return gx
 
     def get_additional_grad(self):

@@ -1,0 +1,63 @@
+"""nts_gat_aggregate_bwd: both gradients of the attention-weighted aggregation from one pass.  The gradient
+of the rows equals nts_spmm_gather_heads bit for bit (same edges in the same order); the gradient of
+alpha is compared with float64 products: a sum of n products in fp32, in any order, is off by at most
+n * 2^-24 times the sum of the terms' magnitudes."""
+import numpy as np
+import pytest
+import torch
+
+from neutronbench_amd.abi import call, ptr
+from neutronbench_amd.layout import u32_to_i64
+from neutronbench_amd.layout import SampledLayer, as_u32
+from neutronbench_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(device, V, E, seed):
+    src, dst = synth.rmat_edges(V, E, seed=seed, device=device)
+    co, ri = synth.build_csc(src, dst, V)
+    return SampledLayer.from_device_hop(as_u32(co), as_u32(ri), torch.arange(V, dtype=torch.int32, device=device), V)
+
+
+# heads x width: every lane class (4, 8, 16 lanes a head; one to four vectors a lane; 16- and 4-byte lanes), head
+# counts that do not fill a group, several groups of heads, and widths that take one pass per gradient
+SHAPES = [(1, 1), (1, 4), (1, 47), (2, 41), (4, 32), (8, 8), (3, 16), (5, 12), (8, 41), (1, 64), (1, 63), (1, 65), (1, 256),
+          (2, 132), (1, 260), (33, 4), (7, 5)]
+
+
+@pytest.mark.parametrize("H,Fh", SHAPES)
+@pytest.mark.parametrize("V,E", [(700, 5000), (3000, 90000)])
+@pytest.mark.parametrize("skew", [0, 1])
+def test_both_gradients(device, H, Fh, V, E, skew):
+    """skew = 1: arrays off 16-byte boundaries."""
+    layer = _layer(device, V, E, 7)
+    F, Vs, s = H * Fh, layer.src_size, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=device).manual_seed(H * 1000 + Fh)
+
+    def rows(n, width):
+        return torch.randn(n * width + skew, generator=g, device=device)[skew:].view(n, width)
+
+    x, gout, alpha = rows(Vs, F), rows(V, F), rows(E, H)
+    gx, want = torch.full((Vs, F), 3.0, device=device), torch.full((Vs, F), 3.0, device=device)
+    galpha = torch.full((E, H), float("nan"), device=device)
+    for accumulate in (0, 1):
+        call("nts_gat_aggregate_bwd", ptr(gx), ptr(galpha), ptr(x), ptr(gout), ptr(alpha), ptr(layer.dev_csr_to_csc),
+             ptr(layer.dev_r_o()), ptr(layer.dev_c_i()), ptr(layer.dev_c_o()), ptr(layer.dev_r_i()), V, Vs, E, H, Fh,
+             accumulate, s)
+        call("nts_spmm_gather_heads", ptr(gout), ptr(want), ptr(alpha), ptr(layer.dev_csr_to_csc), ptr(layer.dev_r_o()),
+             ptr(layer.dev_c_i()), Vs, E, H, Fh, accumulate, s)
+        assert torch.equal(gx, want)
+    co, ri = u32_to_i64(layer.dev_c_o()), u32_to_i64(layer.dev_r_i())
+    own = torch.repeat_interleave(torch.arange(V, device=device), co[1:] - co[:-1])
+    terms = (x[ri].double() * gout[own].double()).view(E, H, Fh)
+    bound = Fh * 2.0 ** -24 * terms.abs().sum(2) + 1e-30
+    assert ((galpha.double() - terms.sum(2)).abs() <= bound).all()
+
+
+def test_empty_structure(device):
+    gx = torch.full((5, 8), 2.0, device=device)
+    ro = torch.zeros(6, dtype=torch.int32, device=device)
+    call("nts_gat_aggregate_bwd", ptr(gx), 0, 0, 0, 0, 0, ptr(ro), 0, ptr(ro), 0, 5, 5, 0, 2, 4, 0,
+         torch.cuda.current_stream().cuda_stream)
+    assert np.array_equal(gx.cpu().numpy(), np.zeros((5, 8), np.float32))
