@@ -61,8 +61,10 @@ long nts_trace_ranges_emitted(void);
  * order from a memory pool of the library's own, one per device, which keeps freed blocks for the
  * next call instead of returning them to the driver at every synchronisation: the pool holds on to
  * the largest scratch any call has needed (the reference allocates such buffers with cudaMalloc per
- * call, cuda/ntsCUDAGraphOP.cu:595-653).  nts_scratch_trim returns the current device's unused
- * scratch to the driver; work queued earlier is not affected. */
+ * call, cuda/ntsCUDAGraphOP.cu:595-653).  The memory of schedules (their arrays, partial sums and what making
+ * one needs) is kept likewise when a schedule is destroyed, up to 16 GiB per device, for the next schedule
+ * of about that size.  nts_scratch_trim returns the current device's unused scratch and such idle blocks
+ * to the driver; work queued earlier is not affected. */
 int nts_scratch_trim(void);
 /* Scratch blocks the library has taken from its pool so far in this process (every call that needs
  * scratch takes one or two): lets a caller check that a code path allocates nothing. */

@@ -5,6 +5,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <utility>
+
 #include "nts_hip.h"
 
 namespace nts {
@@ -63,7 +65,7 @@ struct TraceRange {
 // fresh allocation): the pool holds on to the largest scratch any call has needed.
 hipError_t scratch_alloc(void **ptr, size_t bytes, hipStream_t stream);
 hipError_t scratch_free(void *ptr, hipStream_t stream);
-hipError_t scratch_trim();  // gives the current device's unused scratch back to the driver
+hipError_t scratch_trim();  // gives the current device's unused scratch and idle blocks back to the driver
 long scratch_alloc_count();  // scratch blocks handed out so far by this process
 
 // A scratch block that is returned to the pool when its scope ends, whichever way the function is
@@ -87,6 +89,36 @@ struct ScratchBlock {
     if (ptr) (void)scratch_free(ptr, stream);
   }
 };
+
+// Device memory of the schedules (their arrays, partial sums and what making one needs): gigabytes that come
+// and go with the objects.  Memory handed back to the driver is cleared there, at about 35 GB/s, and an allocation that
+// meets that clearing waits for it: making and dropping a schedule of 10^8 edges over and over took 80 to 130 ms a
+// time instead of 18, with hipMalloc and with a stream-ordered pool alike (the pool gives blocks back
+// whatever its threshold once it holds several sizes).  So blocks that fall idle are kept, at most
+// kIdleBytes and kIdleBlocks of them per device, for the next taker of about their size; nts_scratch_trim
+// gives them back.  A block is given back only when no work on any stream uses it any more.
+struct DeviceBlock {
+  void *ptr = nullptr;
+  size_t bytes = 0;
+  int device = 0;
+  DeviceBlock() = default;
+  DeviceBlock(const DeviceBlock &) = delete;
+  DeviceBlock &operator=(const DeviceBlock &) = delete;
+  hipError_t take(size_t want);  // an idle block of want .. want + want / 2 bytes, or a new one
+  hipError_t give();             // the caller has waited for all work that uses it
+  ~DeviceBlock() { (void)give(); }
+  template <typename T>
+  T *as() const {
+    return static_cast<T *>(ptr);
+  }
+  void swap(DeviceBlock &other) {
+    std::swap(ptr, other.ptr);
+    std::swap(bytes, other.bytes);
+    std::swap(device, other.device);
+  }
+};
+constexpr size_t kIdleBytes = static_cast<size_t>(16) << 30;
+constexpr size_t kIdleBlocks = 32;
 
 inline bool aligned_to(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
@@ -211,6 +243,24 @@ __device__ __forceinline__ uint32_t owners_of_step(const uint32_t *__restrict__ 
   const uint32_t last = __shfl(win, kWave - 1, kWave);
   if (e >= total) return n;
   return last <= e ? owner_of(off, n, e) : d0 + pos;
+}
+
+// owners_of_step for a walk over long rows: `row` enters as a row with off[row] <= base, `row_end` as the
+// end of a row that holds `base` (0 at the start of a walk).  While the 64 positions lie inside that row
+// nothing is loaded; otherwise the row of the step's last position is carried on.  On a graph of 500
+// edges a row nine steps in ten are of the first kind (plan_sort_keys_kernel, 114.8 M edges: 0.58 -> 0.55 ms,
+// plan_scan_edges_kernel 0.81 -> 0.77 ms).
+__device__ __forceinline__ uint32_t owners_of_row_step(const uint32_t *__restrict__ off, uint32_t n, uint32_t base,
+                                                       uint32_t &row, uint32_t &row_end) {
+  if (row_end > base && row_end - base >= static_cast<uint32_t>(kWave)) return row;
+  const uint32_t own = owners_of_step(off, n, base, row);
+  const uint32_t last = __shfl(own, kWave - 1, kWave);
+  row_end = 0;
+  if (last < n) {
+    row = last;
+    row_end = off[last + 1];
+  }
+  return own;
 }
 
 // Exclusive prefix of `mine` over the THREADS threads of a block, in thread order; *total = the sum.

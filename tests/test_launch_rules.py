@@ -17,3 +17,10 @@ def test_default_piece_length_follows_the_edge_count(edges, longest):
     assert n_splits == 1 and n_partials == 2
     pieces = items[items[:, 3] != NO_SLOT]
     assert sorted((pieces[:, 2] - pieces[:, 1]).tolist()) == [1, longest]
+
+
+def test_root_of_a_degree_in_32_bits():
+    """The weights' roots: for every degree a float can hold, the 32-bit root is the 64-bit one rounded."""
+    deg = np.concatenate([np.arange(1, 1 << 20), np.arange((1 << 24) - (1 << 16), 1 << 24),
+                          np.random.default_rng(1).integers(1, 1 << 24, 1 << 20)]).astype(np.uint32)
+    assert np.array_equal(np.sqrt(deg.astype(np.float32)), np.sqrt(deg.astype(np.float64)).astype(np.float32))
