@@ -27,7 +27,11 @@ inline dim3 wave_block() { return dim3(kWavesPerBlock * kWave); }
 // edges per step, every lane looks up the feature row its edge copies from (the source id, or the
 // destination that owns the edge, followed along the wavefront's contiguous span of edges), and
 // sub-wavefront groups of G lanes then move 64/G rows at a time.  Work per wave does not depend on
-// any vertex's degree.
+// any vertex's degree.  Bound by the writes of the messages (1.27 GB: a fill takes 187 us; 412 -> 287 us from the
+// destinations, 460 -> 367 from the sources, which also read as much from the caches): the next four
+// rows are requested before these four are stored, because a wavefront's loads and stores complete in order and a load
+// behind the stores would wait for them; and the stores leave the feature rows in the caches
+// (outgrows_caches).
 
 enum CopyMode { kFromSrc = 0, kFromDst = 1, kAddFromDst = 2 };
 
@@ -49,6 +53,31 @@ __device__ __forceinline__ uint32_t owner_of_wave(const uint32_t *__restrict__ o
   return lo;
 }
 
+// Messages beyond half of the 256 MB last-level cache are gone from it before the next operator asks for them,
+// and on their way they push out the feature rows and offsets that every operator reads: they are moved
+// with non-temporal loads and stores.  Smaller ones stay in the cache for the next operator.  An operator chain
+// (copies, softmax, sums, forward and backward), us, ordinary -> non-temporal: 26 MB of messages 528 -> 630,
+// 51 MB 455 -> 489, 205 MB 950 -> 854, 1,024 MB 2,490 -> 2,306.
+constexpr uint64_t kStreamedBytes = 128ull << 20;
+__device__ __forceinline__ bool outgrows_caches(uint64_t message_bytes) { return message_bytes > kStreamedBytes; }
+__device__ __forceinline__ void store_streamed(float *p, float v) { __builtin_nontemporal_store(v, p); }
+__device__ __forceinline__ void store_streamed(float4 *p, float4 v) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const f4 w = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(w, reinterpret_cast<f4 *>(p));
+}
+
+__device__ __forceinline__ void vsum(float &r, float a, float b) { r = a + b; }
+__device__ __forceinline__ void vsum(float4 &r, float4 a, float4 b) {
+  r = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+__device__ __forceinline__ float load_streamed(const float *p) { return __builtin_nontemporal_load(p); }
+__device__ __forceinline__ float4 load_streamed(const float4 *p) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const f4 w = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(p));
+  return make_float4(w.x, w.y, w.z, w.w);
+}
+
 template <typename V, int G>
 __global__ __launch_bounds__(256) void edge_copy_kernel(V *__restrict__ msg, const V *__restrict__ feat,
                                                         const uint32_t *__restrict__ ri,
@@ -59,6 +88,8 @@ __global__ __launch_bounds__(256) void edge_copy_kernel(V *__restrict__ msg, con
   const uint32_t lane = lane_id();
   const uint32_t gl = lane & (G - 1), grp = lane / G;
   constexpr uint32_t kEdgesPerStep = kWave / G;
+  constexpr int U = G < 4 ? G : 4;  // rows of a group requested together
+  const bool streamed = outgrows_caches(static_cast<uint64_t>(E) * Fv * sizeof(V));
   const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   // A wavefront walks a contiguous span of wave steps: the destination that owns each step's edges
@@ -81,23 +112,48 @@ __global__ __launch_bounds__(256) void edge_copy_kernel(V *__restrict__ msg, con
     } else {
       row = owners_of_step(co, Vd, static_cast<uint32_t>(base), d0);
     }
+    auto holder_of = [&](uint32_t j) { return j * kEdgesPerStep + grp; };  // lane that looked up this group's edge
+    if (Fv <= G) {
+      const bool col_live = gl < Fv;
+      auto request = [&](uint32_t j0, V(&v)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const uint32_t holder = holder_of(j0 + u), r = __shfl(row, holder, kWave);
+          if (base + holder < E && col_live) v[u] = feat[static_cast<size_t>(r) * Fv + gl];
+        }
+      };
+      V cur[U], nxt[U];
+      request(0, cur);
+#pragma unroll
+      for (uint32_t j0 = 0; j0 < G; j0 += U) {
+        if (j0 + U < G) request(j0 + U, nxt);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const uint64_t ee = base + holder_of(j0 + u);
+          if (ee < E && col_live) {
+            V *dst = msg + ee * Fv + gl;
+            V v = cur[u];
+            if (mode == kAddFromDst) vsum(v, *dst, v);
+            if (streamed) store_streamed(dst, v);
+            else *dst = v;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+      }
+      continue;
+    }
     for (uint32_t j = 0; j < G; ++j) {
-      const uint32_t holder = j * kEdgesPerStep + grp;  // lane that looked up this group's edge
-      const uint32_t r = __shfl(row, holder, kWave);
+      const uint32_t holder = holder_of(j), r = __shfl(row, holder, kWave);
       const uint64_t ee = base + holder;
       if (ee < E) {
         const V *src = feat + static_cast<size_t>(r) * Fv;
         V *dst = msg + ee * Fv;
         for (uint32_t c = gl; c < Fv; c += G) {
           V v = src[c];
-          if (mode == kAddFromDst) {
-            const V o = dst[c];
-            float *vf = reinterpret_cast<float *>(&v);
-            const float *of = reinterpret_cast<const float *>(&o);
-#pragma unroll
-            for (int t = 0; t < static_cast<int>(sizeof(V) / 4); ++t) vf[t] = of[t] + vf[t];
-          }
-          dst[c] = v;
+          if (mode == kAddFromDst) vsum(v, dst[c], v);
+          if (streamed) store_streamed(dst + c, v);
+          else dst[c] = v;
         }
       }
     }
@@ -117,7 +173,7 @@ __global__ __launch_bounds__(256) void edge_copy_kernel(V *__restrict__ msg, con
 constexpr uint32_t kNoLimit = 0xFFFFFFFFu;
 constexpr uint32_t kLongRowEdges = 1024;    // edges of a row above which the block kernel takes over
 constexpr uint64_t kGiantValues = 131072;   // softmax segments above this many values are cut into pieces
-constexpr uint64_t kGiantRowEdges = 16384;  // edges of a row above which it is cut into pieces for several blocks
+constexpr uint64_t kGiantRowBytes = 1u << 20;  // row of edge rows above which it is cut into pieces for several blocks
 constexpr uint32_t kLongRowValues = 32768;  // the same for softmax segments, in values (edges * heads)
 constexpr uint32_t kLongMinVertices = 16384;  // vertex count below which the extra launches are not worth it
 constexpr int kLongBlock = 1024;
@@ -274,7 +330,8 @@ __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out,
                                 accumulate, long_part);
   }
   const uint32_t n_pieces = lw.hdr[1];
-  for (uint32_t p = blockIdx.x; p < n_pieces; p += lw.blocks) {
+  // the pieces start with the blocks that the rows left idle
+  for (uint32_t p = (blockIdx.x + lw.blocks - n_rows % lw.blocks) % lw.blocks; p < n_pieces; p += lw.blocks) {
     const uint4 pc = lw.pieces[p];
     block_sum_edge_rows<V, 256>(lw.partial + static_cast<size_t>(p) * Fv, msg, perm, pc.z, pc.w, Fv, lw.tile, 0,
                                 long_part);
@@ -335,6 +392,7 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
   // The wavefronts share the rows by weight, a row counting one plus its edges: wavefront w takes the
   // rows r with w C <= (off[r] - off[0]) + r < (w + 1) C.
   const uint32_t off0 = off[0];
+  const bool streamed = outgrows_caches(static_cast<uint64_t>(off[rows] - off0) * Fv * sizeof(V));
   const uint64_t total = static_cast<uint64_t>(off[rows] - off0) + rows;
   const uint64_t share = (total + n_waves - 1) / n_waves;
   const uint64_t x0 = wave * share < total ? wave * share : total;
@@ -342,92 +400,97 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
   if (x0 == x1) return;
   const uint32_t r_begin = first_row_of_weight(off, rows, off0, x0);
   const uint32_t r_end = first_row_of_weight(off, rows, off0, x1);
-  for (uint64_t base = r_begin; base < r_end; base += kWave) {
-    const uint32_t n_set = r_end - base < kWave ? static_cast<uint32_t>(r_end - base) : kWave;
-    uint32_t my_e1 = 0;
-    if (lane < n_set) my_e1 = off[base + lane + 1];
-    uint32_t pos = off[base];                       // next edge to add (wave-uniform)
-    const uint32_t range_end = wave_read(my_e1, n_set - 1);
-    uint32_t j = 0;                                 // current row of the set
-    float acc[OWN];
+  // The whole walk once per kind of load: a choice at each load keeps them from being in flight together.
+  auto walk = [&](auto load) {
+    for (uint64_t base = r_begin; base < r_end; base += kWave) {
+      const uint32_t n_set = r_end - base < kWave ? static_cast<uint32_t>(r_end - base) : kWave;
+      uint32_t my_e1 = 0;
+      if (lane < n_set) my_e1 = off[base + lane + 1];
+      uint32_t pos = off[base];                       // next edge to add (wave-uniform)
+      const uint32_t range_end = wave_read(my_e1, n_set - 1);
+      uint32_t j = 0;                                 // current row of the set
+      float acc[OWN];
 #pragma unroll
-    for (int o = 0; o < OWN; ++o) acc[o] = 0.f;
-    V cur[U];
-    auto load_round = [&](uint32_t k) {
+      for (int o = 0; o < OWN; ++o) acc[o] = 0.f;
+      V cur[U];
+      auto load_round = [&](uint32_t k) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        cur[u] = V{};
-        const uint32_t idx = k + u * kSlots + slot;
-        if (idx < range_end && col_live) cur[u] = msg[static_cast<size_t>(idx) * Fv + col];
-      }
-    };
-    // Rows that end at `pos` are complete: written out (a skipped long row is not), next row.
-    auto finish_rows = [&](bool skip_first) {
-      bool skip = skip_first;
-      while (j < n_set && wave_read(my_e1, j) == pos) {
-        if (!skip) {
+        for (int u = 0; u < U; ++u) {
+          cur[u] = V{};
+          const uint32_t idx = k + u * kSlots + slot;
+          if (idx < range_end && col_live) cur[u] = load(msg + static_cast<size_t>(idx) * Fv + col);
+        }
+      };
+      // Rows that end at `pos` are complete: written out (a skipped long row is not), next row.
+      auto finish_rows = [&](bool skip_first) {
+        bool skip = skip_first;
+        while (j < n_set && wave_read(my_e1, j) == pos) {
+          if (!skip) {
+#pragma unroll
+            for (int o = 0; o < OWN; ++o) {
+              const uint32_t c = lane + o * kWave;
+              if (c < comps) {
+                float *p = reinterpret_cast<float *>(out) + (base + j) * comps + c;
+                float v = acc[o];
+                if (accumulate) v += *p;
+                *p = v;
+              }
+            }
+          }
+          skip = false;
+#pragma unroll
+          for (int o = 0; o < OWN; ++o) acc[o] = 0.f;
+          ++j;
+        }
+      };
+      finish_rows(false);  // empty rows at the head of the set
+      uint32_t loaded = 0xFFFFFFFFu;  // first edge of the round held in `cur`
+      while (j < n_set) {
+        const uint32_t row_end = wave_read(my_e1, j);
+        if (row_end - pos > long_limit) {  // pos is this row's first edge: nothing of it has been added
+          pos = row_end;
+          finish_rows(true);
+          continue;
+        }
+        const uint32_t ts = pos;  // this round covers [ts, ts + kRound)
+        if (loaded != ts) load_round(ts);
+        __builtin_amdgcn_wave_barrier();  // the previous round's reads of the tile are done
+#pragma unroll
+        for (int u = 0; u < U; ++u) reinterpret_cast<V *>(tile)[u * kWave + lane] = cur[u];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        loaded = ts + kRound;
+        if (loaded < range_end) load_round(loaded);  // in flight while this round is added up
+        const uint32_t tile_end = range_end - ts < kRound ? range_end : ts + kRound;
+        while (pos < tile_end && j < n_set) {
+          const uint32_t e1 = wave_read(my_e1, j);
+          if (e1 - pos > long_limit) break;  // a long row starts here (a shorter one never has that much left)
+          const uint32_t end = e1 < tile_end ? e1 : tile_end;
 #pragma unroll
           for (int o = 0; o < OWN; ++o) {
-            const uint32_t c = lane + o * kWave;
-            if (c < comps) {
-              float *p = reinterpret_cast<float *>(out) + (base + j) * comps + c;
-              float v = acc[o];
-              if (accumulate) v += *p;
-              *p = v;
+            if (lane + o * kWave < comps) {
+              const float *t = tile + (pos - ts) * kPitch + lane + o * kWave;
+              float a = acc[o];
+              uint32_t i = pos;
+              for (; i + 4 <= end; i += 4, t += 4 * kPitch) {
+                a += t[0];
+                a += t[kPitch];
+                a += t[2 * kPitch];
+                a += t[3 * kPitch];
+              }
+              for (; i < end; ++i, t += kPitch) a += t[0];
+              acc[o] = a;
             }
           }
+          pos = end;
+          if (pos == e1) finish_rows(false);
         }
-        skip = false;
-#pragma unroll
-        for (int o = 0; o < OWN; ++o) acc[o] = 0.f;
-        ++j;
-      }
-    };
-    finish_rows(false);  // empty rows at the head of the set
-    uint32_t loaded = 0xFFFFFFFFu;  // first edge of the round held in `cur`
-    while (j < n_set) {
-      const uint32_t row_end = wave_read(my_e1, j);
-      if (row_end - pos > long_limit) {  // pos is this row's first edge: nothing of it has been added
-        pos = row_end;
-        finish_rows(true);
-        continue;
-      }
-      const uint32_t ts = pos;  // this round covers [ts, ts + kRound)
-      if (loaded != ts) load_round(ts);
-      __builtin_amdgcn_wave_barrier();  // the previous round's reads of the tile are done
-#pragma unroll
-      for (int u = 0; u < U; ++u) reinterpret_cast<V *>(tile)[u * kWave + lane] = cur[u];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      loaded = ts + kRound;
-      if (loaded < range_end) load_round(loaded);  // in flight while this round is added up
-      const uint32_t tile_end = range_end - ts < kRound ? range_end : ts + kRound;
-      while (pos < tile_end && j < n_set) {
-        const uint32_t e1 = wave_read(my_e1, j);
-        if (e1 - pos > long_limit) break;  // a long row starts here (a shorter one never has that much left)
-        const uint32_t end = e1 < tile_end ? e1 : tile_end;
-#pragma unroll
-        for (int o = 0; o < OWN; ++o) {
-          if (lane + o * kWave < comps) {
-            const float *t = tile + (pos - ts) * kPitch + lane + o * kWave;
-            float a = acc[o];
-            uint32_t i = pos;
-            for (; i + 4 <= end; i += 4, t += 4 * kPitch) {
-              a += t[0];
-              a += t[kPitch];
-              a += t[2 * kPitch];
-              a += t[3 * kPitch];
-            }
-            for (; i < end; ++i, t += kPitch) a += t[0];
-            acc[o] = a;
-          }
-        }
-        pos = end;
-        if (pos == e1) finish_rows(false);
       }
     }
-  }
+  };
+  if (streamed) walk([](const V *p) { return load_streamed(p); });
+  else walk([](const V *p) { return *p; });
 }
 
 // The same sums for rows that fit one group (Fv <= G), with the rows of a wavefront handed out
@@ -477,6 +540,7 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
   const uint64_t wave = (static_cast<uint64_t>(blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / kWave;
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x - lw.blocks) * blockDim.x / kWave;
   const bool col_live = col < Fv;
+  const bool streamed = outgrows_caches(static_cast<uint64_t>(off[rows] - off[0]) * Fv * sizeof(V));
   for (uint64_t base = wave * kSet; base < rows; base += n_waves * kSet) {
     uint32_t my_e0 = 0, my_e1 = 0;
     bool mine = false;
@@ -537,6 +601,17 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
     bool have = false;
     uint32_t row = 0, k = 0, e1 = 0;
     float a[NF];
+    // The edge ids of a group's next round are requested while the rows of this one are on their way, so a
+    // round is one memory latency and not two.
+    uint32_t id[8];
+    auto request_ids = [&](uint32_t from) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const uint32_t idx = from + u * S + slice;
+        id[u] = 0;
+        if (idx < e1) id[u] = perm ? perm[idx] : idx;
+      }
+    };
     while (true) {
       // Groups without a row take the lowest pending rows, in group order.
       const uint64_t need_mask = __ballot(!have && gl == 0);
@@ -556,6 +631,7 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
         have = true;
         k = new_e0;
         e1 = new_e1;
+        request_ids(k);
 #pragma unroll
         for (int t = 0; t < NF; ++t) a[t] = 0.f;
       }
@@ -566,15 +642,17 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
         // ...), added in order
         V v[8];
         const uint32_t n = e1 - k < 8u * S ? e1 - k : 8u * S;
+        auto request_rows = [&](auto load) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          v[u] = V{};
-          const uint32_t idx = u * S + slice;
-          if (idx < n && col_live) {
-            const uint32_t e = perm ? perm[k + idx] : k + idx;
-            v[u] = msg[static_cast<size_t>(e) * Fv + col];
+          for (int u = 0; u < 8; ++u) {
+            v[u] = V{};
+            const uint32_t idx = u * S + slice;
+            if (idx < n && col_live) v[u] = load(msg + static_cast<size_t>(id[u]) * Fv + col);
           }
-        }
+        };
+        if (streamed) request_rows([](const V *p) { return load_streamed(p); });
+        else request_rows([](const V *p) { return *p; });
+        if (k + n < e1) request_ids(k + n);
         if (S == 1) {
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
@@ -678,17 +756,18 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
 // launch (a 300,000-edge hub next to 10^4 rows of a few thousand edges) is cut into pieces that
 // separate blocks reduce, and a last kernel combines the pieces in order.  The caller's argument
 // lists carry no edge count, so everything is sized by fixed capacities and decided on the device:
-// up to kGiantCap rows are listed (further ones simply stay with the one-block-per-row kernel), and
-// the piece length is chosen so that the listed rows need at most kPieceCap pieces.
-constexpr uint32_t kGiantCap = 1024;
+// a row is giant above the limit of its operator or above a 1/kGiantCap share of all edges, whichever
+// is more, so there are never more than kGiantCap of them whatever order they are found in, and
+// the piece length is chosen so that they need at most kPieceCap pieces.
+constexpr uint32_t kGiantCap = 4096;
 constexpr uint32_t kPieceCap = 8192;
-constexpr uint32_t kGiantMinPiece = 4096;  // edges
+constexpr uint32_t kGiantMinPiece = 4096;  // edges, for the softmax segments
 
-// hdr: [0] giant rows seen (may exceed kGiantCap until the plan kernel clamps it), [1] pieces,
+// hdr: [0] giant rows, [1] pieces,
 //      [2] edges per piece, [4..5] edges of the listed giant rows (64-bit), [6] the long-row counter
 //      (`count` points here, so that one fill clears all of them).
 // list[0 .. *count) = rows r with (off[r+1] - off[r]) * width > limit that are not listed as giant
-// (any order); giant_rows[0 .. min(hdr[0], kGiantCap)) = rows above giant_limit values.
+// (any order); giant_rows[0 .. hdr[0]) = rows above giant_limit values and above the share.
 __global__ __launch_bounds__(256) void collect_long_rows_kernel(uint32_t *__restrict__ list,
                                                                 uint32_t *__restrict__ count,
                                                                 uint32_t *__restrict__ giant_rows,
@@ -700,7 +779,7 @@ __global__ __launch_bounds__(256) void collect_long_rows_kernel(uint32_t *__rest
   if (r >= rows) return;
   const uint32_t deg = off[r + 1] - off[r];
   const uint64_t n = static_cast<uint64_t>(deg) * width;
-  if (n > giant_limit) {
+  if (n > giant_limit && deg > (off[rows] - off[0]) / kGiantCap) {
     const uint32_t gi = atomicAdd(&hdr[0], 1u);
     if (gi < kGiantCap) {
       giant_rows[gi] = r;
@@ -711,38 +790,45 @@ __global__ __launch_bounds__(256) void collect_long_rows_kernel(uint32_t *__rest
   if (n > limit) list[atomicAdd(count, 1u)] = r;
 }
 
-// One block: fixes the piece length, gives every listed giant row its first piece (a serial prefix
-// over at most kGiantCap rows) and writes the piece table (list position, row, first edge, end).
+// One block: fixes the piece length, gives every listed giant row its first piece (every thread counts
+// the pieces of a run of rows, then one prefix over the block) and writes the piece table (list
+// position, row, first edge, end), a wavefront a row.
 __global__ __launch_bounds__(256) void giant_plan_kernel(uint32_t *__restrict__ hdr,
                                                          const uint32_t *__restrict__ giant_rows,
                                                          uint32_t *__restrict__ first, uint4 *__restrict__ pieces,
-                                                         const uint32_t *__restrict__ off) {
-  __shared__ uint32_t n_sh, len_sh;
-  if (threadIdx.x == 0) {
-    const uint32_t n = hdr[0] < kGiantCap ? hdr[0] : kGiantCap;
-    const unsigned long long edges = *reinterpret_cast<const unsigned long long *>(hdr + 4);
-    unsigned long long len = (edges + (kPieceCap - kGiantCap) - 1) / (kPieceCap - kGiantCap);
-    if (len < kGiantMinPiece) len = kGiantMinPiece;
-    uint32_t p = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-      first[i] = p;
-      const uint32_t r = giant_rows[i];
-      p += static_cast<uint32_t>((off[r + 1] - off[r] + len - 1) / len);
-    }
-    first[n] = p;
-    hdr[0] = n;
-    hdr[1] = p;
-    hdr[2] = static_cast<uint32_t>(len);
-    n_sh = n;
-    len_sh = static_cast<uint32_t>(len);
-  }
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < n_sh; i += blockDim.x) {
+                                                         const uint32_t *__restrict__ off, uint32_t min_piece) {
+  __shared__ uint32_t wave_sums[256 / kWave];
+  const uint32_t n = hdr[0] < kGiantCap ? hdr[0] : kGiantCap;
+  const unsigned long long edges = *reinterpret_cast<const unsigned long long *>(hdr + 4);
+  const unsigned long long even = (edges + (kPieceCap - kGiantCap) - 1) / (kPieceCap - kGiantCap);
+  const uint32_t len = even < min_piece ? min_piece : static_cast<uint32_t>(even);
+  auto pieces_of = [&](uint32_t i) -> uint32_t {
     const uint32_t r = giant_rows[i];
-    const uint32_t e1 = off[r + 1];
-    uint32_t p = first[i];
-    for (uint64_t k = off[r]; k < e1; k += len_sh, ++p)
-      pieces[p] = make_uint4(i, r, static_cast<uint32_t>(k), static_cast<uint32_t>(k + len_sh < e1 ? k + len_sh : e1));
+    return (off[r + 1] - off[r] - 1) / len + 1;
+  };
+  const uint32_t per = (n + 255) / 256;
+  const uint32_t i0 = min(n, threadIdx.x * per), i1 = min(n, i0 + per);
+  uint32_t mine = 0, total = 0;
+  for (uint32_t i = i0; i < i1; ++i) mine += pieces_of(i);
+  uint32_t p = block_prefix<256>(mine, wave_sums, &total);
+  for (uint32_t i = i0; i < i1; ++i) {
+    first[i] = p;
+    p += pieces_of(i);
+  }
+  if (threadIdx.x == 0) {
+    first[n] = total;
+    hdr[0] = n;
+    hdr[1] = total;
+    hdr[2] = len;
+  }
+  __syncthreads();  // `first` is read by other threads of this block below
+  for (uint32_t i = threadIdx.x / kWave; i < n; i += 256 / kWave) {
+    const uint32_t r = giant_rows[i];
+    const uint32_t e0 = off[r], e1 = off[r + 1], p0 = first[i], n_pieces = (e1 - e0 - 1) / len + 1;
+    for (uint32_t q = lane_id(); q < n_pieces; q += kWave) {
+      const uint32_t k = e0 + q * len;
+      pieces[p0 + q] = make_uint4(i, r, k, e1 - k < len ? e1 : k + len);
+    }
   }
 }
 
@@ -790,7 +876,15 @@ __global__ __launch_bounds__(256) void giant_sum_combine_kernel(float *__restric
     const uint32_t p0 = first[i], p1 = first[i + 1];
     for (uint32_t c = threadIdx.x; c < F; c += blockDim.x) {
       float a = 0.f;
-      for (uint32_t p = p0; p < p1; ++p) a += partial[static_cast<size_t>(p) * F + c];
+      uint32_t p = p0;
+      for (; p + 8 <= p1; p += 8) {  // eight pieces requested at once, added in order
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = partial[static_cast<size_t>(p + u) * F + c];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) a += v[u];
+      }
+      for (; p < p1; ++p) a += partial[static_cast<size_t>(p) * F + c];
       float *dst = out + static_cast<size_t>(r) * F + c;
       *dst = accumulate ? *dst + a : a;
     }
@@ -1890,10 +1984,10 @@ struct LongRows {
 // count makes hubs likely, the ones above `giant_limit` values separately (with their piece table);
 // returns with lr.list == nullptr when the long path is not used.
 int collect_long_rows(LongRows &lr, const uint32_t *off, uint32_t rows, uint32_t width, uint32_t limit,
-                      uint64_t giant_limit, hipStream_t stream) {
+                      uint64_t giant_limit, uint32_t min_piece, hipStream_t stream) {
   if (rows < kLongMinVertices) return NTS_OK;
   const size_t list_bytes = (static_cast<size_t>(rows) + 7) / 8 * 8 * sizeof(uint32_t);  // list, 32-byte multiple
-  const size_t small_bytes = (8 + kGiantCap + kGiantCap + 8) * sizeof(uint32_t);         // hdr (with the counter), rows, first
+  const size_t small_bytes = (8 + kGiantCap + kGiantCap + 8) * sizeof(uint32_t);  // hdr (with the counter), rows, first
   NTS_HIP_TRY(lr.block.alloc(list_bytes + small_bytes + kPieceCap * sizeof(uint4), stream));
   unsigned char *buf = static_cast<unsigned char *>(lr.block.ptr);
   lr.list = reinterpret_cast<uint32_t *>(buf);
@@ -1906,7 +2000,8 @@ int collect_long_rows(LongRows &lr, const uint32_t *off, uint32_t rows, uint32_t
   hipLaunchKernelGGL(collect_long_rows_kernel, dim3(ceil_div(rows, 256)), dim3(256), 0, stream, lr.list, lr.count,
                      lr.giant_rows, lr.hdr, off, rows, width, limit, giant_limit);
   NTS_LAUNCH_CHECK("collect_long_rows_kernel");
-  hipLaunchKernelGGL(giant_plan_kernel, dim3(1), dim3(256), 0, stream, lr.hdr, lr.giant_rows, lr.first, lr.pieces, off);
+  hipLaunchKernelGGL(giant_plan_kernel, dim3(1), dim3(256), 0, stream, lr.hdr, lr.giant_rows, lr.first, lr.pieces, off,
+                     min_piece);
   NTS_LAUNCH_CHECK("giant_plan_kernel");
   return NTS_OK;
 }
@@ -1962,8 +2057,10 @@ template <typename V>
 void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_t *perm, uint32_t rows, uint32_t Fv,
                         int accumulate, uint32_t limit, const LongRowWork<V> &lw, hipStream_t stream) {
   if (rows_launch_takes_long_rows(rows, Fv) && !perm && stream_contiguous_rows()) {
-    // a wavefront streams the contiguous edges of 64 rows at a time
-    const uint32_t blocks = ceil_div(rows, 4 * kWave);
+    // a wavefront streams the contiguous edges of up to 64 rows at a time
+    // (16 rows of 128 bytes and more: 64 leave an Arxiv-shaped vertex set with a third of the wavefronts that
+    // the chip holds, 1.27 GB of edge rows 423 -> 373 us)
+    const uint32_t blocks = ceil_div(rows, Fv * sizeof(V) >= 128 ? 4 * 16 : 4 * kWave);
     const dim3 grid((blocks < 16384u ? blocks : 16384u) + lw.blocks);
 #define NTS_STREAM(GG)                                                                                          \
   hipLaunchKernelGGL((gather_edge_to_row_stream_kernel<V, GG>), grid, dim3(256), 0, stream, out, msg, off, rows, Fv, \
@@ -2023,7 +2120,15 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   if (rows == 0) return NTS_OK;
   if (!out || !msg || !off) return fail(NTS_ERR_INVALID, who);
   LongRows lr;
-  if (int rc = collect_long_rows(lr, off, rows, 1u, kLongRowEdges, kGiantRowEdges, stream)) return rc;
+  // A block reads a row at 20 to 40 GB/s, whatever the rest of the chip does, so the bound is one on bytes: up
+  // to 64 bytes an edge row it is 16,384 edges in pieces of 4,096; at 512 bytes 2,048 in pieces of 512
+  // (one block and up to 8 MB before: the sums over 1.27 GB of edge rows 463 -> 422 us, through a
+  // permutation 669 -> 605).
+  uint64_t giant_edges = kGiantRowBytes / (4ull * F);
+  giant_edges = giant_edges > 16384 ? 16384 : giant_edges < kLongRowEdges ? kLongRowEdges : giant_edges;
+  if (int rc = collect_long_rows(lr, off, rows, 1u, kLongRowEdges, giant_edges, static_cast<uint32_t>(giant_edges / 4),
+                                 stream))
+    return rc;
   const uint32_t limit = lr.list ? kLongRowEdges : kNoLimit;
   // 16-byte vectors for the row kernels and the block kernels alike
   const bool v4 = F % 4 == 0 && aligned_to(out, 16) && aligned_to(msg, 16);
@@ -2166,7 +2271,7 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   // stated is still computed, by one wavefront.
   const bool no_hubs = max_degree != 0 && static_cast<uint64_t>(max_degree) * H <= kLongRowValues;
   if (pow2 && !no_hubs)
-    if (int rc = collect_long_rows(lr, co, Vd, H, kLongRowValues, kGiantValues, stream)) return rc;
+    if (int rc = collect_long_rows(lr, co, Vd, H, kLongRowValues, kGiantValues, kGiantMinPiece, stream)) return rc;
   const uint32_t max_values = lr.list ? kLongRowValues : kNoLimit;
   // The block kernels of the hub rows and the kernels of the giant ones' pieces run on the side lane,
   // beside the launches for all other rows below (they write other rows); their scratch is taken
