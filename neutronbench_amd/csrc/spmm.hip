@@ -506,7 +506,8 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
 //   out[s, h, :]  = sum_k alpha[e, h] * gout[d, h, :]          (the aggregation, in edge order)
 //   galpha[e, h]  = < x[s, h, :], gout[d, h, :] >
 // The row gout[d] is what either gradient gathers, so the second costs the products and a 4 * H byte
-// store per edge instead of a pass of its own over E rows (DESIGN has the figures).
+// store per edge instead of a pass of its own over E rows (126 M edges, 4 heads of 32: an attention layer's
+// forward and backward 32.5 -> 27.2 ms, of which nts_sddmm_heads was 8.1; 2.48 M edges, one head of 47: 1,115 -> 853 us).
 // A group of G lanes owns a row (or a piece of one) and G / LH heads of it: LH lanes per head, each with
 // NJ vectors of VEC floats at (sub + LH * j) * VEC of the head's slice, so that a head never shares a lane
 // with another whatever its width (41 or 47 floats: 16 lanes with three floats each).  x[s] stays in
