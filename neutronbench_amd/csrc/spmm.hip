@@ -1333,7 +1333,7 @@ struct PlanCounters {  // device words read back to the host
   uint32_t unsorted_long_row;   // a row that would be cut does not ascend
   uint32_t n_splits;
   uint32_t bad_offsets, bad_total;
-  uint32_t pad;
+  uint32_t first_edge;          // offsets[0]
 };
 
 __device__ __forceinline__ uint32_t lower_bound_index(const uint32_t *__restrict__ idx, uint32_t lo, uint32_t hi,
@@ -1434,6 +1434,7 @@ __global__ __launch_bounds__(256) void plan_check_offsets_kernel(const uint32_t 
   const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r < rows && off[r + 1] < off[r]) counters->bad_offsets = 1u;
   if (r == 0 && off[rows] != edges) counters->bad_total = 1u;
+  if (r == 0) counters->first_edge = off[0];
 }
 
 // One pass over the edges: every wavefront walks a contiguous span of edges and carries the row along
@@ -1897,11 +1898,14 @@ int build_plan(nts_spmm_plan_t **plan_out, const uint32_t *offsets_dev, const st
   return NTS_OK;
 }
 
-// Builds the schedule of make_schedule on the device (kernels above).
+// Builds the schedule of make_schedule on the device (kernels above).  *fell_back is set, and nothing built,
+// where the first row does not start at edge 0: the edges before it belong to no row, while the kernels
+// give every edge to the row before it (row 0 would be ordered together with them).
 int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const uint32_t *indices,
                       uint32_t index_base, uint32_t n_index, uint32_t rows, uint32_t edges, uint32_t chunk,
-                      uint32_t n_slabs, hipStream_t stream) {
+                      uint32_t n_slabs, hipStream_t stream, bool *fell_back) {
   using nts::Item;
+  *fell_back = false;
   nts::PlanShape sh;
   sh.chunk = chunk;
   sh.n_slabs = n_slabs;
@@ -1962,6 +1966,10 @@ int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const
   NTS_HIP_TRY(read_counters());
   if (host_counters.bad_total) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_create: offsets[rows] != edges");
   if (host_counters.bad_offsets) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_create: offsets not ascending");
+  if (host_counters.first_edge) {
+    *fell_back = true;
+    return NTS_OK;
+  }
   const uint32_t edge_blocks = std::min(nts::ceil_div(edges, 1024), 2048u);
   auto scan_edges = [&](const uint32_t *idx) -> hipError_t {
     hipLaunchKernelGGL(nts::plan_scan_edges_kernel, dim3(edge_blocks), dim3(256), 0, stream, offsets, idx, rows, edges,
@@ -2120,15 +2128,19 @@ int nts_spmm_plan_create_slabs(nts_spmm_plan_t **plan_out, const uint32_t *offse
   if (edges != 0 && !indices) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_create_slabs: null indices");
   const uint32_t chunk = chunk_edges ? chunk_edges : 512u, slabs = n_slabs ? n_slabs : 32u;
   // The schedule is built on the device where that reproduces the host's (source ranges in use, sizes
-  // within the 32-bit sort keys and the range table); NTS_SPMM_PLAN_HOST=1 forces the host path.
+  // within the 32-bit sort keys and the range table, rows from edge 0 on); NTS_SPMM_PLAN_HOST=1 forces the host path.
   static const bool force_host = [] {
     const char *e = getenv("NTS_SPMM_PLAN_HOST");
     return e && e[0] != '0';
   }();
   if (!force_host && slabs > 1 && n_index > 0 && rows > 0 && edges > 0 &&
       static_cast<uint64_t>(slabs) * (static_cast<uint64_t>(chunk) + 1) < (1ull << 32) && slabs <= 4096 &&
-      static_cast<uint64_t>(rows) * slabs < (1ull << 31))
-    return build_plan_device(plan_out, offsets, indices, index_base, n_index, rows, edges, chunk, slabs, stream);
+      static_cast<uint64_t>(rows) * slabs < (1ull << 31)) {
+    bool fell_back = false;
+    const int rc = build_plan_device(plan_out, offsets, indices, index_base, n_index, rows, edges, chunk, slabs, stream,
+                                     &fell_back);
+    if (rc || !fell_back) return rc;
+  }
   std::vector<uint32_t> off;
   if (int rc = read_offsets(off, offsets, rows, edges, stream)) return rc;
   std::vector<uint32_t> idx(edges);

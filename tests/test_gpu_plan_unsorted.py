@@ -67,6 +67,32 @@ def test_offsets_are_checked_before_they_are_followed(device):
         assert not handle.value and "offsets" in abi.last_error()
 
 
+def test_edges_before_the_first_row_stay_out_of_it(device):
+    """offsets[0] > 0: those edges belong to no row and carry a source that no row has; row 0 is a hub."""
+    Vd, Vs, F = 700, 3000, 20
+    co, ri, deg = power_law_block(Vd + 3, Vs, 5, sort_rows=False, hubs=(9000, 600))
+    co, deg = co[3:].copy(), deg[3:]
+    lead = int(co[0])
+    assert lead and deg[0] == 9000
+    ri %= np.uint32(Vs - 1)
+    ri[:lead] = Vs - 1
+    want, _, _ = schedule(co, ri, Vs, 64, 8)
+    co_d, ri_d = _arrays(co, ri, device)
+    handle, s = ctypes.c_void_p(), torch.cuda.current_stream().cuda_stream
+    call("nts_spmm_plan_create_slabs", ctypes.byref(handle), ptr(co_d), ptr(ri_d), 0, Vs, Vd, int(co[-1]), 64, 8, s)
+    items = np.zeros((want.shape[0], 4), dtype=np.uint32)
+    call("nts_spmm_plan_copy_schedule", handle, items.ctypes.data, items.shape[0], None, 0)
+    assert np.array_equal(items, want)
+    x = torch.randint(-8, 9, (Vs, F), device=device).float()
+    x[Vs - 1] = 1e9
+    out = torch.empty(Vd, F, device=device)
+    call("nts_spmm_gather_planned", handle, ptr(x), ptr(out), 0, ptr(co_d), ptr(ri_d), 0, F, 0, s)
+    own = torch.repeat_interleave(torch.arange(Vd, device=device), torch.from_numpy(deg).to(device))
+    ref = torch.zeros(Vd, F, device=device).index_add_(0, own, x[torch.from_numpy(ri[lead:].astype(np.int64)).to(device)])
+    assert torch.equal(out, ref)
+    call("nts_spmm_plan_destroy", handle)
+
+
 def test_one_row_of_many_edges(device):
     n = 300000
     ri = torch.randperm(n, device=device).to(torch.int32)
