@@ -557,7 +557,8 @@ __global__ __launch_bounds__(256) void attention_grad_kernel(const float *__rest
     live[j] = head_live && c < Fh;
     col[j] = head * Fh + (c < Fh ? c : 0u);  // idle lanes re-read the head's first columns
     acc[j] = vzero<VEC>();
-    xr[j] = *reinterpret_cast<const V *>(x + static_cast<size_t>(row) * F + col[j]);
+    xr[j] = vzero<VEC>();
+    if (e0 < e1) xr[j] = *reinterpret_cast<const V *>(x + static_cast<size_t>(row) * F + col[j]);  // (no edge: x need not hold the row)
   }
   auto fetch_pair = [&](uint32_t e, uint32_t &pi, uint32_t &ps) {
     pi = ps = 0;
