@@ -24,3 +24,18 @@ def test_root_of_a_degree_in_32_bits():
     deg = np.concatenate([np.arange(1, 1 << 20), np.arange((1 << 24) - (1 << 16), 1 << 24),
                           np.random.default_rng(1).integers(1, 1 << 24, 1 << 20)]).astype(np.uint32)
     assert np.array_equal(np.sqrt(deg.astype(np.float32)), np.sqrt(deg.astype(np.float64)).astype(np.float32))
+
+
+@pytest.mark.parametrize("chunk", [1, 7, 64, 100000])
+def test_pieces_of_one_range_are_issued_by_length(chunk):
+    """Longest first, pieces of equal length in the order of their slots; the whole rows behind them likewise by row."""
+    deg = np.random.default_rng(chunk).integers(0, 300, 500)
+    co = np.zeros(deg.size + 1, dtype=np.uint32)
+    co[1:] = np.cumsum(deg)
+    items, n_splits, n_partials = schedule(co, None, 0, chunk, 0)
+    n = items[:, 2].astype(np.int64) - items[:, 1]
+    assert n_splits == int((deg > chunk).sum()) and n_partials == int((items[:, 3] != NO_SLOT).sum())
+    for part, key in ((slice(0, n_partials), 3), (slice(n_partials, None), 0)):
+        order = np.lexsort((items[part, key], -n[part]))
+        assert np.array_equal(order, np.arange(order.size))
+    assert int(n.sum()) == int(co[-1])
