@@ -5,8 +5,10 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <initializer_list>
 #include <utility>
 
+#include "idle_blocks.hpp"
 #include "nts_hip.h"
 
 namespace nts {
@@ -96,27 +98,23 @@ struct ScratchBlock {
 // time instead of 18, with hipMalloc and with a stream-ordered pool alike (the pool gives blocks back
 // whatever its threshold once it holds several sizes).  So blocks that fall idle are kept, at most
 // kIdleBytes and kIdleBlocks of them per device, for the next taker of about their size; nts_scratch_trim
-// gives them back.  A block is given back only when no work on any stream uses it any more.
-struct DeviceBlock {
-  void *ptr = nullptr;
-  size_t bytes = 0;
-  int device = 0;
+// gives them back.  A block reaches the next taker only after a wait for the work that uses it has succeeded; one
+// that goes out of scope before that is freed by the driver.
+struct DeviceBlock : BlockRef {
   DeviceBlock() = default;
   DeviceBlock(const DeviceBlock &) = delete;
   DeviceBlock &operator=(const DeviceBlock &) = delete;
-  hipError_t take(size_t want);  // an idle block of want .. want + want / 2 bytes, or a new one
-  hipError_t give();             // the caller has waited for all work that uses it
-  ~DeviceBlock() { (void)give(); }
+  hipError_t take(size_t want);   // an idle block of want .. want + want / 2 bytes, or a new one
+  hipError_t give(bool unused);   // unused: the caller has waited, with success, for all work that uses it
+  ~DeviceBlock() { (void)give(false); }
   template <typename T>
   T *as() const {
     return static_cast<T *>(ptr);
   }
-  void swap(DeviceBlock &other) {
-    std::swap(ptr, other.ptr);
-    std::swap(bytes, other.bytes);
-    std::swap(device, other.device);
-  }
+  void swap(DeviceBlock &other) { std::swap(static_cast<BlockRef &>(*this), static_cast<BlockRef &>(other)); }
 };
+// Waits for the blocks' own devices (the caller's current one may be another) and gives the blocks back.
+hipError_t retire_blocks(std::initializer_list<DeviceBlock *> blocks);
 constexpr size_t kIdleBytes = static_cast<size_t>(16) << 30;
 constexpr size_t kIdleBlocks = 32;
 

@@ -156,75 +156,46 @@ hipError_t scratch_alloc(void **ptr, size_t bytes, hipStream_t stream) {
 hipError_t scratch_free(void *ptr, hipStream_t stream) { return hipFreeAsync(ptr, stream); }
 
 namespace {
-struct IdleBlock {
-  void *ptr;
-  size_t bytes;
-  int device;
-};
-std::mutex g_idle_mutex;
-std::vector<IdleBlock> g_idle;
-
-// Frees the idle blocks of `device`, smallest first, until at most `keep_bytes` and `keep_blocks` are left.
-// Caller holds g_idle_mutex.
-hipError_t drop_idle(int device, size_t keep_bytes, size_t keep_blocks) {
-  hipError_t err = hipSuccess;
-  while (true) {
-    size_t total = 0, count = 0, at = g_idle.size();
-    for (size_t i = 0; i < g_idle.size(); ++i) {
-      if (g_idle[i].device != device) continue;
-      total += g_idle[i].bytes;
-      ++count;
-      if (at == g_idle.size() || g_idle[i].bytes < g_idle[at].bytes) at = i;
-    }
-    if (total <= keep_bytes && count <= keep_blocks) return err;
-    const hipError_t e = hipFree(g_idle[at].ptr);
-    if (e != hipSuccess) err = e;
-    g_idle.erase(g_idle.begin() + static_cast<std::ptrdiff_t>(at));
+struct HipMemory {
+  using Error = hipError_t;
+  static constexpr hipError_t kSuccess = hipSuccess;
+  static hipError_t current_device(int *device) { return hipGetDevice(device); }
+  // hipFree waits for all streams of the memory's device.  hipDeviceSynchronize would do, but it is refused, and
+  // ends the capture, while any stream is captured, in the relaxed mode too, where hipMalloc and hipFree are not.
+  static hipError_t wait_for_device(int device) {
+    int before = device;
+    hipError_t err = hipGetDevice(&before);
+    if (err == hipSuccess && before != device) err = hipSetDevice(device);
+    if (err != hipSuccess) return err;
+    void *mark = nullptr;
+    err = hipMalloc(&mark, 256);
+    if (err == hipSuccess) err = hipFree(mark);
+    if (before == device) return err;
+    const hipError_t back = hipSetDevice(before);
+    return err != hipSuccess ? err : back;
   }
+  static hipError_t allocate(void **ptr, size_t bytes) { return hipMalloc(ptr, bytes); }
+  static hipError_t release(void *ptr) { return hipFree(ptr); }
+  static bool out_of_memory(hipError_t err) { return err == hipErrorOutOfMemory; }
+  static void clear_error() { (void)hipGetLastError(); }
+};
+// Never destroyed: a schedule may outlive the library's own static objects at the end of the process.
+IdleBlocks<HipMemory> &idle_blocks() {
+  static IdleBlocks<HipMemory> &blocks = *new IdleBlocks<HipMemory>(kIdleBytes, kIdleBlocks);
+  return blocks;
 }
 }  // namespace
 
 hipError_t DeviceBlock::take(size_t want) {
-  if (ptr) {
-    const hipError_t e = give();
-    if (e != hipSuccess) return e;
-  }
-  if (want == 0) return hipSuccess;
-  hipError_t err = hipGetDevice(&device);
-  if (err != hipSuccess) return err;
-  std::lock_guard<std::mutex> lock(g_idle_mutex);
-  size_t best = g_idle.size();
-  for (size_t i = 0; i < g_idle.size(); ++i)
-    if (g_idle[i].device == device && g_idle[i].bytes >= want && g_idle[i].bytes - want <= want / 2 &&
-        (best == g_idle.size() || g_idle[i].bytes < g_idle[best].bytes))
-      best = i;
-  if (best < g_idle.size()) {
-    ptr = g_idle[best].ptr;
-    bytes = g_idle[best].bytes;
-    g_idle.erase(g_idle.begin() + static_cast<std::ptrdiff_t>(best));
-    return hipSuccess;
-  }
-  err = hipMalloc(&ptr, want);
-  if (err == hipErrorOutOfMemory) {  // what lies idle may be what is missing
-    (void)hipGetLastError();
-    (void)drop_idle(device, 0, 0);
-    err = hipMalloc(&ptr, want);
-  }
-  if (err != hipSuccess) {
-    ptr = nullptr;
-    return err;
-  }
-  bytes = want;
-  return hipSuccess;
+  const hipError_t err = give(false);
+  return err == hipSuccess ? idle_blocks().take(want, *this) : err;
 }
 
-hipError_t DeviceBlock::give() {
-  if (!ptr) return hipSuccess;
-  std::lock_guard<std::mutex> lock(g_idle_mutex);
-  g_idle.push_back(IdleBlock{ptr, bytes, device});
-  ptr = nullptr;
-  bytes = 0;
-  return drop_idle(device, kIdleBytes, kIdleBlocks);
+hipError_t DeviceBlock::give(bool unused) { return idle_blocks().give(*this, unused); }
+
+hipError_t retire_blocks(std::initializer_list<DeviceBlock *> blocks) {
+  std::vector<BlockRef *> refs(blocks.begin(), blocks.end());
+  return idle_blocks().retire(refs.data(), refs.size());
 }
 
 hipError_t scratch_trim() {
@@ -234,8 +205,7 @@ hipError_t scratch_trim() {
   if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   const hipError_t pool = g_scratch_pool[dev] ? hipMemPoolTrimTo(g_scratch_pool[dev], 0) : hipSuccess;
-  std::lock_guard<std::mutex> idle_lock(g_idle_mutex);
-  const hipError_t idle = drop_idle(dev, 0, 0);
+  const hipError_t idle = idle_blocks().trim(dev);
   return pool != hipSuccess ? pool : idle;
 }
 

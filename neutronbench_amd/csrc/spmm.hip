@@ -25,6 +25,7 @@
 #include <rocprim/iterator/transform_iterator.hpp>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <mutex>
 #include <new>
@@ -1940,12 +1941,17 @@ int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const
   const size_t tmp1_bytes = nts::up256(std::max(scan_bytes, sort_rows_bytes));
   const size_t cell_words = nts::up256((cells + 1) * sizeof(uint32_t));
   const size_t row_words = nts::up256((static_cast<size_t>(rows) + 1) * sizeof(uint32_t));
-  // Every block is given back after the last wait for the stream, the error paths included.
+  // Every block is given back after the last wait for the stream, the error paths included; where that
+  // wait fails the driver frees them.
   nts::DeviceBlock work, work2, sort_work, sorted_block, ids_block;
-  struct WaitFirst {
+  struct GiveBack {
     hipStream_t s;
-    ~WaitFirst() { (void)hipStreamSynchronize(s); }
-  } wait_first{stream};
+    std::array<nts::DeviceBlock *, 5> blocks;
+    ~GiveBack() {
+      const bool unused = hipStreamSynchronize(s) == hipSuccess;
+      for (nts::DeviceBlock *b : blocks) (void)b->give(unused);
+    }
+  } give_back{stream, {&work, &work2, &sort_work, &sorted_block, &ids_block}};
   NTS_HIP_TRY(work.take(3 * cell_words + 6 * row_words + 256 + tmp1_bytes));
   unsigned char *cursor = work.as<unsigned char>();
   auto take = [&cursor](size_t bytes) {
@@ -2197,19 +2203,13 @@ int nts_spmm_plan_destroy(nts_spmm_plan_t *plan) {
   NTS_TRACE_RANGE("nts_spmm_plan_destroy");
   if (!plan) return NTS_OK;
   { std::lock_guard<std::mutex> lock(plan->mu); }  // a call that is still enqueueing finishes first
-  // Work queued on any stream may still read the arrays.
-  const hipError_t waited = hipDeviceSynchronize();
+  // Work queued on any stream of the plan's device may still read the arrays.
+  const hipError_t given = nts::retire_blocks({&plan->items_block, &plan->splits_block, &plan->sorted_block,
+                                               &plan->ids_block, &plan->partial_block, &plan->padded_block});
   const hipError_t event = plan->done ? hipEventDestroy(plan->done) : hipSuccess;
-  hipError_t given = hipSuccess;
-  for (nts::DeviceBlock *b : {&plan->items_block, &plan->splits_block, &plan->sorted_block, &plan->ids_block,
-                              &plan->partial_block, &plan->padded_block}) {
-    const hipError_t e = b->give();
-    if (e != hipSuccess) given = e;
-  }
   delete plan;
-  if (waited != hipSuccess) return nts::fail_hip(waited, "nts_spmm_plan_destroy");
-  if (event != hipSuccess) return nts::fail_hip(event, "nts_spmm_plan_destroy");
   if (given != hipSuccess) return nts::fail_hip(given, "nts_spmm_plan_destroy");
+  if (event != hipSuccess) return nts::fail_hip(event, "nts_spmm_plan_destroy");
   return NTS_OK;
 }
 
@@ -2278,11 +2278,9 @@ int reserve_locked(nts_spmm_plan *plan, uint32_t F, bool heads) {
   // A buffer that grows may still be read by work queued earlier, on any stream.
   auto grow = [](nts::DeviceBlock &block, float **ptr, size_t *floats, size_t want) -> int {
     if (want <= *floats) return NTS_OK;
-    if (*ptr) {
-      NTS_HIP_TRY(hipDeviceSynchronize());
-      *ptr = nullptr;
-      *floats = 0;
-    }
+    *ptr = nullptr;
+    *floats = 0;
+    NTS_HIP_TRY(nts::retire_blocks({&block}));
     NTS_HIP_TRY(block.take(want * sizeof(float)));
     *ptr = block.as<float>();
     *floats = block.bytes / sizeof(float);
