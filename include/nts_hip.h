@@ -63,8 +63,11 @@ long nts_trace_ranges_emitted(void);
  * the largest scratch any call has needed (the reference allocates such buffers with cudaMalloc per
  * call, cuda/ntsCUDAGraphOP.cu:595-653).  The memory of schedules (their arrays, partial sums and what making
  * one needs) is kept likewise when a schedule is destroyed, up to 16 GiB per device, for the next schedule
- * of about that size.  nts_scratch_trim returns the current device's unused scratch and such idle blocks
- * to the driver; work queued earlier is not affected. */
+ * of about that size.  An allocation of the library that finds no other memory is tried again without such idle
+ * blocks, and nts_mem_info counts them as free; an allocator outside the library sees them as used.
+ * nts_scratch_trim returns the current device's unused scratch and idle blocks to the driver; work queued
+ * earlier is not affected.  A program that needs the memory for allocations of its own calls it once its
+ * graph is loaded. */
 int nts_scratch_trim(void);
 /* Scratch blocks the library has taken from its pool so far in this process (every call that needs
  * scratch takes one or two): lets a caller check that a code path allocates nothing. */
@@ -113,7 +116,8 @@ int nts_stream_destroy(nts_stream_t stream);
 int nts_stream_sync(nts_stream_t stream);
 /* cudaDeviceSynchronize as used by zero_buffer / move_* with sync=true. */
 int nts_device_sync(void);
-/* get_gpu_mem / show_gpu_mem (utils/cuda_memory.hpp:6-68): free and total device bytes. */
+/* get_gpu_mem / show_gpu_mem (utils/cuda_memory.hpp:6-68): free and total bytes of the current device; free
+ * includes the idle blocks of destroyed schedules (see nts_scratch_trim). */
 int nts_mem_info(size_t *free_bytes, size_t *total_bytes);
 
 /* 64-bit checksum of one or two uint32 device arrays (position-dependent: moving or changing any

@@ -178,6 +178,20 @@ def ptr(x):
     return x.data_ptr()
 
 
+def allocate(make, *args, **kwargs):
+    """The tensor that `make` (torch.empty, torch.zeros, torch.empty_like) gives.  Where the device has no memory
+    left for it, once more after the library has given back what it keeps for later schedules and calls."""
+    import torch
+
+    try:
+        return make(*args, **kwargs)
+    except torch.OutOfMemoryError:
+        device = kwargs["device"] if "device" in kwargs else args[0].device
+        with torch.cuda.device(device):
+            status("nts_scratch_trim")
+    return make(*args, **kwargs)
+
+
 def last_error():
     return lib().nts_last_error().decode()
 

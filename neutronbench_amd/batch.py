@@ -5,7 +5,7 @@ import ctypes
 
 import torch
 
-from .abi import SampledLayerDesc, call, ptr
+from .abi import SampledLayerDesc, allocate, call, ptr
 from .layout import SampledLayer, as_u32
 from .stream import CudaStream
 
@@ -98,12 +98,12 @@ def sample_hop(graph_co, graph_ri, dst, fanout, seed):
     device = dst.device
     n = dst.numel()
     stream = torch.cuda.current_stream(device).cuda_stream
-    work = torch.empty(call("nts_sample_hop_work_bytes", n) + 256, dtype=torch.uint8, device=device)
+    work = allocate(torch.empty, call("nts_sample_hop_work_bytes", n) + 256, dtype=torch.uint8, device=device)
     base = (work.data_ptr() + 255) // 256 * 256
-    co = torch.empty(n + 1, dtype=torch.int32, device=device)
+    co = allocate(torch.empty, n + 1, dtype=torch.int32, device=device)
     call("nts_sample_hop_offsets", ptr(co), ptr(graph_co), ptr(dst), n, fanout, base, stream)
     E = int(co[-1].item()) & 0xFFFFFFFF  # one read-back: sizes the edge array
-    ri = torch.empty(E, dtype=torch.int32, device=device)
+    ri = allocate(torch.empty, E, dtype=torch.int32, device=device)
     if E:
         call("nts_sample_hop_neighbors", ptr(ri), ptr(co), ptr(graph_co), ptr(graph_ri), ptr(dst), n, fanout, seed,
              stream)
@@ -156,7 +156,7 @@ class BatchBuilder:
         nbytes = call("nts_batch_builder_arena_bytes", V, E, fan, self.hops, max_batch, int(want_perm))
         if nbytes == 0:
             raise ValueError("nts_batch_builder_arena_bytes: unsupported configuration")
-        self.arena = torch.empty(nbytes + 256, dtype=torch.uint8, device=self.device)
+        self.arena = allocate(torch.empty, nbytes + 256, dtype=torch.uint8, device=self.device)
         self._skew = (-self.arena.data_ptr()) % 256
         handle = ctypes.c_void_p()
         call("nts_batch_builder_create", ctypes.byref(handle), ptr(graph_co), ptr(graph_ri), V, E, fan, self.hops,

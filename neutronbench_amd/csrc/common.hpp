@@ -68,6 +68,10 @@ struct TraceRange {
 hipError_t scratch_alloc(void **ptr, size_t bytes, hipStream_t stream);
 hipError_t scratch_free(void *ptr, hipStream_t stream);
 hipError_t scratch_trim();  // gives the current device's unused scratch and idle blocks back to the driver
+// The library's other allocations of device memory, and the free memory as they see it (idle blocks included).
+hipError_t malloc_device(void **ptr, size_t bytes);
+hipError_t malloc_device_async(void **ptr, size_t bytes, hipStream_t stream);
+hipError_t memory_info(size_t *free_bytes, size_t *total_bytes);
 long scratch_alloc_count();  // scratch blocks handed out so far by this process
 
 // A scratch block that is returned to the pool when its scope ends, whichever way the function is
@@ -98,7 +102,7 @@ struct ScratchBlock {
 // time instead of 18, with hipMalloc and with a stream-ordered pool alike (the pool gives blocks back
 // whatever its threshold once it holds several sizes).  So blocks that fall idle are kept, at most
 // kIdleBytes and kIdleBlocks of them per device, for the next taker of about their size; nts_scratch_trim
-// gives them back.  A block reaches the next taker only after a wait for the work that uses it has succeeded; one
+// gives them back, and so does every allocation of the library that finds no other memory.  A block reaches the next taker only after a wait for the work that uses it has succeeded; one
 // that goes out of scope before that is freed by the driver.
 struct DeviceBlock : BlockRef {
   DeviceBlock() = default;

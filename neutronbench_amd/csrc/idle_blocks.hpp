@@ -44,7 +44,7 @@ class IdleBlocks {
       return Api::kSuccess;
     }
     err = Api::allocate(&block.ptr, want);
-    if (Api::out_of_memory(err)) {  // what lies idle may be what is missing
+    if (Api::out_of_memory(err) && idle_bytes(block.device) != 0) {  // what lies idle may be what is missing
       Api::clear_error();
       (void)drop(block.device, 0, 0);
       err = Api::allocate(&block.ptr, want);
@@ -89,33 +89,55 @@ class IdleBlocks {
     return first;
   }
 
+  // An allocation of another kind on the current device: `allocate` is tried again without the idle blocks
+  // where it runs out of memory.
+  template <class Allocate>
+  Error with_idle_memory(Allocate allocate) {
+    Error err = allocate();
+    int device = 0;
+    if (!Api::out_of_memory(err) || Api::current_device(&device) != Api::kSuccess || held(device) == 0) return err;
+    Api::clear_error();
+    (void)trim(device);
+    return allocate();
+  }
+
+  // Bytes that lie idle on `device`.
+  size_t held(int device) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    return idle_bytes(device);
+  }
+
   Error trim(int device) {
     std::lock_guard<std::mutex> lock(mutex_);
     return drop(device, 0, 0);
   }
 
  private:
-  // Frees the idle blocks of `device`, smallest first, until at most `keep_bytes` and `keep_blocks` are left.
-  // A block that the driver refuses to free stays listed.  Caller holds mutex_.
+  size_t idle_bytes(int device) const {
+    size_t total = 0;
+    for (const BlockRef &b : idle_) total += b.device == device ? b.bytes : 0;
+    return total;
+  }
+
+  // Frees the idle blocks of `device`, the ones that have lain longest first, until at most `keep_bytes` and
+  // `keep_blocks` are left.  A block that the driver refuses to free stays listed.  Caller holds mutex_.
   Error drop(int device, size_t keep_bytes, size_t keep_blocks) {
     while (true) {
-      size_t total = 0, count = 0, at = idle_.size();
+      size_t count = 0, oldest = idle_.size();
       for (size_t i = 0; i < idle_.size(); ++i) {
         if (idle_[i].device != device) continue;
-        total += idle_[i].bytes;
-        ++count;
-        if (at == idle_.size() || idle_[i].bytes < idle_[at].bytes) at = i;
+        if (count++ == 0) oldest = i;
       }
-      if (total <= keep_bytes && count <= keep_blocks) return Api::kSuccess;
-      const Error err = Api::release(idle_[at].ptr);
+      if (count == 0 || (idle_bytes(device) <= keep_bytes && count <= keep_blocks)) return Api::kSuccess;
+      const Error err = Api::release(idle_[oldest].ptr);
       if (err != Api::kSuccess) return err;
-      idle_.erase(idle_.begin() + static_cast<std::ptrdiff_t>(at));
+      idle_.erase(idle_.begin() + static_cast<std::ptrdiff_t>(oldest));
     }
   }
 
   const size_t keep_bytes_, keep_blocks_;
   std::mutex mutex_;
-  std::vector<BlockRef> idle_;
+  std::vector<BlockRef> idle_;  // in the order in which they were given back
 };
 
 }  // namespace nts

@@ -106,6 +106,37 @@ const TraceApi *trace_api() {
 }
 
 namespace {
+struct HipMemory {
+  using Error = hipError_t;
+  static constexpr hipError_t kSuccess = hipSuccess;
+  static hipError_t current_device(int *device) { return hipGetDevice(device); }
+  // hipFree waits for all streams of the memory's device.  hipDeviceSynchronize would do, but it is refused, and
+  // ends the capture, while any stream is captured, in the relaxed mode too, where hipMalloc and hipFree are not.
+  static hipError_t wait_for_device(int device) {
+    int before = device;
+    hipError_t err = hipGetDevice(&before);
+    if (err == hipSuccess && before != device) err = hipSetDevice(device);
+    if (err != hipSuccess) return err;
+    void *mark = nullptr;
+    err = hipMalloc(&mark, 256);
+    if (err == hipSuccess) err = hipFree(mark);
+    if (before == device) return err;
+    const hipError_t back = hipSetDevice(before);
+    return err != hipSuccess ? err : back;
+  }
+  static hipError_t allocate(void **ptr, size_t bytes) { return hipMalloc(ptr, bytes); }
+  static hipError_t release(void *ptr) { return hipFree(ptr); }
+  static bool out_of_memory(hipError_t err) { return err == hipErrorOutOfMemory; }
+  static void clear_error() { (void)hipGetLastError(); }
+};
+// Never destroyed: a schedule may outlive the library's own static objects at the end of the process.
+IdleBlocks<HipMemory> &idle_blocks() {
+  static IdleBlocks<HipMemory> &blocks = *new IdleBlocks<HipMemory>(kIdleBytes, kIdleBlocks);
+  return blocks;
+}
+}  // namespace
+
+namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_pool_mutex;
 hipMemPool_t g_scratch_pool[kMaxDevices] = {};
@@ -148,43 +179,12 @@ hipError_t scratch_alloc(void **ptr, size_t bytes, hipStream_t stream) {
   hipMemPool_t pool = nullptr;
   if (scratch_pool(&pool) != hipSuccess) {
     (void)hipGetLastError();                   // a device without pool support: the device's default pool
-    return hipMallocAsync(ptr, bytes, stream);
+    return idle_blocks().with_idle_memory([&] { return hipMallocAsync(ptr, bytes, stream); });
   }
-  return hipMallocFromPoolAsync(ptr, bytes, pool, stream);
+  return idle_blocks().with_idle_memory([&] { return hipMallocFromPoolAsync(ptr, bytes, pool, stream); });
 }
 
 hipError_t scratch_free(void *ptr, hipStream_t stream) { return hipFreeAsync(ptr, stream); }
-
-namespace {
-struct HipMemory {
-  using Error = hipError_t;
-  static constexpr hipError_t kSuccess = hipSuccess;
-  static hipError_t current_device(int *device) { return hipGetDevice(device); }
-  // hipFree waits for all streams of the memory's device.  hipDeviceSynchronize would do, but it is refused, and
-  // ends the capture, while any stream is captured, in the relaxed mode too, where hipMalloc and hipFree are not.
-  static hipError_t wait_for_device(int device) {
-    int before = device;
-    hipError_t err = hipGetDevice(&before);
-    if (err == hipSuccess && before != device) err = hipSetDevice(device);
-    if (err != hipSuccess) return err;
-    void *mark = nullptr;
-    err = hipMalloc(&mark, 256);
-    if (err == hipSuccess) err = hipFree(mark);
-    if (before == device) return err;
-    const hipError_t back = hipSetDevice(before);
-    return err != hipSuccess ? err : back;
-  }
-  static hipError_t allocate(void **ptr, size_t bytes) { return hipMalloc(ptr, bytes); }
-  static hipError_t release(void *ptr) { return hipFree(ptr); }
-  static bool out_of_memory(hipError_t err) { return err == hipErrorOutOfMemory; }
-  static void clear_error() { (void)hipGetLastError(); }
-};
-// Never destroyed: a schedule may outlive the library's own static objects at the end of the process.
-IdleBlocks<HipMemory> &idle_blocks() {
-  static IdleBlocks<HipMemory> &blocks = *new IdleBlocks<HipMemory>(kIdleBytes, kIdleBlocks);
-  return blocks;
-}
-}  // namespace
 
 hipError_t DeviceBlock::take(size_t want) {
   const hipError_t err = give(false);
@@ -196,6 +196,22 @@ hipError_t DeviceBlock::give(bool unused) { return idle_blocks().give(*this, unu
 hipError_t retire_blocks(std::initializer_list<DeviceBlock *> blocks) {
   std::vector<BlockRef *> refs(blocks.begin(), blocks.end());
   return idle_blocks().retire(refs.data(), refs.size());
+}
+
+hipError_t malloc_device(void **ptr, size_t bytes) {
+  return idle_blocks().with_idle_memory([&] { return hipMalloc(ptr, bytes); });
+}
+
+hipError_t malloc_device_async(void **ptr, size_t bytes, hipStream_t stream) {
+  return idle_blocks().with_idle_memory([&] { return hipMallocAsync(ptr, bytes, stream); });
+}
+
+hipError_t memory_info(size_t *free_bytes, size_t *total_bytes) {
+  int device = 0;
+  hipError_t err = hipGetDevice(&device);
+  if (err == hipSuccess) err = hipMemGetInfo(free_bytes, total_bytes);
+  if (err == hipSuccess) *free_bytes += idle_blocks().held(device);
+  return err;
 }
 
 hipError_t scratch_trim() {
@@ -233,7 +249,7 @@ int nts_malloc_device(void **ptr, size_t bytes) {
   if (!ptr) return fail(NTS_ERR_INVALID, "nts_malloc_device: null out-pointer");
   *ptr = nullptr;
   if (bytes == 0) return NTS_OK;
-  NTS_HIP_TRY(hipMalloc(ptr, bytes));
+  NTS_HIP_TRY(nts::malloc_device(ptr, bytes));
   return NTS_OK;
 }
 
@@ -247,7 +263,7 @@ int nts_malloc_device_async(void **ptr, size_t bytes, nts_stream_t stream) {
   if (!ptr) return fail(NTS_ERR_INVALID, "nts_malloc_device_async: null out-pointer");
   *ptr = nullptr;
   if (bytes == 0) return NTS_OK;
-  NTS_HIP_TRY(hipMallocAsync(ptr, bytes, stream));
+  NTS_HIP_TRY(nts::malloc_device_async(ptr, bytes, stream));
   return NTS_OK;
 }
 
@@ -446,7 +462,7 @@ int nts_event_elapsed_ms(float *ms, nts_event_t start, nts_event_t stop) {
 
 int nts_mem_info(size_t *free_bytes, size_t *total_bytes) {
   if (!free_bytes || !total_bytes) return fail(NTS_ERR_INVALID, "nts_mem_info: null pointer");
-  NTS_HIP_TRY(hipMemGetInfo(free_bytes, total_bytes));
+  NTS_HIP_TRY(nts::memory_info(free_bytes, total_bytes));
   return NTS_OK;
 }
 

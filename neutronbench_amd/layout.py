@@ -12,7 +12,7 @@ import time
 
 import torch
 
-from .abi import call, ptr
+from .abi import allocate, call, ptr
 
 
 def _stream(device):
@@ -112,13 +112,14 @@ class FullGraphChunk:
         """`pairs`: int32 device tensor [E, 2] holding the .edge file's records (src, dst)."""
         device = pairs.device
         E = pairs.shape[0]
-        co32 = torch.empty(V + 1, dtype=torch.int32, device=device)
-        ro32 = torch.empty(V + 1, dtype=torch.int32, device=device)
-        ri32 = torch.empty(E, dtype=torch.int32, device=device)
-        ci32 = torch.empty(E, dtype=torch.int32, device=device)
-        ewf = torch.empty(E, dtype=torch.float32, device=device)
-        ewb = torch.empty(E, dtype=torch.float32, device=device)
-        work = torch.empty(call("nts_chunk_from_edges_work_bytes", V, E) + 256, dtype=torch.uint8, device=device)
+        co32 = allocate(torch.empty, V + 1, dtype=torch.int32, device=device)
+        ro32 = allocate(torch.empty, V + 1, dtype=torch.int32, device=device)
+        ri32 = allocate(torch.empty, E, dtype=torch.int32, device=device)
+        ci32 = allocate(torch.empty, E, dtype=torch.int32, device=device)
+        ewf = allocate(torch.empty, E, dtype=torch.float32, device=device)
+        ewb = allocate(torch.empty, E, dtype=torch.float32, device=device)
+        work_bytes = call("nts_chunk_from_edges_work_bytes", V, E)
+        work = allocate(torch.empty, work_bytes + 256, dtype=torch.uint8, device=device)
         wptr = (work.data_ptr() + 255) // 256 * 256
         call("nts_chunk_from_edges", ptr(co32), ptr(ri32), ptr(ewf), ptr(ro32), ptr(ci32), ptr(ewb), ptr(pairs), E, V,
              wptr, _stream(device))
@@ -135,7 +136,10 @@ class FullGraphChunk:
         E = edge_file_count(path)
         host = torch.empty((E, 2), dtype=torch.int32, pin_memory=True)
         read_edge_file(path, vertices=V, out=host.numpy().view("uint32"))
-        return cls.from_edge_pairs(host.to(device, non_blocking=True), V, chunk_edges, n_slabs)
+        chunk = cls.from_edge_pairs(host.to(device, non_blocking=True), V, chunk_edges, n_slabs)
+        with torch.cuda.device(device):
+            call("nts_scratch_trim")  # the graph is loaded: the memory that making its schedules took is the program's again
+        return chunk
 
 
 class SampledLayer:
@@ -179,11 +183,11 @@ class SampledLayer:
         Vd, E = destination.numel(), row_indices_global.numel()
         stream = _stream(device)
         work_bytes = call("nts_relabel_sources_work_bytes", V)
-        work = torch.empty(work_bytes + 256, dtype=torch.uint8, device=device)
+        work = allocate(torch.empty, work_bytes + 256, dtype=torch.uint8, device=device)
         base = (work.data_ptr() + 255) // 256 * 256
-        source = torch.empty(max(min(E, V), 1), dtype=torch.int32, device=device)
-        n_source = torch.zeros(1, dtype=torch.int32, device=device)
-        local = torch.empty(E, dtype=torch.int32, device=device)
+        source = allocate(torch.empty, max(min(E, V), 1), dtype=torch.int32, device=device)
+        n_source = allocate(torch.zeros, 1, dtype=torch.int32, device=device)
+        local = allocate(torch.empty, E, dtype=torch.int32, device=device)
         call("nts_relabel_sources", ptr(source), ptr(n_source), ptr(local), ptr(row_indices_global), E, V, base, stream)
         Vs = int(n_source.item())  # the one read-back of the construction: sizes the CSR arrays
         self.v_size, self.e_size, self.src_size = Vd, E, Vs
@@ -195,14 +199,14 @@ class SampledLayer:
     def _finish_on_device(self, want_perm):
         device = self.dev_column_offset.device
         Vd, E, Vs = self.v_size, self.e_size, self.src_size
-        self.dev_row_offset = torch.empty(Vs + 1, dtype=torch.int32, device=device)
-        self.dev_column_indices = torch.empty(E, dtype=torch.int32, device=device)
-        self.dev_csr_to_csc = torch.empty(E, dtype=torch.int32, device=device) if want_perm else None
-        self.dev_edge_weight_forward = torch.empty(E, dtype=torch.float32, device=device)
-        self.dev_edge_weight_backward = torch.empty(E, dtype=torch.float32, device=device)
+        self.dev_row_offset = allocate(torch.empty, Vs + 1, dtype=torch.int32, device=device)
+        self.dev_column_indices = allocate(torch.empty, E, dtype=torch.int32, device=device)
+        self.dev_csr_to_csc = allocate(torch.empty, E, dtype=torch.int32, device=device) if want_perm else None
+        self.dev_edge_weight_forward = allocate(torch.empty, E, dtype=torch.float32, device=device)
+        self.dev_edge_weight_backward = allocate(torch.empty, E, dtype=torch.float32, device=device)
         stream = _stream(device)
         work_bytes = call("nts_csr_from_csc_work_bytes", Vd, Vs, E)
-        work = torch.empty(max(work_bytes, 256) + 256, dtype=torch.uint8, device=device)
+        work = allocate(torch.empty, max(work_bytes, 256) + 256, dtype=torch.uint8, device=device)
         base = (work.data_ptr() + 255) // 256 * 256
         call("nts_csr_from_csc", ptr(self.dev_row_offset), ptr(self.dev_column_indices), ptr(self.dev_csr_to_csc),
              ptr(self.dev_column_offset), ptr(self.dev_row_indices), Vd, Vs, E, base, stream)

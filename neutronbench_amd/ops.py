@@ -9,7 +9,7 @@ that allocate their output like the reference does and call the HIP library thro
 """
 import torch
 
-from .abi import call, ptr
+from .abi import allocate, call, ptr
 from .stream import CudaStream
 
 
@@ -28,7 +28,7 @@ class ForwardSingleGPUfuseOp:
 
     def _run(self, plan, x, offsets, indices, weight, base):
         _check2d(x)
-        out = torch.empty_like(x)
+        out = allocate(torch.empty_like, x)
         call("nts_spmm_gather_planned", plan.handle, ptr(x), ptr(out), ptr(weight) if self.with_weight else 0,
              ptr(offsets), ptr(indices), base, x.shape[1], 0, torch.cuda.current_stream(x.device).cuda_stream)
         return out
@@ -57,7 +57,7 @@ class SingleGPUSampleGraphOp:
         _check2d(f_input)
         sg = self.sg
         F = f_input.shape[1]
-        out = torch.zeros(sg.v_size, F, dtype=torch.float32, device=f_input.device)
+        out = allocate(torch.zeros, sg.v_size, F, dtype=torch.float32, device=f_input.device)
         if 0 < sg.max_in_degree <= 256:
             # the sampler bounded every destination's edges by its fanout: one launch, nothing to cut
             call("nts_spmm_gather_bounded", ptr(f_input), ptr(out), ptr(sg.dev_ewf()), ptr(sg.dev_c_o()),
@@ -73,7 +73,7 @@ class SingleGPUSampleGraphOp:
         _check2d(f_output_grad)
         sg = self.sg
         F = f_output_grad.shape[1]
-        gin = torch.zeros(sg.src_size, F, dtype=torch.float32, device=f_output_grad.device)
+        gin = allocate(torch.zeros, sg.src_size, F, dtype=torch.float32, device=f_output_grad.device)
         self.cs.Gather_By_Src_From_Dst(f_output_grad, gin, sg.dev_ewb(), sg.dev_r_o(), sg.dev_c_i(), 0, 0, 0, 0,
                                        sg.e_size, sg.src_size, F, True, False)
         if self.sync:
@@ -91,14 +91,14 @@ class SingleGPUEdgeSoftMax:
 
     def forward(self, f_input):
         _check2d(f_input)
-        out = torch.empty_like(f_input)
+        out = allocate(torch.empty_like, f_input)
         self.cs.Edge_Softmax_Forward_Block(out, f_input, None, None, self.co, self.Vd, f_input.shape[1])
         self.cached = out
         return out
 
     def backward(self, f_output_grad):
         _check2d(f_output_grad)
-        gin = torch.empty_like(f_output_grad)
+        gin = allocate(torch.empty_like, f_output_grad)
         self.cs.Edge_Softmax_Backward_Block(gin, f_output_grad, self.cached, None, self.co, self.Vd,
                                             f_output_grad.shape[1])
         return gin
@@ -114,14 +114,14 @@ class SingleGPUScatterSrc:
     def forward(self, x):
         _check2d(x)
         sg = self.sg
-        msg = torch.empty(sg.e_size, x.shape[1], dtype=torch.float32, device=x.device)
+        msg = allocate(torch.empty, sg.e_size, x.shape[1], dtype=torch.float32, device=x.device)
         self.cs.Scatter_Src_Mirror_to_Msg(msg, x, sg.dev_r_i(), sg.dev_c_o(), None, sg.v_size, x.shape[1])
         return msg
 
     def backward(self, g_msg):
         _check2d(g_msg)
         sg = self.sg
-        out = torch.zeros(sg.src_size, g_msg.shape[1], dtype=torch.float32, device=g_msg.device)
+        out = allocate(torch.zeros, sg.src_size, g_msg.shape[1], dtype=torch.float32, device=g_msg.device)
         self.cs.Gather_Msg_To_Src_Mirror(out, g_msg, sg.dev_r_o(), sg.dev_csr_to_csc, sg.src_size, g_msg.shape[1])
         return out
 
@@ -136,14 +136,14 @@ class SingleGPUScatterDst:
     def forward(self, x):
         _check2d(x)
         sg = self.sg
-        msg = torch.empty(sg.e_size, x.shape[1], dtype=torch.float32, device=x.device)
+        msg = allocate(torch.empty, sg.e_size, x.shape[1], dtype=torch.float32, device=x.device)
         self.cs.Scatter_Dst_to_Msg(msg, x, sg.dev_r_i(), sg.dev_c_o(), sg.v_size, x.shape[1])
         return msg
 
     def backward(self, g_msg):
         _check2d(g_msg)
         sg = self.sg
-        out = torch.zeros(sg.v_size, g_msg.shape[1], dtype=torch.float32, device=g_msg.device)
+        out = allocate(torch.zeros, sg.v_size, g_msg.shape[1], dtype=torch.float32, device=g_msg.device)
         self.cs.Gather_Msg_to_Dst(out, g_msg, sg.dev_r_i(), sg.dev_c_o(), sg.v_size, g_msg.shape[1])
         return out
 
@@ -158,14 +158,14 @@ class SingleGPUAggregateDst:
     def forward(self, msg):
         _check2d(msg)
         sg = self.sg
-        out = torch.zeros(sg.v_size, msg.shape[1], dtype=torch.float32, device=msg.device)
+        out = allocate(torch.zeros, sg.v_size, msg.shape[1], dtype=torch.float32, device=msg.device)
         self.cs.Gather_Msg_to_Dst(out, msg, sg.dev_r_i(), sg.dev_c_o(), sg.v_size, msg.shape[1])
         return out
 
     def backward(self, g_out):
         _check2d(g_out)
         sg = self.sg
-        g_msg = torch.empty(sg.e_size, g_out.shape[1], dtype=torch.float32, device=g_out.device)
+        g_msg = allocate(torch.empty, sg.e_size, g_out.shape[1], dtype=torch.float32, device=g_out.device)
         self.cs.Scatter_Dst_to_Msg(g_msg, g_out, sg.dev_r_i(), sg.dev_c_o(), sg.v_size, g_out.shape[1])
         return g_msg
 
@@ -183,7 +183,7 @@ class GATAttentionOp:
         _check2d(er)
         sg = self.sg
         H = el.shape[1]
-        alpha = torch.empty(sg.e_size, H, dtype=torch.float32, device=el.device)
+        alpha = allocate(torch.empty, sg.e_size, H, dtype=torch.float32, device=el.device)
         stream = torch.cuda.current_stream(el.device).cuda_stream
         call("nts_gat_attention_fwd_bounded", ptr(alpha), ptr(el), ptr(er), ptr(sg.dev_c_o()), ptr(sg.dev_r_i()),
              sg.v_size, H, self.slope, getattr(sg, "max_in_degree", 0), stream)
@@ -196,12 +196,12 @@ class GATAttentionOp:
         H = g_alpha.shape[1]
         dev = g_alpha.device
         stream = torch.cuda.current_stream(dev).cuda_stream
-        gs = torch.empty_like(g_alpha)
-        self.ger = torch.empty(sg.v_size, H, dtype=torch.float32, device=dev)
+        gs = allocate(torch.empty_like, g_alpha)
+        self.ger = allocate(torch.empty, sg.v_size, H, dtype=torch.float32, device=dev)
         call("nts_gat_attention_bwd_bounded", ptr(gs), ptr(self.ger), ptr(g_alpha), ptr(self.alpha), ptr(self.el),
              ptr(self.er), ptr(sg.dev_c_o()), ptr(sg.dev_r_i()), sg.v_size, H, self.slope,
              getattr(sg, "max_in_degree", 0), stream)
-        gel = torch.empty(sg.src_size, H, dtype=torch.float32, device=dev)
+        gel = allocate(torch.empty, sg.src_size, H, dtype=torch.float32, device=dev)
         call("nts_gather_edge_to_src", ptr(gel), ptr(gs), ptr(sg.dev_r_o()), ptr(sg.dev_csr_to_csc), sg.src_size, H, 0,
              stream)
         return gel
@@ -223,7 +223,7 @@ class GATAggregateOp:
         _check2d(alpha)
         sg = self.sg
         Fh = x.shape[1] // self.H
-        out = torch.empty(sg.v_size, x.shape[1], dtype=torch.float32, device=x.device)
+        out = allocate(torch.empty, sg.v_size, x.shape[1], dtype=torch.float32, device=x.device)
         stream = torch.cuda.current_stream(x.device).cuda_stream
         call("nts_spmm_gather_heads_bounded", ptr(x), ptr(out), ptr(alpha), 0, ptr(sg.dev_c_o()), ptr(sg.dev_r_i()),
              sg.v_size, sg.e_size, self.H, Fh, 0, getattr(sg, "max_in_degree", 0), stream)
@@ -236,8 +236,8 @@ class GATAggregateOp:
         Fh = g_out.shape[1] // self.H
         dev = g_out.device
         stream = torch.cuda.current_stream(dev).cuda_stream
-        gx = torch.empty(sg.src_size, g_out.shape[1], dtype=torch.float32, device=dev)
-        self.galpha = torch.empty(sg.e_size, self.H, dtype=torch.float32, device=dev)
+        gx = allocate(torch.empty, sg.src_size, g_out.shape[1], dtype=torch.float32, device=dev)
+        self.galpha = allocate(torch.empty, sg.e_size, self.H, dtype=torch.float32, device=dev)
         call("nts_gat_aggregate_bwd", ptr(gx), ptr(self.galpha), ptr(self.x), ptr(g_out), ptr(self.alpha),
              ptr(sg.dev_csr_to_csc), ptr(sg.dev_r_o()), ptr(sg.dev_c_i()), ptr(sg.dev_c_o()), ptr(sg.dev_r_i()),
              sg.v_size, sg.src_size, sg.e_size, self.H, Fh, 0, stream)

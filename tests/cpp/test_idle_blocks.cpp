@@ -105,10 +105,13 @@ int sizes_and_bounds() {
   CHECK(pool.give(a, true) == 0 && take_log() == "");
   CHECK(pool.take(199, b) == 0 && take_log() == "a199 ");   // 300 is more than half above 199
   CHECK(pool.take(200, b) == 0 && take_log() == "" && b.bytes == 300);
-  CHECK(pool.give(b, true) == 0 && pool.give(c, true) == 0);  // 1,200 bytes: one goes
-  CHECK(take_log() == "f ");
+  CHECK(pool.give(b, true) == 0 && pool.give(c, true) == 0);  // 1,200 bytes: the one that has lain longer goes
+  CHECK(take_log() == "f " && pool.held(0) == 900 && pool.held(1) == 0);
+  CHECK(pool.take(100, a) == 0 && pool.take(100, b) == 0 && take_log() == "a100 a100 ");
+  CHECK(pool.give(a, true) == 0 && take_log() == "" && pool.held(0) == 1000);
+  CHECK(pool.give(b, true) == 0 && take_log() == "f " && pool.held(0) == 200);  // three blocks: the oldest, not the smallest
   CHECK(pool.trim(1) == 0 && take_log() == "");
-  CHECK(pool.trim(0) == 0 && take_log() == "f ");
+  CHECK(pool.trim(0) == 0 && take_log() == "f f " && pool.held(0) == 0);
   return 0;
 }
 
@@ -120,15 +123,40 @@ int an_allocation_that_fails_gets_the_idle_memory() {
   take_log();
   g_allocations_that_fail = 1;
   CHECK(pool.take(5000, b) == 0 && take_log() == "a5000 c f a5000 ");
+  CHECK(pool.give(b, true) == 0);
   g_allocations_that_fail = 2;
   CHECK(pool.take(6000, a) == 2 && !a.ptr);
+  take_log();
+  g_allocations_that_fail = 1;
+  CHECK(pool.take(6000, a) == 2 && take_log() == "a6000 ");  // nothing idle: not tried again
+  return 0;
+}
+
+// Scratch and the allocations of the C interface, which do not come from the list.
+int other_allocations_get_the_idle_memory() {
+  Pool pool(1 << 20, 8);
+  BlockRef a;
+  void *p = nullptr;
+  auto other = [&] { return Api::allocate(&p, 77); };
+  g_device = 0;
+  CHECK(pool.take(100, a) == 0 && pool.give(a, true) == 0);
+  take_log();
+  CHECK(pool.with_idle_memory(other) == 0 && take_log() == "a77 " && pool.held(0) == 100);
+  g_device = 1;  // the other device's idle memory would not help
+  g_allocations_that_fail = 1;
+  CHECK(pool.with_idle_memory(other) == 2 && take_log() == "a77 " && pool.held(0) == 100);
+  g_device = 0;
+  g_allocations_that_fail = 1;
+  CHECK(pool.with_idle_memory(other) == 0 && take_log() == "a77 c f a77 " && pool.held(0) == 0);
+  g_allocations_that_fail = 1;
+  CHECK(pool.with_idle_memory(other) == 2 && take_log() == "a77 ");
   return 0;
 }
 }  // namespace
 
 int main() {
   if (waits_for_the_blocks_own_device() || a_block_whose_wait_failed_is_not_handed_on() || sizes_and_bounds() ||
-      an_allocation_that_fails_gets_the_idle_memory())
+      an_allocation_that_fails_gets_the_idle_memory() || other_allocations_get_the_idle_memory())
     return 1;
   printf("ok\n");
   return 0;

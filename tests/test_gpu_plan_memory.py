@@ -1,5 +1,7 @@
 """Memory that a destroyed schedule leaves to the next one: not before the work that uses it has ended, and not
 at the cost of a capture that runs meanwhile."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -74,3 +76,30 @@ def test_destroyed_while_a_stream_is_captured(device):
         graph.replay()
         torch.cuda.synchronize()
         assert bool((y == 2.0 * k).all())
+
+
+def test_idle_memory_is_free_to_the_library_and_given_back(device):
+    """A schedule with 1 GiB of partial sums: destroyed, it leaves nts_mem_info what it was, the next one of its size
+    takes the same memory, and nts_scratch_trim returns it to the driver."""
+    co = torch.arange(0, (1 << 21) + 1, 64, dtype=torch.int32, device=device)
+    rows, edges = co.numel() - 1, int(co[-1])
+    torch.cuda.synchronize()
+    call("nts_scratch_trim")
+
+    def library_free():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        call("nts_mem_info", ctypes.byref(free), ctypes.byref(total))
+        return free.value
+
+    before, slack = library_free(), 64 << 20
+    for k in range(3):
+        plan = SpmmPlan(co, rows, edges, 32)
+        plan.reserve(1 << 12)
+        used = before - library_free()
+        assert used > (1 << 30) - slack
+        driver = torch.cuda.mem_get_info()[0]
+        plan.close()
+        assert abs(library_free() - before) < slack
+        assert abs(torch.cuda.mem_get_info()[0] - driver) < slack  # kept: the next schedule takes it
+    call("nts_scratch_trim")
+    assert torch.cuda.mem_get_info()[0] - driver > (1 << 30) - slack
