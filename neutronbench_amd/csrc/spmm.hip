@@ -1914,8 +1914,10 @@ int build_plan(nts_spmm_plan_t **plan_out, const uint32_t *offsets_dev, const st
 }
 
 // Builds the schedule of make_schedule on the device (kernels above).  *fell_back is set, and nothing built,
-// where the first row does not start at edge 0: the edges before it belong to no row, while the kernels
-// give every edge to the row before it (row 0 would be ordered together with them).
+//  - where the first row does not start at edge 0: the edges before it belong to no row, while the kernels
+//    give every edge to the row before it (row 0 would be ordered together with them);
+//  - where rows have to be ordered and the sort's memory, some 36 bytes an edge with the ordered copies, is not to
+//    be had: the host orders them with the copies alone on the device, 8 bytes an edge.
 int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const uint32_t *indices,
                       uint32_t index_base, uint32_t n_index, uint32_t rows, uint32_t edges, uint32_t chunk,
                       uint32_t n_slabs, hipStream_t stream, bool *fell_back) {
@@ -2009,10 +2011,16 @@ int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const
     NTS_HIP_TRY(rocprim::radix_sort_pairs(nullptr, sort_edges_bytes, nul64, nul64, ids_in, nul, edges, 0u,
                                           index_bits + row_bits, stream, false));
     const size_t key_bytes = nts::up256(static_cast<size_t>(edges) * sizeof(unsigned long long));
-    NTS_HIP_TRY(sorted_block.take(static_cast<size_t>(edges) * sizeof(uint32_t)));
-    NTS_HIP_TRY(ids_block.take(static_cast<size_t>(edges) * sizeof(uint32_t)));
+    hipError_t taken = sorted_block.take(static_cast<size_t>(edges) * sizeof(uint32_t));
+    if (taken == hipSuccess) taken = ids_block.take(static_cast<size_t>(edges) * sizeof(uint32_t));
+    if (taken == hipSuccess) taken = sort_work.take(2 * key_bytes + nts::up256(sort_edges_bytes));
+    if (taken == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      *fell_back = true;
+      return NTS_OK;
+    }
+    NTS_HIP_TRY(taken);
     uint32_t *sorted_idx = sorted_block.as<uint32_t>(), *edge_ids = ids_block.as<uint32_t>();
-    NTS_HIP_TRY(sort_work.take(2 * key_bytes + nts::up256(sort_edges_bytes)));
     unsigned char *sort_bytes = sort_work.as<unsigned char>();
     unsigned long long *keys = reinterpret_cast<unsigned long long *>(sort_bytes);
     unsigned long long *keys_out = reinterpret_cast<unsigned long long *>(sort_bytes + key_bytes);

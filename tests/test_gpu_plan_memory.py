@@ -103,3 +103,34 @@ def test_idle_memory_is_free_to_the_library_and_given_back(device):
         assert abs(torch.cuda.mem_get_info()[0] - driver) < slack  # kept: the next schedule takes it
     call("nts_scratch_trim")
     assert torch.cuda.mem_get_info()[0] - driver > (1 << 30) - slack
+
+
+def test_ordering_falls_back_to_the_host_without_memory_for_the_sort(device):
+    """30 M edges in rows that do not ascend, with 640 MiB left on the device: the sort alone takes over 900 MB, the
+    ordered copies 240.  The same schedule, and the same sums, as with all of the memory."""
+    rows, n_src, edges, F = 3000, 100000, 30000000, 4
+    g = torch.Generator(device=device).manual_seed(6)
+    ri = torch.randint(0, n_src, (edges,), generator=g, device=device, dtype=torch.int32)
+    co = torch.arange(0, edges + 1, edges // rows, dtype=torch.int32, device=device)
+    x = torch.randint(-8, 9, (n_src, F), generator=g, device=device).float()
+
+    def schedule_and_sums():
+        plan = SpmmPlan(co, rows, edges, 512, ri, n_src, 8)
+        items = np.zeros((plan.info()["items"], 4), dtype=np.uint32)
+        call("nts_spmm_plan_copy_schedule", plan.handle, items.ctypes.data, items.shape[0], None, 0)
+        out = torch.empty(rows, F, device=device)
+        _gather(plan, x, out, co, ri, torch.cuda.current_stream().cuda_stream)
+        plan.close()
+        call("nts_scratch_trim")
+        return items, out
+
+    want, sums = schedule_and_sums()
+    torch.cuda.empty_cache()
+    torch.cuda.synchronize()
+    fill = torch.empty(torch.cuda.mem_get_info()[0] - (640 << 20), dtype=torch.uint8, device=device)
+    try:
+        items, out = schedule_and_sums()
+    finally:
+        del fill
+        torch.cuda.empty_cache()
+    assert np.array_equal(items, want) and torch.equal(out, sums)
