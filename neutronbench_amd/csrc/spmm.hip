@@ -1704,15 +1704,87 @@ struct Schedule {
   uint64_t repeated_edges = 0;
 };
 
+// The schedule without source ranges.  What it is made of follows from the lengths alone, so everything is placed
+// by counting: one pass over the rows counts, the next writes each entry where it belongs (pieces by descending
+// length, equal ones by slot; whole rows by descending length, equal ones by row; split rows by descending piece
+// count).  No piece is written twice: with the short pieces of default_chunk there are often as many of them as rows,
+// and making a list of them that was ordered afterwards took 275 us of a schedule (60 K vertices, 600 K edges) where
+// the few 4,096-edge pieces of before had taken 212; placed at once it is 208 (30 K, 300 K: 152 -> 107; 5 K, 500 K,
+// 19,000 items instead of 5,000: 102 -> 58).
+void make_one_range_schedule(Schedule &out, const uint32_t *off, uint32_t rows, uint32_t chunk) {
+  if (rows == 0) return;
+  chunk = std::min(chunk, std::max(off[rows] - off[0], 1u));  // a longer piece cuts nothing
+  std::vector<uint32_t> whole_at(static_cast<size_t>(chunk) + 2, 0u), rest_at(static_cast<size_t>(chunk) + 1, 0u);
+  std::vector<uint32_t> long_rows;
+  uint32_t n_full = 0, n_partials = 0, most = 0;
+  for (uint32_t r = 0; r < rows; ++r) {
+    const uint32_t deg = off[r + 1] - off[r];
+    if (deg <= chunk) {
+      ++whole_at[chunk - deg + 1];
+      continue;
+    }
+    const uint32_t full = deg / chunk, rest = deg - full * chunk, n = full + (rest ? 1u : 0u);
+    long_rows.push_back(r);
+    n_full += full;
+    n_partials += n;
+    most = std::max(most, n);
+    if (rest) ++rest_at[chunk - rest];
+  }
+  // rest_at[chunk - n] = position of the first piece of n < chunk edges; the full ones come before them
+  uint32_t next = n_full;
+  for (uint32_t &at : rest_at) {
+    const uint32_t n = at;
+    at = next;
+    next += n;
+  }
+  whole_at[0] = n_partials;
+  for (size_t i = 1; i < whole_at.size(); ++i) whole_at[i] += whole_at[i - 1];
+  std::vector<uint32_t> split_at(static_cast<size_t>(most) + 2, 0u);
+  for (uint32_t r : long_rows) ++split_at[most - (off[r + 1] - off[r] - 1) / chunk];
+  for (size_t i = 1; i < split_at.size(); ++i) split_at[i] += split_at[i - 1];
+
+  std::vector<uint4> &items = out.items;
+  items.reserve(static_cast<size_t>(n_partials) + rows);  // (the split rows follow for the upload)
+  items.resize(static_cast<size_t>(n_partials) + rows - long_rows.size());
+  out.splits.resize(long_rows.size());
+  uint32_t slot = 0, full_at = 0;
+  for (uint32_t r : long_rows) {
+    const uint32_t first = slot, end = off[r + 1];
+    uint32_t k = off[r];
+    for (; end - k >= chunk; k += chunk) items[full_at++] = make_uint4(r, k, k + chunk, slot++);
+    if (k < end) items[rest_at[chunk - (end - k)]++] = make_uint4(r, k, end, slot++);
+    out.splits[split_at[most - (slot - first)]++] = make_uint4(r, first, slot - first, 0u);
+  }
+  for (uint32_t r = 0; r < rows; ++r) {
+    const uint32_t deg = off[r + 1] - off[r];
+    if (deg <= chunk) items[whole_at[chunk - deg]++] = make_uint4(r, off[r], off[r + 1], nts::kNoSlot);
+  }
+  out.n_partials = n_partials;
+}
+
 // Host-only: needs nothing but the two index arrays.
 void make_schedule(Schedule &out, const uint32_t *off, const uint32_t *idx_in, uint32_t rows, uint32_t chunk,
                    uint32_t n_slabs, uint32_t n_index) {
   const uint32_t *idx = idx_in;
+  auto count_repeated = [&] {
+    std::atomic<uint64_t> repeated(0);
+    parallel_blocks(rows, [&](uint32_t r0, uint32_t r1) {
+      uint64_t n = 0;
+      for (uint32_t r = r0; r < r1; ++r)
+        for (uint32_t k = off[r] + 1; k < off[r + 1]; ++k) n += idx[k] == idx[k - 1];
+      repeated.fetch_add(n, std::memory_order_relaxed);
+    });
+    out.repeated_edges = repeated.load();
+  };
+  if (n_slabs <= 1 || idx == nullptr || n_index == 0) {
+    make_one_range_schedule(out, off, rows, chunk);
+    if (idx) count_repeated();
+    return;
+  }
   std::vector<Piece> pieces;
   std::vector<uint4> &splits = out.splits;
   uint32_t n_partials = 0;
   std::vector<uint32_t> bucket(static_cast<size_t>(chunk) + 2, 0u);
-  const bool slabbed = n_slabs > 1 && idx != nullptr && n_index > 0;
   // Source ranges come in three widths and a row is cut at the width that suits its length: every
   // piece costs one partial row (written, then read by the second stage), so shorter rows get
   // fewer, wider ranges.
@@ -1724,47 +1796,45 @@ void make_schedule(Schedule &out, const uint32_t *off, const uint32_t *idx_in, u
   // same time gather from the same part of the source rows whatever the width of their ranges.
   // (Twice or four times as many, narrower ranges for rows above 2,048 .. 16,384 edges were
   // measured as well: no gain on the 114.8 M-edge power-law graph.)
-  const uint32_t fine = slabbed ? n_slabs : 1;
-  const uint64_t fine_width = slabbed ? (static_cast<uint64_t>(n_index) + fine - 1) / fine : 0;
-  const uint32_t wide_ranges = slabbed && n_slabs >= 8 ? n_slabs / 4 : 0;
+  const uint32_t fine = n_slabs;
+  const uint64_t fine_width = (static_cast<uint64_t>(n_index) + fine - 1) / fine;
+  const uint32_t wide_ranges = n_slabs >= 8 ? n_slabs / 4 : 0;
   std::vector<uint8_t> was_cut(wide_ranges ? rows : 0, 0);
-  if (slabbed) {
-    // Rows long enough to be cut by source range must ascend.  Edge files are not always sorted
-    // (the reference's loader leaves a CSR row in thread-arrival order), so such rows are sorted in
-    // a copy of the index array that the schedule then gathers through; a stable sort, so equal
-    // indices keep their edge order.  Sums of those rows are associated in source order.
-    const uint32_t cut_above = wide_ranges ? chunk / 4 : chunk;
-    std::vector<uint8_t> unsorted(rows, 0);
-    std::atomic<bool> any(false);
+  // Rows long enough to be cut by source range must ascend.  Edge files are not always sorted
+  // (the reference's loader leaves a CSR row in thread-arrival order), so such rows are sorted in
+  // a copy of the index array that the schedule then gathers through; a stable sort, so equal
+  // indices keep their edge order.  Sums of those rows are associated in source order.
+  const uint32_t cut_above = wide_ranges ? chunk / 4 : chunk;
+  std::vector<uint8_t> unsorted(rows, 0);
+  std::atomic<bool> any(false);
+  parallel_blocks(rows, [&](uint32_t r0, uint32_t r1) {
+    for (uint32_t r = r0; r < r1; ++r) {
+      const uint32_t b = off[r], e = off[r + 1];
+      if (e - b <= cut_above) continue;
+      for (uint32_t k = b + 1; k < e; ++k)
+        if (idx_in[k - 1] > idx_in[k]) {
+          unsorted[r] = 1;
+          any.store(true, std::memory_order_relaxed);
+          break;
+        }
+    }
+  });
+  if (any.load()) {
+    const uint32_t edges = off[rows];
+    out.sorted_idx.assign(idx_in, idx_in + edges);
+    out.edge_ids.resize(edges);
+    parallel_blocks(edges, [&](uint32_t e0, uint32_t e1) {
+      for (uint32_t e = e0; e < e1; ++e) out.edge_ids[e] = e;
+    });
     parallel_blocks(rows, [&](uint32_t r0, uint32_t r1) {
       for (uint32_t r = r0; r < r1; ++r) {
-        const uint32_t b = off[r], e = off[r + 1];
-        if (e - b <= cut_above) continue;
-        for (uint32_t k = b + 1; k < e; ++k)
-          if (idx_in[k - 1] > idx_in[k]) {
-            unsorted[r] = 1;
-            any.store(true, std::memory_order_relaxed);
-            break;
-          }
+        if (!unsorted[r]) continue;
+        uint32_t *ids = out.edge_ids.data() + off[r], *ids_end = out.edge_ids.data() + off[r + 1];
+        std::stable_sort(ids, ids_end, [&](uint32_t a, uint32_t b) { return idx_in[a] < idx_in[b]; });
+        for (uint32_t k = off[r]; k < off[r + 1]; ++k) out.sorted_idx[k] = idx_in[out.edge_ids[k]];
       }
     });
-    if (any.load()) {
-      const uint32_t edges = off[rows];
-      out.sorted_idx.assign(idx_in, idx_in + edges);
-      out.edge_ids.resize(edges);
-      parallel_blocks(edges, [&](uint32_t e0, uint32_t e1) {
-        for (uint32_t e = e0; e < e1; ++e) out.edge_ids[e] = e;
-      });
-      parallel_blocks(rows, [&](uint32_t r0, uint32_t r1) {
-        for (uint32_t r = r0; r < r1; ++r) {
-          if (!unsorted[r]) continue;
-          uint32_t *ids = out.edge_ids.data() + off[r], *ids_end = out.edge_ids.data() + off[r + 1];
-          std::stable_sort(ids, ids_end, [&](uint32_t a, uint32_t b) { return idx_in[a] < idx_in[b]; });
-          for (uint32_t k = off[r]; k < off[r + 1]; ++k) out.sorted_idx[k] = idx_in[out.edge_ids[k]];
-        }
-      });
-      idx = out.sorted_idx.data();
-    }
+    idx = out.sorted_idx.data();
   }
   std::vector<uint32_t> stops;  // (narrow range id, end edge) of the non-empty ranges of one row
   // Cuts edges [b, e) of a row with ascending indices at `ranges` equal ranges; ranges divides fine.
@@ -1786,7 +1856,6 @@ void make_schedule(Schedule &out, const uint32_t *off, const uint32_t *idx_in, u
       cut = stop;
     }
   };
-  if (!slabbed && rows) pieces.reserve(std::min<size_t>((off[rows] - off[0]) / chunk * size_t{2}, size_t{1} << 20));
   for (uint32_t r = 0; r < rows; ++r) {
     const uint32_t b = off[r], e = off[r + 1], deg = e - b;
     if (deg <= chunk) {
@@ -1808,54 +1877,24 @@ void make_schedule(Schedule &out, const uint32_t *off, const uint32_t *idx_in, u
       continue;
     }
     const uint32_t first = n_partials;
-    if (slabbed) {
-      range_stops(b, e, (wide_ranges && deg <= 4 * static_cast<uint64_t>(chunk)) ? n_slabs / 2 : n_slabs);
-      uint32_t from = b;
-      for (size_t q = 0; q < stops.size(); q += 2) {
-        for (uint32_t k = from; k < stops[q + 1]; k += chunk)
-          pieces.push_back(Piece{stops[q], r, k, std::min(stops[q + 1], k + chunk), n_partials++});
-        from = stops[q + 1];
-      }
-    } else {
-      for (uint32_t k = b; k < e; k += chunk) pieces.push_back(Piece{0u, r, k, std::min(e, k + chunk), n_partials++});
+    range_stops(b, e, (wide_ranges && deg <= 4 * static_cast<uint64_t>(chunk)) ? n_slabs / 2 : n_slabs);
+    uint32_t from = b;
+    for (size_t q = 0; q < stops.size(); q += 2) {
+      for (uint32_t k = from; k < stops[q + 1]; k += chunk)
+        pieces.push_back(Piece{stops[q], r, k, std::min(stops[q + 1], k + chunk), n_partials++});
+      from = stops[q + 1];
     }
     splits.push_back(make_uint4(r, first, n_partials - first, 0u));
   }
-  if (idx) {
-    std::atomic<uint64_t> repeated(0);
-    parallel_blocks(rows, [&](uint32_t r0, uint32_t r1) {
-      uint64_t n = 0;
-      for (uint32_t r = r0; r < r1; ++r)
-        for (uint32_t k = off[r] + 1; k < off[r + 1]; ++k) n += idx[k] == idx[k - 1];
-      repeated.fetch_add(n, std::memory_order_relaxed);
-    });
-    out.repeated_edges = repeated.load();
-  }
-  // Split rows by descending piece count, stable: placed by count (a sort of the 2,000 split rows and 11,500 pieces
-  // of a 7 M-edge graph took 0.5 ms of a schedule made without source ranges).
-  uint32_t most = 0;
-  for (const uint4 &sp : splits) most = std::max(most, sp.z);
-  std::vector<uint32_t> at(static_cast<size_t>(most) + 2, 0u);
-  for (const uint4 &sp : splits) ++at[most - sp.z + 1];
-  for (size_t i = 1; i < at.size(); ++i) at[i] += at[i - 1];
-  std::vector<uint4> by_count(splits.size());
-  for (const uint4 &sp : splits) by_count[at[most - sp.z]++] = sp;
-  splits.swap(by_count);
+  count_repeated();
+  std::stable_sort(splits.begin(), splits.end(), [](const uint4 &a, const uint4 &b) { return a.z > b.z; });
+  std::stable_sort(pieces.begin(), pieces.end(), [](const Piece &a, const Piece &b) {
+    if (a.slab != b.slab) return a.slab < b.slab;
+    return (a.e1 - a.e0) > (b.e1 - b.e0);
+  });
   std::vector<uint4> &items = out.items;
   items.reserve(pieces.size() + rows + splits.size());  // (the split rows follow for the upload)
-  if (slabbed) {
-    std::stable_sort(pieces.begin(), pieces.end(), [](const Piece &a, const Piece &b) {
-      if (a.slab != b.slab) return a.slab < b.slab;
-      return (a.e1 - a.e0) > (b.e1 - b.e0);
-    });
-    for (const Piece &pc : pieces) items.push_back(make_uint4(pc.row, pc.e0, pc.e1, pc.slot));
-  } else if (!pieces.empty()) {  // one range: descending length, placed the same way (no piece is above `chunk`)
-    at.assign(static_cast<size_t>(chunk) + 2, 0u);
-    for (const Piece &pc : pieces) ++at[chunk - (pc.e1 - pc.e0) + 1];
-    for (size_t i = 1; i < at.size(); ++i) at[i] += at[i - 1];
-    items.resize(pieces.size());
-    for (const Piece &pc : pieces) items[at[chunk - (pc.e1 - pc.e0)]++] = make_uint4(pc.row, pc.e0, pc.e1, pc.slot);
-  }
+  for (const Piece &pc : pieces) items.push_back(make_uint4(pc.row, pc.e0, pc.e1, pc.slot));
   for (size_t i = 1; i < bucket.size(); ++i) bucket[i] += bucket[i - 1];
   const size_t base = items.size();
   items.resize(base + bucket.back());

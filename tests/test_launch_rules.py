@@ -39,3 +39,26 @@ def test_pieces_of_one_range_are_issued_by_length(chunk):
         order = np.lexsort((items[part, key], -n[part]))
         assert np.array_equal(order, np.arange(order.size))
     assert int(n.sum()) == int(co[-1])
+
+
+@pytest.mark.parametrize("chunk", [1, 3, 32, 299, 300, 301, 2**32 - 1])
+@pytest.mark.parametrize("lead", [0, 5])
+def test_schedule_of_one_range(chunk, lead):
+    """Every entry against the definition: pieces of `chunk` edges and one rest, by length, then the whole rows by
+    length; slots and split rows by row; lengths at the piece length and its multiples, empty rows, edges before the
+    first row, a piece length beyond every row and one that no array could hold a count for."""
+    deg = np.concatenate([[300, 0, 299, 301, 600, 1, 32, 64, 0, 33], np.random.default_rng(9).integers(0, 301, 40)])
+    co = np.zeros(deg.size + 1, dtype=np.uint32)
+    co[1:] = np.cumsum(deg)
+    co += np.uint32(lead)
+    items, n_splits, n_partials = schedule(co, None, 0, chunk, 0)
+    pieces, whole = [], []
+    for r in range(deg.size):
+        b, e = int(co[r]), int(co[r + 1])
+        if e - b <= chunk:
+            whole.append((r, b, e, int(NO_SLOT)))
+        else:
+            pieces += [(r, k, min(e, k + chunk), len(pieces) + j) for j, k in enumerate(range(b, e, chunk))]
+    want = sorted(pieces, key=lambda p: p[1] - p[2]) + sorted(whole, key=lambda p: p[1] - p[2])
+    assert n_splits == int((deg > chunk).sum()) and n_partials == len(pieces)
+    assert np.array_equal(items, np.array(want, dtype=np.uint32))
