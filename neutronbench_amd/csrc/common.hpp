@@ -124,6 +124,16 @@ constexpr size_t kIdleBlocks = 32;
 
 inline bool aligned_to(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
+inline bool is_power_of_two(uint32_t v) { return v && (v & (v - 1)) == 0; }
+
+// Whether nts_sddmm_heads gives every edge a group of lanes (a power of two of them, as many for every head) with
+// *vec floats each; for other widths it takes a wavefront per head of an edge, many times slower.
+inline bool sddmm_by_lanes(const void *in, const void *gout, uint32_t H, uint32_t Fh, uint32_t *vec) {
+  *vec = Fh % 4 == 0 && aligned_to(in, 16) && aligned_to(gout, 16) ? 4 : 1;
+  const uint32_t lanes = H * Fh / *vec;
+  return lanes <= 64 && is_power_of_two(lanes) && is_power_of_two(Fh / *vec);
+}
+
 inline uint32_t ceil_div(uint64_t a, uint64_t b) { return static_cast<uint32_t>((a + b - 1) / b); }
 
 // A count that kernels need: known on the host (`n` null, value = `cap`), or produced earlier in the

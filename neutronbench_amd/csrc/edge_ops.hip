@@ -2526,11 +2526,10 @@ int nts_sddmm_heads(float *galpha, const float *in, const float *gout, const uin
   if (!galpha || !in || !gout || !co || !ri) return fail(NTS_ERR_INVALID, "nts_sddmm_heads: null pointer");
   const uint32_t F = H * Fh;
   const dim3 grid = edge_grid(Vd), block(256);
-  const bool v4 = Fh % 4 == 0 && aligned_to(in, 16) && aligned_to(gout, 16);
-  const uint32_t vec = v4 ? 4 : 1;
-  const uint32_t lanes = F / vec, lanes_per_head = Fh / vec;
-  if (lanes <= kWave && is_pow2(lanes) && is_pow2(lanes_per_head)) {
-    if (v4)
+  uint32_t vec = 1;
+  if (sddmm_by_lanes(in, gout, H, Fh, &vec)) {
+    const uint32_t lanes = F / vec, lanes_per_head = Fh / vec;
+    if (vec == 4)
       hipLaunchKernelGGL(sddmm_edge_kernel<4>, grid, block, 0, stream, galpha, in, gout, co, ri, Vd, H, Fh, lanes,
                          lanes_per_head);
     else

@@ -816,6 +816,13 @@ void launch_attention_grad_lanes(const LaunchArgs &a) {
 template <int VEC>
 void launch_attention_grad(const LaunchArgs &a) {
   const uint32_t vecs = ceil_div(a.heads.Fh, VEC);
+  // Lanes that a narrow head leaves idle are rows that the wavefront does not work on: eight heads of four floats
+  // with four lanes each instead of one, 1.5 M vertices, 5 M edges 704 us, 459 now; two lanes for eight floats 762, 652.
+  // (Not for heads of one or two floats: 30 K vertices, 300 K edges, eight heads of one 59 us, 70 with a lane each.)
+  if constexpr (VEC == 4) {
+    if (vecs <= 1) return launch_attention_grad_lanes<1, 1, VEC>(a);
+    if (vecs <= 2) return launch_attention_grad_lanes<2, 1, VEC>(a);
+  }
   if (vecs <= 4) return launch_attention_grad_lanes<4, 1, VEC>(a);
   if (vecs <= 8) return launch_attention_grad_lanes<8, 1, VEC>(a);
   if (vecs <= 16) return launch_attention_grad_lanes<16, 1, VEC>(a);
@@ -1297,6 +1304,29 @@ int launch_spmm_balanced(LaunchArgs a, uint32_t edges, unsigned char *fixed = nu
   if (err != hipSuccess) return bail(err, "spmm: balanced launch");
   if (!fixed) NTS_HIP_TRY(scratch_free(buf, a.stream));
   return NTS_OK;
+}
+
+// Where a pass per gradient is faster although it gathers the rows twice (both ways measured on R-MAT graphs and on
+// uniformly sampled layers, one to eight heads of 1 to 64 floats; us, fused and separate).
+//  - Graphs of few edges whose rows hold two and more on average have hub rows that no wavefront shares the work of
+//    (kAutoMinEdges), or few that do, and a step of eight edges of the fused kernel, with its sums across lanes,
+//    takes twice a step of the gather: 2.7 K vertices, 13 K edges, eight heads of 8 56, 33; 5 K, 40 K, one of 32 134, 81;
+//    10 K, 100 K, two of 16 51, 39.  From 2^17 edges on the pieces are what a launch lasts, and fused is as fast
+//    (100 K, 300 K, two of 16 66, 62; four of 4 65, 82).  Sampled layers, with little more than an edge a source, have
+//    no such rows: 4 K destinations, 41 K edges, eight heads of 8 7, 14.
+//    For widths that nts_sddmm_heads is slow at, only one head is affected: 5 K, 40 K, 47 floats 151, 80; two of 47 149, 142.
+//  - Rows of at most 64 bytes from kAutoLargeEdges on: reading them again costs less than the fused kernel's idle
+//    lanes and half-filled steps: 1 M vertices, 20 M edges, two heads of 4 1,178, 1,060; four of 4 1,275, 1,173; two of
+//    16 1,266, 1,201; one of 64 1,403, 1,796.
+bool separate_gradients_are_faster(const LaunchArgs &a, uint32_t edges) {
+  const uint32_t H = a.heads.H, Fh = a.heads.Fh;
+  uint32_t vec = 1;
+  const bool by_lanes = sddmm_by_lanes(a.dot_rows, a.in, H, Fh, &vec);
+  if (edges / 2 >= a.n_items) {
+    if (by_lanes && edges < (a.F <= 128 ? 2 * kAutoMinEdges : kAutoMinEdges)) return true;
+    if (!by_lanes && H == 1 && Fh > 4 && edges >= kAutoMinEdges / 4 && edges < kAutoMinEdges) return true;
+  }
+  return by_lanes && a.F <= 16 && edges >= kAutoLargeEdges;
 }
 
 // ---- the same schedule built on the device -----------------------------------------------------------
@@ -2444,9 +2474,10 @@ int nts_gat_aggregate_bwd(float *gx, float *galpha, const float *x, const float 
   a.dot_rows = x;
   a.dot_out = galpha;
   int vec = 1;
-  if (!edges || !perm || !nts::attention_grad_takes(a, &vec)) {
-    // Heads wider than the fused kernel's lanes, or a structure without its edge permutation: one
-    // pass per gradient.
+  if (!edges || !perm || !nts::attention_grad_takes(a, &vec) ||
+      (co && ri && nts::separate_gradients_are_faster(a, edges))) {
+    // Heads wider than the fused kernel's lanes, a structure without its edge permutation, or a size at which it is
+    // faster: one pass per gradient.
     if (edges)
       if (int rc = nts_sddmm_heads(galpha, x, gout, co, ri, Vd, H, Fh, stream)) return rc;
     a.dot_rows = nullptr;

@@ -61,3 +61,40 @@ def test_empty_structure(device):
     call("nts_gat_aggregate_bwd", ptr(gx), 0, 0, 0, 0, 0, ptr(ro), 0, ptr(ro), 0, 5, 5, 0, 2, 4, 0,
          torch.cuda.current_stream().cuda_stream)
     assert np.array_equal(gx.cpu().numpy(), np.zeros((5, 8), np.float32))
+
+
+# a width whose products go by lanes, and one head of a width whose products do not; two heads of it, a layer with little
+# more than an edge a source, and wide rows of many edges stay fused
+@pytest.mark.parametrize("V,E,n_src,H,Fh,separate", [
+    (700, 5000, 0, 2, 16, True), (700, 5000, 0, 4, 64, True), (3000, 90000, 0, 8, 8, True), (3000, 90000, 0, 4, 64, False),
+    (3000, 131072, 0, 8, 8, False), (900, 16384, 0, 1, 47, True), (900, 16383, 0, 1, 47, False), (900, 20000, 0, 2, 47, False),
+    (3000, 65536, 0, 1, 47, False), (2000, 20000, 90000, 2, 16, False), (50000, 4194304, 0, 2, 8, True),
+    (50000, 4194303, 0, 2, 8, False), (50000, 4194304, 0, 2, 16, False)])
+def test_a_pass_per_gradient_where_it_is_faster(device, V, E, n_src, H, Fh, separate):
+    """The way that was taken shows in what the call makes of the CSC's indices, which only nts_sddmm_heads reads: here
+    they all name source 0, while the CSR and its permutation tell the truth.  Without a CSC the call is fused."""
+    F, s = H * Fh, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=device).manual_seed(E)
+    if n_src:
+        ri = torch.randint(0, n_src, (E,), generator=g, device=device)
+        co = torch.arange(0, E + 1, E // V, device=device)
+        layer = SampledLayer.from_device_hop(as_u32(co), as_u32(ri), torch.arange(V, dtype=torch.int32, device=device), n_src)
+    else:
+        layer = _layer(device, V, E, 7)
+    Vs = layer.src_size
+    x, gout, alpha = (torch.randn(n, w, generator=g, device=device) for n, w in ((Vs, F), (V, F), (E, H)))
+    gx, want = torch.empty(Vs, F, device=device), torch.empty(Vs, F, device=device)
+    galpha, of_0, true = (torch.empty(E, H, device=device) for _ in range(3))
+    only_0 = torch.zeros(E, dtype=torch.int32, device=device)
+    call("nts_spmm_gather_heads", ptr(gout), ptr(want), ptr(alpha), ptr(layer.dev_csr_to_csc), ptr(layer.dev_r_o()),
+         ptr(layer.dev_c_i()), Vs, E, H, Fh, 0, s)
+    for out, ri in ((of_0, only_0), (true, layer.dev_r_i())):
+        call("nts_sddmm_heads", ptr(out), ptr(x), ptr(gout), ptr(layer.dev_c_o()), ptr(ri), V, H, Fh, s)
+    for co, ri in ((ptr(layer.dev_c_o()), ptr(only_0)), (0, 0)):
+        call("nts_gat_aggregate_bwd", ptr(gx), ptr(galpha), ptr(x), ptr(gout), ptr(alpha), ptr(layer.dev_csr_to_csc),
+             ptr(layer.dev_r_o()), ptr(layer.dev_c_i()), co, ri, V, Vs, E, H, Fh, 0, s)
+        assert torch.equal(gx, want)
+        if separate and co:
+            assert torch.equal(galpha, of_0)
+        else:  # two sums of the same Fh products in fp32
+            assert (galpha - true).abs().max() <= 2 * Fh * 2.0 ** -24 * (Fh * x.abs().max() * gout.abs().max())
