@@ -420,7 +420,7 @@ int nts_sddmm_heads(float *galpha, const float *in, const float *gout, const uin
  * i.e. nts_spmm_gather_heads over the CSR and nts_sddmm_heads over the CSC, which the call falls back to
  * for heads of more than 64 vectors (256 floats; 64 floats where Fh or an array is off a 16-byte boundary),
  * when perm is NULL (alpha and galpha then as those two calls take them), and, where co and ri are given, at
- * sizes at which they are faster (graphs of few edges with hub rows; rows of at most 16 floats over many).
+ * sizes at which they are faster (wide rows of graphs of few edges).
  * Scratch as nts_spmm_gather.  accumulate applies to gx. */
 int nts_gat_aggregate_bwd(float *gx, float *galpha, const float *x, const float *gout, const float *alpha,
                           const uint32_t *perm, const uint32_t *ro, const uint32_t *ci, const uint32_t *co,

@@ -515,8 +515,22 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
 // registers.  The products of U edges are added over a head's lanes together: each butterfly step
 // halves the edges a lane still holds (U - 1 exchanges for U edges instead of U log2 LH), which leaves
 // lane `sub` with edge sub's sum and spreads the stores over the lanes.
+// A wavefront's loads and stores complete in order, and a load behind stores would wait for them: the sums of a step
+// are stored when the rows of the next one are on their way, in a loop whose accesses depend on no condition (so that
+// the wait for the rows can leave the stores out).  A long row's step is then one memory latency and not two: 5 K
+// vertices, 40 K edges, four heads of 4 135 -> 70 us; 30 K, 300 K, of 16 66 -> 47.  Where throughput bounds it the figures are close: 1 M, 20 M, four of 32 1,911 -> 1,863 us.
+// Requesting the rows of two steps ahead was slower everywhere (0.85 times: a third fewer wavefronts fit).
+//
+// Wavefronts per SIMD that the registers are held down for.  The rows of wide groups come from memory, and six
+// wavefronts with two spilled values outside the loop beat four (1.5 M vertices, 5 M edges, four heads of 32 1,050 -> 854
+// us); narrower ones lose more by the spills than they gain (30 K, 300 K, eight of 4 with six 93, without 52 us).
 template <int G, int LH, int NJ, int VEC>
-__global__ __launch_bounds__(256) void attention_grad_kernel(const float *__restrict__ gout, float *__restrict__ out,
+constexpr int grad_waves() {
+  if (VEC != 4 || NJ != 1 || LH == 1) return 1;
+  return LH < 8 ? 5 : G >= 32 ? 6 : 1;
+}
+template <int G, int LH, int NJ, int VEC>
+__global__ __launch_bounds__(256, (grad_waves<G, LH, NJ, VEC>())) void attention_grad_kernel(const float *__restrict__ gout, float *__restrict__ out,
                                                              const float *__restrict__ alpha,
                                                              const uint32_t *__restrict__ offsets,
                                                              const uint32_t *__restrict__ indices, uint32_t n_items,
@@ -555,82 +569,119 @@ __global__ __launch_bounds__(256) void attention_grad_kernel(const float *__rest
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const uint32_t c = (sub + LH * j) * VEC;
-    live[j] = head_live && c < Fh;
+    live[j] = c < Fh;
     col[j] = head * Fh + (c < Fh ? c : 0u);  // idle lanes re-read the head's first columns
     acc[j] = vzero<VEC>();
     xr[j] = vzero<VEC>();
     if (e0 < e1) xr[j] = *reinterpret_cast<const V *>(x + static_cast<size_t>(row) * F + col[j]);  // (no edge: x need not hold the row)
   }
-  auto fetch_pair = [&](uint32_t e, uint32_t &pi, uint32_t &ps) {
-    pi = ps = 0;
-    if (e < e1) {
-      pi = indices[e];
-      ps = heads.perm[e];
+  const uint32_t n_edges = e1 - e0;
+  // Lane l of a group holds the pair of edge l % U of a step, one step ahead; beyond the row the last edge's.
+  uint32_t my_i, my_s, nxt_i, nxt_s;
+  auto fetch_pair = [&](uint32_t k, uint32_t &pi, uint32_t &ps) {
+    const uint32_t at = e0 + min(k + (gl & (U - 1)), n_edges - 1);
+    pi = indices[at];
+    ps = heads.perm[at];
+  };
+  V v[U][NJ];
+  float p[U];
+  // Lane `sub` of a head answers for the edges S * i + sub % S of a step: it loads their weights and stores their sums.
+  const uint32_t mine = sub & (S - 1);
+  uint32_t id[U / S];
+  float w[U / S];
+  auto gather_row = [&](int u, bool there) {
+    const uint32_t si = __shfl(my_i, u, G);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      if (there) v[u][j] = *reinterpret_cast<const V *>(gout + static_cast<size_t>(si) * F + col[j]);
+  };
+  auto gather_weight = [&](int i, bool there) {
+    id[i] = __shfl(my_s, S * i + mine, G);
+    if (there) w[i] = alpha[static_cast<size_t>(id[i]) * H + head];
+  };
+  auto products = [&](uint32_t left) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float wu = LH == 1 ? w[u / S] : __shfl(w[u / S], u % S, LH);
+      p[u] = 0.f;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        if (static_cast<uint32_t>(u) < left) vfma(acc[j], v[u][j], wu);
+        const float q = vdot(v[u][j], xr[j]);
+        p[u] += live[j] ? q : 0.f;
+      }
+    }
+    int cnt = U;
+#pragma unroll
+    for (int m = 1; m < LH; m <<= 1) {
+      if (cnt > 1) {
+        const bool upper = sub & m;
+#pragma unroll
+        for (int i = 0; i < U / 2; ++i) {
+          if (i < cnt / 2) {
+            const float keep = upper ? p[2 * i + 1] : p[2 * i];
+            const float send = upper ? p[2 * i] : p[2 * i + 1];
+            p[i] = keep + __shfl_xor(send, m, kWave);
+          }
+        }
+        cnt /= 2;
+      } else {
+        p[0] += __shfl_xor(p[0], m, kWave);
+      }
     }
   };
-  uint32_t nxt_i, nxt_s;
-  fetch_pair(e0 + gl, nxt_i, nxt_s);
-  for (uint32_t eb = e0; eb < e1; eb += G) {
-    const uint32_t n = min(static_cast<uint32_t>(G), e1 - eb);
-    const uint32_t my_i = nxt_i, my_s = nxt_s;
-    fetch_pair(eb + G + gl, nxt_i, nxt_s);
-    for (uint32_t j0 = 0; j0 < n; j0 += U) {
-      const uint32_t left = n - j0;
-      V v[U][NJ];
-      float wv[U], p[U];
+  uint32_t k = 0;
+  if (n_edges) fetch_pair(0, my_i, my_s);
+  if (n_edges >= U) {
+    fetch_pair(U, nxt_i, nxt_s);
+    uint32_t done[U / S];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint32_t si = __shfl(my_i, (j0 + u) & (G - 1), G);
-        const uint32_t ss = __shfl(my_s, (j0 + u) & (G - 1), G);
-        wv[u] = 0.f;
+    for (int i = 0; i < U / S; ++i) done[i] = __shfl(my_s, S * i + mine, G);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) v[u][j] = vzero<VEC>();
-        if (static_cast<uint32_t>(u) < left) {
+    for (int u = 0; u < U; ++u) p[u] = 0.f;
+    do {
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) v[u][j] = *reinterpret_cast<const V *>(gout + static_cast<size_t>(si) * F + col[j]);
-          wv[u] = alpha[static_cast<size_t>(ss) * H + head];
-        }
-      }
+      for (int i = 0; i < U / S; ++i) gather_weight(i, true);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        p[u] = 0.f;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          if (static_cast<uint32_t>(u) < left) vfma(acc[j], v[u][j], wv[u]);
-          const float q = vdot(v[u][j], xr[j]);
-          p[u] += live[j] ? q : 0.f;
-        }
-      }
-      int cnt = U;
-#pragma unroll
-      for (int m = 1; m < LH; m <<= 1) {
-        if (cnt > 1) {
-          const bool upper = sub & m;
-#pragma unroll
-          for (int i = 0; i < U / 2; ++i) {
-            if (i < cnt / 2) {
-              const float keep = upper ? p[2 * i + 1] : p[2 * i];
-              const float send = upper ? p[2 * i] : p[2 * i + 1];
-              p[i] = keep + __shfl_xor(send, m, kWave);
-            }
-          }
-          cnt /= 2;
-        } else {
-          p[0] += __shfl_xor(p[0], m, kWave);
-        }
-      }
+      for (int u = 0; u < U; ++u) gather_row(u, true);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < U / S; ++i) {
-        const uint32_t u = S * i + (sub & (S - 1));
-        const uint32_t id = __shfl(my_s, (j0 + u) & (G - 1), G);
-        if (head_live && sub < S && u < left) galpha[static_cast<size_t>(id) * H + head] = p[i];
+        galpha[static_cast<size_t>(done[i]) * H + head] = p[i];
+        done[i] = id[i];
       }
+      k += U;
+      my_i = nxt_i;
+      my_s = nxt_s;
+      fetch_pair(k + U, nxt_i, nxt_s);
+      __builtin_amdgcn_sched_barrier(0);
+      products(U);
+    } while (n_edges - k >= U);
+#pragma unroll
+    for (int i = 0; i < U / S; ++i) galpha[static_cast<size_t>(done[i]) * H + head] = p[i];
+  }
+  const uint32_t left = n_edges - k;
+  if (left) {
+#pragma unroll
+    for (int i = 0; i < U / S; ++i) {
+      w[i] = 0.f;
+      gather_weight(i, S * i + mine < left);
     }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) v[u][j] = vzero<VEC>();
+      gather_row(u, static_cast<uint32_t>(u) < left);
+    }
+    products(left);
+#pragma unroll
+    for (int i = 0; i < U / S; ++i)
+      if (head_live && sub < S && S * i + mine < left) galpha[static_cast<size_t>(id[i]) * H + head] = p[i];
   }
   float *dst = (slot == kNoSlot) ? out + static_cast<size_t>(row) * F : partial + static_cast<size_t>(slot) * F;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    if (live[j]) {
+    if (head_live && live[j]) {
       V *q = reinterpret_cast<V *>(dst + col[j]);
       V r = acc[j];
       if (accumulate && slot == kNoSlot) vadd(r, *q);
@@ -1306,27 +1357,21 @@ int launch_spmm_balanced(LaunchArgs a, uint32_t edges, unsigned char *fixed = nu
   return NTS_OK;
 }
 
-// Where a pass per gradient is faster although it gathers the rows twice (both ways measured on R-MAT graphs and on
-// uniformly sampled layers, one to eight heads of 1 to 64 floats; us, fused and separate).
-//  - Graphs of few edges whose rows hold two and more on average have hub rows that no wavefront shares the work of
-//    (kAutoMinEdges), or few that do, and a step of eight edges of the fused kernel, with its sums across lanes,
-//    takes twice a step of the gather: 2.7 K vertices, 13 K edges, eight heads of 8 56, 33; 5 K, 40 K, one of 32 134, 81;
-//    10 K, 100 K, two of 16 51, 39.  From 2^17 edges on the pieces are what a launch lasts, and fused is as fast
-//    (100 K, 300 K, two of 16 66, 62; four of 4 65, 82).  Sampled layers, with little more than an edge a source, have
-//    no such rows: 4 K destinations, 41 K edges, eight heads of 8 7, 14.
-//    For widths that nts_sddmm_heads is slow at, only one head is affected: 5 K, 40 K, 47 floats 151, 80; two of 47 149, 142.
-//  - Rows of at most 64 bytes from kAutoLargeEdges on: reading them again costs less than the fused kernel's idle
-//    lanes and half-filled steps: 1 M vertices, 20 M edges, two heads of 4 1,178, 1,060; four of 4 1,275, 1,173; two of
-//    16 1,266, 1,201; one of 64 1,403, 1,796.
+// Where a pass per gradient is faster although it gathers the rows twice: graphs of few edges, whose hub rows no
+// wavefront shares the work of (kAutoMinEdges), so that a launch lasts as long as the longest row.  A step of eight edges
+// of the fused kernel, with its sums across the lanes, takes longer than one of the gather of wide rows; the other pass
+// has no such chain.  Fused and separate, us: 5 K vertices, 40 K edges, eight heads of 8 91, 65; one of 64 81, 68;
+// of 128 121, 73; two of 64 97, 73; but four of 4 70, 106, one of 32 75, 81 (rows below 64 floats stay fused)
+// and four of 64 97, 100.  For widths that nts_sddmm_heads is slow at, only one head of 4-byte lanes is affected: 5 K, 40 K, 47
+// floats 100, 80; two of 47 99, 142; 2.7 K, 13 K, 47 floats 42, 58.  With fewer than four edges a row on average there are
+// no such rows, or they matter less: 10 K, 25 K, two of 64 36, 45; a sampled layer of 4 K destinations, 41 K edges, eight
+// heads of 8 7, 14.
 bool separate_gradients_are_faster(const LaunchArgs &a, uint32_t edges) {
+  if (edges >= kAutoMinEdges || edges / 4 < a.n_items) return false;
   const uint32_t H = a.heads.H, Fh = a.heads.Fh;
   uint32_t vec = 1;
-  const bool by_lanes = sddmm_by_lanes(a.dot_rows, a.in, H, Fh, &vec);
-  if (edges / 2 >= a.n_items) {
-    if (by_lanes && edges < (a.F <= 128 ? 2 * kAutoMinEdges : kAutoMinEdges)) return true;
-    if (!by_lanes && H == 1 && Fh > 4 && edges >= kAutoMinEdges / 4 && edges < kAutoMinEdges) return true;
-  }
-  return by_lanes && a.F <= 16 && edges >= kAutoLargeEdges;
+  if (sddmm_by_lanes(a.dot_rows, a.in, H, Fh, &vec)) return a.F >= 64;
+  return H == 1 && vec == 1 && Fh > 32 && edges >= kAutoMinEdges / 4;
 }
 
 // ---- the same schedule built on the device -----------------------------------------------------------

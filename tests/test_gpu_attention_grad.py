@@ -63,13 +63,13 @@ def test_empty_structure(device):
     assert np.array_equal(gx.cpu().numpy(), np.zeros((5, 8), np.float32))
 
 
-# a width whose products go by lanes, and one head of a width whose products do not; two heads of it, a layer with little
-# more than an edge a source, and wide rows of many edges stay fused
+# rows of 64 floats and more whose products go by lanes, and one head of 4-byte lanes; two heads of those, narrower rows,
+# 65,536 edges and a layer with little more than an edge a source stay fused
 @pytest.mark.parametrize("V,E,n_src,H,Fh,separate", [
-    (700, 5000, 0, 2, 16, True), (700, 5000, 0, 4, 64, True), (3000, 90000, 0, 8, 8, True), (3000, 90000, 0, 4, 64, False),
-    (3000, 131072, 0, 8, 8, False), (900, 16384, 0, 1, 47, True), (900, 16383, 0, 1, 47, False), (900, 20000, 0, 2, 47, False),
-    (3000, 65536, 0, 1, 47, False), (2000, 20000, 90000, 2, 16, False), (50000, 4194304, 0, 2, 8, True),
-    (50000, 4194303, 0, 2, 8, False), (50000, 4194304, 0, 2, 16, False)])
+    (700, 5000, 0, 2, 32, True), (700, 5000, 0, 4, 64, True), (700, 5000, 0, 2, 16, False), (700, 5000, 0, 4, 12, False),
+    (3000, 65535, 0, 8, 8, True), (3000, 65536, 0, 8, 8, False), (900, 16384, 0, 1, 47, True), (900, 16383, 0, 1, 47, False),
+    (900, 20000, 0, 2, 47, False), (900, 20000, 0, 1, 48, False), (900, 20000, 0, 1, 31, False), (3000, 65536, 0, 1, 47, False),
+    (2000, 20000, 90000, 2, 32, False)])
 def test_a_pass_per_gradient_where_it_is_faster(device, V, E, n_src, H, Fh, separate):
     """The way that was taken shows in what the call makes of the CSC's indices, which only nts_sddmm_heads reads: here
     they all name source 0, while the CSR and its permutation tell the truth.  Without a CSC the call is fused."""
