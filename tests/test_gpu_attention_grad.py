@@ -98,3 +98,92 @@ def test_a_pass_per_gradient_where_it_is_faster(device, V, E, n_src, H, Fh, sepa
             assert torch.equal(galpha, of_0)
         else:  # two sums of the same Fh products in fp32
             assert (galpha - true).abs().max() <= 2 * Fh * 2.0 ** -24 * (Fh * x.abs().max() * gout.abs().max())
+
+
+@pytest.mark.parametrize("H,Fh", [(4, 32), (8, 41), (2, 8), (8, 4), (1, 47), (1, 256)])
+def test_large_calls(device, H, Fh):
+    """From 2^22 edges on the pieces of long rows are ordered by source before they are issued, and their sums are
+    added by another kernel for rows of more than 256 floats.  An odd edge count; hubs of 256, 257 and 200,000 edges."""
+    V, n_src, F = 40000, 30000, H * Fh
+    g = torch.Generator(device=device).manual_seed(H * 1000 + Fh)
+    hubs = [(0, 200000), (1, 257), (2, 256), (29999, 90001), (17, 8), (18, 7)]
+    parts = [torch.full((n,), s, device=device) for s, n in hubs]
+    E = (1 << 22) + 4097
+    rest = E - sum(n for _, n in hubs)
+    parts.append(100 + (torch.rand(rest, generator=g, device=device) ** 4 * 29000).long())
+    ri = torch.cat(parts)[torch.randperm(E, generator=g, device=device)]
+    dst = torch.sort(torch.randint(0, V, (E,), generator=g, device=device)).values
+    co = torch.zeros(V + 1, dtype=torch.int64, device=device)
+    co[1:] = torch.cumsum(torch.bincount(dst, minlength=V), 0)
+    layer = SampledLayer.from_device_hop(as_u32(co), as_u32(ri), torch.arange(V, dtype=torch.int32, device=device), n_src)
+    Vs, s = layer.src_size, torch.cuda.current_stream().cuda_stream
+    x, gout, alpha = (torch.randn(n, w, generator=g, device=device) for n, w in ((Vs, F), (V, F), (E, H)))
+    gx, want = torch.full((Vs, F), 3.0, device=device), torch.full((Vs, F), 3.0, device=device)
+    for accumulate in (0, 1):
+        galpha = torch.full((E, H), float("nan"), device=device)
+        call("nts_gat_aggregate_bwd", ptr(gx), ptr(galpha), ptr(x), ptr(gout), ptr(alpha), ptr(layer.dev_csr_to_csc),
+             ptr(layer.dev_r_o()), ptr(layer.dev_c_i()), ptr(layer.dev_c_o()), ptr(layer.dev_r_i()), V, Vs, E, H, Fh,
+             accumulate, s)
+        call("nts_spmm_gather_heads", ptr(gout), ptr(want), ptr(alpha), ptr(layer.dev_csr_to_csc), ptr(layer.dev_r_o()),
+             ptr(layer.dev_c_i()), Vs, E, H, Fh, accumulate, s)
+        assert torch.equal(gx, want)
+        local = u32_to_i64(layer.dev_r_i())
+        for e in range(0, E, 1 << 19):  # a part of the edges at a time
+            part = slice(e, min(E, e + (1 << 19)))
+            terms = (x[local[part]].double() * gout[dst[part]].double()).view(-1, H, Fh)
+            bound = Fh * 2.0 ** -24 * terms.abs().sum(2) + 1e-30
+            assert ((galpha[part].double() - terms.sum(2)).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("H,Fh", [(4, 32), (2, 41), (8, 4), (2, 8), (1, 47), (1, 3), (3, 16), (2, 96)])
+@pytest.mark.parametrize("where", ["x", "gout", "alpha"])
+def test_infinities_and_nan_stay_where_they_belong(device, H, Fh, where):
+    """Idle lanes re-read the first columns of a head, and masked steps hold rows of other edges: what is not finite
+    there must not reach another head, edge or row."""
+    V, E = 900, 30000
+    layer = _layer(device, V, E, 11)
+    F, Vs, s = H * Fh, layer.src_size, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=device).manual_seed(5)
+    t = {"x": torch.randn(Vs, F, generator=g, device=device), "gout": torch.randn(V, F, generator=g, device=device),
+         "alpha": torch.randn(E, H, generator=g, device=device)}
+    a = t[where]
+    for value in (float("nan"), float("inf"), float("-inf")):
+        a.view(-1)[torch.randint(0, a.numel(), (a.shape[0] // 40,), generator=g, device=device)] = value
+    gx, want = torch.empty(Vs, F, device=device), torch.empty(Vs, F, device=device)
+    galpha = torch.empty(E, H, device=device)
+    call("nts_gat_aggregate_bwd", ptr(gx), ptr(galpha), ptr(t["x"]), ptr(t["gout"]), ptr(t["alpha"]),
+         ptr(layer.dev_csr_to_csc), ptr(layer.dev_r_o()), ptr(layer.dev_c_i()), 0, 0, V, Vs, E, H, Fh, 0, s)
+    call("nts_spmm_gather_heads", ptr(t["gout"]), ptr(want), ptr(t["alpha"]), ptr(layer.dev_csr_to_csc), ptr(layer.dev_r_o()),
+         ptr(layer.dev_c_i()), Vs, E, H, Fh, 0, s)
+    assert torch.equal(torch.isnan(gx), torch.isnan(want))
+    assert torch.equal(gx.nan_to_num(7.0, 8.0, 9.0), want.nan_to_num(7.0, 8.0, 9.0))
+    co, ri = u32_to_i64(layer.dev_c_o()), u32_to_i64(layer.dev_r_i())
+    own = torch.repeat_interleave(torch.arange(V, device=device), co[1:] - co[:-1])
+    exact = (t["x"][ri].double() * t["gout"][own].double()).view(E, H, Fh).sum(2)
+    assert torch.equal(torch.isnan(galpha), torch.isnan(exact)) and torch.equal(torch.isinf(galpha), torch.isinf(exact))
+    inf = torch.isinf(exact)
+    assert torch.equal(galpha[inf].double(), exact[inf])
+    fine = torch.isfinite(exact)
+    size = (t["x"][ri].double() * t["gout"][own].double()).view(E, H, Fh).abs().sum(2)
+    assert ((galpha.double() - exact).abs()[fine] <= (Fh * 2.0 ** -24 * size + 1e-30)[fine]).all()
+
+
+@pytest.mark.parametrize("H,Fh", [(4, 32), (1, 47)])
+def test_rows_of_x_without_an_edge_are_not_needed(device, H, Fh):
+    """Sources that no edge names lie behind the others, and x ends before them."""
+    V, E, named, Vs = 700, 9000, 400, 1000
+    g = torch.Generator(device=device).manual_seed(8)
+    src = torch.cat([torch.arange(named, device=device), torch.randint(0, named, (E - named,), generator=g, device=device)])
+    dst = torch.randint(0, V, (E,), generator=g, device=device)
+    order = torch.sort(src, stable=True).indices
+    ro = torch.zeros(Vs + 1, dtype=torch.int32, device=device)
+    ro[1:] = torch.cumsum(torch.bincount(src, minlength=Vs), 0)
+    ci, perm = dst[order].to(torch.int32), order.to(torch.int32)
+    F, s = H * Fh, torch.cuda.current_stream().cuda_stream
+    x, gout, alpha = (torch.randn(n, w, generator=g, device=device) for n, w in ((named, F), (V, F), (E, H)))
+    gx, galpha = torch.full((Vs, F), 3.0, device=device), torch.empty(E, H, device=device)
+    call("nts_gat_aggregate_bwd", ptr(gx), ptr(galpha), ptr(x), ptr(gout), ptr(alpha), ptr(perm), ptr(ro), ptr(ci), 0, 0, V,
+         Vs, E, H, Fh, 0, s)
+    assert bool((gx[named:] == 0).all())
+    terms = (x[src].double() * gout[dst].double()).view(E, H, Fh)
+    assert ((galpha.double() - terms.sum(2)).abs() <= Fh * 2.0 ** -24 * terms.abs().sum(2) + 1e-30).all()
