@@ -2053,14 +2053,23 @@ bool stream_contiguous_rows() {
   return value;
 }
 
+// A wavefront streams the contiguous edges of up to 64 rows at a time, and of fewer where that would leave it without
+// the 8,192 wavefronts that the chip holds: whatever the width, 64 rows cost a small vertex set its parallelism and 16
+// cost a large one a wavefront's start-up per four rows' worth of work.  us, 64 / 16 rows a wavefront: 50 K rows, 5 M
+// edges F = 4 191 / 95, F = 128 833 / 599; 169 K, 2.48 M F = 4 88 / 80, F = 32 117 / 108, F = 128 348 / 307; 1 M, 2.5 M F = 4
+// 135 / 168, F = 32 166 / 211, F = 64 224 / 259, F = 128 436 / 439; 2.4 M, 60 M within 3 %.
+uint32_t streamed_rows_per_wave(uint32_t rows) {
+  constexpr uint32_t kChipWaves = 8192;
+  uint32_t per = kWave;
+  while (per > 16 && rows / per < kChipWaves) per /= 2;
+  return per;
+}
+
 template <typename V>
 void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_t *perm, uint32_t rows, uint32_t Fv,
                         int accumulate, uint32_t limit, const LongRowWork<V> &lw, hipStream_t stream) {
   if (rows_launch_takes_long_rows(rows, Fv) && !perm && stream_contiguous_rows()) {
-    // a wavefront streams the contiguous edges of up to 64 rows at a time
-    // (16 rows of 128 bytes and more: 64 leave an Arxiv-shaped vertex set with a third of the wavefronts that
-    // the chip holds, 1.27 GB of edge rows 423 -> 373 us)
-    const uint32_t blocks = ceil_div(rows, Fv * sizeof(V) >= 128 ? 4 * 16 : 4 * kWave);
+    const uint32_t blocks = ceil_div(rows, 4 * streamed_rows_per_wave(rows));
     const dim3 grid((blocks < 16384u ? blocks : 16384u) + lw.blocks);
 #define NTS_STREAM(GG)                                                                                          \
   hipLaunchKernelGGL((gather_edge_to_row_stream_kernel<V, GG>), grid, dim3(256), 0, stream, out, msg, off, rows, Fv, \
