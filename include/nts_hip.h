@@ -222,8 +222,10 @@ int nts_spmm_gather_static_scratch(const float *in, float *out, const float *w, 
 typedef struct nts_spmm_plan nts_spmm_plan_t;
 int nts_spmm_plan_create(nts_spmm_plan_t **plan, const uint32_t *offsets, uint32_t rows,
                          uint32_t edges, uint32_t chunk_edges, nts_stream_t stream);
-/* The same schedule, made cache-aware: `indices` (the gather index array that belongs to `offsets`)
- * is read back once as well, and the pieces of split rows whose indices ascend are cut at the
+/* The same schedule, made cache-aware.  It is built where `offsets` and `indices` (the gather index array that belongs
+ * to `offsets`) lie; they are read back to the host, once, only if offsets[0] > 0, if the memory that ordering rows takes
+ * (some 36 bytes an edge) is not to be had, or if NTS_SPMM_PLAN_HOST=1 is set.  The call synchronises `stream`.
+ * The pieces of split rows whose indices ascend are cut at the
  * boundaries of `n_slabs` equal ranges of [index_base, index_base + n_index) and issued slab by slab,
  * so that concurrently running wavefronts gather from the same range of source rows (each XCD's
  * L2 then holds that range's hot rows).  n_slabs = 0 and chunk_edges = 0 select the defaults (32
