@@ -51,3 +51,20 @@ def test_copies_and_sums(device, F, mega):
                 call("nts_gather_edge_to_src", ptr(out), ptr(msg), ptr(co), ptr(order.to(torch.int32)), V, F, 0, s)
         assert torch.equal(got[0], got[1])
         assert ((got[0].double() - want).abs() <= n * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("rows", [4096, 262143, 262144, 524287, 524288])
+@pytest.mark.parametrize("F", [1, 17, 32])
+def test_streamed_sums_at_the_steps_of_rows_a_wavefront(device, rows, F):
+    """16, 32 and 64 rows a wavefront change at 262,144 and 524,288 rows; whole numbers, so that any order is exact."""
+    rng = np.random.default_rng(rows + F)
+    deg = rng.integers(0, 5, rows)
+    deg[rng.integers(0, rows, 20)] = rng.integers(60, 2000, 20)
+    off = torch.from_numpy(np.concatenate([[0], np.cumsum(deg)])).to(device)
+    E = int(off[-1])
+    msg = torch.randint(-8, 9, (E, F), device=device).float()
+    out = torch.full((rows, F), 3.0, device=device)
+    call("nts_gather_edge_to_dst", ptr(out), ptr(msg), ptr(off.to(torch.int32)), rows, F, 0,
+         torch.cuda.current_stream().cuda_stream)
+    own = torch.repeat_interleave(torch.arange(rows, device=device), off[1:] - off[:-1])
+    assert torch.equal(out, torch.zeros(rows, F, device=device).index_add_(0, own, msg))
