@@ -172,9 +172,12 @@ __global__ __launch_bounds__(256) void edge_copy_kernel(V *__restrict__ msg, con
 
 constexpr uint32_t kNoLimit = 0xFFFFFFFFu;
 constexpr uint32_t kLongRowEdges = 1024;    // edges of a row above which the block kernel takes over
-constexpr uint64_t kGiantValues = 131072;   // softmax segments above this many values are cut into pieces
+constexpr uint64_t kGiantValues = 131072;   // softmax segments above this many values are cut into pieces, at most
 constexpr uint64_t kGiantRowBytes = 1u << 20;  // row of edge rows above which it is cut into pieces for several blocks
-constexpr uint32_t kLongRowValues = 32768;  // the same for softmax segments, in values (edges * heads)
+constexpr uint32_t kLongRowValues = 32768;  // the same for softmax segments, in values (edges * heads), at most
+constexpr uint32_t kLongRowMinValues = 2048;   // and at least
+constexpr uint64_t kGiantMinValues = 32768;
+constexpr uint32_t kByTotal = 0;               // in place of a line: long_segment_values of the call's values
 constexpr uint32_t kLongMinVertices = 16384;  // vertex count below which the extra launches are not worth it
 constexpr int kLongBlock = 1024;
 
@@ -763,11 +766,28 @@ constexpr uint32_t kGiantCap = 4096;
 constexpr uint32_t kPieceCap = 8192;
 constexpr uint32_t kGiantMinPiece = 4096;  // edges, for the softmax segments
 
+// Values above which a softmax segment is a block's and not a wavefront's, and above which it is cut into pieces.
+// A launch lasts at least as long as its longest segment, which a wavefront reads 512 values and a block 8,192 at a time,
+// so the lines follow the values of the whole call: with both fixed at their upper ends the hub rows of a 2.48 M-edge
+// graph (one head) took the wavefront launches 99 us forward and 96 backward, and now 4 and 25 beside a block launch of 19 and 18
+// (attention layer of 47 columns, both directions: 844 -> 644 us).  From 33.5 M values up the ends are reached: a
+// block's two barriers a segment then cost what it gains (126 M edges, four heads, 4,096 against 32,768 values
+// for a wavefront: 1.43, 1.36 ms).
+__device__ __forceinline__ uint32_t long_segment_values(uint64_t total_values) {
+  const uint64_t v = total_values / 1024;
+  return v < kLongRowMinValues ? kLongRowMinValues : v < kLongRowValues ? static_cast<uint32_t>(v) : kLongRowValues;
+}
+__device__ __forceinline__ uint64_t giant_segment_values(uint64_t total_values) {
+  const uint64_t v = total_values / 256;
+  return v < kGiantMinValues ? kGiantMinValues : v < kGiantValues ? v : kGiantValues;
+}
+
 // hdr: [0] giant rows, [1] pieces,
 //      [2] edges per piece, [4..5] edges of the listed giant rows (64-bit), [6] the long-row counter
 //      (`count` points here, so that one fill clears all of them).
 // list[0 .. *count) = rows r with (off[r+1] - off[r]) * width > limit that are not listed as giant
-// (any order); giant_rows[0 .. hdr[0]) = rows above giant_limit values and above the share.
+// (any order); giant_rows[0 .. hdr[0]) = rows above giant_limit values and above the share.  limit
+// kByTotal: a softmax call, whose lines lie where its values put them.
 __global__ __launch_bounds__(256) void collect_long_rows_kernel(uint32_t *__restrict__ list,
                                                                 uint32_t *__restrict__ count,
                                                                 uint32_t *__restrict__ giant_rows,
@@ -779,6 +799,11 @@ __global__ __launch_bounds__(256) void collect_long_rows_kernel(uint32_t *__rest
   if (r >= rows) return;
   const uint32_t deg = off[r + 1] - off[r];
   const uint64_t n = static_cast<uint64_t>(deg) * width;
+  if (limit == kByTotal) {
+    const uint64_t total = static_cast<uint64_t>(off[rows] - off[0]) * width;
+    limit = long_segment_values(total);
+    giant_limit = giant_segment_values(total);
+  }
   if (n > giant_limit && deg > (off[rows] - off[0]) / kGiantCap) {
     const uint32_t gi = atomicAdd(&hdr[0], 1u);
     if (gi < kGiantCap) {
@@ -978,6 +1003,7 @@ constexpr uint32_t kShortValues = kShortG * kShortK;
 constexpr int kWaveK = 8;          // values per lane the wave kernel can hold in registers
 constexpr uint32_t kWaveRegValues = kWave * kWaveK;
 constexpr uint32_t kWaveMidValues = kWave * 32;  // the fused forward's launch for the class above that: 32 per lane
+static_assert(kWaveMidValues <= kLongRowMinValues, "the register classes lie below the block kernels' line");
 
 // One strided pass over a segment with U loads in flight: positions first, first + stride, ...
 // below n; `load(i)` fetches, `use(i, v)` consumes, in ascending position order.
@@ -1266,6 +1292,7 @@ __global__ __launch_bounds__(256) void edge_softmax_fwd_kernel(float *__restrict
                                                                const uint32_t *__restrict__ ri, uint32_t Vd,
                                                                uint32_t H, float slope, uint32_t min_values,
                                                                uint32_t max_values, uint32_t vec4) {
+  if (max_values == kByTotal) max_values = long_segment_values(static_cast<uint64_t>(co[Vd] - co[0]) * H);
   const uint32_t lane = lane_id();
   const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
@@ -1402,6 +1429,7 @@ __global__ __launch_bounds__(256) void edge_softmax_bwd_kernel(float *__restrict
                                                                const uint32_t *__restrict__ ri, uint32_t Vd,
                                                                uint32_t H, float slope, uint32_t min_values,
                                                                uint32_t max_values, uint32_t vec4) {
+  if (max_values == kByTotal) max_values = long_segment_values(static_cast<uint64_t>(co[Vd] - co[0]) * H);
   const uint32_t lane = lane_id();
   const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
@@ -2280,8 +2308,8 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   // stated is still computed, by one wavefront.
   const bool no_hubs = max_degree != 0 && static_cast<uint64_t>(max_degree) * H <= kLongRowValues;
   if (pow2 && !no_hubs)
-    if (int rc = collect_long_rows(lr, co, Vd, H, kLongRowValues, kGiantValues, kGiantMinPiece, stream)) return rc;
-  const uint32_t max_values = lr.list ? kLongRowValues : kNoLimit;
+    if (int rc = collect_long_rows(lr, co, Vd, H, kByTotal, 0, kGiantMinPiece, stream)) return rc;
+  const uint32_t max_values = lr.list ? kByTotal : kNoLimit;
   // The block kernels of the hub rows and the kernels of the giant ones' pieces run on the side lane,
   // beside the launches for all other rows below (they write other rows); their scratch is taken
   // before the fork, so that whatever the pool ordered for it on `stream` lies before it too.
@@ -2383,15 +2411,11 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
                      Vd, H, slope, LO, HI, vec4)
     if (pow2 && fused) {
       // the register-resident segments, then the longer ones
-      const uint32_t regs_hi = max_values < kWaveRegValues ? max_values : kWaveRegValues;
-      NTS_FWD(true, true, 1, min_values, regs_hi);
+      NTS_FWD(true, true, 1, min_values, kWaveRegValues);
       // 513 .. 2,048 values in a launch of their own: 16 or 32 values per lane in registers, one pass over
       // memory, and the registers that costs are not the other classes' (64 per lane measured slower)
-      if (max_values > kWaveRegValues) {
-        const uint32_t mid_hi = max_values < kWaveMidValues ? max_values : kWaveMidValues;
-        NTS_FWD(true, true, 3, kWaveRegValues + 1, mid_hi);
-        if (max_values > kWaveMidValues) NTS_FWD(true, true, 2, kWaveMidValues + 1, max_values);
-      }
+      NTS_FWD(true, true, 3, kWaveRegValues + 1, kWaveMidValues);
+      NTS_FWD(true, true, 2, kWaveMidValues + 1, max_values);
     } else if (pow2) {
       NTS_FWD(false, true, 0, min_values, max_values);
     } else {
@@ -2404,11 +2428,10 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   hipLaunchKernelGGL((edge_softmax_bwd_kernel<FU, P2, PART>), grid, block, 0, stream, out, ger, x_or_gy, y, el, er, co, \
                      ri, Vd, H, slope, LO, HI, vec4)
     if (pow2 && fused) {
-      const uint32_t regs_hi = max_values < kWaveRegValues ? max_values : kWaveRegValues;
-      NTS_BWD(true, true, 1, min_values, regs_hi);
+      NTS_BWD(true, true, 1, min_values, kWaveRegValues);
       // (a launch of its own for the class above that, held in registers as in the forward pass, measured no
       // gain up to 1,024 values and 3.36 -> 3.57 ms up to 2,048: the backward holds two arrays per lane)
-      if (max_values > kWaveRegValues) NTS_BWD(true, true, 2, kWaveRegValues + 1, max_values);
+      NTS_BWD(true, true, 2, kWaveRegValues + 1, max_values);
     } else if (pow2) {
       NTS_BWD(false, true, 0, min_values, max_values);
     } else {
