@@ -1160,25 +1160,44 @@ __global__ __launch_bounds__(256) void auto_fill_kernel(Item *__restrict__ items
   if (i < p_max) items[i] = make_uint4(0u, 0u, 0u, i);
 }
 
-__global__ __launch_bounds__(256) void auto_cut_kernel(Item *__restrict__ items, uint4 *__restrict__ splits,
-                                                       uint32_t *__restrict__ ctr, const uint32_t *__restrict__ off,
-                                                       uint32_t rows, uint32_t chunk, uint32_t p_max, uint32_t s_max) {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
-  const uint32_t b = off[r], e = off[r + 1], deg = e - b;
-  if (deg <= chunk) return;
-  uint32_t n = (deg + chunk - 1) / chunk;
-  const uint32_t first = atomicAdd(&ctr[0], n);
+// A block asks for the slots of its 1,024 rows at once, because requests to one counter are served some 10 ns apart, and
+// the lanes of a wavefront write its rows' pieces one each, wherever they belong: a hub row of 20,000 edges is 80
+// pieces, which one thread wrote one after the other (2.48 M edges, 169 K rows: 20.7 -> 7.6 us,
+// 12.4 with a request per wavefront).
+constexpr int kCutBlock = 1024;
+__global__ __launch_bounds__(kCutBlock) void auto_cut_kernel(Item *__restrict__ items, uint4 *__restrict__ splits,
+                                                             uint32_t *__restrict__ ctr,
+                                                             const uint32_t *__restrict__ off, uint32_t rows,
+                                                             uint32_t chunk, uint32_t p_max, uint32_t s_max) {
+  __shared__ uint32_t wave_sums[kCutBlock / kWave], slot_of_block, list_of_block;
+  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & (kWave - 1);
+  const uint32_t b = off[r < rows ? r : rows], e = off[r < rows ? r + 1 : rows], deg = e - b;
+  const uint32_t n = deg > chunk ? (deg + chunk - 1) / chunk : 0u;
+  uint32_t n_pieces = 0, n_rows = 0;
+  const uint32_t piece = block_prefix<kCutBlock>(n, wave_sums, &n_pieces);  // pieces and cut rows before this one
+  const uint32_t nth = block_prefix<kCutBlock>(n != 0 ? 1u : 0u, wave_sums, &n_rows);
+  if (n_rows == 0) return;
+  if (threadIdx.x == 0) {
+    slot_of_block = atomicAdd(&ctr[0], n_pieces);
+    list_of_block = atomicAdd(&ctr[1], n_rows);
+  }
+  __syncthreads();
   // Slots at or beyond p_max do not exist (only possible when the caller's edge count is smaller than
   // offsets[rows]): such pieces are not created and not read.
-  if (first >= p_max) return;
-  if (first + n > p_max) n = p_max - first;
-  for (uint32_t j = 0; j < n; ++j) {
-    const uint32_t e0 = b + j * chunk;
-    items[first + j] = make_uint4(r, e0, min(e, e0 + chunk), first + j);
+  const uint32_t first = slot_of_block + piece, s = list_of_block + nth;
+  if (n != 0 && first < p_max && s < s_max) splits[s] = make_uint4(r, first, min(n, p_max - first), 0u);
+  const uint32_t wave_first_slot = wave_read(first, 0), upto = first + n - wave_first_slot;
+  const uint32_t total = wave_read(upto, kWave - 1);
+  for (uint32_t t0 = 0; t0 < total; t0 += kWave) {
+    const uint32_t t = t0 + lane;
+    uint32_t own = 0;  // lanes whose pieces all lie before piece t
+#pragma unroll
+    for (uint32_t step = kWave / 2; step >= 1; step >>= 1)
+      if (__shfl(upto, own + step - 1, kWave) <= t) own += step;
+    const uint32_t before = __shfl(upto - n, own, kWave), rb = __shfl(b, own, kWave), re = __shfl(e, own, kWave);
+    const uint32_t at = wave_first_slot + t, e0 = rb + (t - before) * chunk;
+    if (t < total && at < p_max) items[at] = make_uint4(r - lane + own, e0, min(re, e0 + chunk), at);
   }
-  const uint32_t s = atomicAdd(&ctr[1], 1u);
-  if (s < s_max) splits[s] = make_uint4(r, first, n, 0u);
 }
 
 // Block (x, y): adds the partials of listed row x in slot order into out (256 columns per block, tile y).
@@ -1234,7 +1253,7 @@ int launch_spmm_cut_small(const LaunchArgs &a, uint32_t edges, unsigned char *fi
   uint4 *splits = reinterpret_cast<uint4 *>(buf + 256 + n_items_b);
   float *partial = reinterpret_cast<float *>(buf + 256 + n_items_b + n_splits_b);
   hipLaunchKernelGGL(auto_fill_kernel, dim3(ceil_div(p_max, 256)), dim3(256), 0, a.stream, items, ctr, p_max);
-  hipLaunchKernelGGL(auto_cut_kernel, dim3(ceil_div(rows, 256)), dim3(256), 0, a.stream, items, splits, ctr, a.offsets,
+  hipLaunchKernelGGL(auto_cut_kernel, dim3(ceil_div(rows, kCutBlock)), dim3(kCutBlock), 0, a.stream, items, splits, ctr, a.offsets,
                      rows, chunk, p_max, s_max);
   LaunchArgs pc = a;
   pc.n_items = p_max;
