@@ -6,6 +6,8 @@
 // degree); per-destination reductions give one wavefront to one destination (or source) row, lanes
 // spanning the feature / head dimension.  Sums run in edge order or through fixed-shape cross-lane
 // butterflies, and nothing uses float atomics, so every result is bit-reproducible.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace nts {
@@ -497,7 +499,7 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
 }
 
 // The same sums for rows that fit one group (Fv <= G), with the rows of a wavefront handed out
-// dynamically: a wavefront takes 64 consecutive rows, reads their offsets with one coalesced load,
+// dynamically: a wavefront takes `set` (at most 64) consecutive rows, reads their offsets with one coalesced load,
 // and its 64/G groups then pull rows from that set one after the other -- a group that finishes a
 // short row takes the next pending one instead of idling until the longest row of a fixed
 // assignment is done.  Every group adds its row's edge rows in order (eight loads in flight), so
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
                                                                           const uint32_t *__restrict__ perm,
                                                                           uint32_t rows, uint32_t Fv, int accumulate,
                                                                           uint32_t long_limit, uint32_t coop_limit,
-                                                                          LongRowWork<V> lw) {
+                                                                          uint32_t set, LongRowWork<V> lw) {
   if (blockIdx.x < lw.blocks) {
     sum_long_rows_in_this_block(out, msg, off, perm, Fv, accumulate, lw);
     return;
@@ -532,9 +534,6 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
   constexpr int kCoopU = sizeof(V) == 16 ? 4 : 8;           // loads per lane and round on the cooperative path
   constexpr uint32_t kCoopFloats = kWave * kCoopU * (sizeof(V) / 4);  // floats of a wavefront's tile
   __shared__ float coop_tile[kCoop ? 4 : 1][kCoop ? kCoopFloats : 1];
-  // Rows a wavefront takes at a time: eight per lane group, so that a wavefront with two groups
-  // (128-byte-wide vectors) is not left with 32 rows per group while others have finished.
-  constexpr uint32_t kSet = (kWave / (G * S)) * 8 < kWave ? (kWave / (G * S)) * 8 : kWave;
   constexpr int NF = sizeof(V) / 4;
   const uint32_t lane = lane_id();
   constexpr int GG = G * S;  // lanes that share a row
@@ -544,10 +543,10 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x - lw.blocks) * blockDim.x / kWave;
   const bool col_live = col < Fv;
   const bool streamed = outgrows_caches(static_cast<uint64_t>(off[rows] - off[0]) * Fv * sizeof(V));
-  for (uint64_t base = wave * kSet; base < rows; base += n_waves * kSet) {
+  for (uint64_t base = wave * set; base < rows; base += n_waves * set) {
     uint32_t my_e0 = 0, my_e1 = 0;
     bool mine = false;
-    if (lane < kSet && base + lane < rows) {
+    if (lane < set && base + lane < rows) {
       my_e0 = off[base + lane];
       my_e1 = off[base + lane + 1];
       mine = my_e1 - my_e0 <= long_limit;  // longer rows belong to the block kernels
@@ -2093,6 +2092,18 @@ uint32_t streamed_rows_per_wave(uint32_t rows) {
   return per;
 }
 
+// Rows that a wavefront of the permuted sums hands out at a time: eight per lane group, so that a wavefront with two
+// groups (128-byte-wide vectors) is not left with 32 rows per group while others have finished, and fewer, down to eight,
+// where that leaves the chip without its 8,192 wavefronts.  us, always eight per group / so: 16.5 K rows, 300 K edges F = 4
+// 69 / 46, F = 16 133 / 54, F = 128 214 / 206; 100 K, 8 M F = 1 209 / 172, F = 32 682 / 411; 169 K, 2.48 M F = 1 78 / 67, F = 32
+// 193 / 145 (not below 16 rows: 16.5 K F = 16 68, 100 K F = 32 441); from 524,288 rows up the same.
+uint32_t balanced_rows_per_wave(uint32_t rows, uint32_t lanes) {
+  constexpr uint32_t kChipWaves = 8192;
+  uint32_t set = std::min<uint32_t>(kWave / lanes * 8, kWave);
+  while (set > 8 && rows / set < kChipWaves) set /= 2;
+  return set;
+}
+
 template <typename V>
 void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_t *perm, uint32_t rows, uint32_t Fv,
                         int accumulate, uint32_t limit, const LongRowWork<V> &lw, hipStream_t stream) {
@@ -2118,11 +2129,11 @@ void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_
     // One group covers a row: wavefronts hand their 64 rows out dynamically (strided launch).
 #define NTS_BALANCED(GG, SS)                                                                                    \
   do {                                                                                                          \
-    const uint32_t set = (kWave / ((GG) * (SS))) * 8 < kWave ? (kWave / ((GG) * (SS))) * 8 : kWave;            \
+    const uint32_t set = balanced_rows_per_wave(rows, (GG) * (SS));                                            \
     const uint32_t blocks = ceil_div(rows, 4 * set); /* at most `set` rows per wavefront at a time */          \
     hipLaunchKernelGGL((gather_edge_to_row_balanced_kernel<V, GG, SS>),                                         \
                        dim3((blocks < 16384u ? blocks : 16384u) + lw.blocks), dim3(256), 0, stream, out, msg, off, \
-                       perm, rows, Fv, accumulate, limit, coop_limit(), lw);                                    \
+                       perm, rows, Fv, accumulate, limit, coop_limit(), set, lw);                                   \
   } while (0)
     switch (lanes_for(Fv)) {  // rows narrower than eight lanes are shared by eight lanes all the same
       case 1: NTS_BALANCED(1, 8); break;

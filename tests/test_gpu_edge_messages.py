@@ -68,3 +68,22 @@ def test_streamed_sums_at_the_steps_of_rows_a_wavefront(device, rows, F):
          torch.cuda.current_stream().cuda_stream)
     own = torch.repeat_interleave(torch.arange(rows, device=device), off[1:] - off[:-1])
     assert torch.equal(out, torch.zeros(rows, F, device=device).index_add_(0, own, msg))
+
+
+@pytest.mark.parametrize("rows", [4096, 65535, 65537, 131071, 262143, 524288])
+@pytest.mark.parametrize("F", [1, 8, 33, 128])
+def test_permuted_sums_at_the_steps_of_rows_a_wavefront(device, rows, F):
+    """8 to 64 rows a wavefront, by the number of rows and their width; whole numbers, so that any order is exact."""
+    rng = np.random.default_rng(rows + F)
+    deg = rng.integers(0, 4, rows)
+    deg[rng.integers(0, rows, 20)] = rng.integers(60, 2000, 20)
+    off = torch.from_numpy(np.concatenate([[0], np.cumsum(deg)])).to(device)
+    E = int(off[-1])
+    msg = torch.randint(-8, 9, (E, F), device=device).float()
+    perm = torch.randperm(E, device=device)
+    off32, perm32 = off.to(torch.int32), perm.to(torch.int32)
+    out = torch.full((rows, F), 3.0, device=device)
+    call("nts_gather_edge_to_src", ptr(out), ptr(msg), ptr(off32), ptr(perm32), rows, F, 0,
+         torch.cuda.current_stream().cuda_stream)
+    own = torch.repeat_interleave(torch.arange(rows, device=device), off[1:] - off[:-1])
+    assert torch.equal(out, torch.zeros(rows, F, device=device).index_add_(0, own, msg[perm]))
