@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void spmm_wave_kernel(const float *__restrict_
                                                         const uint32_t *__restrict__ offsets,
                                                         const uint32_t *__restrict__ indices, uint32_t index_base,
                                                         uint32_t n_items, uint32_t n_list, uint32_t F,
-                                                        uint32_t col_base, const Item *__restrict__ items,
+                                                        uint32_t first_col, uint32_t panels, const Item *__restrict__ items,
                                                         float *__restrict__ partial,
                                                         int accumulate, HeadArgs heads, uint32_t row_edge_limit,
                                                         const uint32_t *__restrict__ edge_ids, uint32_t in_ld,
@@ -156,7 +156,8 @@ __global__ __launch_bounds__(256) void spmm_wave_kernel(const float *__restrict_
   using V = typename Vec<VEC>::type;
   constexpr int U = unroll_for(NACC, VEC);
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  const uint32_t item = blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
+  const uint32_t col_base = first_col + blockIdx.x % panels * (kWave * VEC * NACC);
+  const uint32_t item = blockIdx.x / panels * (blockDim.x / kWave) + (threadIdx.x / kWave);
   if (item >= n_items) return;
 
   // Work items [0, n_list) come from the list, the ones after it are the rows 0, 1, ... themselves
@@ -365,11 +366,12 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
                                                          const Item *__restrict__ items, float *__restrict__ partial,
                                                          int accumulate, HeadArgs heads,
                                                          uint32_t row_edge_limit,
-                                                         const uint32_t *__restrict__ edge_ids) {
+                                                         const uint32_t *__restrict__ edge_ids, uint32_t panels) {
   using V = typename Vec<VEC>::type;
   constexpr int U = G >= 8 ? 8 : 4;  // edges per step: their rows are requested together
   const uint32_t gl = threadIdx.x & (G - 1);
-  const uint32_t item = (blockIdx.x * blockDim.x + threadIdx.x) / G;
+  const uint32_t panel = blockIdx.x % panels;
+  const uint32_t item = (blockIdx.x / panels * blockDim.x + threadIdx.x) / G;
   if (item >= n_items) return;  // whole groups leave together; shuffles stay inside a group
 
   uint32_t row, e0, e1, slot;
@@ -386,7 +388,7 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
     slot = kNoSlot;
     if (e1 - e0 > row_edge_limit) return;  // a long row: its pieces are separate work items
   }
-  const uint32_t col = gl * VEC;
+  const uint32_t col = (panel * G + gl) * VEC;
   const bool live = col < F;
   const uint32_t lcol = live ? col : F - VEC;  // idle lanes re-read the last columns, never store
   const uint32_t head = HEADS ? lcol / heads.Fh : 0u;
@@ -829,6 +831,7 @@ struct LaunchArgs {
   uint32_t in_ld = 0;                          // row stride of `in` in floats (0 = F)
   uint32_t partial_ld = 0;                     // row stride of `partial` in floats (0 = F)
   bool dup_runs = false;                       // rows hold runs of equal indices worth loading once per run
+  uint32_t scheduled_rows = 0;                 // rows of the schedule that `items` comes from (0: no schedule)
   uint32_t rows_after_items = 0;               // with items: this many whole rows follow the listed items in the launch
   const float *dot_rows = nullptr;             // with dot_out: the rows whose products with the gathered ones
   float *dot_out = nullptr;                    // are the gradient of alpha (attention_grad_kernel)
@@ -883,16 +886,16 @@ void launch_attention_grad(const LaunchArgs &a) {
 }
 
 template <int VEC, int NACC>
-void launch_wave(const LaunchArgs &a, uint32_t col_base) {
+void launch_wave(const LaunchArgs &a, uint32_t col_base, uint32_t panels) {
   constexpr int kWavesPerBlock = 4;
   const uint32_t n_list = a.items ? a.n_items : 0u, n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
   const uint32_t blocks = ceil_div(n_total, kWavesPerBlock);
-  const dim3 grid(blocks), block(kWavesPerBlock * kWave);
+  const dim3 grid(blocks * panels), block(kWavesPerBlock * kWave);
   // Neighbour pairs always go through the wave-private LDS tile (a register-broadcast variant measured
   // the same: 12.44 ms against 12.40 ms for the 114.8 M-edge F=602 gather).
 #define NTS_LAUNCH_WAVE(HD, RM, RUNS)                                                                                  \
   hipLaunchKernelGGL((spmm_wave_kernel<VEC, NACC, true, HD, RM, RUNS>), grid, block, 0, a.stream, a.in, a.out, a.w,    \
-                     a.offsets, a.indices, a.index_base, n_total, n_list, a.F, col_base, a.items, a.partial,         \
+                     a.offsets, a.indices, a.index_base, n_total, n_list, a.F, col_base, panels, a.items, a.partial, \
                      a.accumulate,                                                                                     \
                      a.heads, a.row_edge_limit, a.edge_ids, a.in_ld ? a.in_ld : a.F,                                  \
                      a.partial_ld ? a.partial_ld : a.F,                                                                \
@@ -910,15 +913,15 @@ void launch_wave(const LaunchArgs &a, uint32_t col_base) {
 }
 
 template <int G, int VEC>
-void launch_group(const LaunchArgs &a) {
+void launch_group(const LaunchArgs &a, uint32_t panels = 1) {
   const uint32_t per_block = 256 / G;
   const uint32_t n_list = a.items ? a.n_items : 0u, n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
-  const uint32_t blocks = ceil_div(n_total, per_block);
+  const uint32_t blocks = ceil_div(n_total, per_block) * panels;
 #define NTS_LAUNCH_GROUP(HD, RM, RUNS)                                                                                  \
   hipLaunchKernelGGL((spmm_group_kernel<G, VEC, HD, RM, RUNS>), dim3(blocks), dim3(256), 0, a.stream, a.in, a.out, a.w, \
                      a.offsets, a.indices, a.index_base, n_total, n_list, a.F, a.items, a.partial, a.accumulate,        \
                      a.heads,                                                                                          \
-                     a.row_edge_limit, a.edge_ids)
+                     a.row_edge_limit, a.edge_ids, panels)
   if (a.edge_ids) {
     if (a.heads.H) NTS_LAUNCH_GROUP(true, true, false);
     else if (a.dup_runs) NTS_LAUNCH_GROUP(false, true, true);
@@ -931,32 +934,40 @@ void launch_group(const LaunchArgs &a) {
 #undef NTS_LAUNCH_GROUP
 }
 
+constexpr uint32_t kChipWaves = 8192;                      // wavefronts that the chip holds
+constexpr uint64_t kAllL2Bytes = 8ull * (4 << 20);         // the L2s of its eight XCDs
+
 template <int VEC>
 void launch_wave_vec(const LaunchArgs &a) {
   // Column panels of at most 10 accumulators per lane, balanced; wider rows are covered by several
-  // launches over disjoint column ranges (each panel re-walks the edge list; outputs are disjoint).
+  // launches over disjoint column ranges (each panel re-walks the edge list; outputs are disjoint), or, where one
+  // panel does not fill the chip, by one launch whose blocks alternate between them.  us, apart / together, F = 1,433: 2.7 K
+  // items 32 / 18, 5.2 K 35 / 23, 8.8 K 44 / 40, 21 K 78 / 86 (all panels of a row at once need more of the caches), 172 K 1,733 / 2,067.
   constexpr uint32_t kMaxAcc = 10;
   const uint32_t per_acc = kWave * VEC;
   const uint32_t total_acc = ceil_div(a.F, per_acc);
   const uint32_t panels = ceil_div(total_acc, kMaxAcc);
   const uint32_t acc_per_panel = ceil_div(total_acc, panels);
+  const uint32_t n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
+  const bool together = panels > 1 && n_total <= kChipWaves;
   uint32_t col_base = 0;
   while (col_base < a.F) {
     const uint32_t remaining = a.F - col_base;
     uint32_t nacc = ceil_div(remaining, per_acc);
     if (nacc > acc_per_panel) nacc = acc_per_panel;
     switch (nacc) {
-      case 1: launch_wave<VEC, 1>(a, col_base); break;
-      case 2: launch_wave<VEC, 2>(a, col_base); break;
-      case 3: launch_wave<VEC, 3>(a, col_base); break;
-      case 4: launch_wave<VEC, 4>(a, col_base); break;
-      case 5: launch_wave<VEC, 5>(a, col_base); break;
-      case 6: launch_wave<VEC, 6>(a, col_base); break;
-      case 7: launch_wave<VEC, 7>(a, col_base); break;
-      case 8: launch_wave<VEC, 8>(a, col_base); break;
-      case 9: launch_wave<VEC, 9>(a, col_base); break;
-      default: launch_wave<VEC, 10>(a, col_base); break;
+      case 1: launch_wave<VEC, 1>(a, col_base, together ? panels : 1u); break;
+      case 2: launch_wave<VEC, 2>(a, col_base, together ? panels : 1u); break;
+      case 3: launch_wave<VEC, 3>(a, col_base, together ? panels : 1u); break;
+      case 4: launch_wave<VEC, 4>(a, col_base, together ? panels : 1u); break;
+      case 5: launch_wave<VEC, 5>(a, col_base, together ? panels : 1u); break;
+      case 6: launch_wave<VEC, 6>(a, col_base, together ? panels : 1u); break;
+      case 7: launch_wave<VEC, 7>(a, col_base, together ? panels : 1u); break;
+      case 8: launch_wave<VEC, 8>(a, col_base, together ? panels : 1u); break;
+      case 9: launch_wave<VEC, 9>(a, col_base, together ? panels : 1u); break;
+      default: launch_wave<VEC, 10>(a, col_base, together ? panels : 1u); break;
     }
+    if (together) return;
     col_base += nacc * per_acc;
   }
 }
@@ -981,6 +992,21 @@ int pick_vec(const LaunchArgs &a) {
   return 1;
 }
 
+// Column panels whose blocks alternate, so that an XCD (blocks are dealt out to the eight in turn) meets one panel only and
+// its 4 MB L2 holds a share of the gathered matrix that is as many times smaller.  A panel has to be whole lines (512
+// bytes, or 256 of a row of 512) and the number of panels has to divide eight; shorter requests cost more than they gain (64 bytes:
+// 2.8 times the time, 128: as much as without), and so do panels that share lines.  us without / with: 169 K rows, 2.48 M
+// edges F = 128 111 / 98, 256 251 / 221, 512 584 / 451; 500 K, 20 M with source ranges 722 / 690, 1,437 / 1,388, 3,137 /
+// 2,746; 2.45 M, 126 M 5,221 / 5,108, 11,255 / 10,386; F = 300, 384 and 500 as panels of 128 331 / 404, 396 / 424, 609 / 526
+// and 1,968 / 2,312, 2,249 / 2,362, 3,330 / 3,071.  Rows of 512 bytes that the L2s hold together lose (20 K rows, 4 M edges 93 / 95), rows
+// loaded once per run of equal indices (233 K, 114.8 M F = 128 2,277 / 2,346), heads (169 K 155 / 199: the weights are read
+// once a panel) and calls without a schedule (133 / 149: mostly short rows) too.
+uint32_t die_panels(const LaunchArgs &a, int vec) {
+  if (vec != 4 || !a.scheduled_rows || a.heads.H || a.dup_runs || a.in_ld) return 0;
+  if (a.F == 128) return static_cast<uint64_t>(a.scheduled_rows) * a.F * sizeof(float) > kAllL2Bytes ? 2 : 0;
+  return a.F == 256 ? 2 : a.F == 512 ? 4 : 0;
+}
+
 void launch_spmm(const LaunchArgs &a) {
   if (a.n_items == 0) return;
   if (a.dot_out) {
@@ -990,6 +1016,7 @@ void launch_spmm(const LaunchArgs &a) {
   }
   const int vec = pick_vec(a);
   const uint32_t F = a.F;
+  if (const uint32_t panels = die_panels(a, vec)) return F == 128 ? launch_group<16, 4>(a, panels) : launch_group<32, 4>(a, panels);
   // Narrow rows: sub-wavefront groups so that lanes are not left idle.
   if (vec == 4 && F <= 16) return launch_group<4, 4>(a);
   if (vec == 4 && F <= 32) return launch_group<8, 4>(a);
@@ -2617,6 +2644,7 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
     a.edge_ids = plan->edge_ids;
   }
   a.dup_runs = use_runs(plan);
+  a.scheduled_rows = plan->rows;
   if (const uint32_t ld = padded_stride(plan, F, false)) {
     // Rows off 16-byte boundaries: gather from a padded copy with 16-byte lanes.
     const uint64_t vecs = static_cast<uint64_t>(plan->n_index) * (ld / 4);

@@ -1,0 +1,56 @@
+"""Scheduled aggregation in column panels: rows of 128, 256 and 512 floats, whose blocks alternate between panels, and
+rows of more than 640 four-byte lanes, whose panels are one launch while the items are few.  The panels of an item add
+the same edges in the same order as one pass over narrower rows does, so the columns that both have are equal bit by bit."""
+import pytest
+import torch
+
+from neutronbench_amd import synth
+from neutronbench_amd.abi import call, ptr
+from neutronbench_amd.layout import SpmmPlan
+
+pytestmark = pytest.mark.gpu
+
+
+def graph(rows, edges, seed, device, rising):
+    src, dst = synth.rmat_edges(rows, edges, seed=seed, device=device, sort=True)
+    order = torch.sort(dst, stable=True).indices
+    idx = src[order].to(torch.int32)
+    off = torch.zeros(rows + 1, dtype=torch.int64, device=device)
+    off[1:] = torch.bincount(dst, minlength=rows).cumsum(0)
+    if not rising:  # rows that do not ascend are gathered through the schedule's own copy of the indices
+        idx = idx.flip(0)
+        off = off[-1] - off.flip(0)
+    return off.to(torch.int32), idx.contiguous()
+
+
+# 65,536 rows of 512 bytes are what the L2s hold together; ranges 1 and 8, one of them over rows that do not ascend
+@pytest.mark.parametrize("rows,edges,ranges,rising", [(65536, 300000, 1, True), (65537, 300000, 1, True),
+                                                      (70001, 900000, 8, True), (70001, 900000, 8, False)])
+@pytest.mark.parametrize("F", [128, 256, 512])
+def test_panels_of_whole_lines(device, rows, edges, ranges, rising, F):
+    off, idx = graph(rows, edges, 7, device, rising)
+    plan = SpmmPlan(off, rows, edges, 64, idx, rows, ranges) if ranges > 1 else SpmmPlan(off, rows, edges, 64)
+    compare(device, plan, off, idx, rows, edges, F, F - 4)
+
+
+# 8,192 items are what the chip holds; 640 columns are one panel of 4-byte lanes, 2,560 of 16-byte lanes
+@pytest.mark.parametrize("rows", [100, 8191, 8192, 8193])
+@pytest.mark.parametrize("F,narrow", [(641, 639), (1433, 637), (2564, 2560)])
+def test_wide_rows(device, rows, F, narrow):
+    edges = 3 * rows
+    off, idx = graph(rows, edges, 5, device, True)
+    compare(device, SpmmPlan(off, rows, edges, 4096), off, idx, rows, edges, F, narrow)
+
+
+def compare(device, plan, off, idx, rows, edges, F, narrow):
+    g = torch.Generator(device=device).manual_seed(F)
+    x, w = torch.randn(rows, F, generator=g, device=device), torch.rand(edges, generator=g, device=device)
+    s = torch.cuda.current_stream().cuda_stream
+    for accumulate in (0, 1):
+        init = torch.randn(rows, F, generator=g, device=device)
+        full = init.clone() if accumulate else torch.full((rows, F), float("nan"), device=device)
+        call("nts_spmm_gather_planned", plan.handle, ptr(x), ptr(full), ptr(w), ptr(off), ptr(idx), 0, F, accumulate, s)
+        for c0 in (0, F - narrow):
+            part, xs = init[:, c0:c0 + narrow].contiguous(), x[:, c0:c0 + narrow].contiguous()
+            call("nts_spmm_gather_planned", plan.handle, ptr(xs), ptr(part), ptr(w), ptr(off), ptr(idx), 0, narrow, accumulate, s)
+            assert torch.equal(full[:, c0:c0 + narrow], part)
