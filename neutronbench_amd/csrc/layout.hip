@@ -10,11 +10,13 @@
 #include <rocprim/iterator/transform_iterator.hpp>
 
 #include "common.hpp"
+#include "edge_sort.hpp"
 
 namespace nts {
 namespace {
 
-// ro[s] = number of sorted keys < s, for s in [0, Vs]; keys ascending, E of them.
+// ro[s] = number of sorted keys < s, for s in [0, Vs]; keys ascending, E of them, STEP words apart.
+template <int STEP>
 __global__ __launch_bounds__(256) void offsets_from_sorted_kernel(uint32_t *__restrict__ ro,
                                                                   const uint32_t *__restrict__ keys, DevCount Vs,
                                                                   DevCount E) {
@@ -23,7 +25,7 @@ __global__ __launch_bounds__(256) void offsets_from_sorted_kernel(uint32_t *__re
   uint32_t lo = 0, hi = E.get();  // first position whose key >= s
   while (lo < hi) {
     const uint32_t mid = lo + (hi - lo) / 2;
-    if (keys[mid] < s) lo = mid + 1; else hi = mid;
+    if (keys[static_cast<size_t>(mid) * STEP] < s) lo = mid + 1; else hi = mid;
   }
   ro[s] = lo;
 }
@@ -568,6 +570,7 @@ int nts_csr_from_csc(uint32_t *ro, uint32_t *ci, uint32_t *perm, const uint32_t 
 
 size_t nts_chunk_from_edges_work_bytes(uint32_t V, uint32_t E) {
   (void)V;
+  if (E >= kTiledSortEdges) return 2 * align_up(static_cast<size_t>(E) * sizeof(SortElement), 256) + sort_table_bytes(E) + 256;
   size_t tmp = 0;
   if (sort_pairs_temp_bytes(E, &tmp) != hipSuccess) return 0;
   return 3 * align_up(static_cast<size_t>(E) * sizeof(uint32_t), 256) + align_up(tmp, 256) + 256;
@@ -585,27 +588,49 @@ int nts_chunk_from_edges(uint32_t *co, uint32_t *ri, float *ewf, uint32_t *ro, u
   if (!ri || !ci || !pairs || !work) return fail(NTS_ERR_INVALID, "nts_chunk_from_edges: null pointer");
   if (!aligned_to(work, 256) || !aligned_to(pairs, 8))
     return fail(NTS_ERR_INVALID, "nts_chunk_from_edges: work must be 256-byte and pairs 8-byte aligned");
-  const size_t arr = align_up(static_cast<size_t>(E) * sizeof(uint32_t), 256);
   unsigned char *w = static_cast<unsigned char *>(work);
-  uint32_t *a = reinterpret_cast<uint32_t *>(w);            // file-order sources, later destination-sorted keys
-  uint32_t *b = reinterpret_cast<uint32_t *>(w + arr);      // file-order destinations
-  uint32_t *c = reinterpret_cast<uint32_t *>(w + 2 * arr);  // sources in (source, file) order
-  void *tmp_ptr = w + 3 * arr;
-  size_t tmp = 0;
-  NTS_HIP_TRY(sort_pairs_temp_bytes(E, &tmp));
   const unsigned bits = bits_for(V);
-  hipLaunchKernelGGL(split_pairs_kernel, dim3(ceil_div(E, 256)), dim3(256), 0, stream, a, b,
-                     reinterpret_cast<const uint2 *>(pairs), E);
-  NTS_LAUNCH_CHECK("split_pairs_kernel");
-  // The edge list ordered by source, file order kept inside a source (stable sort): the CSR rows.
-  NTS_HIP_TRY(rocprim::radix_sort_pairs(tmp_ptr, tmp, a, c, b, ci, E, 0u, bits, stream, false));
-  hipLaunchKernelGGL(offsets_from_sorted_kernel, dim3(ceil_div(static_cast<uint64_t>(V) + 1, 256)), dim3(256), 0,
-                     stream, ro, c, host_count(V), host_count(E));
-  NTS_LAUNCH_CHECK("offsets_from_sorted_kernel(ro)");
-  // That list re-ordered by destination, again stable: the CSC rows (sources ascending inside a row).
-  NTS_HIP_TRY(rocprim::radix_sort_pairs(tmp_ptr, tmp, ci, a, c, ri, E, 0u, bits, stream, false));
-  hipLaunchKernelGGL(offsets_from_sorted_kernel, dim3(ceil_div(static_cast<uint64_t>(V) + 1, 256)), dim3(256), 0,
-                     stream, co, a, host_count(V), host_count(E));
+  const dim3 grid(ceil_div(static_cast<uint64_t>(V) + 1, 256));
+  const uint32_t *destinations;  // of the CSC's edges
+  // The edge list ordered by source, file order kept inside a source (stable sort): the CSR rows; and that list
+  // re-ordered by destination, again stable: the CSC rows (sources ascending inside a row).
+  if (E >= kTiledSortEdges) {
+    // A record of the file is an element, its source in the low half.
+    const size_t arr = align_up(static_cast<size_t>(E) * sizeof(SortElement), 256);
+    SortElement *a = reinterpret_cast<SortElement *>(w), *b = reinterpret_cast<SortElement *>(w + arr), *by_source = nullptr;
+    NTS_HIP_TRY(sort_elements(reinterpret_cast<const SortElement *>(pairs), a, b, E, 0, bits, w + 2 * arr, stream,
+                              [&](SortElement *to) {
+                                by_source = to;
+                                return SortSplit{to, nullptr, ci};
+                              }));
+    hipLaunchKernelGGL(offsets_from_sorted_kernel<2>, grid, dim3(256), 0, stream, ro,
+                       reinterpret_cast<const uint32_t *>(by_source), host_count(V), host_count(E));
+    NTS_LAUNCH_CHECK("offsets_from_sorted_kernel(ro)");
+    uint32_t *keys = nullptr;
+    NTS_HIP_TRY(sort_elements(by_source, a, b, E, 32, bits, w + 2 * arr, stream, [&](SortElement *to) {
+      keys = reinterpret_cast<uint32_t *>(to);
+      return SortSplit{nullptr, ri, keys};
+    }));
+    destinations = keys;
+  } else {
+    const size_t arr = align_up(static_cast<size_t>(E) * sizeof(uint32_t), 256);
+    uint32_t *a = reinterpret_cast<uint32_t *>(w);            // file-order sources, later destination-sorted keys
+    uint32_t *b = reinterpret_cast<uint32_t *>(w + arr);      // file-order destinations
+    uint32_t *c = reinterpret_cast<uint32_t *>(w + 2 * arr);  // sources in (source, file) order
+    void *tmp_ptr = w + 3 * arr;
+    size_t tmp = 0;
+    NTS_HIP_TRY(sort_pairs_temp_bytes(E, &tmp));
+    hipLaunchKernelGGL(split_pairs_kernel, dim3(ceil_div(E, 256)), dim3(256), 0, stream, a, b,
+                       reinterpret_cast<const uint2 *>(pairs), E);
+    NTS_LAUNCH_CHECK("split_pairs_kernel");
+    NTS_HIP_TRY(rocprim::radix_sort_pairs(tmp_ptr, tmp, a, c, b, ci, E, 0u, bits, stream, false));
+    hipLaunchKernelGGL(offsets_from_sorted_kernel<1>, grid, dim3(256), 0, stream, ro, c, host_count(V), host_count(E));
+    NTS_LAUNCH_CHECK("offsets_from_sorted_kernel(ro)");
+    NTS_HIP_TRY(rocprim::radix_sort_pairs(tmp_ptr, tmp, ci, a, c, ri, E, 0u, bits, stream, false));
+    destinations = a;
+  }
+  hipLaunchKernelGGL(offsets_from_sorted_kernel<1>, grid, dim3(256), 0, stream, co, destinations, host_count(V),
+                     host_count(E));
   NTS_LAUNCH_CHECK("offsets_from_sorted_kernel(co)");
   if (ewf || ewb) return nts_gcn_edge_weights(ewf, ewb, co, ri, ro, ci, V, V, stream);
   return NTS_OK;

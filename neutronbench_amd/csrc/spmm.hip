@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "edge_sort.hpp"
 
 // Fixed scratch of nts_spmm_gather_static_scratch, the entry point for callers that must not allocate:
 // each device that loads this library holds one copy of the array until the process ends.  Host code
@@ -1457,6 +1458,7 @@ struct PlanCounters {  // device words read back to the host
   uint32_t n_splits;
   uint32_t bad_offsets, bad_total;
   uint32_t first_edge;          // offsets[0]
+  uint32_t longest_row;
 };
 
 __device__ __forceinline__ uint32_t lower_bound_index(const uint32_t *__restrict__ idx, uint32_t lo, uint32_t hi,
@@ -1555,7 +1557,13 @@ __global__ __launch_bounds__(256) void plan_finish_kernel(Item *__restrict__ ite
 __global__ __launch_bounds__(256) void plan_check_offsets_kernel(const uint32_t *__restrict__ off, uint32_t rows,
                                                                  uint32_t edges, PlanCounters *__restrict__ counters) {
   const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ uint32_t longest;
+  if (threadIdx.x == 0) longest = 0;
+  __syncthreads();
   if (r < rows && off[r + 1] < off[r]) counters->bad_offsets = 1u;
+  else if (r < rows) atomicMax(&longest, off[r + 1] - off[r]);
+  __syncthreads();
+  if (threadIdx.x == 0) atomicMax(&counters->longest_row, longest);
   if (r == 0 && off[rows] != edges) counters->bad_total = 1u;
   if (r == 0) counters->first_edge = off[0];
 }
@@ -1626,13 +1634,14 @@ __global__ __launch_bounds__(256) void plan_scan_edges_kernel(const uint32_t *__
 }
 
 // Keys of the stable sort that orders the flagged rows by index and leaves every other row as it is:
-// (row, index) for an edge of a flagged row, (row, 0) otherwise.
+// (row, index) for an edge of a flagged row, (row, 0) otherwise; local_bits: the edge's place in its row below that, so that
+// the element sorted is all there is to move.
 __global__ __launch_bounds__(256) void plan_sort_keys_kernel(unsigned long long *__restrict__ keys,
                                                              const uint32_t *__restrict__ off,
                                                              const uint32_t *__restrict__ idx, uint32_t index_base,
                                                              uint32_t rows, uint32_t edges,
                                                              const unsigned char *__restrict__ unsorted,
-                                                             unsigned index_bits) {
+                                                             unsigned index_bits, unsigned local_bits) {
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
@@ -1646,10 +1655,27 @@ __global__ __launch_bounds__(256) void plan_sort_keys_kernel(unsigned long long 
   for (uint64_t step = first_step; step < end_step; ++step) {
     const uint32_t base = static_cast<uint32_t>(step * kWave), k = base + lane;
     const uint32_t own = owners_of_row_step(off, rows, base, row, row_end);
-    if (k < edges)
-      keys[k] = (static_cast<unsigned long long>(own) << index_bits) | (unsorted[own] ? (idx[k] - index_base) & mask : 0u);
+    if (k >= edges) continue;
+    const unsigned long long key =
+        (static_cast<unsigned long long>(own) << index_bits) | (unsorted[own] ? (idx[k] - index_base) & mask : 0u);
+    keys[k] = local_bits ? key << local_bits | (k - off[own]) : key;
   }
 }
+
+// The last pass of the sort of (row, index, place in the row) elements: the index array in the new order and every edge's
+// position in the caller's.  An edge of a row that is left as it is stays where it was.
+struct TakeSorted {
+  uint32_t *sorted_idx, *edge_ids;
+  const uint32_t *off, *idx;
+  const unsigned char *unsorted;
+  uint32_t index_base, index_mask;
+  unsigned index_bits, local_bits;
+  __device__ __forceinline__ void operator()(uint32_t at, SortElement v) const {
+    const uint32_t row = static_cast<uint32_t>(v >> local_bits >> index_bits);
+    edge_ids[at] = off[row] + (static_cast<uint32_t>(v) & ((1u << local_bits) - 1u));
+    sorted_idx[at] = unsorted[row] ? static_cast<uint32_t>(v >> local_bits) & index_mask : idx[at] - index_base;
+  }
+};
 
 // The index array in the new order.  An edge of an ordered row carries its index in its key; only the
 // other rows' are fetched through the edge ids (all of them: 1.0 ms for 114.8 M edges, scattered within
@@ -2165,11 +2191,16 @@ int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const
     const uint64_t index_range = host_counters.largest_index - index_base;  // 32-bit difference: at most 32 bits
     while (index_range >> index_bits) ++index_bits;
     while (static_cast<uint64_t>(rows - 1) >> row_bits) ++row_bits;
+    unsigned local_bits = 1;
+    while (static_cast<uint64_t>(host_counters.longest_row - 1) >> local_bits) ++local_bits;
+    // The sort of whole tiles where a row, an index and a place in the row fit an element.
+    const bool tiled = edges >= nts::kTiledSortEdges && row_bits + index_bits + local_bits <= 64 && local_bits < 32;
     unsigned long long *nul64 = nullptr;
-    size_t sort_edges_bytes = 0;
+    size_t sort_edges_bytes = nts::sort_table_bytes(edges);
     rocprim::counting_iterator<uint32_t> ids_in(0u);
-    NTS_HIP_TRY(rocprim::radix_sort_pairs(nullptr, sort_edges_bytes, nul64, nul64, ids_in, nul, edges, 0u,
-                                          index_bits + row_bits, stream, false));
+    if (!tiled)
+      NTS_HIP_TRY(rocprim::radix_sort_pairs(nullptr, sort_edges_bytes, nul64, nul64, ids_in, nul, edges, 0u,
+                                            index_bits + row_bits, stream, false));
     const size_t key_bytes = nts::up256(static_cast<size_t>(edges) * sizeof(unsigned long long));
     hipError_t taken = sorted_block.take(static_cast<size_t>(edges) * sizeof(uint32_t));
     if (taken == hipSuccess) taken = ids_block.take(static_cast<size_t>(edges) * sizeof(uint32_t));
@@ -2185,13 +2216,20 @@ int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const
     unsigned long long *keys = reinterpret_cast<unsigned long long *>(sort_bytes);
     unsigned long long *keys_out = reinterpret_cast<unsigned long long *>(sort_bytes + key_bytes);
     hipLaunchKernelGGL(nts::plan_sort_keys_kernel, dim3(edge_blocks), dim3(256), 0, stream, keys, offsets, indices,
-                       index_base, rows, edges, unsorted, index_bits);
+                       index_base, rows, edges, unsorted, index_bits, tiled ? local_bits : 0u);
     NTS_LAUNCH_CHECK("plan_sort_keys_kernel");
-    NTS_HIP_TRY(rocprim::radix_sort_pairs(sort_bytes + 2 * key_bytes, sort_edges_bytes, keys, keys_out, ids_in, edge_ids,
-                                          edges, 0u, index_bits + row_bits, stream, false));
-    hipLaunchKernelGGL(nts::plan_take_indices_kernel, dim3(edge_blocks), dim3(256), 0, stream, sorted_idx, keys_out,
-                       indices, index_base, edge_ids, edges, unsorted, index_bits);
-    NTS_LAUNCH_CHECK("plan_take_indices_kernel");
+    if (tiled) {
+      const nts::TakeSorted take{sorted_idx, edge_ids, offsets, indices, unsorted, index_base,
+                                 static_cast<uint32_t>((1ull << index_bits) - 1), index_bits, local_bits};
+      NTS_HIP_TRY(nts::sort_elements(keys, keys, keys_out, edges, local_bits, index_bits + row_bits,
+                                     sort_bytes + 2 * key_bytes, stream, [&](nts::SortElement *) { return take; }));
+    } else {
+      NTS_HIP_TRY(rocprim::radix_sort_pairs(sort_bytes + 2 * key_bytes, sort_edges_bytes, keys, keys_out, ids_in, edge_ids,
+                                            edges, 0u, index_bits + row_bits, stream, false));
+      hipLaunchKernelGGL(nts::plan_take_indices_kernel, dim3(edge_blocks), dim3(256), 0, stream, sorted_idx, keys_out,
+                         indices, index_base, edge_ids, edges, unsorted, index_bits);
+      NTS_LAUNCH_CHECK("plan_take_indices_kernel");
+    }
     indices = sorted_idx;
     index_base = 0;
     NTS_HIP_TRY(hipMemsetAsync(counters, 0, sizeof(nts::PlanCounters), stream));
