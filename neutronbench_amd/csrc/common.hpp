@@ -257,23 +257,30 @@ __device__ __forceinline__ uint32_t owners_of_step(const uint32_t *__restrict__ 
   return last <= e ? owner_of(off, n, e) : d0 + pos;
 }
 
-// owners_of_step for a walk over long rows: `row` enters as a row with off[row] <= base, `row_end` as the
-// end of a row that holds `base` (0 at the start of a walk).  While the 64 positions lie inside that row
-// nothing is loaded; otherwise the row of the step's last position is carried on.  On a graph of 500
-// edges a row nine steps in ten are of the first kind (plan_sort_keys_kernel, 114.8 M edges: 0.58 -> 0.55 ms,
-// plan_scan_edges_kernel 0.81 -> 0.77 ms).
+// owners_of_step for a walk over long rows: `row` enters as a row with off[row] <= base, `row_begin` and `row_end` as the
+// bounds of a row that holds `base` and began before it (0 at the start of a walk).  While the 64 positions lie inside
+// that row nothing is loaded; otherwise the row of the step's last position is carried on.  On a graph of 500
+// edges a row nine steps in ten are of the first kind.
+__device__ __forceinline__ bool step_inside_row(uint32_t base, uint32_t row_end) {
+  return row_end > base && row_end - base >= static_cast<uint32_t>(kWave);
+}
 __device__ __forceinline__ uint32_t owners_of_row_step(const uint32_t *__restrict__ off, uint32_t n, uint32_t base,
-                                                       uint32_t &row, uint32_t &row_end) {
-  if (row_end > base && row_end - base >= static_cast<uint32_t>(kWave)) return row;
+                                                       uint32_t &row, uint32_t &row_begin, uint32_t &row_end) {
+  if (step_inside_row(base, row_end)) return row;
   const uint32_t own = owners_of_step(off, n, base, row);
   const uint32_t last = __shfl(own, kWave - 1, kWave);
-  row_end = 0;
+  row_begin = row_end = 0;
   if (last < n) {
     row = last;
+    row_begin = off[last];
     row_end = off[last + 1];
   }
   return own;
 }
+// Steps of such a walk whose indices are requested together: with one at a time a wavefront's step was a memory latency or
+// two (114.8 M edges, plan_scan_edges_kernel 328 -> 255 us, plan_sort_keys_kernel 619 -> 363; the weights, bound by the rate of
+// random degrees, do not gain).
+constexpr int kWalkSteps = 4;
 
 // Exclusive prefix of `mine` over the THREADS threads of a block, in thread order; *total = the sum.
 template <int THREADS>

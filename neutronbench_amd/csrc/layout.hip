@@ -132,10 +132,10 @@ __global__ __launch_bounds__(256) void edge_weights_kernel(float *__restrict__ e
     const uint64_t steps = (static_cast<uint64_t>(E) + kWave - 1) / kWave, per_wave = (steps + n_waves - 1) / n_waves;
     const uint64_t first_step = wave * per_wave, end_step = first_step + per_wave < steps ? first_step + per_wave : steps;
     if (first_step >= end_step) return;
-    uint32_t row = owner_of(own_off, n_own, static_cast<uint32_t>(first_step * kWave)), row_end = 0;
+    uint32_t row = owner_of(own_off, n_own, static_cast<uint32_t>(first_step * kWave)), row_begin = 0, row_end = 0;
     for (uint64_t step = first_step; step < end_step; ++step) {
       const uint32_t base = static_cast<uint32_t>(step * kWave), e = base + lane;
-      const uint32_t o = owners_of_row_step(own_off, n_own, base, row, row_end);
+      const uint32_t o = owners_of_row_step(own_off, n_own, base, row, row_begin, row_end);
       if (e >= E) continue;
       const uint32_t own_deg = degree_at(own_off, o);
       const uint32_t t = other_idx[e];

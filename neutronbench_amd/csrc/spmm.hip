@@ -1427,7 +1427,7 @@ bool separate_gradients_are_faster(const LaunchArgs &a, uint32_t edges) {
 // to the host and scheduling there costs seconds per 10^8 edges.  The kernels below build the item
 // list of make_schedule -- the same pieces, slots, order of pieces, order of whole rows and order of
 // split rows, entry for entry -- from the arrays where they lie:
-//   plan_cut_rows_kernel      one thread per row: the row's range count by its length, a lower_bound per
+//   plan_cut_rows_kernel      16 lanes per row: the row's range count by its length, a lower_bound per
 //                             range boundary, pieces per (row, range) into a [rows, n_slabs] table
 //   exclusive scan of the table = first partial slot of every (row, range); its total = slots
 //   plan_emit_pieces_kernel   one thread per non-empty (row, range): its pieces and their sort keys
@@ -1439,7 +1439,7 @@ bool separate_gradients_are_faster(const LaunchArgs &a, uint32_t edges) {
 // Rows long enough to be cut must ascend.  plan_scan_edges_kernel flags the ones that do not; if there are
 // any, a stable radix sort of (row, index) keys orders them in a copy of the index array that the schedule
 // then cuts and gathers through, with the caller's position of every edge beside it (an edge list in
-// random order, 114.8 M edges: 6 ms, where sorting the rows on 16 host threads took 0.9 s).
+// random order, 114.8 M edges: 3.2 ms, where sorting the rows on 16 host threads took 0.9 s).
 
 struct PlanShape {
   uint32_t chunk, n_slabs, wide_ranges;
@@ -1470,11 +1470,15 @@ __device__ __forceinline__ uint32_t lower_bound_index(const uint32_t *__restrict
   return lo;
 }
 
+// kCutLanes lanes per row, each searching the whole row for the end of its range: one thread that searched range after
+// range from where the last one ended was 32 searches in a row (114.8 M edges, 233 K rows: 280 -> 80 us).
+constexpr uint32_t kCutLanes = 16;
 __global__ __launch_bounds__(256) void plan_cut_rows_kernel(uint32_t *__restrict__ counts, uint32_t *__restrict__ stops,
                                                             const uint32_t *__restrict__ off,
                                                             const uint32_t *__restrict__ idx, uint32_t index_base,
                                                             uint32_t rows, PlanShape sh) {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t gl = threadIdx.x & (kCutLanes - 1), group = (threadIdx.x & (kWave - 1)) / kCutLanes;
+  const uint32_t r = blockIdx.x * (blockDim.x / kCutLanes) + threadIdx.x / kCutLanes;
   if (r >= rows) return;
   const uint32_t b = off[r], e = off[r + 1], deg = e - b;
   const uint32_t R = sh.ranges_for(deg);
@@ -1483,17 +1487,20 @@ __global__ __launch_bounds__(256) void plan_cut_rows_kernel(uint32_t *__restrict
   uint32_t *stp = stops + static_cast<size_t>(r) * sh.n_slabs;
   const uint32_t per = sh.n_slabs / R;
   uint32_t cut = b, nonempty = 0;
-  for (uint32_t c = 0; c < R; ++c) {
+  for (uint32_t c0 = 0; c0 < R; c0 += kCutLanes) {
+    const uint32_t c = c0 + gl;
     const uint64_t hi = static_cast<uint64_t>(c + 1) * per * sh.fine_width;  // first index of the next range
-    const uint32_t stop = (c + 1 == R || cut >= e) ? e : lower_bound_index(idx, cut, e, hi, index_base);
-    const uint32_t n = stop - cut;
-    cnt[c] = deg > sh.chunk ? (n + sh.chunk - 1) / sh.chunk : (n ? 1u : 0u);
-    stp[c] = stop;
-    nonempty += n ? 1u : 0u;
-    cut = stop;
+    const uint32_t stop = c + 1 >= R ? e : lower_bound_index(idx, cut, e, hi, index_base);
+    const uint32_t up = __shfl_up(stop, 1, kCutLanes), n = stop - (gl ? up : cut);
+    if (c < R) {
+      cnt[c] = deg > sh.chunk ? (n + sh.chunk - 1) / sh.chunk : (n ? 1u : 0u);
+      stp[c] = stop;
+    }
+    nonempty += __popcll(__ballot(c < R && n) >> (group * kCutLanes) & ((1ull << kCutLanes) - 1));
+    cut = __shfl(stop, kCutLanes - 1, kCutLanes);
   }
   if (deg <= sh.chunk && nonempty <= 1)  // all edges in one wide range: the row stays whole
-    for (uint32_t c = 0; c < R; ++c) cnt[c] = 0;
+    for (uint32_t c = gl; c < R; c += kCutLanes) cnt[c] = 0;
 }
 
 __global__ __launch_bounds__(256) void plan_emit_pieces_kernel(Item *__restrict__ pieces, uint32_t *__restrict__ keys,
@@ -1573,7 +1580,7 @@ __global__ __launch_bounds__(256) void plan_check_offsets_kernel(const uint32_t 
 // that repeat the index before them in their row, finds the largest index, and flags the rows of more
 // than `cut_above` edges whose indices do not ascend.  Bound by the one read of the index array; an edge
 // list in random order has a descent at every second edge, so nothing is listed or counted per descent
-// (the list's counter alone took 42 ms for 114.8 M edges; the pass takes 0.32 ms whatever the order).
+// (the list's counter alone took 42 ms for 114.8 M edges; the pass takes 0.23 to 0.3 ms whatever the order).
 __global__ __launch_bounds__(256) void plan_scan_edges_kernel(const uint32_t *__restrict__ off,
                                                               const uint32_t *__restrict__ idx, uint32_t rows,
                                                               uint32_t edges, uint32_t cut_above,
@@ -1586,29 +1593,46 @@ __global__ __launch_bounds__(256) void plan_scan_edges_kernel(const uint32_t *__
   const uint64_t per_wave = (total_steps + n_waves - 1) / n_waves;
   const uint64_t first_step = wave * per_wave;
   const uint64_t end_step = first_step + per_wave < total_steps ? first_step + per_wave : total_steps;
-  uint32_t row = 0, row_end = 0;  // a wavefront without a span still takes part in the block's sums
+  uint32_t row = 0, row_begin = 0, row_end = 0;  // a wavefront without a span still takes part in the block's sums
   if (first_step < end_step) row = owner_of(off, rows, static_cast<uint32_t>(first_step * kWave));
   unsigned long long equal = 0;
-  uint32_t largest = 0, descends = 0;
-  uint32_t nxt = 0, before = 0;  // the indices of the next step are requested while this one is looked at
-  if (first_step * kWave + lane < edges) nxt = idx[first_step * kWave + lane];
+  uint32_t largest = 0, descends = 0, flagged = 0;  // flagged: the row at hand is
+  uint32_t before = 0;
   if (first_step && first_step < end_step) before = idx[first_step * kWave - 1];
-  for (uint64_t step = first_step; step < end_step; ++step) {
-    const uint32_t base = static_cast<uint32_t>(step * kWave), k = base + lane;
-    const uint32_t b = nxt;
-    uint32_t a = __shfl_up(b, 1, kWave);
-    if (lane == 0) a = before;
-    before = wave_read(b, kWave - 1);
-    if (static_cast<uint64_t>(base) + kWave + lane < edges) nxt = idx[base + kWave + lane];
-    const uint32_t own = owners_of_row_step(off, rows, base, row, row_end);
-    if (k >= edges) continue;
-    largest = max(largest, b);
-    const uint32_t start = off[own];
-    if (k == start) continue;
-    equal += a == b ? 1u : 0u;
-    if (a > b && off[own + 1] - start > cut_above) {
-      unsorted[own] = 1;  // the same value from every lane that finds one
-      descends = 1;
+  for (uint64_t step4 = first_step; step4 < end_step; step4 += kWalkSteps) {
+    uint32_t v[kWalkSteps];
+#pragma unroll
+    for (int u = 0; u < kWalkSteps; ++u) {
+      const uint64_t k = (step4 + u) * kWave + lane;
+      v[u] = step4 + u < end_step && k < edges ? idx[k] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < kWalkSteps; ++u) {
+      if (step4 + u >= end_step) break;
+      const uint32_t base = static_cast<uint32_t>((step4 + u) * kWave), k = base + lane, b = v[u];
+      uint32_t a = __shfl_up(b, 1, kWave);
+      if (lane == 0) a = before;
+      before = wave_read(b, kWave - 1);
+      if (step_inside_row(base, row_end)) {  // no row starts here
+        largest = max(largest, b);
+        equal += a == b ? 1u : 0u;
+        if (!flagged && row_end - row_begin > cut_above && __ballot(a > b)) {
+          flagged = descends = 1;
+          if (lane == 0) unsorted[row] = 1;
+        }
+        continue;
+      }
+      flagged = 0;
+      const uint32_t own = owners_of_row_step(off, rows, base, row, row_begin, row_end);
+      if (k >= edges) continue;
+      largest = max(largest, b);
+      const uint32_t start = off[own];
+      if (k == start) continue;
+      equal += a == b ? 1u : 0u;
+      if (a > b && off[own + 1] - start > cut_above) {
+        unsorted[own] = 1;  // the same value from every lane that finds one
+        descends = 1;
+      }
     }
   }
 #pragma unroll
@@ -1651,14 +1675,32 @@ __global__ __launch_bounds__(256) void plan_sort_keys_kernel(unsigned long long 
   const uint64_t end_step = first_step + per_wave < total_steps ? first_step + per_wave : total_steps;
   if (first_step >= end_step) return;
   const uint32_t mask = static_cast<uint32_t>((1ull << index_bits) - 1);
-  uint32_t row = owner_of(off, rows, static_cast<uint32_t>(first_step * kWave)), row_end = 0;
-  for (uint64_t step = first_step; step < end_step; ++step) {
-    const uint32_t base = static_cast<uint32_t>(step * kWave), k = base + lane;
-    const uint32_t own = owners_of_row_step(off, rows, base, row, row_end);
-    if (k >= edges) continue;
+  uint32_t row = owner_of(off, rows, static_cast<uint32_t>(first_step * kWave)), row_begin = 0, row_end = 0;
+  uint32_t flagged = 0;  // the row at hand is
+  auto put = [&](uint32_t k, uint32_t own, uint32_t own_begin, uint32_t is_unsorted, uint32_t index) {
     const unsigned long long key =
-        (static_cast<unsigned long long>(own) << index_bits) | (unsorted[own] ? (idx[k] - index_base) & mask : 0u);
-    keys[k] = local_bits ? key << local_bits | (k - off[own]) : key;
+        (static_cast<unsigned long long>(own) << index_bits) | (is_unsorted ? (index - index_base) & mask : 0u);
+    keys[k] = local_bits ? key << local_bits | (k - own_begin) : key;
+  };
+  for (uint64_t step4 = first_step; step4 < end_step; step4 += kWalkSteps) {
+    uint32_t v[kWalkSteps];
+#pragma unroll
+    for (int u = 0; u < kWalkSteps; ++u) {
+      const uint64_t k = (step4 + u) * kWave + lane;
+      v[u] = step4 + u < end_step && k < edges ? idx[k] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < kWalkSteps; ++u) {
+      if (step4 + u >= end_step) break;
+      const uint32_t base = static_cast<uint32_t>((step4 + u) * kWave), k = base + lane;
+      if (step_inside_row(base, row_end)) {
+        put(k, row, row_begin, flagged, v[u]);
+        continue;
+      }
+      const uint32_t own = owners_of_row_step(off, rows, base, row, row_begin, row_end);
+      flagged = row_end ? unsorted[row] : 0u;
+      if (k < edges) put(k, own, off[own], unsorted[own], v[u]);
+    }
   }
 }
 
@@ -2235,8 +2277,8 @@ int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const
     NTS_HIP_TRY(hipMemsetAsync(counters, 0, sizeof(nts::PlanCounters), stream));
     NTS_HIP_TRY(scan_edges(indices));  // counts the repeated edges of the copy
   }
-  hipLaunchKernelGGL(nts::plan_cut_rows_kernel, dim3(row_blocks), dim3(256), 0, stream, counts, stops, offsets, indices,
-                     index_base, rows, sh);
+  hipLaunchKernelGGL(nts::plan_cut_rows_kernel, dim3(nts::ceil_div(rows, 256 / nts::kCutLanes)), dim3(256), 0, stream, counts,
+                     stops, offsets, indices, index_base, rows, sh);
   NTS_LAUNCH_CHECK("plan_cut_rows_kernel");
   NTS_HIP_TRY(rocprim::exclusive_scan(tmp1, scan_bytes, counts, slot_base, 0u, cells + 1, rocprim::plus<uint32_t>(),
                                       stream, false));
