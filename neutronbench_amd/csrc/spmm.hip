@@ -80,6 +80,36 @@ struct Vec<4> {
   using type = float4;
 };
 
+// Vectors of a row that starts at any float (SHARED): the memory path takes 16-byte lanes at multiples of four bytes.
+typedef float Floats4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int VEC, bool SHARED>
+__device__ __forceinline__ typename Vec<VEC>::type load_row(const float *p) {
+  if constexpr (VEC == 4 && SHARED) {
+    const Floats4 v = *reinterpret_cast<const Floats4 *>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+  } else {
+    return *reinterpret_cast<const typename Vec<VEC>::type *>(p);
+  }
+}
+// The floats `skip` .. VEC - 1 of r, to p + skip on; with `accumulate` added to what is there.
+template <int VEC>
+__device__ __forceinline__ void store_row(float *p, typename Vec<VEC>::type r, uint32_t skip, bool accumulate) {
+  if constexpr (VEC == 4) {
+    if (skip == 0) {
+      if (accumulate) {
+        const Floats4 o = *reinterpret_cast<const Floats4 *>(p);
+        r = make_float4(r.x + o.x, r.y + o.y, r.z + o.z, r.w + o.w);
+      }
+      *reinterpret_cast<Floats4 *>(p) = Floats4{r.x, r.y, r.z, r.w};
+      return;
+    }
+  }
+  const float *f = reinterpret_cast<const float *>(&r);
+#pragma unroll
+  for (uint32_t i = 0; i < VEC; ++i)
+    if (i >= skip) p[i] = accumulate ? f[i] + p[i] : f[i];
+}
+
 template <int VEC>
 __device__ __forceinline__ typename Vec<VEC>::type vzero();
 template <>
@@ -355,11 +385,21 @@ __global__ __launch_bounds__(256) void spmm_wave_kernel(const float *__restrict_
   }
 }
 
-// Sub-wavefront variant for narrow rows: G lanes per row (G = 4, 8, 16 or 32), 64/G rows per
-// wavefront, one VEC-wide accumulator per lane (F <= G*VEC).  Neighbour pairs are fetched G at a
-// time per group and broadcast inside the group with cross-lane shuffles.
-template <int G, int VEC, bool HEADS, bool REMAP, bool RUNS>
-__global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict__ in, float *__restrict__ out,
+// Sub-wavefront variant for narrow rows: G lanes per row, 64/G rows per wavefront, one VEC-wide accumulator per lane.
+// Neighbour pairs are fetched G at a time per group and broadcast inside the group with cross-lane shuffles.
+// A lane's vector never crosses the end of its head (or row): where the width is no multiple of VEC the last lane's starts
+// earlier, shares columns with the lane before it and stores only its own.  16-byte lanes at any float instead of a
+// wavefront of 4-byte ones for a row of 47 floats: 500 K rows, 20 M edges with source ranges 809 -> 416 us, and from 33 to 127
+// floats 800-1,046 -> 343-861; 1 M, 3 M without a schedule 306 -> 210.
+// With per-head weights the registers are held down to what six wavefronts per SIMD have (98 -> 80; the gather waits
+// for memory): four heads of 32 on 169 K rows, 2.48 M edges 175 -> 146 us, 1 M, 3 M 499 -> 403, 500 K, 20 M 1,066 -> 970; eight
+// wavefronts 157, 419 and 1,028.
+template <int G, bool HEADS, bool RUNS>
+constexpr int group_waves() {
+  return HEADS ? 6 : !RUNS && G <= 16 ? 8 : 1;
+}
+template <bool SHARED, int G, int VEC, int U, bool HEADS, bool REMAP, bool RUNS>
+__global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_group_kernel(const float *__restrict__ in, float *__restrict__ out,
                                                          const float *__restrict__ w,
                                                          const uint32_t *__restrict__ offsets,
                                                          const uint32_t *__restrict__ indices, uint32_t index_base,
@@ -369,7 +409,7 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
                                                          uint32_t row_edge_limit,
                                                          const uint32_t *__restrict__ edge_ids, uint32_t panels) {
   using V = typename Vec<VEC>::type;
-  constexpr int U = G >= 8 ? 8 : 4;  // edges per step: their rows are requested together
+  static_assert(U <= G, "a step's pairs come from one tile");  // U edges per step: their rows are requested together
   const uint32_t gl = threadIdx.x & (G - 1);
   const uint32_t panel = blockIdx.x % panels;
   const uint32_t item = (blockIdx.x / panels * blockDim.x + threadIdx.x) / G;
@@ -389,10 +429,22 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
     slot = kNoSlot;
     if (e1 - e0 > row_edge_limit) return;  // a long row: its pieces are separate work items
   }
-  const uint32_t col = (panel * G + gl) * VEC;
-  const bool live = col < F;
-  const uint32_t lcol = live ? col : F - VEC;  // idle lanes re-read the last columns, never store
-  const uint32_t head = HEADS ? lcol / heads.Fh : 0u;
+  // This lane's first column, the one its loads start at, and its head.  SHARED: of `per_head` lanes a head the last one
+  // starts earlier where the head ends; otherwise idle lanes re-read the last columns and never store.
+  uint32_t col = (panel * G + gl) * VEC, lcol, head = 0;
+  bool live;
+  if (SHARED) {
+    const uint32_t q = panel * G + gl, Fh = HEADS ? heads.Fh : F, per_head = (Fh + VEC - 1) / VEC;
+    if (HEADS) head = min(q / per_head, heads.H - 1);
+    const uint32_t first = (q - head * per_head) * VEC;
+    live = first < Fh;
+    col = head * Fh + first;
+    lcol = head * Fh + min(first, Fh - VEC);
+  } else {
+    live = col < F;
+    lcol = live ? col : F - VEC;
+    if (HEADS) head = lcol / heads.Fh;
+  }
   V acc = vzero<VEC>();
 
   // The (index, weight) pairs of the next G edges are requested while the current ones are used, so
@@ -436,7 +488,7 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
         for (int u = 0; u < U; ++u) {
           fresh[u] = si[u] != (u ? si[u - 1] : held_i);
           v[u] = vzero<VEC>();
-          if (fresh[u]) v[u] = *reinterpret_cast<const V *>(in + static_cast<size_t>(si[u]) * F + lcol);
+          if (fresh[u]) v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si[u]) * F + lcol);
           wv[u] = HEADS ? w[static_cast<size_t>(ss[u]) * heads.H + head] : __uint_as_float(ss[u]);
         }
 #pragma unroll
@@ -449,7 +501,7 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        v[u] = *reinterpret_cast<const V *>(in + static_cast<size_t>(si[u]) * F + lcol);
+        v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si[u]) * F + lcol);
         wv[u] = HEADS ? w[static_cast<size_t>(ss[u]) * heads.H + head] : __uint_as_float(ss[u]);
       }
 #pragma unroll
@@ -471,7 +523,7 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
         v[u] = vzero<VEC>();
         wv[u] = 0.f;
         if (static_cast<uint32_t>(u) < left) {
-          v[u] = *reinterpret_cast<const V *>(in + static_cast<size_t>(si) * F + lcol);
+          v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si) * F + lcol);
           wv[u] = HEADS ? w[static_cast<size_t>(ss) * heads.H + head] : __uint_as_float(ss);
         }
       }
@@ -486,21 +538,25 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(const float *__restrict
       const uint32_t ss = __shfl(my_s, j, G);
       const float wgt = HEADS ? w[static_cast<size_t>(ss) * heads.H + head] : __uint_as_float(ss);
       if (RUNS) {
-        if (si != held_i) held = *reinterpret_cast<const V *>(in + static_cast<size_t>(si) * F + lcol);
+        if (si != held_i) held = load_row<VEC, SHARED>(in + static_cast<size_t>(si) * F + lcol);
         held_i = si;
         vfma(acc, held, wgt);
         continue;
       }
-      vfma(acc, *reinterpret_cast<const V *>(in + static_cast<size_t>(si) * F + lcol), wgt);
+      vfma(acc, load_row<VEC, SHARED>(in + static_cast<size_t>(si) * F + lcol), wgt);
     }
   }
 
   if (live) {
     float *dst = (slot == kNoSlot) ? out + static_cast<size_t>(row) * F : partial + static_cast<size_t>(slot) * F;
-    V *p = reinterpret_cast<V *>(dst + col);
-    V r = acc;
-    if (accumulate && slot == kNoSlot) vadd(r, *p);
-    *p = r;
+    if (SHARED) {
+      store_row<VEC>(dst + lcol, acc, col - lcol, accumulate && slot == kNoSlot);
+    } else {
+      V *p = reinterpret_cast<V *>(dst + col);
+      V r = acc;
+      if (accumulate && slot == kNoSlot) vadd(r, *p);
+      *p = r;
+    }
   }
 }
 
@@ -833,6 +889,7 @@ struct LaunchArgs {
   uint32_t partial_ld = 0;                     // row stride of `partial` in floats (0 = F)
   bool dup_runs = false;                       // rows hold runs of equal indices worth loading once per run
   uint32_t scheduled_rows = 0;                 // rows of the schedule that `items` comes from (0: no schedule)
+  uint32_t scheduled_edges = 0;                // and its edges
   uint32_t rows_after_items = 0;               // with items: this many whole rows follow the listed items in the launch
   const float *dot_rows = nullptr;             // with dot_out: the rows whose products with the gathered ones
   float *dot_out = nullptr;                    // are the gradient of alpha (attention_grad_kernel)
@@ -913,13 +970,13 @@ void launch_wave(const LaunchArgs &a, uint32_t col_base, uint32_t panels) {
 #undef NTS_LAUNCH_WAVE
 }
 
-template <int G, int VEC>
+template <int G, int VEC, int U = 8, bool SHARED = false>
 void launch_group(const LaunchArgs &a, uint32_t panels = 1) {
   const uint32_t per_block = 256 / G;
   const uint32_t n_list = a.items ? a.n_items : 0u, n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
   const uint32_t blocks = ceil_div(n_total, per_block) * panels;
 #define NTS_LAUNCH_GROUP(HD, RM, RUNS)                                                                                  \
-  hipLaunchKernelGGL((spmm_group_kernel<G, VEC, HD, RM, RUNS>), dim3(blocks), dim3(256), 0, a.stream, a.in, a.out, a.w, \
+  hipLaunchKernelGGL((spmm_group_kernel<SHARED, G, VEC, U, HD, RM, RUNS>), dim3(blocks), dim3(256), 0, a.stream, a.in, a.out, a.w, \
                      a.offsets, a.indices, a.index_base, n_total, n_list, a.F, a.items, a.partial, a.accumulate,        \
                      a.heads,                                                                                          \
                      a.row_edge_limit, a.edge_ids, panels)
@@ -1008,6 +1065,55 @@ uint32_t die_panels(const LaunchArgs &a, int vec) {
   return a.F == 256 ? 2 : a.F == 512 ? 4 : 0;
 }
 
+// Lanes of a narrow row, by what bounds the launch.  Lanes of one float (16 or 32 a row, 64 up to 64 floats) cover more pairs a
+// tile and leave fewer rows to a wavefront, which is what counts while a launch lasts as long as its long rows and
+// pieces; lanes of four floats take fewer instructions a row, which counts where the chip is full.  us, four floats / one:
+//   scheduled, F = 16   2.7 K rows, 11 K edges 33 / 16, 169 K, 2.48 M 117 / 44, 1 M, 3 M 137 / 66, 500 K, 20 M 350 / 165
+//   scheduled, F = 32   2.7 K 23 / 15, 60 K, 600 K 63 / 32, 169 K 72 / 49, 500 K, 1.5 M 73 / 57, 300 K, 4.5 M 85 / 77; but
+//                       50 K, 8 M 78 / 95, 1 M, 3 M 97 / 106, 500 K, 20 M 243 / 280: six million edges, a row counting four
+//   scheduled, F = 64   2.7 K 20 / 15, 20 K, 300 K 46 / 29, 60 K 54 / 39, 50 K, 8 M 112 / 101; but 169 K 71 / 74, 500 K, 20 M
+//                       376 / 452, and rows with runs of equal indices 20 K 63 / 78
+//   no schedule, F = 16 5 K, 40 K 66 / 26, 60 K, 600 K 63 / 42, 300 K, 4.5 M 178 / 165; but 50 K, 8 M, mostly pieces, 152 / 158 and
+//                       1 M, 3 M 131 / 135
+//   no schedule, F = 32 20 K 39 / 33, 60 K 53 / 45; but 169 K 82 / 90
+//   no schedule, F = 64 5 K 36 / 24, 20 K 40 / 31, 60 K 51 / 51
+// Up to eight floats a group of that many lanes where pieces are most of the work or the rows are many (F = 3, 16 lanes and 4:
+// 50 K, 8 M 157 / 140, 1 M, 3 M 134 / 120).  Sixteen edges a step instead of eight where the rows are few: scheduled F = 16
+// 169 K 53 -> 44, 1 M 66 -> 71; F = 32 60 K 40 -> 32, 169 K 49 -> 53; no schedule 5 K 47 -> 41, 20 K 34 -> 35.
+// Rows off 16-byte boundaries of 25 lanes and more take a wavefront of 4-byte lanes where the chip is full of dense rows:
+// F = 127 50 K, 8 M 267 / 243, 300 K, 4.5 M 304 / 295; but 60 K 54 / 71, 1 M, 3 M 377 / 411; F = 201 50 K, 8 M 438 / 383, 169 K 227 / 219, 60 K
+// 63 / 117; no schedule 5 K 30 / 76, 169 K 243 / 272, 300 K 496 / 535, but 1 M, 3 M 648 / 642 and F = 129 525 / 486.
+enum NarrowLanes {
+  kFloats4, kFloats8, kFloats16, kFloats16x16, kFloats32, kFloats32x16, kFloats64, kVectors4, kVectors8, kVectors16, kVectors32, kVectors64, kWide
+};
+NarrowLanes narrow_lanes(const LaunchArgs &a, int vec) {
+  const uint32_t F = a.F, H = a.heads.H, width = H ? a.heads.Fh : F;
+  const uint32_t lanes = (H ? H : 1u) * ceil_div(width, 4);
+  const uint32_t n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
+  const bool scheduled = a.scheduled_rows != 0, no_vectors = width < 4;
+  const bool few = scheduled ? a.scheduled_edges + 4ull * a.scheduled_rows <= 6000000 : n_total <= 1u << (F <= 16 ? 14 : 16);
+  const bool pieces = !scheduled && a.rows_after_items && a.n_items > a.rows_after_items;
+  if (F <= 16) {
+    if (F <= 8 && (pieces || (!scheduled && n_total > 1u << 18))) return F <= 4 ? kFloats4 : kFloats8;
+    if (no_vectors || scheduled || !(pieces || n_total > 1u << 19)) return few ? kFloats16x16 : kFloats16;
+  } else if (F <= 32) {
+    if (no_vectors || few) return n_total <= (scheduled ? 1u << 17 : 1u << 14) ? kFloats32x16 : kFloats32;
+  } else if (F <= 64 && !a.dup_runs && n_total <= (scheduled ? 1u << 17 : 1u << 15)) {
+    return kFloats64;
+  }
+  if (no_vectors) return kWide;
+  if (lanes <= 4) return kVectors4;
+  if (lanes <= 8) return kVectors8;
+  if (lanes <= 16) return kVectors16;
+  if (vec == 4) return lanes <= 32 ? kVectors32 : kWide;
+  const bool short_schedule = scheduled && few && n_total <= 1u << 17;
+  if (lanes <= 32) {
+    const bool dense = scheduled && !a.dup_runs && lanes > 24 && a.scheduled_edges / 8 > a.scheduled_rows;
+    return dense && !short_schedule ? kWide : kVectors32;
+  }
+  return lanes <= 64 && !pieces && (scheduled ? short_schedule : n_total <= 3u << 17) ? kVectors64 : kWide;
+}
+
 void launch_spmm(const LaunchArgs &a) {
   if (a.n_items == 0) return;
   if (a.dot_out) {
@@ -1018,15 +1124,23 @@ void launch_spmm(const LaunchArgs &a) {
   const int vec = pick_vec(a);
   const uint32_t F = a.F;
   if (const uint32_t panels = die_panels(a, vec)) return F == 128 ? launch_group<16, 4>(a, panels) : launch_group<32, 4>(a, panels);
-  // Narrow rows: sub-wavefront groups so that lanes are not left idle.
-  if (vec == 4 && F <= 16) return launch_group<4, 4>(a);
-  if (vec == 4 && F <= 32) return launch_group<8, 4>(a);
-  if (vec == 4 && F <= 64) return launch_group<16, 4>(a);
-  if (vec == 4 && F <= 128) return launch_group<32, 4>(a);
-  if (vec == 1 && F <= 4) return launch_group<4, 1>(a);
-  if (vec == 1 && F <= 8) return launch_group<8, 1>(a);
-  if (vec == 1 && F <= 16) return launch_group<16, 1>(a);
-  if (vec == 1 && F <= 32) return launch_group<32, 1>(a);
+  if (!a.in_ld) {
+    switch (narrow_lanes(a, vec)) {
+      case kFloats4: return launch_group<4, 1, 4>(a);
+      case kFloats8: return launch_group<8, 1>(a);
+      case kFloats16: return launch_group<16, 1>(a);
+      case kFloats16x16: return launch_group<16, 1, 16>(a);
+      case kFloats32: return launch_group<32, 1>(a);
+      case kFloats32x16: return launch_group<32, 1, 16>(a);
+      case kVectors4: return vec == 4 ? launch_group<4, 4, 4>(a) : launch_group<4, 4, 4, true>(a);
+      case kVectors8: return vec == 4 ? launch_group<8, 4>(a) : launch_group<8, 4, 8, true>(a);
+      case kVectors16: return vec == 4 ? launch_group<16, 4>(a) : launch_group<16, 4, 8, true>(a);
+      case kVectors32: return vec == 4 ? launch_group<32, 4>(a) : launch_group<32, 4, 8, true>(a);
+      case kVectors64: return launch_group<64, 4, 8, true>(a);
+      case kFloats64: return launch_wave_vec<1>(a);
+      case kWide: break;
+    }
+  }
   // Wave per row.
   if (vec == 4) return launch_wave_vec<4>(a);
   return launch_wave_vec<1>(a);
@@ -2679,6 +2793,8 @@ int nts_spmm_gather_heads_planned(nts_spmm_plan_t *plan, const float *in, float 
   nts::LaunchArgs a{in,  out,         alpha,         offsets,    indices, 0u, plan->n_items,
                     F,   plan->items, plan->partial, accumulate, stream};
   a.heads = nts::HeadArgs{perm, H, Fh};
+  a.scheduled_rows = plan->rows;
+  a.scheduled_edges = plan->edges;
   if (plan->sorted_idx) {
     a.indices = plan->sorted_idx;
     a.edge_ids = plan->edge_ids;
@@ -2725,6 +2841,7 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
   }
   a.dup_runs = use_runs(plan);
   a.scheduled_rows = plan->rows;
+  a.scheduled_edges = plan->edges;
   if (const uint32_t ld = padded_stride(plan, F, false)) {
     // Rows off 16-byte boundaries: gather from a padded copy with 16-byte lanes.
     const uint64_t vecs = static_cast<uint64_t>(plan->n_index) * (ld / 4);
