@@ -136,6 +136,13 @@ __device__ __forceinline__ void vfma(float4 &a, float4 x, float w) {
   a.z = fmaf(x.z, w, a.z);
   a.w = fmaf(x.w, w, a.w);
 }
+// Zero in place of the first `skip` floats: the columns that the lane before has too count once in a product.
+__device__ __forceinline__ void drop_first(float &, uint32_t) {}
+__device__ __forceinline__ void drop_first(float4 &a, uint32_t skip) {
+  a.x = skip > 0 ? 0.f : a.x;
+  a.y = skip > 1 ? 0.f : a.y;
+  a.z = skip > 2 ? 0.f : a.z;
+}
 __device__ __forceinline__ float vdot(float a, float b) { return a * b; }
 __device__ __forceinline__ float vdot(float4 a, float4 b) {
   return fmaf(a.w, b.w, fmaf(a.z, b.z, fmaf(a.y, b.y, a.x * b.x)));
@@ -588,7 +595,7 @@ constexpr int grad_waves() {
   if (VEC != 4 || NJ != 1 || LH == 1) return 1;
   return LH < 8 ? 5 : G >= 32 ? 6 : 1;
 }
-template <int G, int LH, int NJ, int VEC>
+template <int G, int LH, int NJ, int VEC, bool SHARED>
 __global__ __launch_bounds__(256, (grad_waves<G, LH, NJ, VEC>())) void attention_grad_kernel(const float *__restrict__ gout, float *__restrict__ out,
                                                              const float *__restrict__ alpha,
                                                              const uint32_t *__restrict__ offsets,
@@ -622,17 +629,19 @@ __global__ __launch_bounds__(256, (grad_waves<G, LH, NJ, VEC>())) void attention
   const uint32_t my_head = blockIdx.y * (G / LH) + gl / LH;
   const bool head_live = my_head < H;
   const uint32_t head = head_live ? my_head : H - 1;
-  uint32_t col[NJ];
+  uint32_t col[NJ], skip[NJ];
   bool live[NJ];
   V acc[NJ], xr[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    const uint32_t c = (sub + LH * j) * VEC;
+    const uint32_t c = (sub + LH * j) * VEC, from = SHARED ? min(c, Fh - VEC) : c;
     live[j] = c < Fh;
-    col[j] = head * Fh + (c < Fh ? c : 0u);  // idle lanes re-read the head's first columns
+    skip[j] = live[j] ? c - from : 0u;
+    col[j] = head * Fh + (c < Fh ? from : 0u);  // idle lanes re-read the head's first columns
     acc[j] = vzero<VEC>();
     xr[j] = vzero<VEC>();
-    if (e0 < e1) xr[j] = *reinterpret_cast<const V *>(x + static_cast<size_t>(row) * F + col[j]);  // (no edge: x need not hold the row)
+    if (e0 < e1) xr[j] = load_row<VEC, SHARED>(x + static_cast<size_t>(row) * F + col[j]);  // (no edge: x need not hold the row)
+    if (SHARED) drop_first(xr[j], skip[j]);
   }
   const uint32_t n_edges = e1 - e0;
   // Lane l of a group holds the pair of edge l % U of a step, one step ahead; beyond the row the last edge's.
@@ -652,7 +661,7 @@ __global__ __launch_bounds__(256, (grad_waves<G, LH, NJ, VEC>())) void attention
     const uint32_t si = __shfl(my_i, u, G);
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-      if (there) v[u][j] = *reinterpret_cast<const V *>(gout + static_cast<size_t>(si) * F + col[j]);
+      if (there) v[u][j] = load_row<VEC, SHARED>(gout + static_cast<size_t>(si) * F + col[j]);
   };
   auto gather_weight = [&](int i, bool there) {
     id[i] = __shfl(my_s, S * i + mine, G);
@@ -666,7 +675,9 @@ __global__ __launch_bounds__(256, (grad_waves<G, LH, NJ, VEC>())) void attention
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         if (static_cast<uint32_t>(u) < left) vfma(acc[j], v[u][j], wu);
-        const float q = vdot(v[u][j], xr[j]);
+        V own = v[u][j];
+        if (SHARED) drop_first(own, skip[j]);  // (also here: zero times an infinity is no zero)
+        const float q = vdot(own, xr[j]);
         p[u] += live[j] ? q : 0.f;
       }
     }
@@ -741,6 +752,10 @@ __global__ __launch_bounds__(256, (grad_waves<G, LH, NJ, VEC>())) void attention
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     if (head_live && live[j]) {
+      if (SHARED) {
+        store_row<VEC>(dst + col[j], acc[j], skip[j], accumulate && slot == kNoSlot);
+        continue;
+      }
       V *q = reinterpret_cast<V *>(dst + col[j]);
       V r = acc[j];
       if (accumulate && slot == kNoSlot) vadd(r, *q);
@@ -898,49 +913,64 @@ struct LaunchArgs {
 // Lanes per head and vectors per lane of attention_grad_kernel for heads of `vecs` vectors; 16 lanes with up to
 // four vectors each cover 64 vectors, wider heads are not its business.
 constexpr uint32_t kGradMaxVecs = 64;
-bool attention_grad_takes(const LaunchArgs &a, int *vec) {
-  const bool a16 = aligned_to(a.in, 16) && aligned_to(a.out, 16) && aligned_to(a.dot_rows, 16);
-  *vec = a.heads.Fh % 4 == 0 && a16 ? 4 : 1;
-  return a.heads.Fh / *vec <= kGradMaxVecs;
+bool attention_grad_takes(const LaunchArgs &a) { return ceil_div(a.heads.Fh, a.heads.Fh >= 4 ? 4 : 1) <= kGradMaxVecs; }
+
+// Rows off 16-byte boundaries: lanes of one float or of four that start at any float.  One float a lane spreads a step's
+// products over more lanes, four take fewer registers and instructions for wide rows.  us, one float / four:
+//   heads x floats   5 K rows, 40 K edges   20 K, 300 K   169 K, 2.48 M   1 M, 4 M     500 K, 20 M
+//   1 x 5            62 / 99                40 / 48       113 / 120       195 / 219    928 / 950
+//   1 x 17           86 / 94                47 / 49       130 / 135       277 / 235    1,031 / 1,014
+//   4 x 10           66 / 91                47 / 49       175 / 161       614 / 404    1,575 / 1,266
+//   1 x 47           --                     50 / 49       167 / 164       405 / 400    1,227 / 1,201
+//   8 x 13           73 / 92                64 / 51       432 / 254       1,311 / 649  3,298 / 1,746
+//   8 x 47           96 / 104               87 / 93       704 / 714       2,012 / 2,052
+// Heads of 65 to 256 floats of such rows took a pass per gradient: 1 x 101 127 -> 65 on 20 K, 622 -> 245, 1,458 -> 640, 4,713 -> 1,679.
+bool grad_floats_are_faster(const LaunchArgs &a) {
+  const uint32_t Fh = a.heads.Fh, rows = a.n_items + (a.items ? a.rows_after_items : 0u);
+  if (Fh > kGradMaxVecs) return false;
+  const uint64_t lanes = static_cast<uint64_t>(a.heads.H) * (Fh <= 4 ? 4 : Fh <= 8 ? 8 : ceil_div(Fh, 16) * 16);
+  if (Fh < 4 || lanes <= 16 || (lanes <= 32 && rows <= 1u << 19)) return true;
+  if (Fh > 32) return Fh <= 48 && a.heads.H >= 4;
+  return rows <= (lanes <= 64 ? 1u << 15 : 1u << 13);
 }
 
-template <int G, int LH, int NJ, int VEC>
+template <int G, int LH, int NJ, int VEC, bool SHARED>
 void launch_attention_grad_as(const LaunchArgs &a) {
   const uint32_t n_list = a.items ? a.n_items : 0u, n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
   const dim3 grid(ceil_div(n_total, 256 / G), ceil_div(a.heads.H, G / LH));
-  hipLaunchKernelGGL((attention_grad_kernel<G, LH, NJ, VEC>), grid, dim3(256), 0, a.stream, a.in, a.out, a.w, a.offsets,
+  hipLaunchKernelGGL((attention_grad_kernel<G, LH, NJ, VEC, SHARED>), grid, dim3(256), 0, a.stream, a.in, a.out, a.w, a.offsets,
                      a.indices, n_total, n_list, a.F, a.items, a.partial, a.accumulate, a.heads, a.row_edge_limit,
                      a.dot_rows, a.dot_out);
 }
 
-template <int LH, int NJ, int VEC>
+template <int LH, int NJ, int VEC, bool SHARED>
 void launch_attention_grad_lanes(const LaunchArgs &a) {
   // As many heads side by side as there are, in groups of 8 (a tile of edge pairs is one per lane) to 64 lanes.
   const uint32_t H = a.heads.H;
   if constexpr (LH <= 8) {
-    if (H * LH <= 8) return launch_attention_grad_as<8, LH, NJ, VEC>(a);
+    if (H * LH <= 8) return launch_attention_grad_as<8, LH, NJ, VEC, SHARED>(a);
   }
-  if (H * LH <= 16) return launch_attention_grad_as<16, LH, NJ, VEC>(a);
-  if (H * LH <= 32) return launch_attention_grad_as<32, LH, NJ, VEC>(a);
-  return launch_attention_grad_as<64, LH, NJ, VEC>(a);
+  if (H * LH <= 16) return launch_attention_grad_as<16, LH, NJ, VEC, SHARED>(a);
+  if (H * LH <= 32) return launch_attention_grad_as<32, LH, NJ, VEC, SHARED>(a);
+  return launch_attention_grad_as<64, LH, NJ, VEC, SHARED>(a);
 }
 
-template <int VEC>
+template <int VEC, bool SHARED = false>
 void launch_attention_grad(const LaunchArgs &a) {
   const uint32_t vecs = ceil_div(a.heads.Fh, VEC);
   // Lanes that a narrow head leaves idle are rows that the wavefront does not work on: eight heads of four floats
   // with four lanes each instead of one, 1.5 M vertices, 5 M edges 704 us, 459 now; two lanes for eight floats 762, 652.
   // (Not for heads of one or two floats: 30 K vertices, 300 K edges, eight heads of one 59 us, 70 with a lane each.)
   if constexpr (VEC == 4) {
-    if (vecs <= 1) return launch_attention_grad_lanes<1, 1, VEC>(a);
-    if (vecs <= 2) return launch_attention_grad_lanes<2, 1, VEC>(a);
+    if (vecs <= 1) return launch_attention_grad_lanes<1, 1, VEC, SHARED>(a);
+    if (vecs <= 2) return launch_attention_grad_lanes<2, 1, VEC, SHARED>(a);
   }
-  if (vecs <= 4) return launch_attention_grad_lanes<4, 1, VEC>(a);
-  if (vecs <= 8) return launch_attention_grad_lanes<8, 1, VEC>(a);
-  if (vecs <= 16) return launch_attention_grad_lanes<16, 1, VEC>(a);
-  if (vecs <= 32) return launch_attention_grad_lanes<16, 2, VEC>(a);
-  if (vecs <= 48) return launch_attention_grad_lanes<16, 3, VEC>(a);
-  return launch_attention_grad_lanes<16, 4, VEC>(a);
+  if (vecs <= 4) return launch_attention_grad_lanes<4, 1, VEC, SHARED>(a);
+  if (vecs <= 8) return launch_attention_grad_lanes<8, 1, VEC, SHARED>(a);
+  if (vecs <= 16) return launch_attention_grad_lanes<16, 1, VEC, SHARED>(a);
+  if (vecs <= 32) return launch_attention_grad_lanes<16, 2, VEC, SHARED>(a);
+  if (vecs <= 48) return launch_attention_grad_lanes<16, 3, VEC, SHARED>(a);
+  return launch_attention_grad_lanes<16, 4, VEC, SHARED>(a);
 }
 
 template <int VEC, int NACC>
@@ -1117,9 +1147,9 @@ NarrowLanes narrow_lanes(const LaunchArgs &a, int vec) {
 void launch_spmm(const LaunchArgs &a) {
   if (a.n_items == 0) return;
   if (a.dot_out) {
-    int dot_vec = 1;
-    attention_grad_takes(a, &dot_vec);
-    return dot_vec == 4 ? launch_attention_grad<4>(a) : launch_attention_grad<1>(a);
+    const bool a16 = aligned_to(a.in, 16) && aligned_to(a.out, 16) && aligned_to(a.dot_rows, 16);
+    if (a.heads.Fh % 4 == 0 && a16) return launch_attention_grad<4>(a);
+    return grad_floats_are_faster(a) ? launch_attention_grad<1>(a) : launch_attention_grad<4, true>(a);
   }
   const int vec = pick_vec(a);
   const uint32_t F = a.F;
@@ -1523,8 +1553,8 @@ int launch_spmm_balanced(LaunchArgs a, uint32_t edges, unsigned char *fixed = nu
 // of the fused kernel, with its sums across the lanes, takes longer than one of the gather of wide rows; the other pass
 // has no such chain.  Fused and separate, us: 5 K vertices, 40 K edges, eight heads of 8 91, 65; one of 64 81, 68;
 // of 128 121, 73; two of 64 97, 73; but four of 4 70, 106, one of 32 75, 81 (rows below 64 floats stay fused)
-// and four of 64 97, 100.  For widths that nts_sddmm_heads is slow at, only one head of 4-byte lanes is affected: 5 K, 40 K, 47
-// floats 100, 80; two of 47 99, 142; 2.7 K, 13 K, 47 floats 42, 58.  With fewer than four edges a row on average there are
+// and four of 64 97, 100.  For widths that nts_sddmm_heads is slow at, only one head off 16-byte boundaries is affected: 5 K, 40 K, 47
+// floats 94, 80, 201 209, 143; two of 47 97, 142; 2.7 K, 13 K, 47 floats 39, 58 (and 5 K, 20 K 43, 60: the line could lie higher).  With fewer than four edges a row on average there are
 // no such rows, or they matter less: 10 K, 25 K, two of 64 36, 45; a sampled layer of 4 K destinations, 41 K edges, eight
 // heads of 8 7, 14.
 bool separate_gradients_are_faster(const LaunchArgs &a, uint32_t edges) {
@@ -2758,8 +2788,7 @@ int nts_gat_aggregate_bwd(float *gx, float *galpha, const float *x, const float 
   a.heads = nts::HeadArgs{perm, H, Fh};
   a.dot_rows = x;
   a.dot_out = galpha;
-  int vec = 1;
-  if (!edges || !perm || !nts::attention_grad_takes(a, &vec) ||
+  if (!edges || !perm || !nts::attention_grad_takes(a) ||
       (co && ri && nts::separate_gradients_are_faster(a, edges))) {
     // Heads wider than the fused kernel's lanes, a structure without its edge permutation, or a size at which it is
     // faster: one pass per gradient.
