@@ -405,7 +405,7 @@ template <int G, bool HEADS, bool RUNS>
 constexpr int group_waves() {
   return HEADS ? 6 : !RUNS && G <= 16 ? 8 : 1;
 }
-template <bool SHARED, int G, int VEC, int U, bool HEADS, bool REMAP, bool RUNS>
+template <bool SHARED, bool PANELS, int G, int VEC, int U, bool HEADS, bool REMAP, bool RUNS>
 __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_group_kernel(const float *__restrict__ in, float *__restrict__ out,
                                                          const float *__restrict__ w,
                                                          const uint32_t *__restrict__ offsets,
@@ -418,8 +418,8 @@ __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_gro
   using V = typename Vec<VEC>::type;
   static_assert(U <= G, "a step's pairs come from one tile");  // U edges per step: their rows are requested together
   const uint32_t gl = threadIdx.x & (G - 1);
-  const uint32_t panel = blockIdx.x % panels;
-  const uint32_t item = (blockIdx.x / panels * blockDim.x + threadIdx.x) / G;
+  const uint32_t panel = PANELS ? blockIdx.x % panels : 0u;
+  const uint32_t item = ((PANELS ? blockIdx.x / panels : blockIdx.x) * blockDim.x + threadIdx.x) / G;
   if (item >= n_items) return;  // whole groups leave together; shuffles stay inside a group
 
   uint32_t row, e0, e1, slot;
@@ -1000,13 +1000,13 @@ void launch_wave(const LaunchArgs &a, uint32_t col_base, uint32_t panels) {
 #undef NTS_LAUNCH_WAVE
 }
 
-template <int G, int VEC, int U = 8, bool SHARED = false>
+template <int G, int VEC, int U = 8, bool SHARED = false, bool PANELS = false>
 void launch_group(const LaunchArgs &a, uint32_t panels = 1) {
   const uint32_t per_block = 256 / G;
   const uint32_t n_list = a.items ? a.n_items : 0u, n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
   const uint32_t blocks = ceil_div(n_total, per_block) * panels;
 #define NTS_LAUNCH_GROUP(HD, RM, RUNS)                                                                                  \
-  hipLaunchKernelGGL((spmm_group_kernel<SHARED, G, VEC, U, HD, RM, RUNS>), dim3(blocks), dim3(256), 0, a.stream, a.in, a.out, a.w, \
+  hipLaunchKernelGGL((spmm_group_kernel<SHARED, PANELS, G, VEC, U, HD, RM, RUNS>), dim3(blocks), dim3(256), 0, a.stream, a.in, a.out, a.w, \
                      a.offsets, a.indices, a.index_base, n_total, n_list, a.F, a.items, a.partial, a.accumulate,        \
                      a.heads,                                                                                          \
                      a.row_edge_limit, a.edge_ids, panels)
@@ -1153,7 +1153,7 @@ void launch_spmm(const LaunchArgs &a) {
   }
   const int vec = pick_vec(a);
   const uint32_t F = a.F;
-  if (const uint32_t panels = die_panels(a, vec)) return F == 128 ? launch_group<16, 4>(a, panels) : launch_group<32, 4>(a, panels);
+  if (const uint32_t panels = die_panels(a, vec)) return F == 128 ? launch_group<16, 4, 8, false, true>(a, panels) : launch_group<32, 4, 8, false, true>(a, panels);
   if (!a.in_ld) {
     switch (narrow_lanes(a, vec)) {
       case kFloats4: return launch_group<4, 1, 4>(a);
