@@ -400,7 +400,9 @@ __global__ __launch_bounds__(256) void spmm_wave_kernel(const float *__restrict_
 // floats 800-1,046 -> 343-861; 1 M, 3 M without a schedule 306 -> 210.
 // With per-head weights the registers are held down to what six wavefronts per SIMD have (98 -> 80; the gather waits
 // for memory): four heads of 32 on 169 K rows, 2.48 M edges 175 -> 146 us, 1 M, 3 M 499 -> 403, 500 K, 20 M 1,066 -> 970; eight
-// wavefronts 157, 419 and 1,028.
+// wavefronts 157, 419 and 1,028.  Without, groups of up to 16 lanes are held to eight (72 -> 63 registers: 1 M, 3 M without a
+// schedule F = 64 219 -> 208, F = 47 211 -> 201); 32 lanes would spill in the loop (2.45 M, 126 M F = 100 and 128 20.4 -> 21.1 ms a
+// step), and rows with runs, held to seven, lose the overlap of their loads (60 K, 600 K F = 17 48 -> 101 us).
 template <int G, bool HEADS, bool RUNS>
 constexpr int group_waves() {
   return HEADS ? 6 : !RUNS && G <= 16 ? 8 : 1;
