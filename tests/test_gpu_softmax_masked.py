@@ -1,0 +1,51 @@
+"""Masked scores (-inf) in the softmax operators: segments of every class -- lane group, registers, wavefront, block, pieces --
+whose first values, most values, or whole pieces are masked.  A masked edge gets exactly 0; the others are held to the
+bound of test_gpu_softmax_lines.py.  A head whose every value is masked has no softmax: NaN, as torch gives it."""
+import pytest
+import torch
+
+from neutronbench_amd.abi import call, ptr
+
+pytestmark = pytest.mark.gpu
+
+V, ROWS = 16500, (100, 500, 1500, 2100, 3000, 30000, 60000, 140000)  # values of a segment; 4,096 edges are a piece
+
+
+@pytest.mark.parametrize("H", [1, 4, 3])  # 3: no power of two, a pass per head
+@pytest.mark.parametrize("masked", ["first", "a tenth", "second half", "all but the last", "all"])
+def test_masked_scores(device, H, masked):
+    deg = torch.zeros(V, dtype=torch.int64)
+    deg[7:7 + len(ROWS)] = torch.tensor([n // H for n in ROWS])
+    deg[100:] = 50
+    deg = deg.to(device)
+    off = torch.cat([deg.new_zeros(1), deg.cumsum(0)])
+    E, co = int(off[-1]), off.to(torch.int32)
+    g = torch.Generator(device=device).manual_seed(H)
+    x = torch.randn(E, H, generator=g, device=device)
+    mask = torch.zeros(E, dtype=torch.bool, device=device)
+    for r in range(7, 7 + len(ROWS)):
+        e0, e1 = int(off[r]), int(off[r + 1])
+        mask[e0:e1] = {"first": lambda k, n: k < 1, "a tenth": lambda k, n: k % 10 == 0, "second half": lambda k, n: k >= n // 2,
+                       "all but the last": lambda k, n: k < n - 1, "all": lambda k, n: k >= 0}[masked](
+                           torch.arange(e1 - e0, device=device), e1 - e0)
+    x[mask] = -torch.inf
+    own = torch.repeat_interleave(torch.arange(V, device=device), deg)
+    wide = x.double()
+    top = torch.full((V, H), -torch.inf, dtype=torch.float64, device=device)
+    top.scatter_reduce_(0, own[:, None].expand(E, H), wide, "amax")
+    ex = (wide - top[own]).exp()
+    want = ex / torch.zeros(V, H, dtype=torch.float64, device=device).index_add_(0, own, ex)[own]
+    bound = ((deg * H).double()[own, None] / 64 + 64) * 2.0 ** -24 + 4e-6
+    s = torch.cuda.current_stream().cuda_stream
+    # the fused form: el of a source of its own per edge, er zero, slope 1
+    el, er, ri = x, torch.zeros(V, H, device=device), torch.arange(E, dtype=torch.int32, device=device)
+    for bounded in (None, 0, int(deg.max())):
+        y = torch.full((E, H), 7.0, device=device)
+        if bounded is None:
+            call("nts_edge_softmax_fwd", ptr(y), ptr(x), ptr(co), V, H, s)
+        else:
+            call("nts_gat_attention_fwd_bounded", ptr(y), ptr(el), ptr(er), ptr(co), ptr(ri), V, H, 1.0, bounded, s)
+        none = want.isnan()
+        assert torch.equal(y.isnan(), none)
+        assert bool(((y.double() - want).abs() <= bound * want)[~none].all())
+        assert bool((y[mask] == 0).all()) or masked == "all"
