@@ -1325,7 +1325,7 @@ inline size_t up256(size_t v) { return (v + 255) / 256 * 256; }
 // either: a long row takes its consecutive partial slots from a counter (integer atomic: which slots a
 // row gets varies from call to call, the order of its pieces inside them and therefore every sum does
 // not), and lists itself for the second stage.
-//   ctr[0] = slots handed out, ctr[1] = rows listed.  Items are pre-filled as empty, so the slots beyond
+//   ctr[0] = slots handed out, ctr[1] = rows listed (one 64-bit counter).  Items are pre-filled as empty, so the slots beyond
 //   the live count cost a wavefront that writes zeros to a slot nobody reads.
 __global__ __launch_bounds__(256) void auto_fill_kernel(Item *__restrict__ items, uint32_t *__restrict__ ctr,
                                                         uint32_t p_max) {
@@ -1343,7 +1343,8 @@ __global__ __launch_bounds__(kCutBlock) void auto_cut_kernel(Item *__restrict__ 
                                                              uint32_t *__restrict__ ctr,
                                                              const uint32_t *__restrict__ off, uint32_t rows,
                                                              uint32_t chunk, uint32_t p_max, uint32_t s_max) {
-  __shared__ uint32_t wave_sums[kCutBlock / kWave], slot_of_block, list_of_block;
+  __shared__ uint32_t wave_sums[kCutBlock / kWave];
+  __shared__ unsigned long long places_of_block;
   const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & (kWave - 1);
   const uint32_t b = off[r < rows ? r : rows], e = off[r < rows ? r + 1 : rows], deg = e - b;
   const uint32_t n = deg > chunk ? (deg + chunk - 1) / chunk : 0u;
@@ -1351,15 +1352,18 @@ __global__ __launch_bounds__(kCutBlock) void auto_cut_kernel(Item *__restrict__ 
   const uint32_t piece = block_prefix<kCutBlock>(n, wave_sums, &n_pieces);  // pieces and cut rows before this one
   const uint32_t nth = block_prefix<kCutBlock>(n != 0 ? 1u : 0u, wave_sums, &n_rows);
   if (n_rows == 0) return;
-  if (threadIdx.x == 0) {
-    slot_of_block = atomicAdd(&ctr[0], n_pieces);
-    list_of_block = atomicAdd(&ctr[1], n_rows);
-  }
+  if (threadIdx.x == 0)  // both counters at once: rows are listed in the order of their slots
+    places_of_block = atomicAdd(reinterpret_cast<unsigned long long *>(ctr),
+                                static_cast<unsigned long long>(n_rows) << 32 | n_pieces);
   __syncthreads();
+  const uint32_t first = static_cast<uint32_t>(places_of_block) + piece;
+  const uint32_t s = static_cast<uint32_t>(places_of_block >> 32) + nth;
   // Slots at or beyond p_max do not exist (only possible when the caller's edge count is smaller than
-  // offsets[rows]): such pieces are not created and not read.
-  const uint32_t first = slot_of_block + piece, s = list_of_block + nth;
-  if (n != 0 && first < p_max && s < s_max) splits[s] = make_uint4(r, first, min(n, p_max - first), 0u);
+  // offsets[rows]): such pieces are not created, and a row without any is listed with none, so that every entry that
+  // the second stage reads was written.  A row with a slot always finds a place: the rows before it in the list took
+  // two slots each at least, and p_max <= 2 s_max - 1 or every row has a place.
+  if (n != 0 && s < s_max)
+    splits[s] = first < p_max ? make_uint4(r, first, min(n, p_max - first), 0u) : make_uint4(0u, 0u, 0u, 0u);
   const uint32_t wave_first_slot = wave_read(first, 0), upto = first + n - wave_first_slot;
   const uint32_t total = wave_read(upto, kWave - 1);
   for (uint32_t t0 = 0; t0 < total; t0 += kWave) {

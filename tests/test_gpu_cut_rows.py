@@ -37,3 +37,40 @@ def test_rows_around_the_piece_length(device, rows, F):
         assert ((out.double() - want).abs() <= (deg.double()[:, None] + 1) * 2.0 ** -24 * size).all()
         outs.append(out)
     assert torch.equal(*outs)
+
+
+ENTRIES = {
+    "plain": lambda x, y, w, off, idx, rows, E, F, s: call("nts_spmm_gather", ptr(x), y, ptr(w), ptr(off), ptr(idx), 0, rows, E, F, 0, s),
+    "static": lambda x, y, w, off, idx, rows, E, F, s: call("nts_spmm_gather_static_scratch", ptr(x), y, ptr(w), ptr(off), ptr(idx),
+                                                            0, rows, E, F, 0, s),
+    "heads": lambda x, y, w, off, idx, rows, E, F, s: call("nts_spmm_gather_heads", ptr(x), y, ptr(w), 0, ptr(off), ptr(idx), rows, E,
+                                                           1, F, 0, s),
+}
+
+
+@pytest.mark.parametrize("entry", list(ENTRIES))
+@pytest.mark.parametrize("rows,each", [(1000, 1000), (100, 20000), (5000, 300), (3000, 257)])
+def test_fewer_edges_stated_than_there_are(device, entry, rows, each):
+    """65,536 edges stated: slots for 256 pieces and one more per possible row.  Rows that got all their slots are right, at
+    most one got some of them, the others keep what they held; nothing is written anywhere else."""
+    F, V, stated = 8, 4000, 65536
+    print(f"case {entry} {rows} {each}", flush=True)
+    g = torch.Generator(device=device).manual_seed(rows)
+    E = rows * each
+    x, w = torch.randn(V, F, generator=g, device=device), torch.rand(E, generator=g, device=device)
+    idx = torch.randint(V, (E,), generator=g, device=device)
+    off = torch.arange(0, E + 1, each, dtype=torch.int32, device=device)
+    terms = (x[idx].double() * w[:, None].double()).view(rows, each, F)
+    n_slots, per_row = stated // 256 + min(rows, stated // 256) + 1, -(-each // 256)
+    for _ in range(3):
+        buf = torch.full((rows + 64, F), 7.0, device=device)
+        ENTRIES[entry](x, buf.data_ptr() + 32 * F * 4, w, off, idx.to(torch.int32), rows, stated, F,
+                       torch.cuda.current_stream().cuda_stream)
+        out = buf[32:32 + rows].double()
+        assert bool((buf[:32] == 7).all()) and bool((buf[32 + rows:] == 7).all())
+        right = ((out - terms.sum(1)).abs() <= (each + 1) * 2.0 ** -24 * terms.abs().sum(1)).all(1)
+        kept = (out == 7).all(1)
+        some = ~right & ~kept
+        assert int(right.sum()) == n_slots // per_row and int(some.sum()) == (1 if n_slots % per_row else 0)
+        part = min(each, n_slots % per_row * 256)
+        assert bool(((out[some] - terms[some, :part].sum(1)).abs() <= (each + 1) * 2.0 ** -24 * terms[some].abs().sum(1)).all())
