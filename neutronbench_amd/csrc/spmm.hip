@@ -1336,35 +1336,48 @@ __global__ __launch_bounds__(256) void auto_fill_kernel(Item *__restrict__ items
 
 // A block asks for the slots of its 1,024 rows at once, because requests to one counter are served some 10 ns apart, and
 // the lanes of a wavefront write its rows' pieces one each, wherever they belong: a hub row of 20,000 edges is 80
-// pieces, which one thread wrote one after the other (2.48 M edges, 169 K rows: 20.7 -> 7.6 us,
-// 12.4 with a request per wavefront).
+// pieces, which one thread wrote one after the other (2.48 M edges, 169 K rows: 20.7 -> 4.9 us; a request per
+// wavefront is slower).  Most blocks and wavefronts of a sampled layer have no row to cut and leave after one look:
+// with a prefix over the block for every one of them 90 K rows took 5.0 us instead of 3.9.
 constexpr int kCutBlock = 1024;
 __global__ __launch_bounds__(kCutBlock) void auto_cut_kernel(Item *__restrict__ items, uint4 *__restrict__ splits,
                                                              uint32_t *__restrict__ ctr,
                                                              const uint32_t *__restrict__ off, uint32_t rows,
                                                              uint32_t chunk, uint32_t p_max, uint32_t s_max) {
-  __shared__ uint32_t wave_sums[kCutBlock / kWave];
-  __shared__ unsigned long long places_of_block;
+  // Slots (low half) and rows (high half) that the block's wavefronts ask for, and where the block's start.
+  __shared__ unsigned long long asked, places_of_block;
   const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & (kWave - 1);
   const uint32_t b = off[r < rows ? r : rows], e = off[r < rows ? r + 1 : rows], deg = e - b;
   const uint32_t n = deg > chunk ? (deg + chunk - 1) / chunk : 0u;
-  uint32_t n_pieces = 0, n_rows = 0;
-  const uint32_t piece = block_prefix<kCutBlock>(n, wave_sums, &n_pieces);  // pieces and cut rows before this one
-  const uint32_t nth = block_prefix<kCutBlock>(n != 0 ? 1u : 0u, wave_sums, &n_rows);
-  if (n_rows == 0) return;
-  if (threadIdx.x == 0)  // both counters at once: rows are listed in the order of their slots
-    places_of_block = atomicAdd(reinterpret_cast<unsigned long long *>(ctr),
-                                static_cast<unsigned long long>(n_rows) << 32 | n_pieces);
+  if (threadIdx.x == 0) asked = 0;
   __syncthreads();
-  const uint32_t first = static_cast<uint32_t>(places_of_block) + piece;
-  const uint32_t s = static_cast<uint32_t>(places_of_block >> 32) + nth;
+  const uint64_t cut = __ballot(n != 0);
+  uint32_t upto = n;  // pieces of the wavefront's rows up to this one
+  unsigned long long before_wave = 0;
+  if (cut) {
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const uint32_t up = __shfl_up(upto, d, kWave);
+      if (lane >= static_cast<uint32_t>(d)) upto += up;
+    }
+    if (lane == kWave - 1) before_wave = atomicAdd(&asked, static_cast<unsigned long long>(__popcll(cut)) << 32 | upto);
+  }
+  __syncthreads();
+  if (asked == 0) return;
+  if (threadIdx.x == 0)  // both counters at once: rows are listed in the order of their slots
+    places_of_block = atomicAdd(reinterpret_cast<unsigned long long *>(ctr), asked);
+  __syncthreads();
+  if (!cut) return;
+  const unsigned long long places = places_of_block + before_wave;  // (the last lane's)
+  const uint32_t wave_slot = wave_read(static_cast<uint32_t>(places), kWave - 1);
+  const uint32_t wave_place = wave_read(static_cast<uint32_t>(places >> 32), kWave - 1);
+  const uint32_t first = wave_slot + upto - n, s = wave_place + __popcll(cut & ((1ull << lane) - 1ull));
   // Slots at or beyond p_max do not exist (only possible when the caller's edge count is smaller than
   // offsets[rows]): such pieces are not created, and a row without any is listed with none, so that every entry that
   // the second stage reads was written.  A row with a slot always finds a place: the rows before it in the list took
   // two slots each at least, and p_max <= 2 s_max - 1 or every row has a place.
   if (n != 0 && s < s_max)
     splits[s] = first < p_max ? make_uint4(r, first, min(n, p_max - first), 0u) : make_uint4(0u, 0u, 0u, 0u);
-  const uint32_t wave_first_slot = wave_read(first, 0), upto = first + n - wave_first_slot;
   const uint32_t total = wave_read(upto, kWave - 1);
   for (uint32_t t0 = 0; t0 < total; t0 += kWave) {
     const uint32_t t = t0 + lane;
@@ -1373,7 +1386,7 @@ __global__ __launch_bounds__(kCutBlock) void auto_cut_kernel(Item *__restrict__ 
     for (uint32_t step = kWave / 2; step >= 1; step >>= 1)
       if (__shfl(upto, own + step - 1, kWave) <= t) own += step;
     const uint32_t before = __shfl(upto - n, own, kWave), rb = __shfl(b, own, kWave), re = __shfl(e, own, kWave);
-    const uint32_t at = wave_first_slot + t, e0 = rb + (t - before) * chunk;
+    const uint32_t at = wave_slot + t, e0 = rb + (t - before) * chunk;
     if (t < total && at < p_max) items[at] = make_uint4(r - lane + own, e0, min(re, e0 + chunk), at);
   }
 }
