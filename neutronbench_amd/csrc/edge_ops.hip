@@ -98,11 +98,15 @@ __global__ __launch_bounds__(256) void edge_copy_kernel(V *__restrict__ msg, con
   // A wavefront walks a contiguous span of wave steps: the destination that owns each step's edges
   // follows from the previous step's (owners_of_step) instead of a search per lane.  Messages that outgrow the caches are
   // walked in turns of some 32 KB, one wavefront's after the other's, so that those in flight write one stretch of
-  // memory: from destinations 2.48 M edges of 128 floats 228 -> 200 us (a fill of as many bytes 184), 8 M 1,013 -> 934, 40 M
-  // of 16 487 -> 444; from sources 1,286 -> 1,224 (8 M of 128).
+  // memory: from destinations 2.48 M edges of 128 floats 228 -> 200 us (a fill of as many bytes 184), 8 M 1,013 -> 934;
+  // from sources 1,286 -> 1,224 (8 M of 128).
   const uint64_t total_steps = (static_cast<uint64_t>(E) + kWave - 1) / kWave;
   const uint64_t per_wave = (total_steps + n_waves - 1) / n_waves;
-  constexpr bool kTurns = sizeof(V) == 16 && G >= 4;  // (for narrower rows the second loop costs more than the order gives)
+  // Rows of up to four vectors have no second loop: the edges are counted on the device, so messages of every size would pay
+  // for its registers (rows of 16 floats: 64 -> 80, eight wavefronts per SIMD -> six; 1.2 M edges from sources 20.6 us and
+  // 21.8 with it, of 12 floats 18.0, 20.4), and the order gives such rows little (8 M edges of 16 147, 147, from destinations
+  // 91.8, 90.5; 40 M 487, 444).
+  constexpr bool kTurns = sizeof(V) == 16 && G >= 8;
   uint64_t span = per_wave;
   if (kTurns && streamed) {
     const uint32_t turn_steps = Fv < kTurnBytes / (kWave * sizeof(V)) ? kTurnBytes / (kWave * sizeof(V)) / Fv : 1u;
