@@ -516,7 +516,7 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
 }
 
 // The same sums for rows that fit one group (Fv <= G), with the rows of a wavefront handed out
-// dynamically: a wavefront takes `set` (at most 64) consecutive rows, reads their offsets with one coalesced load,
+// dynamically: a wavefront takes kFullSet consecutive rows (FEW: `few_rows`, see balanced_rows_per_wave), reads their offsets with one coalesced load,
 // and its 64/G groups then pull rows from that set one after the other -- a group that finishes a
 // short row takes the next pending one instead of idling until the longest row of a fixed
 // assignment is done.  Every group adds its row's edge rows in order (eight loads in flight), so
@@ -535,14 +535,16 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
 // same running fp32 sum (the tile is padded with zeros, and a sum that starts at +0 is never -0, so
 // the padding changes no bit).  A 1,000-edge row of 16-byte values is four such rounds instead of
 // sixteen dependent ones.
-template <typename V, int G, int S>
+template <int GG>  // lanes that share a row
+constexpr uint32_t kFullSet = kWave / GG * 8u < kWave ? kWave / GG * 8u : static_cast<uint32_t>(kWave);
+template <typename V, int G, int S, bool FEW>
 __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__restrict__ out,
                                                                           const V *__restrict__ msg,
                                                                           const uint32_t *__restrict__ off,
                                                                           const uint32_t *__restrict__ perm,
                                                                           uint32_t rows, uint32_t Fv, int accumulate,
                                                                           uint32_t long_limit, uint32_t coop_limit,
-                                                                          uint32_t set, LongRowWork<V> lw) {
+                                                                          uint32_t few_rows, LongRowWork<V> lw) {
   if (blockIdx.x < lw.blocks) {
     sum_long_rows_in_this_block(out, msg, off, perm, Fv, accumulate, lw);
     return;
@@ -554,6 +556,12 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
   constexpr int NF = sizeof(V) / 4;
   const uint32_t lane = lane_id();
   constexpr int GG = G * S;  // lanes that share a row
+  // A constant where it can be (1 M rows of 3 floats 137 us, 143 without); twice `few_rows` where most rows are a lane's own
+  // business (see below), which eight rows a wavefront leave most lanes without (sampled layers' sums over their sources, four
+  // heads, 236 K rows of 655 K edges 30.2 -> 25.9 us, 90 K of 156 K 13.8 -> 10.6; four times as many 25.2 and 10.2, but then
+  // wavefronts with hub rows last longer: 76 K of 87 K with hubs 22 us, 26, 33, always 64 44).
+  uint32_t set = FEW ? few_rows : kFullSet<GG>;
+  if (FEW && G == 1 && sizeof(V) == 16 && off[rows] - off[0] < 4ull * rows) set = min(2u * few_rows, kFullSet<GG>);
   const uint32_t gl = lane & (GG - 1), grp = lane / GG;
   const uint32_t col = gl & (G - 1), slice = gl / G;
   const uint64_t wave = (static_cast<uint64_t>(blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / kWave;
@@ -2121,9 +2129,8 @@ uint32_t streamed_rows_per_wave(uint32_t rows) {
 // where that leaves the chip without its 8,192 wavefronts.  us, always eight per group / so: 16.5 K rows, 300 K edges F = 4
 // 69 / 46, F = 16 133 / 54, F = 128 214 / 206; 100 K, 8 M F = 1 209 / 172, F = 32 682 / 411; 169 K, 2.48 M F = 1 78 / 67, F = 32
 // 193 / 145 (not below 16 rows: 16.5 K F = 16 68, 100 K F = 32 441); from 524,288 rows up the same.
-uint32_t balanced_rows_per_wave(uint32_t rows, uint32_t lanes) {
+uint32_t balanced_rows_per_wave(uint32_t rows, uint32_t set) {
   constexpr uint32_t kChipWaves = 8192;
-  uint32_t set = std::min<uint32_t>(kWave / lanes * 8, kWave);
   while (set > 8 && rows / set < kChipWaves) set /= 2;
   return set;
 }
@@ -2153,11 +2160,15 @@ void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_
     // One group covers a row: wavefronts hand their 64 rows out dynamically (strided launch).
 #define NTS_BALANCED(GG, SS)                                                                                    \
   do {                                                                                                          \
-    const uint32_t set = balanced_rows_per_wave(rows, (GG) * (SS));                                            \
+    const uint32_t set = balanced_rows_per_wave(rows, kFullSet<(GG) * (SS)>);                                  \
     const uint32_t blocks = ceil_div(rows, 4 * set); /* at most `set` rows per wavefront at a time */          \
-    hipLaunchKernelGGL((gather_edge_to_row_balanced_kernel<V, GG, SS>),                                         \
-                       dim3((blocks < 16384u ? blocks : 16384u) + lw.blocks), dim3(256), 0, stream, out, msg, off, \
-                       perm, rows, Fv, accumulate, limit, coop_limit(), set, lw);                                   \
+    const dim3 grid((blocks < 16384u ? blocks : 16384u) + lw.blocks);                                          \
+    if (set < kFullSet<(GG) * (SS)>)                                                                            \
+      hipLaunchKernelGGL((gather_edge_to_row_balanced_kernel<V, GG, SS, (kFullSet<(GG) * (SS)> > 8)>), grid, dim3(256), 0, stream, out, msg, \
+                         off, perm, rows, Fv, accumulate, limit, coop_limit(), set, lw);                        \
+    else                                                                                                        \
+      hipLaunchKernelGGL((gather_edge_to_row_balanced_kernel<V, GG, SS, false>), grid, dim3(256), 0, stream, out, msg, \
+                         off, perm, rows, Fv, accumulate, limit, coop_limit(), set, lw);                        \
   } while (0)
     switch (lanes_for(Fv)) {  // rows narrower than eight lanes are shared by eight lanes all the same
       case 1: NTS_BALANCED(1, 8); break;

@@ -71,7 +71,7 @@ def test_streamed_sums_at_the_steps_of_rows_a_wavefront(device, rows, F):
 
 
 @pytest.mark.parametrize("rows", [4096, 65535, 65537, 131071, 262143, 524288])
-@pytest.mark.parametrize("F", [1, 8, 33, 128])
+@pytest.mark.parametrize("F", [1, 4, 8, 33, 128])
 def test_permuted_sums_at_the_steps_of_rows_a_wavefront(device, rows, F):
     """8 to 64 rows a wavefront, by the number of rows and their width; whole numbers, so that any order is exact."""
     rng = np.random.default_rng(rows + F)

@@ -50,6 +50,7 @@ FLOAT4 = "15HIP_vector_typeIfLj4EE"
 
 @pytest.mark.parametrize("kernel,most", [
     (f"edge_copy_kernelI{FLOAT4}Li4E", 64),  # rows of up to 16 floats copied to edges
+    (f"gather_edge_to_row_balanced_kernelI{FLOAT4}Li64ELi1ELb0E", 64),  # permuted sums of rows of 132 to 256 floats
 ])
 def test_registers(kernels, kernel, most):
     found = [k for name, k in kernels.items() if kernel in name]
