@@ -906,7 +906,8 @@ struct LaunchArgs {
   uint32_t partial_ld = 0;                     // row stride of `partial` in floats (0 = F)
   bool dup_runs = false;                       // rows hold runs of equal indices worth loading once per run
   uint32_t scheduled_rows = 0;                 // rows of the schedule that `items` comes from (0: no schedule)
-  uint32_t scheduled_edges = 0;                // and its edges
+  uint32_t edges = 0;                          // edges of the rows, as the caller or the schedule has them
+  bool bounded = false;                        // the caller knows that no row has more than kAutoChunk edges
   uint32_t rows_after_items = 0;               // with items: this many whole rows follow the listed items in the launch
   const float *dot_rows = nullptr;             // with dot_out: the rows whose products with the gathered ones
   float *dot_out = nullptr;                    // are the gradient of alpha (attention_grad_kernel)
@@ -1097,53 +1098,120 @@ uint32_t die_panels(const LaunchArgs &a, int vec) {
   return a.F == 256 ? 2 : a.F == 512 ? 4 : 0;
 }
 
-// Lanes of a narrow row, by what bounds the launch.  Lanes of one float (16 or 32 a row, 64 up to 64 floats) cover more pairs a
-// tile and leave fewer rows to a wavefront, which is what counts while a launch lasts as long as its long rows and
-// pieces; lanes of four floats take fewer instructions a row, which counts where the chip is full.  us, four floats / one:
-//   scheduled, F = 16   2.7 K rows, 11 K edges 33 / 16, 169 K, 2.48 M 117 / 44, 1 M, 3 M 137 / 66, 500 K, 20 M 350 / 165
-//   scheduled, F = 32   2.7 K 23 / 15, 60 K, 600 K 63 / 32, 169 K 72 / 49, 500 K, 1.5 M 73 / 57, 300 K, 4.5 M 85 / 77; but
-//                       50 K, 8 M 78 / 95, 1 M, 3 M 97 / 106, 500 K, 20 M 243 / 280: six million edges, a row counting four
-//   scheduled, F = 64   2.7 K 20 / 15, 20 K, 300 K 46 / 29, 60 K 54 / 39, 50 K, 8 M 112 / 101; but 169 K 71 / 74, 500 K, 20 M
-//                       376 / 452, and rows with runs of equal indices 20 K 63 / 78
-//   no schedule, F = 16 5 K, 40 K 66 / 26, 60 K, 600 K 63 / 42, 300 K, 4.5 M 178 / 165; but 50 K, 8 M, mostly pieces, 152 / 158 and
-//                       1 M, 3 M 131 / 135
-//   no schedule, F = 32 20 K 39 / 33, 60 K 53 / 45; but 169 K 82 / 90
-//   no schedule, F = 64 5 K 36 / 24, 20 K 40 / 31, 60 K 51 / 51
-// Up to eight floats a group of that many lanes where pieces are most of the work or the rows are many (F = 3, 16 lanes and 4:
-// 50 K, 8 M 157 / 140, 1 M, 3 M 134 / 120).  Sixteen edges a step instead of eight where the rows are few: scheduled F = 16
-// 169 K 53 -> 44, 1 M 66 -> 71; F = 32 60 K 40 -> 32, 169 K 49 -> 53; no schedule 5 K 47 -> 41, 20 K 34 -> 35.
-// Rows off 16-byte boundaries of 25 lanes and more take a wavefront of 4-byte lanes where the chip is full of dense rows:
-// F = 127 50 K, 8 M 267 / 243, 300 K, 4.5 M 304 / 295; but 60 K 54 / 71, 1 M, 3 M 377 / 411; F = 201 50 K, 8 M 438 / 383, 169 K 227 / 219, 60 K
-// 63 / 117; no schedule 5 K 30 / 76, 169 K 243 / 272, 300 K 496 / 535, but 1 M, 3 M 648 / 642 and F = 129 525 / 486.
+// Lanes of a narrow row.  A group of G lanes fetches G edge pairs at a time and works on one row, so what counts is how
+// long the rows are and how many of them there are:
+//   lanes of one float (16 or 32 a row, 64 up to 64 floats) put fewer rows into a wavefront and request more edges of a
+//     row at once: for launches that last as long as their longest rows or pieces, or that do not fill the chip;
+//   lanes of four floats take fewer instructions a row: where there are many rows.
+// Rows off 16-byte boundaries take the latter too (SHARED), a wavefront of 4-byte lanes otherwise.
 enum NarrowLanes {
   kFloats4, kFloats8, kFloats16, kFloats16x16, kFloats32, kFloats32x16, kFloats64, kVectors4, kVectors8, kVectors16, kVectors32, kVectors64, kWide
 };
+struct RowShape {
+  uint32_t rows, F, lanes;          // lanes: of four floats that a row takes
+  uint64_t edges;
+  bool vectors, aligned;            // rows (heads) of four floats and more; of 16-byte boundaries throughout
+  bool longer(uint64_t n) const { return edges >= n * rows; }  // rows of n edges and more on average
+};
+NarrowLanes fewest_lanes(const RowShape &s) {
+  if (!s.vectors) return s.F <= 4 ? kFloats4 : s.F <= 8 ? kFloats8 : s.F <= 16 ? kFloats16 : s.F <= 32 ? kFloats32 : kWide;
+  if (s.lanes <= 4) return kVectors4;
+  if (s.lanes <= 8) return kVectors8;
+  if (s.lanes <= 16) return kVectors16;
+  return s.lanes <= 32 ? kVectors32 : kWide;
+}
+
+// Rows of a schedule, whose long rows are pieces of their own.  Every line below was measured over 24 graphs of 2 K to 2.4 M
+// rows and 2 to 200 edges a row, in turn over several sets of arrays; us, four floats a lane (the fewest lanes) / others:
+//   F = 16   eight lanes of four (each row's half idle): 100 K rows, 300 K edges 18 -> 16, 1 M, 3 M 89 -> 59, 2.4 M, 6 M 256 -> 174; from
+//            eight edges a row 16 lanes of one float: 60 K, 600 K 25 -> 18, 169 K, 2.48 M 70 -> 33, and there 16 edges a step from
+//            twelve edges a row (169 K 35 -> 33, 300 K, 4.5 M 63 -> 53; 1 M, 8 M 112 -> 118); up to 65,536 rows one float in any case
+//            (20 K, 60 K 11.6 -> 10.5, but 169 K, 500 K 18.6 -> 21)
+//   F = 7    8 lanes of one float, 16 from eight edges a row: 300 K, 900 K 24, 27, 300 K, 4.5 M 79, 62; 5 K, 1 M 28, 30
+//   F = 32   8 lanes of four.  16 lanes 300 K, 4.5 M 98 -> 80, 169 K, 2.48 M 50 -> 44, but 500 K, 20 M 244 -> 262, 500 K, 1.5 M 49 -> 52; 32
+//            of one float 20 K, 60 K 11.9 -> 10.9, but 100 K, 300 K 16 -> 21, 300 K, 900 K 34 -> 43, 500 K, 1.5 M 49 -> 65
+//   F = 31   32 lanes of one float 20 K, 60 K 11.7, eight of four 13.3, 16 12.5; 100 K, 300 K 22, 19, 20; 300 K, 4.5 M 100, 127, 104; 50 K,
+//            8 M 103, 106, 100; with repeated edges 100 K, 20 M F = 17 276, 238, 256
+//   F = 64   16 lanes of four; a wavefront 100 K, 300 K 21 -> 32, 60 K, 600 K 24 -> 32
+//   F = 47   16 lanes of four; a wavefront of 4-byte lanes 300 K, 900 K 75, 44, 100 K, 20 M with ranges 650, 261; but 50 K, 8 M 102, 110
+//   F = 127  32 lanes of four; a wavefront 169 K, 500 K 77, 69, 500 K, 20 M with ranges 1,050, 861; but 50 K, 8 M 207, 221
+//   F = 201  64 lanes of four 8 K, 30 K 15.6 -> 12.8, 20 K, 3 M 130 -> 119; but 50 K, 8 M 324 -> 363, and F = 129 20 K, 3 M 88 -> 103
+NarrowLanes scheduled_lanes(const RowShape &s, bool dup_runs) {
+  const bool large = s.edges > 1u << 20, few = s.rows <= 1u << 15;
+  if (s.F <= 16) {
+    if (s.longer(8)) return s.F <= 8 && !large && s.longer(64) ? kFloats8 : large && s.longer(12) ? kFloats16x16 : kFloats16;
+    if (s.rows <= 1u << 16) return kFloats16;
+    return s.F <= 8 ? kFloats8 : s.vectors ? kVectors8 : kFloats16;
+  }
+  if (!s.vectors) return fewest_lanes(s);
+  if (s.F <= 32) {
+    if (few && (!s.longer(8) || (!s.aligned && !s.longer(128)))) return kFloats32;
+    const bool sixteen = large && s.longer(8) && (s.aligned ? !s.longer(32) : !dup_runs || !s.longer(64));
+    return sixteen || s.lanes > 8 ? kVectors16 : kVectors8;
+  }
+  const bool dense = !s.aligned && !dup_runs && s.longer(128);
+  if (s.lanes <= 16) return dense ? kWide : kVectors16;
+  if (s.lanes <= 32) return dense && s.lanes > 24 ? kWide : kVectors32;
+  return !s.aligned && few && s.lanes >= 48 && s.lanes <= 64 ? kVectors64 : kWide;
+}
+
+// Calls without a schedule.  `bounded`: the caller knows that no row is long (sampled layers), so one launch of whole rows;
+// `pieces` > 0: rows above 256 edges are cut into up to so many; otherwise a launch of whole rows among which one may be
+// long, and lasts as long as that one.  Measured on sampled layers of R-MAT graphs, their transposed structures, and whole
+// graphs; us, the fewest lanes / others:
+//   bounded     F = 16 1 K rows, 5 K edges 6.2 -> 4.1 with 16 of one float, 28 K, 272 K 7.3 -> 6.8; but 133 K, 655 K 12 -> 14; F = 64 1 K
+//               4.9 -> 4.2 with a wavefront; but 16 K, 156 K 8.2 -> 10.2, 32 K of five 6.9 -> 14; F = 32 with 32 of one 5 K, 118 K 6.9 ->
+//               5.1; but 28 K 7.8 -> 8.4, 32 K of five 6.0 -> 6.5; F = 201 64 of four 133 K 97 -> 93, but 5 K, 118 K 15 -> 16
+//   whole rows  F = 16 5 K, 40 K 107 -> 41 with 16 of one float and 16 edges a step; F = 32 68 -> 36 with 32; F = 64 56 -> 37 with a
+//               wavefront; sources of a sampled layer 28 K, 37 K 8.9 -> 10.6; F = 201 78 -> 30 with 64 of four
+//   pieces      F = 16 60 K, 600 K 63 -> 41, 300 K, 4.5 M 177 -> 166; 1 M, 3 M 131 -> 133; F = 8 255 K, 343 K 59 -> 37; F = 7 eight lanes
+//               of one 169 K, 2.48 M 67, 16 73; F = 32 60 K, 600 K 51 -> 45 with 32 of one; but 169 K 82 -> 90; F = 17 100 K, 300 K with
+//               eight of four 41 -> 47, 256 K, 343 K 46 -> 47, 1 M, 3 M 172 -> 131; F = 47 32 K, 100 K with 16 of four 32 -> 39, 54 K, 118 K
+//               33 -> 30, 300 K, 900 K 102 -> 69; F = 201 64 of four 89 K, 156 K 69 -> 51, but rows of 1.4 edges 117 -> 124
+NarrowLanes plain_lanes(const RowShape &s, bool bounded, uint32_t pieces) {
+  const uint32_t items = s.rows + pieces;
+  const bool mostly_pieces = pieces > s.rows;
+  if (s.F <= 16) {
+    if (bounded) {
+      if (s.rows <= 1u << 15) return kFloats16;
+      return s.F <= 4 ? kFloats4 : s.F <= 8 ? kFloats8 : s.aligned ? fewest_lanes(s) : kFloats16;
+    }
+    if (s.F <= 8 && pieces && (mostly_pieces || items > 1u << 18 || s.edges > 1u << 20)) return s.F <= 4 ? kFloats4 : kFloats8;
+    if (s.vectors && (mostly_pieces || items > 1u << 19)) return fewest_lanes(s);
+    return items <= 1u << 14 ? kFloats16x16 : kFloats16;
+  }
+  if (!s.vectors) return fewest_lanes(s);
+  if (s.F <= 32) {
+    if (bounded) {
+      if (s.rows <= 1u << (s.aligned ? 14 : 15)) return kFloats32;
+      return !s.aligned && s.rows <= 1u << 16 ? kVectors16 : fewest_lanes(s);
+    }
+    const bool floats = items <= 1u << (pieces ? 16 : 15) ||
+                        (!s.aligned && !mostly_pieces && s.rows <= 1u << (s.longer(2) ? 17 : 18));
+    return !floats ? fewest_lanes(s) : items <= 1u << 14 && s.longer(2) ? kFloats32x16 : kFloats32;
+  }
+  if (s.F <= 64) {
+    const bool floats = bounded ? s.rows <= 1u << 11 : pieces ? s.rows <= 1u << 15 && (!s.aligned || s.longer(8)) : s.rows <= 3u << 13;
+    return floats ? kFloats64 : fewest_lanes(s);
+  }
+  if (s.lanes <= 32 || s.lanes > 64 || s.aligned || mostly_pieces || items > 3u << 17) return fewest_lanes(s);
+  return (bounded ? !s.longer(16) : pieces ? 2 * s.edges >= 3ull * s.rows : s.rows <= 1u << 15) ? kVectors64 : kWide;
+}
+
 NarrowLanes narrow_lanes(const LaunchArgs &a, int vec) {
-  const uint32_t F = a.F, H = a.heads.H, width = H ? a.heads.Fh : F;
-  const uint32_t lanes = (H ? H : 1u) * ceil_div(width, 4);
+  const uint32_t H = a.heads.H ? a.heads.H : 1u, width = a.heads.H ? a.heads.Fh : a.F;
   const uint32_t n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
-  const bool scheduled = a.scheduled_rows != 0, no_vectors = width < 4;
-  const bool few = scheduled ? a.scheduled_edges + 4ull * a.scheduled_rows <= 6000000 : n_total <= 1u << (F <= 16 ? 14 : 16);
-  const bool pieces = !scheduled && a.rows_after_items && a.n_items > a.rows_after_items;
-  if (F <= 16) {
-    if (F <= 8 && (pieces || (!scheduled && n_total > 1u << 18))) return F <= 4 ? kFloats4 : kFloats8;
-    if (no_vectors || scheduled || !(pieces || n_total > 1u << 19)) return few ? kFloats16x16 : kFloats16;
-  } else if (F <= 32) {
-    if (no_vectors || few) return n_total <= (scheduled ? 1u << 17 : 1u << 14) ? kFloats32x16 : kFloats32;
-  } else if (F <= 64 && !a.dup_runs && n_total <= (scheduled ? 1u << 17 : 1u << 15)) {
-    return kFloats64;
+  RowShape s{n_total, a.F, 0u, a.edges, width >= 4, vec == 4};
+  const uint64_t lanes = static_cast<uint64_t>(H) * ceil_div(width, 4);
+  s.lanes = lanes > 64 ? 65u : static_cast<uint32_t>(lanes);
+  if (n_total >= 1u << 28) return fewest_lanes(s);  // 16 lanes a row would be more threads than a launch can have
+  if (a.scheduled_rows) {
+    s.rows = a.scheduled_rows;
+    return scheduled_lanes(s, a.dup_runs);
   }
-  if (no_vectors) return kWide;
-  if (lanes <= 4) return kVectors4;
-  if (lanes <= 8) return kVectors8;
-  if (lanes <= 16) return kVectors16;
-  if (vec == 4) return lanes <= 32 ? kVectors32 : kWide;
-  const bool short_schedule = scheduled && few && n_total <= 1u << 17;
-  if (lanes <= 32) {
-    const bool dense = scheduled && !a.dup_runs && lanes > 24 && a.scheduled_edges / 8 > a.scheduled_rows;
-    return dense && !short_schedule ? kWide : kVectors32;
-  }
-  return lanes <= 64 && !pieces && (scheduled ? short_schedule : n_total <= 3u << 17) ? kVectors64 : kWide;
+  const uint32_t pieces = a.items ? a.n_items : 0u;
+  s.rows = n_total - pieces;
+  return plain_lanes(s, a.bounded, pieces);
 }
 
 void launch_spmm(const LaunchArgs &a) {
@@ -1469,6 +1537,7 @@ int launch_spmm_cut_small(const LaunchArgs &a, uint32_t edges, unsigned char *fi
 // (nothing is allocated or freed then; a call that needs more is refused).
 int launch_spmm_balanced(LaunchArgs a, uint32_t edges, unsigned char *fixed = nullptr, size_t fixed_cap = 0) {
   const uint32_t rows = a.n_items;
+  a.edges = edges;
   if (edges < kAutoMinEdges) {
     launch_spmm(a);
     return NTS_OK;
@@ -1988,6 +2057,8 @@ int nts_spmm_gather_bounded(const float *in, float *out, const float *w, const u
   if (rows == 0) return NTS_OK;
   nts::LaunchArgs a{in, out, w, offsets, indices, index_base, rows, F, nullptr, nullptr, accumulate, stream};
   if (max_row_edges != 0 && max_row_edges <= nts::kAutoChunk) {
+    a.edges = edges;
+    a.bounded = true;
     // No row can need cutting: one launch, a wavefront (or lane group) per row, no scratch.
     nts::launch_spmm(a);
   } else if (int rc = nts::launch_spmm_balanced(a, edges)) {
@@ -2785,6 +2856,8 @@ int nts_spmm_gather_heads_bounded(const float *in, float *out, const float *alph
   nts::LaunchArgs a{in, out, alpha, offsets, indices, 0u, rows, H * Fh, nullptr, nullptr, accumulate, stream};
   a.heads = nts::HeadArgs{perm, H, Fh};
   if (max_row_edges != 0 && max_row_edges <= nts::kAutoChunk) {
+    a.edges = edges;
+    a.bounded = true;
     nts::launch_spmm(a);
   } else if (int rc = nts::launch_spmm_balanced(a, edges)) {
     return rc;
@@ -2842,7 +2915,7 @@ int nts_spmm_gather_heads_planned(nts_spmm_plan_t *plan, const float *in, float 
                     F,   plan->items, plan->partial, accumulate, stream};
   a.heads = nts::HeadArgs{perm, H, Fh};
   a.scheduled_rows = plan->rows;
-  a.scheduled_edges = plan->edges;
+  a.edges = plan->edges;
   if (plan->sorted_idx) {
     a.indices = plan->sorted_idx;
     a.edge_ids = plan->edge_ids;
@@ -2889,7 +2962,7 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
   }
   a.dup_runs = use_runs(plan);
   a.scheduled_rows = plan->rows;
-  a.scheduled_edges = plan->edges;
+  a.edges = plan->edges;
   if (const uint32_t ld = padded_stride(plan, F, false)) {
     // Rows off 16-byte boundaries: gather from a padded copy with 16-byte lanes.
     const uint64_t vecs = static_cast<uint64_t>(plan->n_index) * (ld / 4);

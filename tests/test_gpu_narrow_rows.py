@@ -91,3 +91,35 @@ def test_heads(device, rows, edges, H, Fh):
     plan = SpmmPlan(off, rows, edges, 64, idx, rows, 4)
     check(device, rows, off, idx, dst, H, Fh, Fh % 4, lambda x, y, w, acc: call(
         "nts_spmm_gather_heads_planned", plan.handle, ptr(x), ptr(y), ptr(w), 0, ptr(off), ptr(idx), H, Fh, acc, s))
+
+
+def even_graph(rows, edges, seed, device):
+    """Rows of about as many edges each, none of 256."""
+    g = torch.Generator(device=device).manual_seed(seed)
+    dst = torch.randint(rows, (edges,), generator=g, device=device).sort().values
+    off = torch.zeros(rows + 1, dtype=torch.int64, device=device)
+    off[1:] = torch.bincount(dst, minlength=rows).cumsum(0)
+    idx = torch.randint(rows, (edges,), generator=g, device=device).to(torch.int32)
+    return off.to(torch.int32), idx, dst
+
+
+# 2,048, 16,384, 32,768 and 65,536 rows are lines of calls that bound their rows, 16 edges a row another
+@pytest.mark.parametrize("rows,edges", [(2048, 40000), (2049, 9000), (16385, 90000), (32768, 100000), (32769, 100000), (65537, 200000)])
+@pytest.mark.parametrize("F", [3, 4, 7, 8, 15, 16, 17, 32, 47, 64, 129, 201])
+def test_bounded_rows(device, rows, edges, F):
+    off, idx, dst = even_graph(rows, edges, 8, device)
+    s = torch.cuda.current_stream().cuda_stream
+    check(device, rows, off, idx, dst, 1, F, F % 4, lambda x, y, w, acc: call(
+        "nts_spmm_gather_bounded", ptr(x), ptr(y), ptr(w), ptr(off), ptr(idx), 0, rows, edges, F, acc, 256, s))
+
+
+# 8, 12, 32, 64 and 128 edges a row, 32,768 and 65,536 rows and 2^20 edges are lines of the schedules
+@pytest.mark.parametrize("rows,edges", [(65537, 500000), (65536, 500000), (120000, 1100000), (90000, 1100000), (33000, 1100000),
+                                        (16400, 1100000), (8000, 1100000), (3000, 200000), (32768, 262144)])
+@pytest.mark.parametrize("F", [3, 7, 8, 13, 16, 17, 32, 47, 65, 127, 201])
+def test_scheduled_rows_by_their_length(device, rows, edges, F):
+    off, idx, dst = even_graph(rows, edges, 9, device)
+    s = torch.cuda.current_stream().cuda_stream
+    plan = SpmmPlan(off, rows, edges, 64)
+    check(device, rows, off, idx, dst, 1, F, F % 4, lambda x, y, w, acc: call(
+        "nts_spmm_gather_planned", plan.handle, ptr(x), ptr(y), ptr(w), ptr(off), ptr(idx), 0, F, acc, s))
