@@ -1094,6 +1094,7 @@ int pick_vec(const LaunchArgs &a) {
 // once a panel) and calls without a schedule (133 / 149: mostly short rows) too.
 uint32_t die_panels(const LaunchArgs &a, int vec) {
   if (vec != 4 || !a.scheduled_rows || a.heads.H || a.dup_runs || a.in_ld) return 0;
+  if (a.n_items >= 1u << 24) return 0;  // (up to 128 threads an item: a launch has fewer than 2^32)
   if (a.F == 128) return static_cast<uint64_t>(a.scheduled_rows) * a.F * sizeof(float) > kAllL2Bytes ? 2 : 0;
   return a.F == 256 ? 2 : a.F == 512 ? 4 : 0;
 }
@@ -1710,29 +1711,32 @@ __global__ __launch_bounds__(256) void plan_cut_rows_kernel(uint32_t *__restrict
                                                             const uint32_t *__restrict__ idx, uint32_t index_base,
                                                             uint32_t rows, PlanShape sh) {
   const uint32_t gl = threadIdx.x & (kCutLanes - 1), group = (threadIdx.x & (kWave - 1)) / kCutLanes;
-  const uint32_t r = blockIdx.x * (blockDim.x / kCutLanes) + threadIdx.x / kCutLanes;
-  if (r >= rows) return;
-  const uint32_t b = off[r], e = off[r + 1], deg = e - b;
-  const uint32_t R = sh.ranges_for(deg);
-  if (R == 0) return;  // the table was cleared: a whole row has no pieces
-  uint32_t *cnt = counts + static_cast<size_t>(r) * sh.n_slabs;
-  uint32_t *stp = stops + static_cast<size_t>(r) * sh.n_slabs;
-  const uint32_t per = sh.n_slabs / R;
-  uint32_t cut = b, nonempty = 0;
-  for (uint32_t c0 = 0; c0 < R; c0 += kCutLanes) {
-    const uint32_t c = c0 + gl;
-    const uint64_t hi = static_cast<uint64_t>(c + 1) * per * sh.fine_width;  // first index of the next range
-    const uint32_t stop = c + 1 >= R ? e : lower_bound_index(idx, cut, e, hi, index_base);
-    const uint32_t up = __shfl_up(stop, 1, kCutLanes), n = stop - (gl ? up : cut);
-    if (c < R) {
-      cnt[c] = deg > sh.chunk ? (n + sh.chunk - 1) / sh.chunk : (n ? 1u : 0u);
-      stp[c] = stop;
+  const uint32_t per_block = blockDim.x / kCutLanes;
+  for (uint64_t r64 = static_cast<uint64_t>(blockIdx.x) * per_block + threadIdx.x / kCutLanes; r64 < rows;
+       r64 += static_cast<uint64_t>(gridDim.x) * per_block) {
+    const uint32_t r = static_cast<uint32_t>(r64);
+    const uint32_t b = off[r], e = off[r + 1], deg = e - b;
+    const uint32_t R = sh.ranges_for(deg);
+    if (R == 0) continue;  // the table was cleared: a whole row has no pieces
+    uint32_t *cnt = counts + static_cast<size_t>(r) * sh.n_slabs;
+    uint32_t *stp = stops + static_cast<size_t>(r) * sh.n_slabs;
+    const uint32_t per = sh.n_slabs / R;
+    uint32_t cut = b, nonempty = 0;
+    for (uint32_t c0 = 0; c0 < R; c0 += kCutLanes) {
+      const uint32_t c = c0 + gl;
+      const uint64_t hi = static_cast<uint64_t>(c + 1) * per * sh.fine_width;  // first index of the next range
+      const uint32_t stop = c + 1 >= R ? e : lower_bound_index(idx, cut, e, hi, index_base);
+      const uint32_t up = __shfl_up(stop, 1, kCutLanes), n = stop - (gl ? up : cut);
+      if (c < R) {
+        cnt[c] = deg > sh.chunk ? (n + sh.chunk - 1) / sh.chunk : (n ? 1u : 0u);
+        stp[c] = stop;
+      }
+      nonempty += __popcll(__ballot(c < R && n) >> (group * kCutLanes) & ((1ull << kCutLanes) - 1));
+      cut = __shfl(stop, kCutLanes - 1, kCutLanes);
     }
-    nonempty += __popcll(__ballot(c < R && n) >> (group * kCutLanes) & ((1ull << kCutLanes) - 1));
-    cut = __shfl(stop, kCutLanes - 1, kCutLanes);
+    if (deg <= sh.chunk && nonempty <= 1)  // all edges in one wide range: the row stays whole
+      for (uint32_t c = gl; c < R; c += kCutLanes) cnt[c] = 0;
   }
-  if (deg <= sh.chunk && nonempty <= 1)  // all edges in one wide range: the row stays whole
-    for (uint32_t c = gl; c < R; c += kCutLanes) cnt[c] = 0;
 }
 
 __global__ __launch_bounds__(256) void plan_emit_pieces_kernel(Item *__restrict__ pieces, uint32_t *__restrict__ keys,
@@ -2511,7 +2515,8 @@ int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const
     NTS_HIP_TRY(hipMemsetAsync(counters, 0, sizeof(nts::PlanCounters), stream));
     NTS_HIP_TRY(scan_edges(indices));  // counts the repeated edges of the copy
   }
-  hipLaunchKernelGGL(nts::plan_cut_rows_kernel, dim3(nts::ceil_div(rows, 256 / nts::kCutLanes)), dim3(256), 0, stream, counts,
+  // (16 threads a row are more than a launch can have from 2^28 rows up)
+  hipLaunchKernelGGL(nts::plan_cut_rows_kernel, dim3(std::min(nts::ceil_div(rows, 256 / nts::kCutLanes), 1u << 20)), dim3(256), 0, stream, counts,
                      stops, offsets, indices, index_base, rows, sh);
   NTS_LAUNCH_CHECK("plan_cut_rows_kernel");
   NTS_HIP_TRY(rocprim::exclusive_scan(tmp1, scan_bytes, counts, slot_base, 0u, cells + 1, rocprim::plus<uint32_t>(),
