@@ -1084,19 +1084,26 @@ int pick_vec(const LaunchArgs &a) {
 }
 
 // Column panels whose blocks alternate, so that an XCD (blocks are dealt out to the eight in turn) meets one panel only and
-// its 4 MB L2 holds a share of the gathered matrix that is as many times smaller.  A panel has to be whole lines (512
-// bytes, or 256 of a row of 512) and the number of panels has to divide eight; shorter requests cost more than they gain (64 bytes:
-// 2.8 times the time, 128: as much as without), and so do panels that share lines.  us without / with: 169 K rows, 2.48 M
+// its 4 MB L2 holds a share of the gathered matrix that is as many times smaller.  A panel is whole lines (512
+// bytes, or 256 of a row of 512) and the number of panels divides eight; shorter requests cost more than they gain (64 bytes:
+// 2.8 times the time, 128: as much as without).  us without / with: 169 K rows, 2.48 M
 // edges F = 128 111 / 98, 256 251 / 221, 512 584 / 451; 500 K, 20 M with source ranges 722 / 690, 1,437 / 1,388, 3,137 /
-// 2,746; 2.45 M, 126 M 5,221 / 5,108, 11,255 / 10,386; F = 300, 384 and 500 as panels of 128 331 / 404, 396 / 424, 609 / 526
-// and 1,968 / 2,312, 2,249 / 2,362, 3,330 / 3,071.  Rows of 512 bytes that the L2s hold together lose (20 K rows, 4 M edges 93 / 95), rows
-// loaded once per run of equal indices (233 K, 114.8 M F = 128 2,277 / 2,346), heads (169 K 155 / 199: the weights are read
-// once a panel) and calls without a schedule (133 / 149: mostly short rows) too.
+// 2,746; 2.45 M, 126 M 5,221 / 5,108, 11,255 / 10,386.  Panels that share lines lose or gain by width and graph (F = 300, 384
+// and 500 as panels of 128 331 / 404, 396 / 424, 609 / 526 and 1,968 / 2,312, 2,249 / 2,362, 3,330 / 3,071) and are not taken; eight
+// panels (F = 1,024) were not measured.  Without them stay:
+//   rows of 512 bytes that the L2s hold together (20 K rows, 4 M edges 93 / 95; wider rows gain there too: F = 256 and 512 2 K, 8 K
+//     11.4 / 11.5, 12.0 / 11.1, 5 K, 60 K 14.3 / 14.2, 18.1 / 16.9, 20 K, 300 K 33 / 32, 58 / 51, 60 K, 600 K 60 / 55, 124 / 96)
+//   rows of 2 KB with fewer than five edges each once they fill the chip, which are read once or twice whatever the caches hold,
+//     while every panel walks the short rows again: 32 K, 100 K 34 / 37, 130 K, 300 K 126 / 139, 300 K, 600 K 267 / 290, 2.45 M, 5 M
+//     2,402 / 2,667, 10 M 3,782 / 4,042; but 2 K, 8 K 12 / 10, 300 K, 1.5 M 492 / 438, 600 K, 3 M 1,008 / 985
+//   rows loaded once per run of equal indices (233 K, 114.8 M F = 128 2,277 / 2,346), heads (169 K 155 / 199: the weights are
+//     read once a panel) and calls without a schedule (133 / 149: mostly short rows)
 uint32_t die_panels(const LaunchArgs &a, int vec) {
   if (vec != 4 || !a.scheduled_rows || a.heads.H || a.dup_runs || a.in_ld) return 0;
   if (a.n_items >= 1u << 24) return 0;  // (up to 128 threads an item: a launch has fewer than 2^32)
   if (a.F == 128) return static_cast<uint64_t>(a.scheduled_rows) * a.F * sizeof(float) > kAllL2Bytes ? 2 : 0;
-  return a.F == 256 ? 2 : a.F == 512 ? 4 : 0;
+  if (a.F == 512) return a.n_items > kChipWaves && a.edges < 5ull * a.scheduled_rows ? 0 : 4;
+  return a.F == 256 ? 2 : 0;
 }
 
 // Lanes of a narrow row.  A group of G lanes fetches G edge pairs at a time and works on one row, so what counts is how

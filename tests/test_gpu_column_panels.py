@@ -33,6 +33,14 @@ def test_panels_of_whole_lines(device, rows, edges, ranges, rising, F):
     compare(device, plan, off, idx, rows, edges, F, F - 4)
 
 
+# few rows, and rows of 2 KB on both sides of five edges each and of 8,192 items
+@pytest.mark.parametrize("rows,edges", [(3, 70), (100, 3000), (2000, 8000), (8192, 24000), (8193, 24000), (30000, 149000), (30000, 151000)])
+@pytest.mark.parametrize("F", [256, 512])
+def test_panels_on_small_graphs(device, rows, edges, F):
+    off, idx = graph(rows, edges, 9, device, True)
+    compare(device, SpmmPlan(off, rows, edges, 4096), off, idx, rows, edges, F, F - 4)
+
+
 # 8,192 items are what the chip holds; 640 columns are one panel of 4-byte lanes, 2,560 of 16-byte lanes
 @pytest.mark.parametrize("rows", [100, 8191, 8192, 8193])
 @pytest.mark.parametrize("F,narrow", [(641, 639), (1433, 637), (2564, 2560)])
