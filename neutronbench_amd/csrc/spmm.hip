@@ -1013,7 +1013,10 @@ void launch_group(const LaunchArgs &a, uint32_t panels = 1) {
                      a.offsets, a.indices, a.index_base, n_total, n_list, a.F, a.items, a.partial, a.accumulate,        \
                      a.heads,                                                                                          \
                      a.row_edge_limit, a.edge_ids, panels)
-  if (a.edge_ids) {
+  if constexpr (PANELS) {  // neither heads nor repeated indices (die_panels)
+    if (a.edge_ids) NTS_LAUNCH_GROUP(false, true, false);
+    else NTS_LAUNCH_GROUP(false, false, false);
+  } else if (a.edge_ids) {
     if (a.heads.H) NTS_LAUNCH_GROUP(true, true, false);
     else if (a.dup_runs) NTS_LAUNCH_GROUP(false, true, true);
     else NTS_LAUNCH_GROUP(false, true, false);
