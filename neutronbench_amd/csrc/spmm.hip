@@ -590,8 +590,10 @@ __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_gro
 // Requesting the rows of two steps ahead was slower everywhere (0.85 times: a third fewer wavefronts fit).
 //
 // Wavefronts per SIMD that the registers are held down for.  The rows of wide groups come from memory, and six
-// wavefronts with two spilled values outside the loop beat four (1.5 M vertices, 5 M edges, four heads of 32 1,050 -> 854
-// us); narrower ones lose more by the spills than they gain (30 K, 300 K, eight of 4 with six 93, without 52 us).
+// wavefronts with one or two spilled values outside the loop beat four (1.5 M vertices, 5 M edges, four heads of 32 1,050 -> 854
+// us); narrower ones lose more by the spills than they gain (30 K, 300 K, eight of 4 with six 93, without 52 us).  The forms
+// that share columns spill two to four, and six still beat five, whose spills are one or two (1 M, 4 M 8 x 17 786, 859 us, 4 x 25 590, 636,
+// 2 x 47 575, 600; 169 K, 2.48 M 304, 316, 235, 236, 235, 223).
 template <int G, int LH, int NJ, int VEC>
 constexpr int grad_waves() {
   if (VEC != 4 || NJ != 1 || LH == 1) return 1;
@@ -927,13 +929,15 @@ bool attention_grad_takes(const LaunchArgs &a) { return ceil_div(a.heads.Fh, a.h
 //   1 x 47           --                     50 / 49       167 / 164       405 / 400    1,227 / 1,201
 //   8 x 13           73 / 92                64 / 51       432 / 254       1,311 / 649  3,298 / 1,746
 //   8 x 47           96 / 104               87 / 93       704 / 714       2,012 / 2,052
+// Two and three heads of 33 to 48 floats take one float a lane where rows are short: 2 x 47 sampled layers 90 K rows, 156 K edges
+// 46 / 48, 54 K, 118 K 44 / 45, but 169 K, 2.48 M 242 / 235; 3 x 47 60 / 63, 54 / 57, 1 M, 4 M 800 / 817, but 169 K 312 / 306.
 // Heads of 65 to 256 floats of such rows took a pass per gradient: 1 x 101 127 -> 65 on 20 K, 622 -> 245, 1,458 -> 640, 4,713 -> 1,679.
 bool grad_floats_are_faster(const LaunchArgs &a) {
   const uint32_t Fh = a.heads.Fh, rows = a.n_items + (a.items ? a.rows_after_items : 0u);
   if (Fh > kGradMaxVecs) return false;
   const uint64_t lanes = static_cast<uint64_t>(a.heads.H) * (Fh <= 4 ? 4 : Fh <= 8 ? 8 : ceil_div(Fh, 16) * 16);
   if (Fh < 4 || lanes <= 16 || (lanes <= 32 && rows <= 1u << 19)) return true;
-  if (Fh > 32) return Fh <= 48 && a.heads.H >= 4;
+  if (Fh > 32) return Fh <= 48 && (a.heads.H >= 4 || (a.heads.H >= 2 && a.edges < 8ull * rows));
   return rows <= (lanes <= 64 ? 1u << 15 : 1u << 13);
 }
 

@@ -56,12 +56,12 @@ def test_both_gradients(device, H, Fh, V, E, skew):
 
 
 # rows off 16-byte boundaries: lanes of one float and of four that share columns, by width, heads and rows (8,192, 32,768 and
-# 524,288 are lines)
-@pytest.mark.parametrize("V,E", [(700, 5000), (9000, 70000), (33000, 70000), (530000, 540000)])
-@pytest.mark.parametrize("H,Fh", [(1, 5), (1, 17), (2, 6), (4, 5), (4, 13), (8, 13), (4, 47), (3, 49), (1, 66), (1, 129), (1, 255)])
+# 524,288 are lines), two and three heads of 33 to 48 floats by the edges a row (eight)
+@pytest.mark.parametrize("V,E", [(700, 5000), (700, 6000), (9000, 70000), (9000, 75000), (33000, 70000), (530000, 540000)])
+@pytest.mark.parametrize("H,Fh", [(1, 5), (1, 17), (2, 6), (4, 5), (4, 13), (8, 13), (2, 33), (3, 47), (4, 47), (3, 49), (1, 66),
+                                  (1, 129), (1, 255)])
 def test_rows_off_16_byte_boundaries(device, H, Fh, V, E):
-    if V < 100000 or H * Fh <= 64:
-        test_both_gradients(device, H, Fh, V, E, 0)
+    test_both_gradients(device, H, Fh, V, E, 0)
 
 
 def test_empty_structure(device):
