@@ -965,9 +965,10 @@ __device__ __forceinline__ float leaky(float s, float slope) { return s > 0.f ? 
 // 2e-9 of the segment's largest term), well inside the 1e-4 these operators are held to.
 __device__ __forceinline__ float softmax_exp(float x) { return __expf(x); }
 
-// What a running sum subtracts from its terms while `m` is the largest value met: m, or 0 while nothing but masked values
-// (-inf) has been met, whose exponentials are then the zeros that they are and not exp(-inf + inf).
-__device__ __forceinline__ float sum_base(float m) { return m == -INFINITY ? 0.f : m; }
+// Where the running maxima of a (maximum, sum of exp(v - maximum)) pair start: the lowest float and not -inf, so that a
+// masked value (-inf) that comes first adds exp(-inf) = 0 and not exp(-inf + inf).  A head without any other value keeps
+// a sum of 0 and becomes 0 / 0.
+constexpr float kLowestMax = -3.402823466e38f;
 
 // Multi-pass softmax forward of one segment with 16-byte lanes (H a multiple of 4, 16-byte aligned
 // arrays): lane l of a group of WIDTH threads takes the vectors l, l + WIDTH, ... of the segment, i.e.
@@ -985,17 +986,16 @@ __device__ __forceinline__ void strided_max_sum_pass4(uint64_t first, uint64_t n
       m[2] = fmaxf(m[2], v[u].z);
       m[3] = fmaxf(m[3], v[u].w);
     }
-    const float base[4] = {sum_base(m[0]), sum_base(m[1]), sum_base(m[2]), sum_base(m[3])};
     float add[4] = {0.f, 0.f, 0.f, 0.f};
     for (int u = 0; u < count; ++u) {
-      add[0] += softmax_exp(v[u].x - base[0]);
-      add[1] += softmax_exp(v[u].y - base[1]);
-      add[2] += softmax_exp(v[u].z - base[2]);
-      add[3] += softmax_exp(v[u].w - base[3]);
+      add[0] += softmax_exp(v[u].x - m[0]);
+      add[1] += softmax_exp(v[u].y - m[1]);
+      add[2] += softmax_exp(v[u].z - m[2]);
+      add[3] += softmax_exp(v[u].w - m[3]);
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      sum[c] = sum[c] * softmax_exp(mx[c] - base[c]) + add[c];  // mx = -inf at the start: the old sum is 0 and stays 0
+      sum[c] = sum[c] * softmax_exp(mx[c] - m[c]) + add[c];  // (at the start the old sum is 0 and stays 0)
       mx[c] = m[c];
     }
   };
@@ -1066,18 +1066,17 @@ __device__ __forceinline__ void strided_max_sum_pass(uint64_t first, uint64_t n,
       seen(i + u * stride, v[u]);
       m = fmaxf(m, v[u]);
     }
-    const float base = sum_base(m);
     float add = 0.f;
 #pragma unroll
-    for (int u = 0; u < U; ++u) add += softmax_exp(v[u] - base);
-    sum = sum * softmax_exp(mx - base) + add;  // mx = -inf at the start: the old sum is 0 and stays 0
+    for (int u = 0; u < U; ++u) add += softmax_exp(v[u] - m);
+    sum = sum * softmax_exp(mx - m) + add;  // (at the start the old sum is 0 and stays 0)
     mx = m;
   }
   for (; i < n; i += stride) {
     const float v = load(i);
     seen(i, v);
-    const float m = fmaxf(mx, v), base = sum_base(m);
-    sum = sum * softmax_exp(mx - base) + softmax_exp(v - base);
+    const float m = fmaxf(mx, v);
+    sum = sum * softmax_exp(mx - m) + softmax_exp(v - m);
     mx = m;
   }
 }
@@ -1357,7 +1356,7 @@ __global__ __launch_bounds__(256) void edge_softmax_fwd_kernel(float *__restrict
           if (FUSED) erv = *reinterpret_cast<const float4 *>(er + static_cast<size_t>(d) * H + h0);
           const float4 *xs4 = reinterpret_cast<const float4 *>(xs);
           float4 *ys4 = reinterpret_cast<float4 *>(ys);
-          float mx4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY}, sum4[4] = {0.f, 0.f, 0.f, 0.f};
+          float mx4[4] = {kLowestMax, kLowestMax, kLowestMax, kLowestMax}, sum4[4] = {0.f, 0.f, 0.f, 0.f};
           strided_max_sum_pass4<4>(
               lane, n / 4, kWave,
               [&](uint64_t i) -> float4 {
@@ -1389,7 +1388,7 @@ __global__ __launch_bounds__(256) void edge_softmax_fwd_kernel(float *__restrict
         const uint32_t h = lane & (H - 1);
         float erv = 0.f;
         if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
-        float mx = -INFINITY, sum = 0.f;
+        float mx = kLowestMax, sum = 0.f;
         strided_max_sum_pass<8>(
             lane, n, kWave,
             [&](uint64_t i) -> float {
@@ -1621,7 +1620,7 @@ __global__ __launch_bounds__(kLongBlock) void edge_softmax_fwd_long_kernel(
     const float *xs = FUSED ? nullptr : x + base;
     float erv = 0.f;
     if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
-    float mx = -INFINITY, sum = 0.f;
+    float mx = kLowestMax, sum = 0.f;
     strided_max_sum_pass<8>(
         threadIdx.x, n, kLongBlock,
         [&](uint64_t j) -> float {
@@ -1710,7 +1709,7 @@ __global__ __launch_bounds__(kLongBlock) void giant_softmax_stats_kernel(
     const float *xs = FUSED ? nullptr : x + base;
     float erv = 0.f;
     if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
-    float mx = -INFINITY;
+    float mx = kLowestMax;
     strided_pass<8>(threadIdx.x, n, kLongBlock,
                     [&](uint64_t j) -> float {
                       if (!FUSED) return xs[j];
@@ -1722,10 +1721,9 @@ __global__ __launch_bounds__(kLongBlock) void giant_softmax_stats_kernel(
                       mx = fmaxf(mx, sc);
                     });
     mx = block_head_reduce<0>(mx, H, red);
-    const float piece_base = sum_base(mx);
     float sum = 0.f;
     strided_pass<8>(threadIdx.x, n, kLongBlock, [&](uint64_t j) -> float { return FUSED ? ys[j] : xs[j]; },
-                    [&](uint64_t, float sc) { sum += softmax_exp(sc - piece_base); });
+                    [&](uint64_t, float sc) { sum += softmax_exp(sc - mx); });
     sum = block_head_reduce<1>(sum, H, red);
     if (threadIdx.x < H) {
       stats[static_cast<size_t>(p) * 2 * H + threadIdx.x] = mx;

@@ -1,6 +1,7 @@
-"""Masked scores (-inf) in the softmax operators: segments of every class -- lane group, registers, wavefront, block, pieces --
-whose first values, most values, or whole pieces are masked.  A masked edge gets exactly 0; the others are held to the
-bound of test_gpu_softmax_lines.py.  A head whose every value is masked has no softmax: NaN, as torch gives it."""
+"""Masked scores (-inf, or the lowest float) in the softmax operators: segments of every class -- lane group, registers,
+wavefront, block, pieces -- whose first values, most values, or whole pieces are masked.  A masked edge gets exactly 0; the
+others are held to the bound of test_gpu_softmax_lines.py.  A head whose every value is masked has no softmax with -inf
+(NaN, as torch gives it) and equal parts with the lowest float."""
 import pytest
 import torch
 
@@ -13,7 +14,8 @@ V, ROWS = 16500, (100, 500, 1500, 2100, 3000, 30000, 60000, 140000)  # values of
 
 @pytest.mark.parametrize("H", [1, 4, 3])  # 3: no power of two, a pass per head
 @pytest.mark.parametrize("masked", ["first", "a tenth", "second half", "all but the last", "all"])
-def test_masked_scores(device, H, masked):
+@pytest.mark.parametrize("value", [-torch.inf, torch.finfo(torch.float32).min])
+def test_masked_scores(device, H, masked, value):
     deg = torch.zeros(V, dtype=torch.int64)
     deg[7:7 + len(ROWS)] = torch.tensor([n // H for n in ROWS])
     deg[100:] = 50
@@ -28,13 +30,19 @@ def test_masked_scores(device, H, masked):
         mask[e0:e1] = {"first": lambda k, n: k < 1, "a tenth": lambda k, n: k % 10 == 0, "second half": lambda k, n: k >= n // 2,
                        "all but the last": lambda k, n: k < n - 1, "all": lambda k, n: k >= 0}[masked](
                            torch.arange(e1 - e0, device=device), e1 - e0)
-    x[mask] = -torch.inf
+    x[mask] = value
     own = torch.repeat_interleave(torch.arange(V, device=device), deg)
     wide = x.double()
-    top = torch.full((V, H), -torch.inf, dtype=torch.float64, device=device)
-    top.scatter_reduce_(0, own[:, None].expand(E, H), wide, "amax")
-    ex = (wide - top[own]).exp()
-    want = ex / torch.zeros(V, H, dtype=torch.float64, device=device).index_add_(0, own, ex)[own]
+
+    def per_row(v, reduce):  # rows 7 .. one by one, the rows of 50 edges together
+        out = torch.zeros(V, H, dtype=torch.float64, device=device)
+        for r in range(7, 7 + len(ROWS)):
+            out[r] = reduce(v[int(off[r]):int(off[r + 1])], 0)
+        out[100:] = reduce(v[int(off[100]):].view(V - 100, 50, H), 1)
+        return out
+
+    ex = (wide - per_row(wide, torch.amax)[own]).exp()
+    want = ex / per_row(ex, torch.sum)[own]
     bound = ((deg * H).double()[own, None] / 64 + 64) * 2.0 ** -24 + 4e-6
     s = torch.cuda.current_stream().cuda_stream
     # the fused form: el of a source of its own per edge, er zero, slope 1
