@@ -224,7 +224,8 @@ int nts_spmm_plan_create(nts_spmm_plan_t **plan, const uint32_t *offsets, uint32
                          uint32_t edges, uint32_t chunk_edges, nts_stream_t stream);
 /* The same schedule, made cache-aware.  It is built where `offsets` and `indices` (the gather index array that belongs
  * to `offsets`) lie; they are read back to the host, once, only if offsets[0] > 0, if the memory that ordering rows takes
- * (some 36 bytes an edge) is not to be had, or if NTS_SPMM_PLAN_HOST=1 is set.  The call synchronises `stream`.
+ * (some 25 bytes an edge; 36 below 65,536 edges, or where a row, an index and a place in the row need more than 64 bits)
+ * is not to be had, or if NTS_SPMM_PLAN_HOST=1 is set.  The call synchronises `stream`.
  * The pieces of split rows whose indices ascend are cut at the
  * boundaries of `n_slabs` equal ranges of [index_base, index_base + n_index) and issued slab by slab,
  * so that concurrently running wavefronts gather from the same range of source rows (each XCD's
@@ -420,8 +421,7 @@ int nts_sddmm_heads(float *galpha, const float *in, const float *gout, const uin
  *   gx[s, h*Fh + f] (+)= sum_{k in CSR(s)} alpha[perm[k], h] * gout[ci[k], h*Fh + f]
  *   galpha[perm[k], h] = < x[s, h*Fh : (h+1)*Fh], gout[ci[k], h*Fh : (h+1)*Fh] >
  * i.e. nts_spmm_gather_heads over the CSR and nts_sddmm_heads over the CSC, which the call falls back to
- * for heads of more than 64 vectors (256 floats; 64 floats where Fh or an array is off a 16-byte boundary),
- * when perm is NULL (alpha and galpha then as those two calls take them), and, where co and ri are given, at
+ * for heads of more than 256 floats, when perm is NULL (alpha and galpha then as those two calls take them), and, where co and ri are given, at
  * sizes at which they are faster (wide rows of graphs of few edges).
  * Scratch as nts_spmm_gather.  accumulate applies to gx. */
 int nts_gat_aggregate_bwd(float *gx, float *galpha, const float *x, const float *gout, const float *alpha,

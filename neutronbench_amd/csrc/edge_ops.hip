@@ -1018,7 +1018,7 @@ __device__ __forceinline__ void strided_max_sum_pass4(uint64_t first, uint64_t n
 // Three kernels share a launch, by segment size n = degree * H (values):
 //   short   n <= 128, power-of-two H <= 16: a group of 16 lanes per destination, the segment held
 //           in registers -- one pass over memory, four destinations per wavefront in flight;
-//   wave    up to kLongRowValues (or any size when the block kernel is not used): one wavefront per
+//   wave    up to long_segment_values of the call (or any size when the block kernel is not used): one wavefront per
 //           destination; segments of at most 512 values are register-resident too, larger ones take
 //           the three passes (max, sum, write) / two passes (dot, write) over memory;
 //   block   longer segments (hub destinations), listed by collect_long_rows.
@@ -2347,8 +2347,9 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
                  float slope, hipStream_t stream, const char *who, uint32_t max_degree = 0) {
   const bool pow2 = is_pow2(H) && H <= kWave;
   LongRows lr;
-  // A caller that bounds every segment below the block kernels' class (a sampled layer: at most `fanout`
-  // edges per destination) needs none of the launches that look for hub rows; a longer segment than
+  // A caller that bounds every segment below the block kernels' class where it begins highest (a sampled layer: at most
+  // `fanout` edges per destination) needs none of the launches that look for hub rows: every segment is a wavefront's,
+  // also one that a call without a bound would hand to a block because its values are few in all.  A longer segment than
   // stated is still computed, by one wavefront.
   const bool no_hubs = max_degree != 0 && static_cast<uint64_t>(max_degree) * H <= kLongRowValues;
   if (pow2 && !no_hubs)

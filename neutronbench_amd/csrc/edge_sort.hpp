@@ -1,4 +1,4 @@
-// Stable radix sort of 64-bit elements by a run of their bits, for edge lists of 10^6 elements and more: a graph's
+// Stable radix sort of 64-bit elements by a run of their bits, for edge lists of 65,536 elements and more: a graph's
 // edges by source and by destination (layout.hip), a schedule's edges by row and index (spmm.hip).
 //
 // Least significant digit first, digits of equal width of at most nine bits, so an 18-bit vertex id is two passes.

@@ -215,8 +215,8 @@ __global__ __launch_bounds__(256) void spmm_wave_kernel(const float *__restrict_
     if (e1 - e0 > row_edge_limit) return;  // a long row: its pieces are separate work items
   }
 
-  // Lanes past the end of the row (only possible in the last accumulator) read the row's last
-  // VEC columns instead, so that loads need no predication; their sums are never stored.
+  // Lanes past the end of the row (in the last accumulator; where one launch covers all panels, in any of the last
+  // panel's) read the row's last VEC columns instead, so that loads need no predication; their sums are never stored.
   uint32_t col[NACC];
   uint32_t lcol[NACC];
   uint32_t head[NACC];
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(256) void spmm_wave_kernel(const float *__restrict_
 // earlier, shares columns with the lane before it and stores only its own.  16-byte lanes at any float instead of a
 // wavefront of 4-byte ones for a row of 47 floats: 500 K rows, 20 M edges with source ranges 809 -> 416 us, and from 33 to 127
 // floats 800-1,046 -> 343-861; 1 M, 3 M without a schedule 306 -> 210.
-// With per-head weights the registers are held down to what six wavefronts per SIMD have (98 -> 80; the gather waits
+// With per-head weights the registers are held down to what six wavefronts per SIMD have (90-96 -> 75-77; the gather waits
 // for memory): four heads of 32 on 169 K rows, 2.48 M edges 175 -> 146 us, 1 M, 3 M 499 -> 403, 500 K, 20 M 1,066 -> 970; eight
 // wavefronts 157, 419 and 1,028.  Without, groups of up to 16 lanes are held to eight (72 -> 63 registers: 1 M, 3 M without a
 // schedule F = 64 219 -> 208, F = 47 211 -> 201); 32 lanes would spill in the loop (2.45 M, 126 M F = 100 and 128 20.4 -> 21.1 ms a
@@ -2408,8 +2408,8 @@ int build_plan(nts_spmm_plan_t **plan_out, const uint32_t *offsets_dev, const st
 // Builds the schedule of make_schedule on the device (kernels above).  *fell_back is set, and nothing built,
 //  - where the first row does not start at edge 0: the edges before it belong to no row, while the kernels
 //    give every edge to the row before it (row 0 would be ordered together with them);
-//  - where rows have to be ordered and the sort's memory, some 36 bytes an edge with the ordered copies, is not to
-//    be had: the host orders them with the copies alone on the device, 8 bytes an edge.
+//  - where rows have to be ordered and the sort's memory, some 25 bytes an edge with the ordered copies (36 with the
+//    library's sort), is not to be had: the host orders them with the copies alone on the device, 8 bytes an edge.
 int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const uint32_t *indices,
                       uint32_t index_base, uint32_t n_index, uint32_t rows, uint32_t edges, uint32_t chunk,
                       uint32_t n_slabs, hipStream_t stream, bool *fell_back) {

@@ -1,6 +1,6 @@
 """Segments on both sides of the lines between the wavefront, block and piece kernels of the softmax operators, which
 lie where the call's own number of values puts them: at 1/1,024 and 1/256 of it, within 2,048 .. 32,768 and
-32,768 .. 131,072 values.
+32,768 .. 131,072 values.  With 16 and 64 heads a segment above the last line is a single piece.
 
 A segment of n values is summed by chains of at most n / 64 additions whose results are added in trees: off by at most
 (n / 64 + 64) 2^-24 of the sum of its terms' magnitudes.  An exponential is off by |x| 2^-24 of itself (|x| < 32 here:
@@ -29,7 +29,7 @@ def degrees(total, H, V):
     return deg
 
 
-@pytest.mark.parametrize("total,H", [(1 << 20, 1), (1 << 20, 4), (10000000, 4), (10000000, 1), (1 << 26, 4), (1 << 26, 16)])
+@pytest.mark.parametrize("total,H", [(1 << 20, 1), (1 << 20, 4), (1 << 20, 16), (1 << 21, 64), (10000000, 4), (10000000, 1), (1 << 26, 4), (1 << 26, 16)])
 def test_softmax_on_both_sides_of_the_lines(device, total, H):
     print(f"case total={total} H={H}", flush=True)
     V, slope = 16500, 0.2
