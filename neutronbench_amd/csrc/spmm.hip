@@ -1146,10 +1146,13 @@ NarrowLanes fewest_lanes(const RowShape &s) {
 //   F = 32   8 lanes of four.  16 lanes 300 K, 4.5 M 98 -> 80, 169 K, 2.48 M 50 -> 44, but 500 K, 20 M 244 -> 262, 500 K, 1.5 M 49 -> 52; 32
 //            of one float 20 K, 60 K 11.9 -> 10.9, but 100 K, 300 K 16 -> 21, 300 K, 900 K 34 -> 43, 500 K, 1.5 M 49 -> 65
 //   F = 31   32 lanes of one float 20 K, 60 K 11.7, eight of four 13.3, 16 12.5; 100 K, 300 K 22, 19, 20; 300 K, 4.5 M 100, 127, 104; 50 K,
-//            8 M 103, 106, 100; with repeated edges 100 K, 20 M F = 17 276, 238, 256
+//            8 M 103, 106, 100; 200 K, 1.7 M 51, 55, 49, 200 K, 7 M 112, 149, 123, 50 K, 4.5 M 65, 80, 71 (F = 21 101, 126, 107 and 64, 74, 66,
+//            but 100 K, 4 M 61, 60, 54); with repeated edges 100 K, 20 M F = 17 276, 238, 256
 //   F = 64   16 lanes of four; a wavefront 100 K, 300 K 21 -> 32, 60 K, 600 K 24 -> 32
-//   F = 47   16 lanes of four; a wavefront of 4-byte lanes 300 K, 900 K 75, 44, 100 K, 20 M with ranges 650, 261; but 50 K, 8 M 102, 110
-//   F = 127  32 lanes of four; a wavefront 169 K, 500 K 77, 69, 500 K, 20 M with ranges 1,050, 861; but 50 K, 8 M 207, 221
+//   F = 47   a wavefront of 4-byte lanes / 16 of four: 300 K, 900 K 75, 44, 120 K, 7.5 M 134, 128, 50 K, 3.2 M 59, 60, 50 K, 4.5 M 69, 80, 20 K,
+//            2.3 M 40, 43, 50 K, 8 M 102, 110; 100 K, 20 M with ranges 650, 261
+//   F = 127  a wavefront / 32 of four: 169 K, 500 K 77, 69, 50 K, 2 M 80, 79, 120 K, 7.5 M 272, 292, 90 K, 8 M 267, 286, 50 K, 8 M 207, 221 (F = 90
+//            120 K, 7.5 M 195, 200, 90 K, 8 M 195, 197); 500 K, 20 M with ranges 1,050, 861
 //   F = 201  64 lanes of four 8 K, 30 K 15.6 -> 12.8, 20 K, 3 M 130 -> 119; but 50 K, 8 M 324 -> 363, and F = 129 20 K, 3 M 88 -> 103
 NarrowLanes scheduled_lanes(const RowShape &s, bool dup_runs) {
   const bool large = s.edges > 1u << 20, few = s.rows <= 1u << 15;
@@ -1160,13 +1163,14 @@ NarrowLanes scheduled_lanes(const RowShape &s, bool dup_runs) {
   }
   if (!s.vectors) return fewest_lanes(s);
   if (s.F <= 32) {
-    if (few && (!s.longer(8) || (!s.aligned && !s.longer(128)))) return kFloats32;
+    const bool one = few || (s.lanes > 6 && s.longer(16) && !dup_runs);
+    if ((few && !s.longer(8)) || (one && !s.aligned && !s.longer(128))) return kFloats32;
     const bool sixteen = large && s.longer(8) && (s.aligned ? !s.longer(32) : !dup_runs || !s.longer(64));
     return sixteen || s.lanes > 8 ? kVectors16 : kVectors8;
   }
-  const bool dense = !s.aligned && !dup_runs && s.longer(128);
-  if (s.lanes <= 16) return dense ? kWide : kVectors16;
-  if (s.lanes <= 32) return dense && s.lanes > 24 ? kWide : kVectors32;
+  const bool ones = !s.aligned && !dup_runs;
+  if (s.lanes <= 16) return ones && s.longer(64) ? kWide : kVectors16;
+  if (s.lanes <= 32) return ones && s.lanes > 24 && s.longer(32) ? kWide : kVectors32;
   return !s.aligned && few && s.lanes >= 48 && s.lanes <= 64 ? kVectors64 : kWide;
 }
 

@@ -113,10 +113,10 @@ def test_bounded_rows(device, rows, edges, F):
         "nts_spmm_gather_bounded", ptr(x), ptr(y), ptr(w), ptr(off), ptr(idx), 0, rows, edges, F, acc, 256, s))
 
 
-# 8, 12, 32, 64 and 128 edges a row, 32,768 and 65,536 rows and 2^20 edges are lines of the schedules
+# 8, 12, 16, 32, 64 and 128 edges a row, 32,768 and 65,536 rows and 2^20 edges are lines of the schedules
 @pytest.mark.parametrize("rows,edges", [(65537, 500000), (65536, 500000), (120000, 1100000), (90000, 1100000), (33000, 1100000),
                                         (16400, 1100000), (8000, 1100000), (3000, 200000), (32768, 262144)])
-@pytest.mark.parametrize("F", [3, 7, 8, 13, 16, 17, 32, 47, 65, 127, 201])
+@pytest.mark.parametrize("F", [3, 7, 8, 13, 16, 17, 31, 32, 47, 65, 127, 201])
 def test_scheduled_rows_by_their_length(device, rows, edges, F):
     off, idx, dst = even_graph(rows, edges, 9, device)
     s = torch.cuda.current_stream().cuda_stream
