@@ -908,6 +908,7 @@ struct LaunchArgs {
   uint32_t partial_ld = 0;                     // row stride of `partial` in floats (0 = F)
   bool dup_runs = false;                       // rows hold runs of equal indices worth loading once per run
   uint32_t scheduled_rows = 0;                 // rows of the schedule that `items` comes from (0: no schedule)
+  bool ranged = false;                         // a schedule with source ranges: rows are cut where these end
   uint32_t edges = 0;                          // edges of the rows, as the caller or the schedule has them
   bool bounded = false;                        // the caller knows that no row has more than kAutoChunk edges
   uint32_t rows_after_items = 0;               // with items: this many whole rows follow the listed items in the launch
@@ -1150,11 +1151,12 @@ NarrowLanes fewest_lanes(const RowShape &s) {
 //            but 100 K, 4 M 61, 60, 54); with repeated edges 100 K, 20 M F = 17 276, 238, 256
 //   F = 64   16 lanes of four; a wavefront 100 K, 300 K 21 -> 32, 60 K, 600 K 24 -> 32
 //   F = 47   a wavefront of 4-byte lanes / 16 of four: 300 K, 900 K 75, 44, 120 K, 7.5 M 134, 128, 50 K, 3.2 M 59, 60, 50 K, 4.5 M 69, 80, 20 K,
-//            2.3 M 40, 43, 50 K, 8 M 102, 110; 100 K, 20 M with ranges 650, 261
+//            2.3 M 40, 43, 50 K, 8 M 102, 110; with source ranges 20 K, 1.8 M 41, 45, 34 K, 6.5 M 115, 117 (F = 33 106, 102), 120 K, 6.4 M 145,
+//            141, 100 K, 16.4 M 283, 264, with repeated edges too 100 K, 20 M 650, 261
 //   F = 127  a wavefront / 32 of four: 169 K, 500 K 77, 69, 50 K, 2 M 80, 79, 120 K, 7.5 M 272, 292, 90 K, 8 M 267, 286, 50 K, 8 M 207, 221 (F = 90
-//            120 K, 7.5 M 195, 200, 90 K, 8 M 195, 197); 500 K, 20 M with ranges 1,050, 861
+//            120 K, 7.5 M 195, 200, 90 K, 8 M 195, 197); with source ranges 34 K, 6.5 M 206, 192, 500 K, 20 M with repeated edges 1,050, 861
 //   F = 201  64 lanes of four 8 K, 30 K 15.6 -> 12.8, 20 K, 3 M 130 -> 119; but 50 K, 8 M 324 -> 363, and F = 129 20 K, 3 M 88 -> 103
-NarrowLanes scheduled_lanes(const RowShape &s, bool dup_runs) {
+NarrowLanes scheduled_lanes(const RowShape &s, bool ranged, bool dup_runs) {
   const bool large = s.edges > 1u << 20, few = s.rows <= 1u << 15;
   if (s.F <= 16) {
     if (s.longer(8)) return s.F <= 8 && !large && s.longer(64) ? kFloats8 : large && s.longer(12) ? kFloats16x16 : kFloats16;
@@ -1168,9 +1170,8 @@ NarrowLanes scheduled_lanes(const RowShape &s, bool dup_runs) {
     const bool sixteen = large && s.longer(8) && (s.aligned ? !s.longer(32) : !dup_runs || !s.longer(64));
     return sixteen || s.lanes > 8 ? kVectors16 : kVectors8;
   }
-  const bool ones = !s.aligned && !dup_runs;
-  if (s.lanes <= 16) return ones && s.longer(64) ? kWide : kVectors16;
-  if (s.lanes <= 32) return ones && s.lanes > 24 && s.longer(32) ? kWide : kVectors32;
+  if (s.lanes <= 16) return !s.aligned && s.longer(64) && (few ? !dup_runs : !ranged) ? kWide : kVectors16;
+  if (s.lanes <= 32) return !s.aligned && s.longer(32) && s.lanes > 24 && !ranged ? kWide : kVectors32;
   return !s.aligned && few && s.lanes >= 48 && s.lanes <= 64 ? kVectors64 : kWide;
 }
 
@@ -1226,7 +1227,7 @@ NarrowLanes narrow_lanes(const LaunchArgs &a, int vec) {
   if (n_total >= 1u << 28) return fewest_lanes(s);  // 16 lanes a row would be more threads than a launch can have
   if (a.scheduled_rows) {
     s.rows = a.scheduled_rows;
-    return scheduled_lanes(s, a.dup_runs);
+    return scheduled_lanes(s, a.ranged, a.dup_runs);
   }
   const uint32_t pieces = a.items ? a.n_items : 0u;
   s.rows = n_total - pieces;
@@ -2055,6 +2056,7 @@ struct nts_spmm_plan {
   // At least 1 in 20 edges repeats the gather index of the edge before it: the wave kernel then loads
   // a row once per run of equal indices (and widths off 16-byte boundaries get the padded copy).
   bool dup_runs = false;
+  bool ranged = false;                // built with source ranges
   uint64_t repeated_edges = 0;
   std::mutex mu;
   hipEvent_t done = nullptr;
@@ -2383,6 +2385,7 @@ int build_plan(nts_spmm_plan_t **plan_out, const uint32_t *offsets_dev, const st
   p->n_index = n_index;
   p->repeated_edges = sched.repeated_edges;
   p->dup_runs = edges > 0 && sched.repeated_edges * 20 >= edges;
+  p->ranged = n_slabs > 1;
   hipError_t err = hipEventCreateWithFlags(&p->done, hipEventDisableTiming);
   items.insert(items.end(), sched.splits.begin(), sched.splits.end());  // one block, one copy
   if (err == hipSuccess && !items.empty()) {
@@ -2574,6 +2577,7 @@ int build_plan_device(nts_spmm_plan_t **plan_out, const uint32_t *offsets, const
   p->n_index = n_index;
   p->repeated_edges = host_counters.repeated;
   p->dup_runs = edges > 0 && p->repeated_edges * 20 >= edges;
+  p->ranged = true;
   auto bail = [&](hipError_t err, const char *what) {
     nts_spmm_plan_destroy(p);
     return nts::fail_hip(err, what);
@@ -2951,6 +2955,7 @@ int nts_spmm_gather_heads_planned(nts_spmm_plan_t *plan, const float *in, float 
                     F,   plan->items, plan->partial, accumulate, stream};
   a.heads = nts::HeadArgs{perm, H, Fh};
   a.scheduled_rows = plan->rows;
+  a.ranged = plan->ranged;
   a.edges = plan->edges;
   if (plan->sorted_idx) {
     a.indices = plan->sorted_idx;
@@ -2998,6 +3003,7 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
   }
   a.dup_runs = use_runs(plan);
   a.scheduled_rows = plan->rows;
+  a.ranged = plan->ranged;
   a.edges = plan->edges;
   if (const uint32_t ld = padded_stride(plan, F, false)) {
     // Rows off 16-byte boundaries: gather from a padded copy with 16-byte lanes.

@@ -123,3 +123,17 @@ def test_scheduled_rows_by_their_length(device, rows, edges, F):
     plan = SpmmPlan(off, rows, edges, 64)
     check(device, rows, off, idx, dst, 1, F, F % 4, lambda x, y, w, acc: call(
         "nts_spmm_gather_planned", plan.handle, ptr(x), ptr(y), ptr(w), ptr(off), ptr(idx), 0, F, acc, s))
+
+
+# source ranges, without and with repeated edges in a row, on both sides of 32,768 rows and of 32 and 64 edges a row
+@pytest.mark.parametrize("rows,edges,repeats", [(16400, 1100000, False), (33000, 1000000, False), (33000, 2300000, False),
+                                                (16400, 1100000, True), (33000, 2300000, True)])
+@pytest.mark.parametrize("F", [31, 33, 47, 64, 101, 127])
+def test_scheduled_rows_with_source_ranges(device, rows, edges, repeats, F):
+    off, idx, dst = even_graph(rows, edges, 10, device)
+    if repeats:
+        idx = idx // 512 * 512
+    s = torch.cuda.current_stream().cuda_stream
+    plan = SpmmPlan(off, rows, edges, 64, idx, rows, 8)
+    check(device, rows, off, idx, dst, 1, F, F % 4, lambda x, y, w, acc: call(
+        "nts_spmm_gather_planned", plan.handle, ptr(x), ptr(y), ptr(w), ptr(off), ptr(idx), 0, F, acc, s))
