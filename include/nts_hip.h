@@ -268,8 +268,8 @@ int nts_spmm_plan_info(const nts_spmm_plan_t *plan, uint32_t *items, uint32_t *s
  * calls load a source row once per run of such edges.  Any out-pointer may be NULL. */
 int nts_spmm_plan_scratch_info(nts_spmm_plan_t *plan, uint32_t F, size_t *partial_bytes, size_t *padded_input_bytes,
                                uint64_t *repeated_edges, int *loads_once_per_run);
-/* Grow the plan's scratch (partial sums of split rows; for a schedule with runs of equal indices
- * also a copy of the input with padded rows, see below) so that a later call of width F allocates
+/* Grow the plan's scratch (partial sums of split rows; for some schedules and widths also a copy of
+ * the input with padded rows, see below) so that a later call of width F allocates
  * nothing. */
 int nts_spmm_plan_reserve(nts_spmm_plan_t *plan, uint32_t F);
 /* NtsScheduler::GatherByDstFromSrc / GatherBySrcFromDst on a full-graph chunk
@@ -281,7 +281,10 @@ int nts_spmm_plan_reserve(nts_spmm_plan_t *plan, uint32_t F);
  * order, so every sum keeps its bits.  Such a schedule also gathers rows that are wider than 128
  * floats and not a multiple of four floats wide from a copy of `in` whose rows are padded to whole
  * 128-byte lines (made by the call, in the plan's scratch, n_index * 4 * ceil(F / 32) * 32 bytes), so
- * that the row loads are 16 bytes per lane.
+ * that the row loads are 16 bytes per lane.  So does a schedule with source ranges and without such runs for rows of 257 to
+ * 768 floats that are not whole lines, if it has 48 edges (24 from 513 floats up) for every row of `in`.  A call that finds no
+ * memory for the copy, or is captured before nts_spmm_plan_reserve or an earlier call has made room for it, gathers from
+ * `in` itself; the sums are the same.
  * Concurrency.  A plan's scratch is shared by all calls on it.  The host side of a call is
  * serialised per plan, and a call on another stream than the previous one first waits, on the
  * device, for that call's last kernel; calls on one plan therefore never overlap on the device,

@@ -403,6 +403,7 @@ __global__ __launch_bounds__(256) void spmm_wave_kernel(const float *__restrict_
 // wavefronts 157, 419 and 1,028.  Without, groups of up to 16 lanes are held to eight (72 -> 63 registers: 1 M, 3 M without a
 // schedule F = 64 219 -> 208, F = 47 211 -> 201); 32 lanes would spill in the loop (2.45 M, 126 M F = 100 and 128 20.4 -> 21.1 ms a
 // step), and rows with runs, held to seven, lose the overlap of their loads (60 K, 600 K F = 17 48 -> 101 us).
+constexpr uint32_t kXcds = 8;
 template <int G, bool HEADS, bool RUNS>
 constexpr int group_waves() {
   return HEADS ? 6 : !RUNS && G <= 16 ? 8 : 1;
@@ -416,12 +417,29 @@ __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_gro
                                                          const Item *__restrict__ items, float *__restrict__ partial,
                                                          int accumulate, HeadArgs heads,
                                                          uint32_t row_edge_limit,
-                                                         const uint32_t *__restrict__ edge_ids, uint32_t panels) {
+                                                         const uint32_t *__restrict__ edge_ids, uint32_t panels,
+                                                         int panel_bits, uint32_t in_ld, uint32_t partial_ld) {
   using V = typename Vec<VEC>::type;
   static_assert(U <= G, "a step's pairs come from one tile");  // U edges per step: their rows are requested together
   const uint32_t gl = threadIdx.x & (G - 1);
-  const uint32_t panel = PANELS ? blockIdx.x % panels : 0u;
-  const uint32_t item = ((PANELS ? blockIdx.x / panels : blockIdx.x) * blockDim.x + threadIdx.x) / G;
+  // Blocks are dealt out to the eight XCDs in turn.  1 << panel_bits panels (up to eight) alternate and an XCD meets one of
+  // them.  Of other numbers, eight blocks of items are 8 * panels units of work, panel by panel, and XCD x takes the units
+  // x * panels and on: an XCD meets as few panels as can be.  (The alternating panels too by that rule: 169 K rows, 2.48 M edges
+  // F = 128 97 -> 100 us.)
+  uint32_t panel = 0, block = blockIdx.x;
+  if (PANELS) {
+    if (panel_bits >= 0) {
+      panel = blockIdx.x & (panels - 1);
+      block = blockIdx.x >> panel_bits;
+    } else {
+      const uint32_t turn = blockIdx.x / kXcds, unit = blockIdx.x % kXcds * panels + turn % panels;
+      panel = unit / kXcds;
+      block = turn / panels * kXcds + unit % kXcds;
+    }
+  } else {
+    in_ld = partial_ld = F;
+  }
+  const uint32_t item = (block * blockDim.x + threadIdx.x) / G;
   if (item >= n_items) return;  // whole groups leave together; shuffles stay inside a group
 
   uint32_t row, e0, e1, slot;
@@ -497,7 +515,7 @@ __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_gro
         for (int u = 0; u < U; ++u) {
           fresh[u] = si[u] != (u ? si[u - 1] : held_i);
           v[u] = vzero<VEC>();
-          if (fresh[u]) v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si[u]) * F + lcol);
+          if (fresh[u]) v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si[u]) * in_ld + lcol);
           wv[u] = HEADS ? w[static_cast<size_t>(ss[u]) * heads.H + head] : __uint_as_float(ss[u]);
         }
 #pragma unroll
@@ -510,7 +528,7 @@ __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_gro
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si[u]) * F + lcol);
+        v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si[u]) * in_ld + lcol);
         wv[u] = HEADS ? w[static_cast<size_t>(ss[u]) * heads.H + head] : __uint_as_float(ss[u]);
       }
 #pragma unroll
@@ -532,7 +550,7 @@ __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_gro
         v[u] = vzero<VEC>();
         wv[u] = 0.f;
         if (static_cast<uint32_t>(u) < left) {
-          v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si) * F + lcol);
+          v[u] = load_row<VEC, SHARED>(in + static_cast<size_t>(si) * in_ld + lcol);
           wv[u] = HEADS ? w[static_cast<size_t>(ss) * heads.H + head] : __uint_as_float(ss);
         }
       }
@@ -547,17 +565,17 @@ __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_gro
       const uint32_t ss = __shfl(my_s, j, G);
       const float wgt = HEADS ? w[static_cast<size_t>(ss) * heads.H + head] : __uint_as_float(ss);
       if (RUNS) {
-        if (si != held_i) held = load_row<VEC, SHARED>(in + static_cast<size_t>(si) * F + lcol);
+        if (si != held_i) held = load_row<VEC, SHARED>(in + static_cast<size_t>(si) * in_ld + lcol);
         held_i = si;
         vfma(acc, held, wgt);
         continue;
       }
-      vfma(acc, load_row<VEC, SHARED>(in + static_cast<size_t>(si) * F + lcol), wgt);
+      vfma(acc, load_row<VEC, SHARED>(in + static_cast<size_t>(si) * in_ld + lcol), wgt);
     }
   }
 
   if (live) {
-    float *dst = (slot == kNoSlot) ? out + static_cast<size_t>(row) * F : partial + static_cast<size_t>(slot) * F;
+    float *dst = (slot == kNoSlot) ? out + static_cast<size_t>(row) * F : partial + static_cast<size_t>(slot) * partial_ld;
     if (SHARED) {
       store_row<VEC>(dst + lcol, acc, col - lcol, accumulate && slot == kNoSlot);
     } else {
@@ -1012,13 +1030,18 @@ template <int G, int VEC, int U = 8, bool SHARED = false, bool PANELS = false>
 void launch_group(const LaunchArgs &a, uint32_t panels = 1) {
   const uint32_t per_block = 256 / G;
   const uint32_t n_list = a.items ? a.n_items : 0u, n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
-  const uint32_t blocks = ceil_div(n_total, per_block) * panels;
+  int panel_bits = -1;
+  for (uint32_t bits = 0; bits < 4; ++bits)
+    if (panels == 1u << bits) panel_bits = static_cast<int>(bits);
+  // where panels do not alternate, whole turns of the XCDs (the last ones' surplus blocks leave at once)
+  const uint32_t turn = PANELS && panel_bits < 0 ? kXcds : 1u;
+  const uint32_t blocks = ceil_div(n_total, per_block * turn) * turn * panels;
 #define NTS_LAUNCH_GROUP(HD, RM, RUNS)                                                                                  \
   hipLaunchKernelGGL((spmm_group_kernel<SHARED, PANELS, G, VEC, U, HD, RM, RUNS>), dim3(blocks), dim3(256), 0, a.stream, a.in, a.out, a.w, \
                      a.offsets, a.indices, a.index_base, n_total, n_list, a.F, a.items, a.partial, a.accumulate,        \
                      a.heads,                                                                                          \
-                     a.row_edge_limit, a.edge_ids, panels)
-  if constexpr (PANELS) {  // neither heads nor repeated indices (die_panels)
+                     a.row_edge_limit, a.edge_ids, panels, panel_bits, a.in_ld ? a.in_ld : a.F, a.partial_ld ? a.partial_ld : a.F)
+  if constexpr (PANELS) {  // neither heads nor repeated indices (panel_lanes)
     if (a.edge_ids) NTS_LAUNCH_GROUP(false, true, false);
     else NTS_LAUNCH_GROUP(false, false, false);
   } else if (a.edge_ids) {
@@ -1091,27 +1114,53 @@ int pick_vec(const LaunchArgs &a) {
   return 1;
 }
 
-// Column panels whose blocks alternate, so that an XCD (blocks are dealt out to the eight in turn) meets one panel only and
-// its 4 MB L2 holds a share of the gathered matrix that is as many times smaller.  A panel is whole lines (512
-// bytes, or 256 of a row of 512) and the number of panels divides eight; shorter requests cost more than they gain (64 bytes:
-// 2.8 times the time, 128: as much as without).  us without / with: 169 K rows, 2.48 M
-// edges F = 128 111 / 98, 256 251 / 221, 512 584 / 451; 500 K, 20 M with source ranges 722 / 690, 1,437 / 1,388, 3,137 /
-// 2,746; 2.45 M, 126 M 5,221 / 5,108, 11,255 / 10,386.  Panels that share lines lose or gain by width and graph (F = 300, 384
-// and 500 as panels of 128 331 / 404, 396 / 424, 609 / 526 and 1,968 / 2,312, 2,249 / 2,362, 3,330 / 3,071) and are not taken; eight
-// panels (F = 1,024) were not measured.  Without them stay:
+// Lanes of a column panel (16 or 32, of four floats each: panels of 256 or 512 bytes), or 0 for rows that are not cut into panels.
+// An XCD meets one or two panels of a row only, so that its 4 MB L2 holds a share of the gathered matrix that is as many times
+// smaller.  us without / with, panels of whole lines (the last one may be shorter):
+//   rows          169 K, 2.48 M   60 K, 4 M   1 M, 6 M        20 M of 500 K   233 K, 114.8 M simple   2.45 M, 126 M (40 M)
+//   128  2 x 16   111 / 98                                    722 / 690       2,651 / 2,660           5,221 / 5,108
+//   192  3 x 16                   171 / 146                                                           (80 M 6,082 / 5,495)
+//   256  2 x 32   251 / 221                                   1,437 / 1,388   4,871 / 4,852           11,255 / 10,386
+//   320  5 x 16                   318 / 241   700 K, 7.5 M 1,316 / 1,157                              (80 M 10,590 / 9,121)
+//   384  3 x 32   409 / 344       407 / 304   1,468 / 1,383   2,255 / 2,051   8,183 / 7,291           (7,496 / 6,924)
+//   512  4 x 32   584 / 451                                   3,137 / 2,746
+//   640  5 x 32                   773 / 523                                   1 M, 40 M 9,217 / 7,301 (80 M 23,238 / 19,127)
+// Rows off whole lines are gathered from a copy padded to them where that pays (padded_stride), the copy included:
+//   300  5 x 16   1 M, 40 M 4,226 / 4,275                     1,963 / 1,947   7,536 / 6,392           15,003 / 14,410
+//   450  4 x 32   200 K, 12 M 1,587 / 1,518                   3,365 / 2,975   9,674 / 9,236           (80 M 16,989 / 16,514)
+//   500  4 x 32   200 K, 12 M 1,803 / 1,588                   3,271 / 3,143   10,629 / 9,531          26,582 / 23,291
+//   602  5 x 32   1 M, 24 M 6,430 / 6,062                     4,414 / 3,879   12,992 / 11,767         31,848 / 28,922
+//   700  11 x 16  200 K, 12 M 2,562 / 2,261; 1 M, 40 M 10,888 / 9,437
+// and without a copy, panels that share a line, by schedules without source ranges whose rows are wide and long: 450 60 K, 4 M
+// 535 / 474, 500 20 K, 4 M 416 / 326, 602 757 / 651, 30 K, 600 K 129 / 108, 700 145 / 126; but 300 60 K, 4 M 330 / 376, 602 300 K, 3 M
+// 1,036 / 1,098, 1 M, 6 M 2,573 / 2,915.  Shorter panels cost more than they give (64 bytes: 2.8 times the time, 128: as much as
+// without), longer ones of 64 lanes lose too (602 233 K 15,300, 500 9,900).  Without them stay:
 //   rows of 512 bytes that the L2s hold together (20 K rows, 4 M edges 93 / 95; wider rows gain there too: F = 256 and 512 2 K, 8 K
 //     11.4 / 11.5, 12.0 / 11.1, 5 K, 60 K 14.3 / 14.2, 18.1 / 16.9, 20 K, 300 K 33 / 32, 58 / 51, 60 K, 600 K 60 / 55, 124 / 96)
-//   rows of 2 KB with fewer than five edges each once they fill the chip, which are read once or twice whatever the caches hold,
-//     while every panel walks the short rows again: 32 K, 100 K 34 / 37, 130 K, 300 K 126 / 139, 300 K, 600 K 267 / 290, 2.45 M, 5 M
-//     2,402 / 2,667, 10 M 3,782 / 4,042; but 2 K, 8 K 12 / 10, 300 K, 1.5 M 492 / 438, 600 K, 3 M 1,008 / 985
-//   rows loaded once per run of equal indices (233 K, 114.8 M F = 128 2,277 / 2,346), heads (169 K 155 / 199: the weights are
-//     read once a panel) and calls without a schedule (133 / 149: mostly short rows)
-uint32_t die_panels(const LaunchArgs &a, int vec) {
-  if (vec != 4 || !a.scheduled_rows || a.heads.H || a.dup_runs || a.in_ld) return 0;
-  if (a.n_items >= 1u << 24) return 0;  // (up to 128 threads an item: a launch has fewer than 2^32)
-  if (a.F == 128) return static_cast<uint64_t>(a.scheduled_rows) * a.F * sizeof(float) > kAllL2Bytes ? 2 : 0;
-  if (a.F == 512) return a.n_items > kChipWaves && a.edges < 5ull * a.scheduled_rows ? 0 : 4;
-  return a.F == 256 ? 2 : 0;
+//   rows of 160 and 224 floats, whose last panel is half idle: 2.45 M, 40 M 3,111 / 3,302, 1 M, 40 M 2,764 / 2,825
+//   rows with fewer than five edges each once they fill the chip, which are read once or twice whatever the caches hold,
+//     while every panel walks the short rows again: F = 512 32 K, 100 K 34 / 37, 130 K, 300 K 126 / 139, 300 K, 600 K 267 / 290, 2.45 M, 5 M
+//     2,402 / 2,667, 10 M 3,782 / 4,042; but 2 K, 8 K 12 / 10, 300 K, 1.5 M 492 / 438, 600 K, 3 M 1,008 / 985; and rows of other widths
+//     that do not fill it (2 K, 16 K F = 192 to 640 13 / 14)
+//   rows loaded once per run of equal indices (233 K, 114.8 M F = 128 2,277 / 2,346; 100 K, 40 M F = 602 3,399 / 3,707), heads (169 K
+//     155 / 199: the weights are read once a panel) and calls without a schedule (133 / 149: mostly short rows)
+constexpr uint32_t kMinPanelEdges = 5;                     // edges a row
+// Panels of 512 bytes, or of 256 where they leave fewer lanes idle.
+uint32_t lanes_for_lines(uint32_t lines) { return lines % 4 == 1 || lines % 4 == 2 ? 16u : 32u; }
+constexpr uint32_t kMaxPanelLines = 24;                    // (wider rows were not measured)
+uint32_t panel_lanes(const LaunchArgs &a, int vec) {
+  if (!a.scheduled_rows || a.heads.H || a.dup_runs) return 0;
+  const uint32_t lines = ceil_div(a.F, 32);
+  if (static_cast<uint64_t>(a.n_items) * (lines + 4) * 8 >= 0xF0000000ull) return 0;  // (a launch has fewer than 2^32 threads)
+  const bool full = a.n_items > kChipWaves, sparse = a.edges < static_cast<uint64_t>(kMinPanelEdges) * a.scheduled_rows;
+  if (a.in_ld) return lines <= kMaxPanelLines ? lanes_for_lines(lines) : 0u;
+  if (vec == 4 && a.F % 32 == 0) {
+    if (a.F == 128) return static_cast<uint64_t>(a.scheduled_rows) * a.F * sizeof(float) > kAllL2Bytes ? 16u : 0u;
+    if (a.F == 256) return 32;
+    if (a.F == 512) return full && sparse ? 0u : 32u;
+    return lines >= 6 && lines != 7 && lines <= kMaxPanelLines && full && !sparse ? lanes_for_lines(lines) : 0u;
+  }
+  return !a.ranged && a.F >= 448 && lines <= kMaxPanelLines && a.n_items > 2 * kChipWaves && a.edges >= 20ull * a.scheduled_rows ? 32u : 0u;
 }
 
 // Lanes of a narrow row.  A group of G lanes fetches G edge pairs at a time and works on one row, so what counts is how
@@ -1243,7 +1292,11 @@ void launch_spmm(const LaunchArgs &a) {
   }
   const int vec = pick_vec(a);
   const uint32_t F = a.F;
-  if (const uint32_t panels = die_panels(a, vec)) return F == 128 ? launch_group<16, 4, 8, false, true>(a, panels) : launch_group<32, 4, 8, false, true>(a, panels);
+  if (const uint32_t lanes = panel_lanes(a, vec)) {
+    const uint32_t panels = ceil_div(F, lanes * 4);
+    if (F % 4 == 0 && vec == 4 && aligned_to(a.out, 16)) return lanes == 16 ? launch_group<16, 4, 8, false, true>(a, panels) : launch_group<32, 4, 8, false, true>(a, panels);
+    return lanes == 16 ? launch_group<16, 4, 8, true, true>(a, panels) : launch_group<32, 4, 8, true, true>(a, panels);
+  }
   if (!a.in_ld) {
     switch (narrow_lanes(a, vec)) {
       case kFloats4: return launch_group<4, 1, 4>(a);
@@ -2771,16 +2824,21 @@ namespace {
 // stride).  Measured on the 114.8 M-edge R-MAT graph at F = 602: with one load per run of equal
 // indices the copy pays (9.75 -> 9.21 ms per pass, the 0.25 ms copy not included; 25.7 -> 25.0 ms per
 // four-pass step with it); without runs it does not (11.05 -> 11.7 ms, and 8.79 -> 8.93 ms on the same
-// graph with its parallel edges removed), so only schedules with runs use it.  NTS_SPMM_PAD=0 / 1 in
-// the environment forces it off / on.
+// graph with its parallel edges removed), but column panels of whole lines do (panel_lanes, which has the figures), for rows
+// of more than 256 floats: the copy costs two passes over the gathered matrix, the panels save a tenth of the gather, so
+// there have to be 48 edges a gathered row, or 24 where rows are wider than 512 floats (300 floats 300 K rows, 10 M edges 1,082 ->
+// 1,114 us, 1 M, 40 M 4,226 -> 4,275; 500 1 M, 24 M 5,213 -> 5,068, 450 4,664 -> 4,868; 602 2.45 M, 40 M 12,905 -> 14,108).
+// NTS_SPMM_PAD=0 / 1 in the environment forces it off / on.
 uint32_t padded_stride(const nts_spmm_plan *plan, uint32_t F, bool heads) {
   static const int forced = [] {
     const char *e = getenv("NTS_SPMM_PAD");
     return e ? (e[0] != '0' ? 1 : 0) : -1;
   }();
-  if (heads || plan->n_index == 0 || F <= 128 || F % 4 == 0) return 0;
-  if (forced == 0 || (forced < 0 && !plan->dup_runs)) return 0;
-  return (F + 31) / 32 * 32;
+  if (heads || plan->n_index == 0 || F <= 128 || forced == 0) return 0;
+  const uint32_t padded = (F + 31) / 32 * 32;
+  if (forced == 1 || plan->dup_runs) return F % 4 ? padded : 0u;
+  const uint64_t least = F > 512 ? 24 : 48;
+  return plan->ranged && F > 256 && F < padded && padded <= 32 * nts::kMaxPanelLines && plan->edges >= least * plan->n_index ? padded : 0u;
 }
 
 // NTS_SPMM_RUNS=0 / 1 forces the one-load-per-run kernel off / on whatever the schedule found.
@@ -2792,11 +2850,11 @@ bool use_runs(const nts_spmm_plan *plan) {
   return forced < 0 ? plan->dup_runs : forced == 1;
 }
 
-// Grows the plan's scratch for width F.  Caller holds plan->mu.
-int reserve_locked(nts_spmm_plan *plan, uint32_t F, bool heads) {
-  const uint32_t ld = padded_stride(plan, F, heads);
-  const size_t want_partial = static_cast<size_t>(plan->n_partials) * (ld ? ld : F);
-  const size_t want_padded = ld ? static_cast<size_t>(plan->n_index) * ld : 0;
+// Grows the plan's scratch for width F and leaves the call's row stride (padded_stride) in *stride: 0 also where the copy
+// has no room yet and there is no memory for it, or `fixed` says that none can be had now (the call gathers from the rows as
+// they are, with the same sums).  Caller holds plan->mu.
+int reserve_locked(nts_spmm_plan *plan, uint32_t F, bool heads, bool fixed, uint32_t *stride) {
+  uint32_t ld = padded_stride(plan, F, heads);
   // A buffer that grows may still be read by work queued earlier, on any stream.
   auto grow = [](nts::DeviceBlock &block, float **ptr, size_t *floats, size_t want) -> int {
     if (want <= *floats) return NTS_OK;
@@ -2808,8 +2866,25 @@ int reserve_locked(nts_spmm_plan *plan, uint32_t F, bool heads) {
     *floats = block.bytes / sizeof(float);
     return NTS_OK;
   };
-  if (int rc = grow(plan->partial_block, &plan->partial, &plan->partial_floats, want_partial)) return rc;
-  return grow(plan->padded_block, &plan->in_padded, &plan->in_padded_floats, want_padded);
+  if (const size_t want = static_cast<size_t>(plan->n_index) * ld; want > plan->in_padded_floats) {
+    if (fixed) {
+      ld = 0;
+    } else if (grow(plan->padded_block, &plan->in_padded, &plan->in_padded_floats, want)) {
+      (void)hipGetLastError();
+      ld = 0;
+    }
+  }
+  const size_t n = plan->n_partials;
+  if (ld && grow(plan->partial_block, &plan->partial, &plan->partial_floats, n * ld)) {
+    // the copy has taken the memory that the partial sums need more
+    (void)hipGetLastError();
+    plan->in_padded = nullptr;
+    plan->in_padded_floats = 0;
+    NTS_HIP_TRY(nts::retire_blocks({&plan->padded_block}));
+    ld = 0;
+  }
+  *stride = ld;
+  return ld ? NTS_OK : grow(plan->partial_block, &plan->partial, &plan->partial_floats, n * F);
 }
 
 // A call on `stream` is about to use the plan's scratch: if the previous call ran on another stream,
@@ -2859,7 +2934,8 @@ int nts_spmm_plan_reserve(nts_spmm_plan_t *plan, uint32_t F) {
   if (!plan) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_reserve: null plan");
   if (F == 0) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_reserve: F is 0");
   std::lock_guard<std::mutex> lock(plan->mu);
-  return reserve_locked(plan, F, false);
+  uint32_t ld = 0;
+  return reserve_locked(plan, F, false, false, &ld);
 }
 
 namespace {
@@ -2949,7 +3025,8 @@ int nts_spmm_gather_heads_planned(nts_spmm_plan_t *plan, const float *in, float 
     return rc;
   if (plan->rows == 0) return NTS_OK;
   std::lock_guard<std::mutex> lock(plan->mu);
-  if (int rc = reserve_locked(plan, F, true)) return rc;
+  uint32_t ld = 0;
+  if (int rc = reserve_locked(plan, F, true, false, &ld)) return rc;
   if (int rc = enter_stream(plan, stream)) return rc;
   nts::LaunchArgs a{in,  out,         alpha,         offsets,    indices, 0u, plan->n_items,
                     F,   plan->items, plan->partial, accumulate, stream};
@@ -2992,7 +3069,8 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
     return rc;
   if (plan->rows == 0) return NTS_OK;
   std::lock_guard<std::mutex> lock(plan->mu);
-  if (int rc = reserve_locked(plan, F, false)) return rc;
+  uint32_t ld = 0;
+  if (int rc = reserve_locked(plan, F, false, stream_is_capturing(stream), &ld)) return rc;
   if (int rc = enter_stream(plan, stream)) return rc;
   nts::LaunchArgs a{in,  out,         w,           offsets,       indices,   index_base, plan->n_items,
                     F,   plan->items, plan->partial, accumulate, stream};
@@ -3005,8 +3083,8 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
   a.scheduled_rows = plan->rows;
   a.ranged = plan->ranged;
   a.edges = plan->edges;
-  if (const uint32_t ld = padded_stride(plan, F, false)) {
-    // Rows off 16-byte boundaries: gather from a padded copy with 16-byte lanes.
+  if (ld) {
+    // Rows off whole lines: gather from a padded copy.
     const uint64_t vecs = static_cast<uint64_t>(plan->n_index) * (ld / 4);
     const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>((vecs + 255) / 256, 1u << 16));
     hipLaunchKernelGGL(nts::pad_rows_kernel, dim3(blocks), dim3(256), 0, stream,

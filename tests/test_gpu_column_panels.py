@@ -50,6 +50,77 @@ def test_wide_rows(device, rows, F, narrow):
     compare(device, SpmmPlan(off, rows, edges, 4096), off, idx, rows, edges, F, narrow)
 
 
+def simple_graph(rows, edges, device, rising):
+    """`edges` of the rows * rows pairs, each at most once, so that no schedule loads a row once per run of equal indices."""
+    g = torch.Generator(device=device).manual_seed(rows)
+    pairs = torch.unique(torch.randint(rows * rows, (edges + edges // 4,), generator=g, device=device))
+    pairs = pairs[torch.randperm(pairs.numel(), generator=g, device=device)[:edges]].sort().values
+    assert pairs.numel() == edges
+    off = torch.zeros(rows + 1, dtype=torch.int64, device=device)
+    off[1:] = torch.bincount(pairs // rows, minlength=rows).cumsum(0)
+    idx = (pairs % rows).to(torch.int32)
+    if not rising:
+        idx, off = idx.flip(0), off[-1] - off.flip(0)
+    return off.to(torch.int32), idx.contiguous()
+
+
+# whole lines: panels of 16 and 32 lanes, last ones of one to four lines; around 8,192 items and five edges a row
+@pytest.mark.parametrize("rows,edges,ranges,rising", [(8192, 81920, 1, True), (8193, 81930, 1, True), (9001, 45004, 1, True),
+                                                      (9001, 45005, 1, True), (9001, 900000, 8, True), (9001, 900000, 8, False)])
+@pytest.mark.parametrize("F", [160, 192, 288, 320, 352, 384, 640, 768, 800])
+def test_panels_of_other_whole_lines(device, rows, edges, ranges, rising, F):
+    off, idx = simple_graph(rows, edges, device, rising)
+    plan = SpmmPlan(off, rows, edges, 64, idx, rows, ranges) if ranges > 1 else SpmmPlan(off, rows, edges, 4096)
+    compare(device, plan, off, idx, rows, edges, F, 100)
+
+
+# copies padded to whole lines: on both sides of 256, 512 and 768 floats, of 24 and of 48 edges a row
+@pytest.mark.parametrize("edges", [48 * 3001, 48 * 3001 - 1, 24 * 3001, 24 * 3001 - 1])
+@pytest.mark.parametrize("rising", [True, False])
+@pytest.mark.parametrize("F", [255, 257, 300, 450, 500, 511, 513, 602, 700, 767, 769])
+def test_panels_of_a_padded_copy(device, edges, rising, F):
+    rows = 3001
+    off, idx = simple_graph(rows, edges, device, rising)
+    plan = SpmmPlan(off, rows, edges, 64, idx, rows, 8)
+    padded = F > 256 and F <= 768 and edges >= (24 if F > 512 else 48) * rows
+    assert plan.scratch_info(F)["padded_input_bytes"] == (rows * 4 * ((F + 31) // 32 * 32) if padded else 0)
+    compare(device, plan, off, idx, rows, edges, F, 100)
+
+
+# panels that share lines: on both sides of 448 and 768 floats, 16,384 items and twenty edges a row
+@pytest.mark.parametrize("rows,edges", [(16384, 330000), (16385, 330000), (17000, 340000), (17000, 339999)])
+@pytest.mark.parametrize("F", [447, 449, 500, 602, 767, 769])
+def test_panels_that_share_lines(device, rows, edges, F):
+    off, idx = simple_graph(rows, edges, device, True)
+    compare(device, SpmmPlan(off, rows, edges, 4096), off, idx, rows, edges, F, 100)
+
+
+def test_captured_call_without_room_for_the_copy(device):
+    """The capture of a call whose copy has no room yet gathers from the rows as they are; one with room, from the copy."""
+    rows, edges, F = 3001, 150050, 602
+    off, idx = simple_graph(rows, edges, device, True)
+    g = torch.Generator(device=device).manual_seed(1)
+    x, w = torch.randn(rows, F, generator=g, device=device), torch.rand(edges, generator=g, device=device)
+    want = torch.empty(rows, F, device=device)
+    other = SpmmPlan(off, rows, edges, 64, idx, rows, 8)
+    call("nts_spmm_gather_planned", other.handle, ptr(x), ptr(want), ptr(w), ptr(off), ptr(idx), 0, F, 0,
+         torch.cuda.current_stream().cuda_stream)
+    for reserved in (640, 602):  # 640 floats are whole lines: room for the partial sums and none for a copy
+        plan = SpmmPlan(off, rows, edges, 64, idx, rows, 8)
+        plan.reserve(reserved)
+        out = torch.empty(rows, F, device=device)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            call("nts_spmm_gather_planned", plan.handle, ptr(x), ptr(out), ptr(w), ptr(off), ptr(idx), 0, F, 0,
+                 torch.cuda.current_stream().cuda_stream)
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+
+
 def compare(device, plan, off, idx, rows, edges, F, narrow):
     g = torch.Generator(device=device).manual_seed(F)
     x, w = torch.randn(rows, F, generator=g, device=device), torch.rand(edges, generator=g, device=device)
