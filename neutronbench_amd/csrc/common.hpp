@@ -214,6 +214,15 @@ __device__ __forceinline__ uint32_t wave_first(uint32_t v) {
   return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
 }
 
+// The wavefront's number within its block, and within the grid's blocks from `first_block` on, in scalar registers: what
+// follows from it (offsets, loop ends, row numbers) is then computed once a wavefront and loaded by scalar requests, where the
+// compiler takes threadIdx.x / 64 for a value of every lane (edge copies: 8 registers a lane fewer; 2.48 M edges of 128 floats, a
+// chain of copies and sums 2,305 -> 2,274 us).
+__device__ __forceinline__ uint32_t wave_of_block() { return wave_first(threadIdx.x / kWave); }
+__device__ __forceinline__ uint64_t wave_of_grid(uint32_t first_block = 0) {
+  return static_cast<uint64_t>(blockIdx.x - first_block) * (blockDim.x / kWave) + wave_of_block();
+}
+
 // Largest r such that off[r] <= pos, searched in off[0 .. n] (off ascending, off[n] > pos): the row
 // that owns edge position `pos`.
 __device__ __forceinline__ uint32_t owner_of(const uint32_t *__restrict__ off, uint32_t n, uint32_t pos) {

@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void edge_copy_kernel(V *__restrict__ msg, con
   constexpr uint32_t kEdgesPerStep = kWave / G;
   constexpr int U = G < 4 ? G : 4;  // rows of a group requested together
   const bool streamed = outgrows_caches(static_cast<uint64_t>(E) * Fv * sizeof(V));
-  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+  const uint64_t wave = wave_of_grid();
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   // A wavefront walks a contiguous span of wave steps: the destination that owns each step's edges
   // follows from the previous step's (owners_of_step) instead of a search per lane.  Messages that outgrow the caches are
@@ -403,13 +403,13 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
   constexpr uint32_t kRound = kSlots * U;         // edge rows per round
   constexpr uint32_t kPitch = G * NF;             // floats of an edge row in the tile
   __shared__ float tiles[4][kWave * U * NF];
-  float *tile = tiles[threadIdx.x / kWave];
+  float *tile = tiles[wave_of_block()];
   const uint32_t lane = lane_id();
   const uint32_t col = lane & (G - 1), slot = lane / G;
   const bool col_live = col < Fv;
   const uint32_t comps = Fv * NF;  // floats of an output row: lane c owns the floats c + 64 k below comps
   constexpr int OWN = (G * NF + kWave - 1) / kWave;  // floats a lane owns at most (1 up to 16 lanes of 16 bytes)
-  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / kWave;
+  const uint64_t wave = wave_of_grid(lw.blocks);
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x - lw.blocks) * blockDim.x / kWave;
   // The wavefronts share the rows by weight, a row counting one plus its edges: wavefront w takes the
   // rows r with w C <= (off[r] - off[0]) + r < (w + 1) C.
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
   if (FEW && G == 1 && sizeof(V) == 16 && off[rows] - off[0] < 4ull * rows) set = min(2u * few_rows, kFullSet<GG>);
   const uint32_t gl = lane & (GG - 1), grp = lane / GG;
   const uint32_t col = gl & (G - 1), slice = gl / G;
-  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / kWave;
+  const uint64_t wave = wave_of_grid(lw.blocks);
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x - lw.blocks) * blockDim.x / kWave;
   const bool col_live = col < Fv;
   const bool streamed = outgrows_caches(static_cast<uint64_t>(off[rows] - off[0]) * Fv * sizeof(V));
@@ -732,7 +732,7 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__r
       constexpr uint32_t kSlots = kWave / G;           // edge rows per load of the wavefront
       constexpr uint32_t kRound = kSlots * kCoopU;     // edge rows per round
       constexpr uint32_t kPitch = G * NF;              // floats of an edge row in the tile
-      float *tile = coop_tile[threadIdx.x / kWave];
+      float *tile = coop_tile[wave_of_block()];
       const uint32_t slot = lane / G;
       const uint32_t comps = Fv * NF;                  // floats of an output row: lane c < comps owns float c
       while (coop) {
@@ -1323,7 +1323,7 @@ __global__ __launch_bounds__(256) void edge_softmax_fwd_kernel(float *__restrict
                                                                uint32_t max_values, uint32_t vec4) {
   if (max_values == kByTotal) max_values = long_segment_values(static_cast<uint64_t>(co[Vd] - co[0]) * H);
   const uint32_t lane = lane_id();
-  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+  const uint64_t wave = wave_of_grid();
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   for (uint64_t first = wave * kWave; first < Vd; first += n_waves * kWave) {
     uint32_t my_e0, my_e1;
@@ -1460,7 +1460,7 @@ __global__ __launch_bounds__(256) void edge_softmax_bwd_kernel(float *__restrict
                                                                uint32_t max_values, uint32_t vec4) {
   if (max_values == kByTotal) max_values = long_segment_values(static_cast<uint64_t>(co[Vd] - co[0]) * H);
   const uint32_t lane = lane_id();
-  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+  const uint64_t wave = wave_of_grid();
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   for (uint64_t first = wave * kWave; first < Vd; first += n_waves * kWave) {
     uint32_t my_e0, my_e1;
@@ -1871,7 +1871,7 @@ __global__ __launch_bounds__(256) void sddmm_edge_kernel(float *__restrict__ gal
   const uint32_t F = H * Fh;
   const uint32_t lane = lane_id();
   const uint32_t gl = lane & (G - 1), grp = lane / G;
-  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+  const uint64_t wave = wave_of_grid();
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   uint32_t d_held = 0xFFFFFFFFu;
   float4 y4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1946,7 +1946,7 @@ __global__ __launch_bounds__(256) void sddmm_edge_generic_kernel(float *__restri
   const uint32_t E = co[Vd];
   const uint32_t F = H * Fh;
   const uint32_t lane = lane_id();
-  const uint64_t wave = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+  const uint64_t wave = wave_of_grid();
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   for (uint64_t base = wave * kWave; base < E; base += n_waves * kWave) {
     const uint64_t e = base + lane;
