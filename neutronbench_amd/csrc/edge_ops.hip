@@ -806,6 +806,31 @@ __device__ __forceinline__ uint64_t giant_segment_values(uint64_t total_values) 
   return v < kGiantMinValues ? kGiantMinValues : v < kGiantValues ? v : kGiantValues;
 }
 
+// The same for a call of few rows (kFewRows), whose launch has blocks of 256 threads for both.
+// The rows, by both sides' times in us, the kernels of many rows / these, edge softmax (H = 1, 4) and attention, forward, backward:
+//   rows, edges     softmax fwd       bwd               attention fwd       bwd
+//   2.7 K, 13 K     7 / 6, 7 / 7      8 / 6, 7 / 6      14 / 7, 18 / 10     11 / 7, 18 / 9
+//   10 K, 3 M       69 / 39, 304 / 129  67 / 40, 307 / 125  327 / 115, 572 / 182  387 / 129, 525 / 180
+//   30 K, 1 M       82 / 40, 94 / 39  85 / 40, 96 / 40  88 / 39, 99 / 55    92 / 42, 106 / 67
+//   60 K, 4 M       84 / 43, 84 / 65  86 / 41, 95 / 76  94 / 70, 135 / 113  99 / 88, 125 / 134
+//   169 K, 2.48 M   65 / 48, 70 / 62  66 / 47, 72 / 64  80 / 65, 139 / 109  84 / 86, 118 / 124
+//   250 K, 3 M      78 / 61, 95 / 75  82 / 57, 97 / 76  101 / 83, 157 / 140 92 / 105, 141 / 161
+//   200 K, 20 M     102 / 84, 245 / 239  108 / 91, 328 / 316  319 / 180, 492 / 459  418 / 282, 525 / 561
+//   100 K, 40 M     160 / 148, 459 / 485  204 / 185, 629 / 671  495 / 457, 766 / 802  526 / 521, 838 / 930
+// Above, one block takes too long over the offsets (1 M rows 30 us).  The fused backward holds two arrays and the signs of the scores a
+// lane, 114 registers for all of its paths together, and loses from some 32 K rows on.
+constexpr uint32_t kFewRows = 1u << 18;
+constexpr uint32_t kFewRowsFusedBackward = 1u << 15;
+constexpr uint32_t kFewPieceValues = 4096;
+__device__ __forceinline__ uint64_t few_long_values(uint64_t total_values) {
+  const uint64_t v = total_values / 2048;
+  return v < 1024 ? 1024 : v < kLongRowValues ? v : kLongRowValues;
+}
+__device__ __forceinline__ uint64_t few_giant_values(uint64_t total_values) {
+  const uint64_t v = total_values / 256;
+  return v < 8192 ? 8192 : v < kGiantValues ? v : kGiantValues;
+}
+
 // hdr: [0] giant rows, [1] pieces,
 //      [2] edges per piece, [4..5] edges of the listed giant rows (64-bit), [6] the long-row counter
 //      (`count` points here, so that one fill clears all of them).
@@ -842,24 +867,23 @@ __global__ __launch_bounds__(256) void collect_long_rows_kernel(uint32_t *__rest
 // One block: fixes the piece length, gives every listed giant row its first piece (every thread counts
 // the pieces of a run of rows, then one prefix over the block) and writes the piece table (list
 // position, row, first edge, end), a wavefront a row.
-__global__ __launch_bounds__(256) void giant_plan_kernel(uint32_t *__restrict__ hdr,
-                                                         const uint32_t *__restrict__ giant_rows,
-                                                         uint32_t *__restrict__ first, uint4 *__restrict__ pieces,
-                                                         const uint32_t *__restrict__ off, uint32_t min_piece) {
-  __shared__ uint32_t wave_sums[256 / kWave];
-  const uint32_t n = hdr[0] < kGiantCap ? hdr[0] : kGiantCap;
-  const unsigned long long edges = *reinterpret_cast<const unsigned long long *>(hdr + 4);
+template <int BLOCK>
+__device__ __forceinline__ void plan_giant_rows(uint32_t listed, unsigned long long edges, uint32_t *hdr, const uint32_t *giant_rows,
+                                                uint32_t *first, uint4 *__restrict__ pieces, const uint32_t *__restrict__ off,
+                                                uint32_t min_piece) {
+  __shared__ uint32_t wave_sums[BLOCK / kWave];
+  const uint32_t n = listed < kGiantCap ? listed : kGiantCap;
   const unsigned long long even = (edges + (kPieceCap - kGiantCap) - 1) / (kPieceCap - kGiantCap);
   const uint32_t len = even < min_piece ? min_piece : static_cast<uint32_t>(even);
   auto pieces_of = [&](uint32_t i) -> uint32_t {
     const uint32_t r = giant_rows[i];
     return (off[r + 1] - off[r] - 1) / len + 1;
   };
-  const uint32_t per = (n + 255) / 256;
+  const uint32_t per = (n + BLOCK - 1) / BLOCK;
   const uint32_t i0 = min(n, threadIdx.x * per), i1 = min(n, i0 + per);
   uint32_t mine = 0, total = 0;
   for (uint32_t i = i0; i < i1; ++i) mine += pieces_of(i);
-  uint32_t p = block_prefix<256>(mine, wave_sums, &total);
+  uint32_t p = block_prefix<BLOCK>(mine, wave_sums, &total);
   for (uint32_t i = i0; i < i1; ++i) {
     first[i] = p;
     p += pieces_of(i);
@@ -871,7 +895,7 @@ __global__ __launch_bounds__(256) void giant_plan_kernel(uint32_t *__restrict__ 
     hdr[2] = len;
   }
   __syncthreads();  // `first` is read by other threads of this block below
-  for (uint32_t i = threadIdx.x / kWave; i < n; i += 256 / kWave) {
+  for (uint32_t i = threadIdx.x / kWave; i < n; i += BLOCK / kWave) {
     const uint32_t r = giant_rows[i];
     const uint32_t e0 = off[r], e1 = off[r + 1], p0 = first[i], n_pieces = (e1 - e0 - 1) / len + 1;
     for (uint32_t q = lane_id(); q < n_pieces; q += kWave) {
@@ -879,6 +903,80 @@ __global__ __launch_bounds__(256) void giant_plan_kernel(uint32_t *__restrict__ 
       pieces[p0 + q] = make_uint4(i, r, k, e1 - k < len ? e1 : k + len);
     }
   }
+}
+
+__global__ __launch_bounds__(256) void giant_plan_kernel(uint32_t *__restrict__ hdr, const uint32_t *__restrict__ giant_rows,
+                                                         uint32_t *__restrict__ first, uint4 *__restrict__ pieces,
+                                                         const uint32_t *__restrict__ off, uint32_t min_piece) {
+  plan_giant_rows<256>(hdr[0], *reinterpret_cast<const unsigned long long *>(hdr + 4), hdr, giant_rows, first, pieces, off, min_piece);
+}
+
+// look(row, edges) for every row, by one block: a thread loads the offsets of four rows at a time, and four times as many at once.
+template <int BLOCK, typename Look>
+__device__ __forceinline__ void each_row_by_block(const uint32_t *__restrict__ off, uint32_t rows, Look look) {
+  typedef uint32_t Words4 __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr uint32_t kStep = 4 * BLOCK;
+  constexpr int U = 4;
+  for (uint32_t base = 0; base < rows; base += U * kStep) {
+    Words4 w[U];
+    uint32_t next[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t r = base + u * kStep + threadIdx.x * 4;
+      w[u] = Words4{0u, 0u, 0u, 0u};
+      next[u] = 0;
+      if (r + 4 <= rows) {
+        w[u] = *reinterpret_cast<const Words4 *>(off + r);
+        next[u] = off[r + 4];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t r = base + u * kStep + threadIdx.x * 4;
+      if (r + 4 <= rows) {
+        look(r, w[u].y - w[u].x);
+        look(r + 1, w[u].z - w[u].y);
+        look(r + 2, w[u].w - w[u].z);
+        look(r + 3, next[u] - w[u].w);
+      } else {
+        for (uint32_t t = r; t < rows; ++t) look(t, off[t + 1] - off[t]);
+      }
+    }
+  }
+}
+
+// The lists, their counters and the piece table in one launch of one block, for a softmax call of few rows (kFewRows): a fill, a
+// launch that lists and one that plans are 14 us and as much of the host's time.
+__global__ __launch_bounds__(kLongBlock) void few_long_rows_kernel(uint32_t *__restrict__ list, uint32_t *__restrict__ count,
+                                                                   uint32_t *giant_rows, uint32_t *hdr, uint32_t *first,
+                                                                   uint4 *__restrict__ pieces, const uint32_t *__restrict__ off,
+                                                                   uint32_t rows, uint32_t width, uint32_t min_piece) {
+  __shared__ uint32_t n_long, n_giant;
+  __shared__ unsigned long long giant_edges;
+  if (threadIdx.x == 0) {
+    n_long = n_giant = 0;
+    giant_edges = 0;
+  }
+  __syncthreads();
+  const uint32_t edges = off[rows] - off[0];
+  const uint64_t total = static_cast<uint64_t>(edges) * width, limit = few_long_values(total), giant_limit = few_giant_values(total);
+  auto look = [&](uint32_t r, uint32_t deg) {
+    const uint64_t n = static_cast<uint64_t>(deg) * width;
+    if (n <= limit) return;
+    if (n > giant_limit && deg > edges / kGiantCap) {
+      const uint32_t gi = atomicAdd(&n_giant, 1u);
+      if (gi < kGiantCap) {
+        giant_rows[gi] = r;
+        atomicAdd(&giant_edges, static_cast<unsigned long long>(deg));
+        return;
+      }
+    }
+    list[atomicAdd(&n_long, 1u)] = r;
+  };
+  each_row_by_block<kLongBlock>(off, rows, look);
+  __syncthreads();
+  if (threadIdx.x == 0) *count = n_long;
+  plan_giant_rows<kLongBlock>(n_giant, giant_edges, hdr, giant_rows, first, pieces, off, min_piece);
 }
 
 // One 1024-thread block per listed long row.
@@ -1285,16 +1383,17 @@ __global__ __launch_bounds__(256) void edge_softmax_short_kernel(float *__restri
   }
 }
 
-// The destinations of [base, base + 64) whose segment size lies in [min_values, max_values], as a
+// The destinations of [base, base + set) whose segment size lies in [min_values, max_values], as a
 // wave-uniform bit mask; every lane keeps the offsets of its own destination for the visit.
 __device__ __forceinline__ uint64_t wave_rows_in_class(const uint32_t *__restrict__ co, uint32_t Vd, uint64_t base,
-                                                       uint32_t H, uint32_t min_values, uint32_t max_values,
+                                                       uint32_t set, uint32_t H, uint32_t min_values, uint32_t max_values,
                                                        uint32_t &my_e0, uint32_t &my_e1) {
-  const uint64_t d = base + lane_id();
+  const uint32_t lane = lane_id();
+  const uint64_t d = base + lane;
   my_e0 = 0;
   my_e1 = 0;
   bool mine = false;
-  if (d < Vd) {
+  if (lane < set && d < Vd) {
     my_e0 = co[d];
     my_e1 = co[d + 1];
     const uint64_t n = static_cast<uint64_t>(my_e1 - my_e0) * H;
@@ -1320,14 +1419,14 @@ __global__ __launch_bounds__(256) void edge_softmax_fwd_kernel(float *__restrict
                                                                const uint32_t *__restrict__ co,
                                                                const uint32_t *__restrict__ ri, uint32_t Vd,
                                                                uint32_t H, float slope, uint32_t min_values,
-                                                               uint32_t max_values, uint32_t vec4) {
+                                                               uint32_t max_values, uint32_t vec4, uint32_t set) {
   if (max_values == kByTotal) max_values = long_segment_values(static_cast<uint64_t>(co[Vd] - co[0]) * H);
   const uint32_t lane = lane_id();
   const uint64_t wave = wave_of_grid();
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
-  for (uint64_t first = wave * kWave; first < Vd; first += n_waves * kWave) {
+  for (uint64_t first = wave * set; first < Vd; first += n_waves * set) {
     uint32_t my_e0, my_e1;
-    uint64_t todo = wave_rows_in_class(co, Vd, first, H, min_values < 1 ? 1 : min_values, max_values, my_e0, my_e1);
+    uint64_t todo = wave_rows_in_class(co, Vd, first, set, H, min_values < 1 ? 1 : min_values, max_values, my_e0, my_e1);
     while (todo) {
       const uint32_t j = static_cast<uint32_t>(__builtin_ctzll(todo));
       todo &= todo - 1;
@@ -1457,14 +1556,14 @@ __global__ __launch_bounds__(256) void edge_softmax_bwd_kernel(float *__restrict
                                                                const uint32_t *__restrict__ co,
                                                                const uint32_t *__restrict__ ri, uint32_t Vd,
                                                                uint32_t H, float slope, uint32_t min_values,
-                                                               uint32_t max_values, uint32_t vec4) {
+                                                               uint32_t max_values, uint32_t vec4, uint32_t set) {
   if (max_values == kByTotal) max_values = long_segment_values(static_cast<uint64_t>(co[Vd] - co[0]) * H);
   const uint32_t lane = lane_id();
   const uint64_t wave = wave_of_grid();
   const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
-  for (uint64_t first = wave * kWave; first < Vd; first += n_waves * kWave) {
+  for (uint64_t first = wave * set; first < Vd; first += n_waves * set) {
     uint32_t my_e0, my_e1;
-    uint64_t todo = wave_rows_in_class(co, Vd, first, H, min_values, max_values, my_e0, my_e1);
+    uint64_t todo = wave_rows_in_class(co, Vd, first, set, H, min_values, max_values, my_e0, my_e1);
     while (todo) {
       const uint32_t j = static_cast<uint32_t>(__builtin_ctzll(todo));
       todo &= todo - 1;
@@ -1590,7 +1689,7 @@ __global__ __launch_bounds__(256) void edge_softmax_bwd_kernel(float *__restrict
 // kernels).  1024 threads walk the segment's values; thread t always meets head t mod H.  Per-head
 // maxima / sums are reduced inside each wave with the head butterfly, then across the 16 waves
 // through LDS in wave order.
-template <int MODE>  // 0 = max, 1 = sum
+template <int MODE, int BLOCK = kLongBlock>  // 0 = max, 1 = sum
 __device__ __forceinline__ float block_head_reduce(float v, uint32_t H, float (*red)[kWave]) {
   const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
   v = head_reduce<MODE>(v, H);
@@ -1598,9 +1697,43 @@ __device__ __forceinline__ float block_head_reduce(float v, uint32_t H, float (*
   __syncthreads();
   const uint32_t h = lane & (H - 1);
   float r = red[0][h];
-  for (uint32_t wv = 1; wv < kLongBlock / kWave; ++wv) r = MODE == 0 ? fmaxf(r, red[wv][h]) : r + red[wv][h];
+  for (uint32_t wv = 1; wv < BLOCK / kWave; ++wv) r = MODE == 0 ? fmaxf(r, red[wv][h]) : r + red[wv][h];
   __syncthreads();
   return r;
+}
+
+// The segment of destination d by one block.
+template <bool FUSED, int BLOCK>
+__device__ __forceinline__ void softmax_fwd_by_block(float *__restrict__ y, const float *__restrict__ x,
+                                                     const float *__restrict__ el, const float *__restrict__ er,
+                                                     const uint32_t *__restrict__ co, const uint32_t *__restrict__ ri, uint32_t d,
+                                                     uint32_t H, float slope, float (*red)[kWave]) {
+  const uint32_t h = threadIdx.x & (H - 1);
+  const uint32_t e0 = co[d], e1 = co[d + 1];
+  const size_t base = static_cast<size_t>(e0) * H;
+  const size_t n = static_cast<size_t>(e1 - e0) * H;
+  float *ys = y + base;
+  const float *xs = FUSED ? nullptr : x + base;
+  float erv = 0.f;
+  if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
+  float mx = kLowestMax, sum = 0.f;
+  strided_max_sum_pass<8>(
+      threadIdx.x, n, BLOCK,
+      [&](uint64_t j) -> float {
+        if (!FUSED) return xs[j];
+        const uint32_t src = ri[e0 + j / H];
+        return leaky(el[static_cast<size_t>(src) * H + h] + erv, slope);
+      },
+      [&](uint64_t j, float sc) {
+        if (FUSED) ys[j] = sc;
+      },
+      mx, sum);
+  const float thread_mx = mx;
+  mx = block_head_reduce<0, BLOCK>(mx, H, red);
+  sum = block_head_reduce<1, BLOCK>(sum * softmax_exp(thread_mx - mx), H, red);
+  const float inv = 1.f / sum;
+  strided_pass<8>(threadIdx.x, n, BLOCK, [&](uint64_t j) -> float { return FUSED ? ys[j] : xs[j]; },
+                  [&](uint64_t j, float sc) { ys[j] = softmax_exp(sc - mx) * inv; });
 }
 
 template <bool FUSED>
@@ -1610,35 +1743,62 @@ __global__ __launch_bounds__(kLongBlock) void edge_softmax_fwd_long_kernel(
     const uint32_t *__restrict__ count, uint32_t H, float slope) {
   __shared__ float red[kLongBlock / kWave][kWave];
   const uint32_t n_rows = *count;
+  for (uint32_t i = blockIdx.x; i < n_rows; i += gridDim.x)
+    softmax_fwd_by_block<FUSED, kLongBlock>(y, x, el, er, co, ri, list[i], H, slope, red);
+}
+
+// gx over the edges [e0, e1) of destination d by one block, with their dot product given; returns with FUSED the sum of gx.
+template <bool FUSED, int BLOCK>
+__device__ __forceinline__ float softmax_bwd_pass(float *__restrict__ gx, const float *__restrict__ gy, const float *__restrict__ y,
+                                                  const float *__restrict__ el, const float *__restrict__ er,
+                                                  const uint32_t *__restrict__ ri, uint32_t d, uint32_t e0, uint32_t e1, uint32_t H,
+                                                  float slope, float dot, float (*red)[kWave]) {
   const uint32_t h = threadIdx.x & (H - 1);
-  for (uint32_t i = blockIdx.x; i < n_rows; i += gridDim.x) {
-    const uint32_t d = list[i];
-    const uint32_t e0 = co[d], e1 = co[d + 1];
-    const size_t base = static_cast<size_t>(e0) * H;
-    const size_t n = static_cast<size_t>(e1 - e0) * H;
-    float *ys = y + base;
-    const float *xs = FUSED ? nullptr : x + base;
-    float erv = 0.f;
-    if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
-    float mx = kLowestMax, sum = 0.f;
-    strided_max_sum_pass<8>(
-        threadIdx.x, n, kLongBlock,
-        [&](uint64_t j) -> float {
-          if (!FUSED) return xs[j];
-          const uint32_t src = ri[e0 + j / H];
-          return leaky(el[static_cast<size_t>(src) * H + h] + erv, slope);
-        },
-        [&](uint64_t j, float sc) {
-          if (FUSED) ys[j] = sc;
-        },
-        mx, sum);
-    const float thread_mx = mx;
-    mx = block_head_reduce<0>(mx, H, red);
-    sum = block_head_reduce<1>(sum * softmax_exp(thread_mx - mx), H, red);
-    const float inv = 1.f / sum;
-    strided_pass<8>(threadIdx.x, n, kLongBlock, [&](uint64_t j) -> float { return FUSED ? ys[j] : xs[j]; },
-                    [&](uint64_t j, float sc) { ys[j] = softmax_exp(sc - mx) * inv; });
-  }
+  const size_t base = static_cast<size_t>(e0) * H;
+  const float *gys = gy + base;
+  const float *ys = y + base;
+  float *gxs = gx + base;
+  float erv = 0.f, gsum = 0.f;
+  if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
+  strided_pass<8>(threadIdx.x, static_cast<uint64_t>(e1 - e0) * H, BLOCK,
+                  [&](uint64_t j) -> float4 {
+                    float pre = 1.f;
+                    if (FUSED) pre = el[static_cast<size_t>(ri[e0 + j / H]) * H + h] + erv;
+                    return make_float4(gys[j], ys[j], pre, 0.f);
+                  },
+                  [&](uint64_t j, float4 v) {
+                    float g = v.y * (v.x - dot);
+                    if (FUSED) {
+                      g *= v.z > 0.f ? 1.f : slope;
+                      gsum += g;
+                    }
+                    gxs[j] = g;
+                  });
+  return FUSED ? block_head_reduce<1, BLOCK>(gsum, H, red) : 0.f;
+}
+
+template <int BLOCK>
+__device__ __forceinline__ float softmax_dot_by_block(const float *__restrict__ gy, const float *__restrict__ y, uint32_t e0,
+                                                      uint32_t e1, uint32_t H, float (*red)[kWave]) {
+  const size_t base = static_cast<size_t>(e0) * H;
+  const float *gys = gy + base;
+  const float *ys = y + base;
+  float dot = 0.f;
+  strided_pass<8>(threadIdx.x, static_cast<uint64_t>(e1 - e0) * H, BLOCK, [&](uint64_t j) -> float2 { return make_float2(gys[j], ys[j]); },
+                  [&](uint64_t, float2 v) { dot += v.x * v.y; });
+  return block_head_reduce<1, BLOCK>(dot, H, red);
+}
+
+template <bool FUSED, int BLOCK>
+__device__ __forceinline__ void softmax_bwd_by_block(float *__restrict__ gx, float *__restrict__ ger, const float *__restrict__ gy,
+                                                     const float *__restrict__ y, const float *__restrict__ el,
+                                                     const float *__restrict__ er, const uint32_t *__restrict__ co,
+                                                     const uint32_t *__restrict__ ri, uint32_t d, uint32_t H, float slope,
+                                                     float (*red)[kWave]) {
+  const uint32_t e0 = co[d], e1 = co[d + 1];
+  const float dot = softmax_dot_by_block<BLOCK>(gy, y, e0, e1, H, red);
+  const float gsum = softmax_bwd_pass<FUSED, BLOCK>(gx, gy, y, el, er, ri, d, e0, e1, H, slope, dot, red);
+  if (FUSED && threadIdx.x < H) ger[static_cast<size_t>(d) * H + threadIdx.x] = gsum;
 }
 
 template <bool FUSED>
@@ -1649,40 +1809,8 @@ __global__ __launch_bounds__(kLongBlock) void edge_softmax_bwd_long_kernel(
     float slope) {
   __shared__ float red[kLongBlock / kWave][kWave];
   const uint32_t n_rows = *count;
-  const uint32_t h = threadIdx.x & (H - 1);
-  for (uint32_t i = blockIdx.x; i < n_rows; i += gridDim.x) {
-    const uint32_t d = list[i];
-    const uint32_t e0 = co[d], e1 = co[d + 1];
-    const size_t base = static_cast<size_t>(e0) * H;
-    const size_t n = static_cast<size_t>(e1 - e0) * H;
-    const float *gys = gy + base;
-    const float *ys = y + base;
-    float *gxs = gx + base;
-    float dot = 0.f;
-    strided_pass<8>(threadIdx.x, n, kLongBlock, [&](uint64_t j) -> float2 { return make_float2(gys[j], ys[j]); },
-                    [&](uint64_t, float2 v) { dot += v.x * v.y; });
-    dot = block_head_reduce<1>(dot, H, red);
-    float erv = 0.f, gsum = 0.f;
-    if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
-    strided_pass<8>(threadIdx.x, n, kLongBlock,
-                    [&](uint64_t j) -> float4 {
-                      float pre = 1.f;
-                      if (FUSED) pre = el[static_cast<size_t>(ri[e0 + j / H]) * H + h] + erv;
-                      return make_float4(gys[j], ys[j], pre, 0.f);
-                    },
-                    [&](uint64_t j, float4 v) {
-                      float g = v.y * (v.x - dot);
-                      if (FUSED) {
-                        g *= v.z > 0.f ? 1.f : slope;
-                        gsum += g;
-                      }
-                      gxs[j] = g;
-                    });
-    if (FUSED) {
-      gsum = block_head_reduce<1>(gsum, H, red);
-      if (threadIdx.x < H) ger[static_cast<size_t>(d) * H + threadIdx.x] = gsum;
-    }
-  }
+  for (uint32_t i = blockIdx.x; i < n_rows; i += gridDim.x)
+    softmax_bwd_by_block<FUSED, kLongBlock>(gx, ger, gy, y, el, er, co, ri, list[i], H, slope, red);
 }
 
 // ---- giant segments of the softmax operators ----------------------------------------------------
@@ -1692,6 +1820,41 @@ __global__ __launch_bounds__(kLongBlock) void edge_softmax_bwd_long_kernel(
 // the destination's maximum is max_p m_p and its sum is sum_p s_p * exp(m_p - m).
 // stats[piece, 0..H) / [H..2H) and rowstat[giant row, 0..H) / [H..2H) hold the two values per head.
 
+template <bool FUSED, int BLOCK>
+__device__ __forceinline__ void giant_softmax_stats(float *__restrict__ stats, float *__restrict__ y, const float *__restrict__ x,
+                                                    const float *__restrict__ el, const float *__restrict__ er,
+                                                    const uint32_t *__restrict__ ri, uint32_t p, uint4 pc, uint32_t H, float slope,
+                                                    float (*red)[kWave]) {
+  const uint32_t h = threadIdx.x & (H - 1);
+  const uint32_t d = pc.y, e0 = pc.z;
+  const size_t base = static_cast<size_t>(e0) * H;
+  const uint64_t n = static_cast<uint64_t>(pc.w - e0) * H;
+  float *ys = y + base;
+  const float *xs = FUSED ? nullptr : x + base;
+  float erv = 0.f;
+  if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
+  float mx = kLowestMax;
+  strided_pass<8>(threadIdx.x, n, BLOCK,
+                  [&](uint64_t j) -> float {
+                    if (!FUSED) return xs[j];
+                    const uint32_t src = ri[e0 + j / H];
+                    return leaky(el[static_cast<size_t>(src) * H + h] + erv, slope);
+                  },
+                  [&](uint64_t j, float sc) {
+                    if (FUSED) ys[j] = sc;
+                    mx = fmaxf(mx, sc);
+                  });
+  mx = block_head_reduce<0, BLOCK>(mx, H, red);
+  float sum = 0.f;
+  strided_pass<8>(threadIdx.x, n, BLOCK, [&](uint64_t j) -> float { return FUSED ? ys[j] : xs[j]; },
+                  [&](uint64_t, float sc) { sum += softmax_exp(sc - mx); });
+  sum = block_head_reduce<1, BLOCK>(sum, H, red);
+  if (threadIdx.x < H) {
+    stats[static_cast<size_t>(p) * 2 * H + threadIdx.x] = mx;
+    stats[static_cast<size_t>(p) * 2 * H + H + threadIdx.x] = sum;
+  }
+}
+
 template <bool FUSED>
 __global__ __launch_bounds__(kLongBlock) void giant_softmax_stats_kernel(
     float *__restrict__ stats, float *__restrict__ y, const float *__restrict__ x, const float *__restrict__ el,
@@ -1699,41 +1862,12 @@ __global__ __launch_bounds__(kLongBlock) void giant_softmax_stats_kernel(
     const uint4 *__restrict__ pieces, uint32_t H, float slope) {
   __shared__ float red[kLongBlock / kWave][kWave];
   const uint32_t n_pieces = hdr[1];
-  const uint32_t h = threadIdx.x & (H - 1);
-  for (uint32_t p = blockIdx.x; p < n_pieces; p += gridDim.x) {
-    const uint4 pc = pieces[p];
-    const uint32_t d = pc.y, e0 = pc.z;
-    const size_t base = static_cast<size_t>(e0) * H;
-    const uint64_t n = static_cast<uint64_t>(pc.w - e0) * H;
-    float *ys = y + base;
-    const float *xs = FUSED ? nullptr : x + base;
-    float erv = 0.f;
-    if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
-    float mx = kLowestMax;
-    strided_pass<8>(threadIdx.x, n, kLongBlock,
-                    [&](uint64_t j) -> float {
-                      if (!FUSED) return xs[j];
-                      const uint32_t src = ri[e0 + j / H];
-                      return leaky(el[static_cast<size_t>(src) * H + h] + erv, slope);
-                    },
-                    [&](uint64_t j, float sc) {
-                      if (FUSED) ys[j] = sc;
-                      mx = fmaxf(mx, sc);
-                    });
-    mx = block_head_reduce<0>(mx, H, red);
-    float sum = 0.f;
-    strided_pass<8>(threadIdx.x, n, kLongBlock, [&](uint64_t j) -> float { return FUSED ? ys[j] : xs[j]; },
-                    [&](uint64_t, float sc) { sum += softmax_exp(sc - mx); });
-    sum = block_head_reduce<1>(sum, H, red);
-    if (threadIdx.x < H) {
-      stats[static_cast<size_t>(p) * 2 * H + threadIdx.x] = mx;
-      stats[static_cast<size_t>(p) * 2 * H + H + threadIdx.x] = sum;
-    }
-  }
+  for (uint32_t p = blockIdx.x; p < n_pieces; p += gridDim.x)
+    giant_softmax_stats<FUSED, kLongBlock>(stats, y, x, el, er, ri, p, pieces[p], H, slope, red);
 }
 
 // MODE 0: online-softmax combine of (m_p, s_p).  MODE 1: plain sum of stats[piece, 0..H) in piece
-// order; the result goes to rowstat[giant row, 0..H) or, when `to_rows` is set, to to_rows[row, 0..H)
+// order (`width` floats of a piece from the next); the result goes to rowstat[giant row, 0..H) or, when `to_rows` is set, to to_rows[row, 0..H)
 // (the per-destination gradient sum of the fused backward).
 template <int MODE>
 __global__ __launch_bounds__(64) void giant_softmax_combine_kernel(float *__restrict__ rowstat,
@@ -1741,11 +1875,10 @@ __global__ __launch_bounds__(64) void giant_softmax_combine_kernel(float *__rest
                                                                    const float *__restrict__ stats,
                                                                    const uint32_t *__restrict__ hdr,
                                                                    const uint32_t *__restrict__ giant_rows,
-                                                                   const uint32_t *__restrict__ first, uint32_t H) {
+                                                                   const uint32_t *__restrict__ first, uint32_t H, uint32_t width) {
   const uint32_t n = hdr[0];
   const uint32_t h = threadIdx.x;
   if (h >= H) return;
-  const uint32_t width = MODE == 0 ? 2 * H : H;
   for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
     const uint32_t p0 = first[i], p1 = first[i + 1];
     if (MODE == 0) {
@@ -1798,14 +1931,7 @@ __global__ __launch_bounds__(kLongBlock) void giant_softmax_dot_kernel(float *__
   const uint32_t n_pieces = hdr[1];
   for (uint32_t p = blockIdx.x; p < n_pieces; p += gridDim.x) {
     const uint4 pc = pieces[p];
-    const size_t base = static_cast<size_t>(pc.z) * H;
-    const uint64_t n = static_cast<uint64_t>(pc.w - pc.z) * H;
-    const float *gys = gy + base;
-    const float *ys = y + base;
-    float dot = 0.f;
-    strided_pass<8>(threadIdx.x, n, kLongBlock, [&](uint64_t j) -> float2 { return make_float2(gys[j], ys[j]); },
-                    [&](uint64_t, float2 v) { dot += v.x * v.y; });
-    dot = block_head_reduce<1>(dot, H, red);
+    const float dot = softmax_dot_by_block<kLongBlock>(gy, y, pc.z, pc.w, H, red);
     if (threadIdx.x < H) stats[static_cast<size_t>(p) * H + threadIdx.x] = dot;
   }
 }
@@ -1822,33 +1948,395 @@ __global__ __launch_bounds__(kLongBlock) void giant_softmax_bwd_apply_kernel(
   const uint32_t h = threadIdx.x & (H - 1);
   for (uint32_t p = blockIdx.x; p < n_pieces; p += gridDim.x) {
     const uint4 pc = pieces[p];
-    const uint32_t d = pc.y, e0 = pc.z;
-    const size_t base = static_cast<size_t>(e0) * H;
-    const uint64_t n = static_cast<uint64_t>(pc.w - e0) * H;
-    const float *gys = gy + base;
-    const float *ys = y + base;
-    float *gxs = gx + base;
     const float dot = rowstat[static_cast<size_t>(pc.x) * 2 * H + h];
-    float erv = 0.f, gsum = 0.f;
-    if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
-    strided_pass<8>(threadIdx.x, n, kLongBlock,
-                    [&](uint64_t j) -> float4 {
-                      float pre = 1.f;
-                      if (FUSED) pre = el[static_cast<size_t>(ri[e0 + j / H]) * H + h] + erv;
-                      return make_float4(gys[j], ys[j], pre, 0.f);
-                    },
-                    [&](uint64_t j, float4 v) {
-                      float g = v.y * (v.x - dot);
-                      if (FUSED) {
-                        g *= v.z > 0.f ? 1.f : slope;
-                        gsum += g;
-                      }
-                      gxs[j] = g;
-                    });
-    if (FUSED) {
-      gsum = block_head_reduce<1>(gsum, H, red);
-      if (threadIdx.x < H) stats[static_cast<size_t>(p) * H + threadIdx.x] = gsum;
+    const float gsum = softmax_bwd_pass<FUSED, kLongBlock>(gx, gy, y, el, er, ri, pc.y, pc.z, pc.w, H, slope, dot, red);
+    if (FUSED && threadIdx.x < H) stats[static_cast<size_t>(p) * H + threadIdx.x] = gsum;
+  }
+}
+
+// ---- softmax operators on few rows ----------------------------------------------------------------
+//
+// Calls of at most kFewRows destinations, heads a power of two up to kShortG: what the kernels above do in nine to eleven
+// launches on two streams, whose gaps and idle ends are most of the time there (and, below a million values, the host's
+// launching them all of it), in one, or three to four where there are hub rows:
+//   few_long_rows_kernel   lists the hub rows and cuts the giant ones (from kLongMinVertices rows up)
+//   few_softmax_kernel     its first blocks take the listed rows and the pieces' statistics; every other wavefront a set of
+//                          consecutive rows, short segments four at a time, each of the longer ones by the whole wavefront
+//   few_giant_apply_kernel combines the statistics of a piece's row itself and writes the piece
+//   giant_softmax_combine_kernel  (fused backward) the sums of the giant rows' gradients
+// stats[piece, 0 .. 2H): (maximum, sum) forward; (dot product, sum of gx) backward.
+constexpr uint64_t kDenseRow = 64;  // edges a row from which a wavefront takes kDenseSet rows together
+constexpr uint32_t kDenseSet = 4;
+template <bool FUSED>
+__device__ __forceinline__ void softmax_fwd_by_wave(float *__restrict__ ys, const float *__restrict__ xs, const float *__restrict__ el,
+                                                    const float *__restrict__ er, const uint32_t *__restrict__ ri, uint32_t d, uint32_t e0,
+                                                    uint64_t n, uint32_t H, float slope, uint32_t lane) {
+  if (n <= kWaveRegValues) {
+    NTS_BY_SLOTS(kWave, softmax_fwd_regs, ys, xs, el, er, ri, d, e0, n, H, slope, lane);
+    return;
+  }
+  const uint32_t h = lane & (H - 1);
+  float erv = 0.f;
+  if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
+  float mx = kLowestMax, sum = 0.f;
+  strided_max_sum_pass<8>(
+      lane, n, kWave,
+      [&](uint64_t i) -> float {
+        if (!FUSED) return xs[i];
+        const uint32_t src = ri[e0 + i / H];
+        return leaky(el[static_cast<size_t>(src) * H + h] + erv, slope);
+      },
+      [&](uint64_t i, float sc) {
+        if (FUSED) ys[i] = sc;
+      },
+      mx, sum);
+  const float lane_mx = mx;
+  mx = head_reduce<0>(mx, H);
+  sum = head_reduce<1>(sum * softmax_exp(lane_mx - mx), H);
+  const float inv = 1.f / sum;
+  strided_pass<8>(lane, n, kWave, [&](uint64_t i) -> float { return FUSED ? ys[i] : xs[i]; },
+                  [&](uint64_t i, float sc) { ys[i] = softmax_exp(sc - mx) * inv; });
+}
+
+template <bool FUSED>
+__device__ __forceinline__ void softmax_bwd_by_wave(float *__restrict__ gxs, float *__restrict__ ger, const float *__restrict__ gys,
+                                                    const float *__restrict__ ys, const float *__restrict__ el,
+                                                    const float *__restrict__ er, const uint32_t *__restrict__ ri, uint32_t d, uint32_t e0,
+                                                    uint64_t n, uint32_t H, float slope, uint32_t lane) {
+  if (n <= kWaveRegValues) {
+    NTS_BY_SLOTS(kWave, softmax_bwd_regs, gxs, ger, gys, ys, el, er, ri, d, e0, n, H, slope, lane);
+    return;
+  }
+  const uint32_t h = lane & (H - 1);
+  float dot = 0.f;
+  strided_pass<8>(lane, n, kWave, [&](uint64_t i) -> float2 { return make_float2(gys[i], ys[i]); },
+                  [&](uint64_t, float2 v) { dot += v.x * v.y; });
+  dot = head_reduce<1>(dot, H);
+  float erv = 0.f, gsum = 0.f;
+  if (FUSED) erv = er[static_cast<size_t>(d) * H + h];
+  strided_pass<8>(lane, n, kWave,
+                  [&](uint64_t i) -> float4 {
+                    float pre = 1.f;
+                    if (FUSED) pre = el[static_cast<size_t>(ri[e0 + i / H]) * H + h] + erv;
+                    return make_float4(gys[i], ys[i], pre, 0.f);
+                  },
+                  [&](uint64_t i, float4 v) {
+                    float g = v.y * (v.x - dot);
+                    if (FUSED) {
+                      g *= v.z > 0.f ? 1.f : slope;
+                      gsum += g;
+                    }
+                    gxs[i] = g;
+                  });
+  if (FUSED) {
+    gsum = head_reduce<1>(gsum, H);
+    if (lane < H) ger[static_cast<size_t>(d) * H + lane] = gsum;
+  }
+}
+
+// The fused operators' segments above the register class with 16-byte lanes (heads a multiple of four, 16-byte aligned arrays), by
+// a wavefront or a block: thread t of WIDTH takes the vectors t, t + WIDTH, ... of the segment, four consecutive heads of one
+// edge each, and always meets the heads h0 = 4 t mod H .. + 3; threads H / 4 apart hold the same ones.  `most` and `all` reduce
+// over these.
+struct Attention4 {
+  const float *el;
+  const uint32_t *ri;
+  uint32_t e0, H, h0;
+  float4 er;
+  float slope;
+  __device__ __forceinline__ Attention4(const float *el_, const float *er_, const uint32_t *ri_, uint32_t d, uint32_t e0_, uint32_t H_,
+                                        float slope_, uint32_t t)
+      : el(el_), ri(ri_), e0(e0_), H(H_), h0((t * 4u) & (H_ - 1)), slope(slope_) {
+    er = *reinterpret_cast<const float4 *>(er_ + static_cast<size_t>(d) * H + h0);
+  }
+  __device__ __forceinline__ float4 sum(uint64_t i) const {  // el + er of vector i
+    const uint32_t src = ri[e0 + static_cast<uint32_t>(i * 4 / H)];
+    const float4 e = *reinterpret_cast<const float4 *>(el + static_cast<size_t>(src) * H + h0);
+    return make_float4(e.x + er.x, e.y + er.y, e.z + er.z, e.w + er.w);
+  }
+  __device__ __forceinline__ float4 score(uint64_t i) const {
+    const float4 v = sum(i);
+    return make_float4(leaky(v.x, slope), leaky(v.y, slope), leaky(v.z, slope), leaky(v.w, slope));
+  }
+};
+// Raw scores to ys, and the (maximum, sum) of each of the four heads.
+template <int WIDTH, typename Most, typename All>
+__device__ __forceinline__ void attention_stats4(float4 *__restrict__ ys, const Attention4 &a, uint64_t nv, uint32_t t, Most most, All all,
+                                                 float (&mx)[4], float (&sum)[4]) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    mx[c] = kLowestMax;
+    sum[c] = 0.f;
+  }
+  strided_max_sum_pass4<4>(t, nv, WIDTH, [&](uint64_t i) { return a.score(i); }, [&](uint64_t i, float4 v) { ys[i] = v; }, mx, sum);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const float own = mx[c];
+    mx[c] = most(own);
+    sum[c] = all(sum[c] * softmax_exp(own - mx[c]));
+  }
+}
+template <int WIDTH>
+__device__ __forceinline__ void attention_write4(float4 *__restrict__ ys, uint64_t nv, uint32_t t, const float (&mx)[4], const float (&sum)[4]) {
+  const float inv[4] = {1.f / sum[0], 1.f / sum[1], 1.f / sum[2], 1.f / sum[3]};
+  strided_pass<4>(t, nv, WIDTH, [&](uint64_t i) -> float4 { return ys[i]; },
+                  [&](uint64_t i, float4 v) {
+                    ys[i] = make_float4(softmax_exp(v.x - mx[0]) * inv[0], softmax_exp(v.y - mx[1]) * inv[1], softmax_exp(v.z - mx[2]) * inv[2],
+                                        softmax_exp(v.w - mx[3]) * inv[3]);
+                  });
+}
+template <int WIDTH, typename All>
+__device__ __forceinline__ void attention_dot4(const float4 *__restrict__ gys, const float4 *__restrict__ ys, uint64_t nv, uint32_t t, All all,
+                                               float (&dot)[4]) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) dot[c] = 0.f;
+  struct Two {
+    float4 g, a;
+  };
+  strided_pass<4>(t, nv, WIDTH, [&](uint64_t i) -> Two { return Two{gys[i], ys[i]}; },
+                  [&](uint64_t, Two v) {
+                    dot[0] += v.g.x * v.a.x;
+                    dot[1] += v.g.y * v.a.y;
+                    dot[2] += v.g.z * v.a.z;
+                    dot[3] += v.g.w * v.a.w;
+                  });
+#pragma unroll
+  for (int c = 0; c < 4; ++c) dot[c] = all(dot[c]);
+}
+// gx of the segment; gsum: its sum over each of the four heads.
+template <int WIDTH, typename All>
+__device__ __forceinline__ void attention_bwd4(float4 *__restrict__ gxs, const float4 *__restrict__ gys, const float4 *__restrict__ ys,
+                                               const Attention4 &a, uint64_t nv, uint32_t t, All all, const float (&dot)[4], float (&gsum)[4]) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) gsum[c] = 0.f;
+  strided_pass<4>(t, nv, WIDTH, [&](uint64_t i) -> float4 { return a.sum(i); },
+                  [&](uint64_t i, float4 s) {
+                    const float4 g = gys[i], y = ys[i];
+                    const float4 r = make_float4(y.x * (g.x - dot[0]) * (s.x > 0.f ? 1.f : a.slope), y.y * (g.y - dot[1]) * (s.y > 0.f ? 1.f : a.slope),
+                                                 y.z * (g.z - dot[2]) * (s.z > 0.f ? 1.f : a.slope), y.w * (g.w - dot[3]) * (s.w > 0.f ? 1.f : a.slope));
+                    gsum[0] += r.x;
+                    gsum[1] += r.y;
+                    gsum[2] += r.z;
+                    gsum[3] += r.w;
+                    gxs[i] = r;
+                  });
+#pragma unroll
+  for (int c = 0; c < 4; ++c) gsum[c] = all(gsum[c]);
+}
+
+struct FewHubs {
+  const uint32_t *list, *count, *hdr, *first;
+  const uint4 *pieces;
+  float *stats;
+  uint32_t blocks;  // of the launch, set aside for them (0: no hub rows are looked for)
+};
+
+// A hub row or a piece of a giant row by one block of 256 threads.
+template <bool FUSED, bool BWD, bool VEC4>
+__device__ __forceinline__ void few_hub_row(float *__restrict__ out, float *__restrict__ ger, const float *__restrict__ x_or_gy,
+                                            const float *__restrict__ y, const float *__restrict__ el, const float *__restrict__ er,
+                                            const uint32_t *__restrict__ co, const uint32_t *__restrict__ ri, uint32_t d, uint32_t H,
+                                            float slope, float (*red)[kWave]) {
+  if constexpr (!VEC4) {
+    if (BWD) softmax_bwd_by_block<FUSED, 256>(out, ger, x_or_gy, y, el, er, co, ri, d, H, slope, red);
+    else softmax_fwd_by_block<FUSED, 256>(out, x_or_gy, el, er, co, ri, d, H, slope, red);
+  } else {
+    const uint32_t t = threadIdx.x, e0 = co[d], hq = H / 4;
+    const uint64_t nv = static_cast<uint64_t>(co[d + 1] - e0) * hq;
+    const Attention4 a(el, er, ri, d, e0, H, slope, t);
+    float4 *outs = reinterpret_cast<float4 *>(out + static_cast<size_t>(e0) * H);
+    auto most = [&](float v) { return block_head_reduce<0, 256>(v, hq, red); };
+    auto all = [&](float v) { return block_head_reduce<1, 256>(v, hq, red); };
+    float s0[4], s1[4];
+    if constexpr (BWD) {
+      const float4 *gys = reinterpret_cast<const float4 *>(x_or_gy + static_cast<size_t>(e0) * H), *ys = reinterpret_cast<const float4 *>(y + static_cast<size_t>(e0) * H);
+      attention_dot4<256>(gys, ys, nv, t, all, s0);
+      attention_bwd4<256>(outs, gys, ys, a, nv, t, all, s0, s1);
+      if (t < hq) *reinterpret_cast<float4 *>(ger + static_cast<size_t>(d) * H + a.h0) = make_float4(s1[0], s1[1], s1[2], s1[3]);
+    } else {
+      attention_stats4<256>(outs, a, nv, t, most, all, s0, s1);
+      attention_write4<256>(outs, nv, t, s0, s1);
     }
+  }
+}
+template <bool FUSED, bool BWD, bool VEC4>
+__device__ __forceinline__ void few_giant_piece(float *__restrict__ stats, float *__restrict__ out, const float *__restrict__ x_or_gy,
+                                                const float *__restrict__ y, const float *__restrict__ el, const float *__restrict__ er,
+                                                const uint32_t *__restrict__ ri, uint32_t p, uint4 pc, uint32_t H, float slope,
+                                                float (*red)[kWave]) {
+  if constexpr (BWD) {
+    const float dot = softmax_dot_by_block<256>(x_or_gy, y, pc.z, pc.w, H, red);
+    if (threadIdx.x < H) stats[static_cast<size_t>(p) * 2 * H + threadIdx.x] = dot;
+  } else if constexpr (!VEC4) {
+    giant_softmax_stats<FUSED, 256>(stats, out, x_or_gy, el, er, ri, p, pc, H, slope, red);
+  } else {
+    const uint32_t t = threadIdx.x, hq = H / 4;
+    const Attention4 a(el, er, ri, pc.y, pc.z, H, slope, t);
+    float mx[4], sum[4];
+    attention_stats4<256>(
+        reinterpret_cast<float4 *>(out + static_cast<size_t>(pc.z) * H), a, static_cast<uint64_t>(pc.w - pc.z) * hq, t,
+        [&](float v) { return block_head_reduce<0, 256>(v, hq, red); }, [&](float v) { return block_head_reduce<1, 256>(v, hq, red); }, mx, sum);
+    if (t < hq) {
+      float *st = stats + static_cast<size_t>(p) * 2 * H + a.h0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        st[c] = mx[c];
+        st[H + c] = sum[c];
+      }
+    }
+  }
+}
+
+template <bool FUSED, bool BWD, bool VEC4>
+__global__ __launch_bounds__(256) void few_softmax_kernel(float *__restrict__ out, float *__restrict__ ger,
+                                                          const float *__restrict__ x_or_gy, const float *__restrict__ y,
+                                                          const float *__restrict__ el, const float *__restrict__ er,
+                                                          const uint32_t *__restrict__ co, const uint32_t *__restrict__ ri,
+                                                          uint32_t Vd, uint32_t H, float slope, uint32_t set, FewHubs hubs) {
+  if (blockIdx.x < hubs.blocks) {
+    __shared__ float red[256 / kWave][kWave];
+    if (!hubs.list) {
+      // Few enough rows for every hub block to find its own: a row is the block's that its number hashes to.  (There are fewer
+      // than 2,048 of them: each holds more than a 1/2,048 share of the values.)
+      __shared__ uint32_t found, rows_here[2048];
+      if (threadIdx.x == 0) found = 0;
+      __syncthreads();
+      const uint64_t limit = few_long_values(static_cast<uint64_t>(co[Vd] - co[0]) * H);
+      each_row_by_block<256>(co, Vd, [&](uint32_t r, uint32_t deg) {
+        if (static_cast<uint64_t>(deg) * H > limit && (r * 2654435761u >> 16) % hubs.blocks == blockIdx.x)
+          if (const uint32_t at = atomicAdd(&found, 1u); at < 2048) rows_here[at] = r;
+      });
+      __syncthreads();
+      const uint32_t n = found < 2048 ? found : 2048;
+      for (uint32_t i = 0; i < n; ++i) few_hub_row<FUSED, BWD, VEC4>(out, ger, x_or_gy, y, el, er, co, ri, rows_here[i], H, slope, red);
+      return;
+    }
+    const uint32_t n_rows = *hubs.count, n_pieces = hubs.hdr[1];
+    for (uint32_t i = blockIdx.x; i < n_rows + n_pieces; i += hubs.blocks) {
+      if (i < n_rows) few_hub_row<FUSED, BWD, VEC4>(out, ger, x_or_gy, y, el, er, co, ri, hubs.list[i], H, slope, red);
+      else few_giant_piece<FUSED, BWD, VEC4>(hubs.stats, out, x_or_gy, y, el, er, ri, i - n_rows, hubs.pieces[i - n_rows], H, slope, red);
+    }
+    return;
+  }
+  const uint32_t lane = lane_id();
+  const uint64_t n_waves = static_cast<uint64_t>(gridDim.x - hubs.blocks) * (256 / kWave);
+  const uint64_t limit = hubs.blocks ? few_long_values(static_cast<uint64_t>(co[Vd] - co[0]) * H) : ~0ull;
+  if (co[Vd] - co[0] >= kDenseRow * Vd) set = set < kDenseSet ? set : kDenseSet;
+  for (uint64_t first = wave_of_grid(hubs.blocks) * set; first < Vd; first += n_waves * set) {
+    uint32_t my_e0 = 0, my_e1 = 0;
+    const bool mine = lane < set && first + lane < Vd;
+    if (mine) {
+      my_e0 = co[first + lane];
+      my_e1 = co[first + lane + 1];
+    }
+    const uint64_t my_n = static_cast<uint64_t>(my_e1 - my_e0) * H;
+    uint64_t todo = __ballot(my_n > kShortValues && my_n <= limit);
+    const uint64_t shorts = __ballot(mine && my_n <= kShortValues && (my_n || (BWD && FUSED)));
+    {
+      const uint32_t gl = lane & (kShortG - 1), grp = lane / kShortG;
+      for (uint64_t left = shorts; left;) {
+        // the next four short rows, one a group
+        uint32_t j = kWave;
+#pragma unroll
+        for (uint32_t g = 0; g < kWave / kShortG; ++g) {
+          if (left) {
+            if (g == grp) j = static_cast<uint32_t>(__builtin_ctzll(left));
+            left &= left - 1;
+          }
+        }
+        const uint32_t e0 = __shfl(my_e0, j & (kWave - 1), kWave), e1 = __shfl(my_e1, j & (kWave - 1), kWave);
+        const uint32_t n = j < kWave ? (e1 - e0) * H : 0u, d = static_cast<uint32_t>(first) + j;
+        const size_t base = static_cast<size_t>(e0) * H;
+        if (BWD) {
+          if (j < kWave) {
+            if (!any_lane(n > 2u * kShortG)) softmax_bwd_regs<FUSED, kShortG, 2>(out + base, ger, x_or_gy + base, y + base, el, er, ri, d, e0, n, H, slope, gl);
+            else softmax_bwd_regs<FUSED, kShortG, kShortK>(out + base, ger, x_or_gy + base, y + base, el, er, ri, d, e0, n, H, slope, gl);
+          }
+        } else if (n) {
+          NTS_BY_SLOTS(kShortG, softmax_fwd_regs, out + base, FUSED ? nullptr : x_or_gy + base, el, er, ri, d, e0, n, H, slope, gl);
+        }
+      }
+    }
+    while (todo) {
+      const uint32_t j = static_cast<uint32_t>(__builtin_ctzll(todo));
+      todo &= todo - 1;
+      const uint32_t d = static_cast<uint32_t>(first) + j;
+      const uint32_t e0 = wave_read(my_e0, j), e1 = wave_read(my_e1, j);
+      const size_t base = static_cast<size_t>(e0) * H;
+      const uint64_t n64 = static_cast<uint64_t>(e1 - e0) * H;
+      if constexpr (VEC4) {
+        if (n64 > kWaveRegValues) {
+          const uint32_t hq = H / 4;
+          const uint64_t nv = n64 / 4;
+          const Attention4 a(el, er, ri, d, e0, H, slope, lane);
+          float4 *outs = reinterpret_cast<float4 *>(out + base);
+          auto most = [&](float v) { return head_reduce<0>(v, hq); };
+          auto all = [&](float v) { return head_reduce<1>(v, hq); };
+          float s0[4], s1[4];
+          if constexpr (BWD) {
+            const float4 *gys = reinterpret_cast<const float4 *>(x_or_gy + base), *ys = reinterpret_cast<const float4 *>(y + base);
+            attention_dot4<kWave>(gys, ys, nv, lane, all, s0);
+            attention_bwd4<kWave>(outs, gys, ys, a, nv, lane, all, s0, s1);
+            if (lane < hq) *reinterpret_cast<float4 *>(ger + static_cast<size_t>(d) * H + a.h0) = make_float4(s1[0], s1[1], s1[2], s1[3]);
+          } else {
+            attention_stats4<kWave>(outs, a, nv, lane, most, all, s0, s1);
+            attention_write4<kWave>(outs, nv, lane, s0, s1);
+          }
+          continue;
+        }
+      }
+      if (BWD) softmax_bwd_by_wave<FUSED>(out + base, ger, x_or_gy + base, y + base, el, er, ri, d, e0, n64, H, slope, lane);
+      else softmax_fwd_by_wave<FUSED>(out + base, FUSED ? nullptr : x_or_gy + base, el, er, ri, d, e0, n64, H, slope, lane);
+    }
+  }
+}
+
+template <bool FUSED, bool BWD, bool VEC4>
+__global__ __launch_bounds__(256) void few_giant_apply_kernel(float *__restrict__ out, const float *__restrict__ x_or_gy,
+                                                              const float *__restrict__ y, const float *__restrict__ el,
+                                                              const float *__restrict__ er, const uint32_t *__restrict__ ri,
+                                                              uint32_t H, float slope, FewHubs hubs) {
+  __shared__ float red[256 / kWave][kWave];
+  const uint32_t n_pieces = hubs.hdr[1];
+  const uint32_t lane = lane_id(), h = lane & (H - 1);
+  for (uint32_t p = blockIdx.x; p < n_pieces; p += gridDim.x) {
+    const uint4 pc = hubs.pieces[p];
+    // lane l takes the pieces l / H, l / H + 64 / H, ... of the row, then the lanes of a head are combined
+    const uint32_t q0 = hubs.first[pc.x] + lane / H, q1 = hubs.first[pc.x + 1];
+    const float *st = hubs.stats + h;
+    if (BWD) {
+      float dot = 0.f;
+      for (uint32_t q = q0; q < q1; q += kWave / H) dot += st[static_cast<size_t>(q) * 2 * H];
+      dot = head_reduce<1>(dot, H);
+      if constexpr (VEC4) {
+        const uint32_t t = threadIdx.x, hq = H / 4;
+        const Attention4 a(el, er, ri, pc.y, pc.z, H, slope, t);
+        const size_t base = static_cast<size_t>(pc.z) * H;
+        float d4[4], gsum[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) d4[c] = __shfl(dot, a.h0 + c, kWave);  // (lane h holds head h)
+        attention_bwd4<256>(reinterpret_cast<float4 *>(out + base), reinterpret_cast<const float4 *>(x_or_gy + base),
+                            reinterpret_cast<const float4 *>(y + base), a, static_cast<uint64_t>(pc.w - pc.z) * hq, t,
+                            [&](float v) { return block_head_reduce<1, 256>(v, hq, red); }, d4, gsum);
+        if (t < hq) *reinterpret_cast<float4 *>(hubs.stats + static_cast<size_t>(p) * 2 * H + H + a.h0) = make_float4(gsum[0], gsum[1], gsum[2], gsum[3]);
+        continue;
+      }
+      const float gsum = softmax_bwd_pass<FUSED, 256>(out, x_or_gy, y, el, er, ri, pc.y, pc.z, pc.w, H, slope, dot, red);
+      if (FUSED && threadIdx.x < H) hubs.stats[static_cast<size_t>(p) * 2 * H + H + threadIdx.x] = gsum;
+      continue;
+    }
+    float mx = kLowestMax, sum = 0.f;
+    for (uint32_t q = q0; q < q1; q += kWave / H) mx = fmaxf(mx, st[static_cast<size_t>(q) * 2 * H]);
+    mx = head_reduce<0>(mx, H);
+    for (uint32_t q = q0; q < q1; q += kWave / H)
+      sum += st[static_cast<size_t>(q) * 2 * H + H] * softmax_exp(st[static_cast<size_t>(q) * 2 * H] - mx);
+    sum = head_reduce<1>(sum, H);
+    const float inv = 1.f / sum;
+    const size_t base = static_cast<size_t>(pc.z) * H;
+    float *ys = out + base;
+    const float *xs = FUSED ? ys : x_or_gy + base;  // the fused forward left the raw score in y
+    strided_pass<8>(threadIdx.x, static_cast<uint64_t>(pc.w - pc.z) * H, 256, [&](uint64_t j) -> float { return xs[j]; },
+                    [&](uint64_t j, float sc) { ys[j] = softmax_exp(sc - mx) * inv; });
   }
 }
 
@@ -2040,8 +2528,7 @@ struct LongRows {
 // Collects the rows whose segment holds more than `limit` values (edges * width) when the vertex
 // count makes hubs likely, the ones above `giant_limit` values separately (with their piece table);
 // returns with lr.list == nullptr when the long path is not used.
-int collect_long_rows(LongRows &lr, const uint32_t *off, uint32_t rows, uint32_t width, uint32_t limit,
-                      uint64_t giant_limit, uint32_t min_piece, hipStream_t stream) {
+int take_long_rows(LongRows &lr, uint32_t rows, hipStream_t stream) {
   if (rows < kLongMinVertices) return NTS_OK;
   const size_t list_bytes = (static_cast<size_t>(rows) + 7) / 8 * 8 * sizeof(uint32_t);  // list, 32-byte multiple
   const size_t small_bytes = (8 + kGiantCap + kGiantCap + 8) * sizeof(uint32_t);  // hdr (with the counter), rows, first
@@ -2053,6 +2540,11 @@ int collect_long_rows(LongRows &lr, const uint32_t *off, uint32_t rows, uint32_t
   lr.giant_rows = lr.hdr + 8;
   lr.first = lr.giant_rows + kGiantCap;
   lr.pieces = reinterpret_cast<uint4 *>(buf + list_bytes + small_bytes);
+  return NTS_OK;
+}
+int collect_long_rows(const LongRows &lr, const uint32_t *off, uint32_t rows, uint32_t width, uint32_t limit,
+                      uint64_t giant_limit, uint32_t min_piece, hipStream_t stream) {
+  if (!lr.list) return NTS_OK;
   if (int rc = nts_memset_zero(lr.hdr, 8 * sizeof(uint32_t), stream)) return rc;  // counters and the ticket
   hipLaunchKernelGGL(collect_long_rows_kernel, dim3(ceil_div(rows, 256)), dim3(256), 0, stream, lr.list, lr.count,
                      lr.giant_rows, lr.hdr, off, rows, width, limit, giant_limit);
@@ -2207,6 +2699,7 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   // permutation 669 -> 605).
   uint64_t giant_edges = kGiantRowBytes / (4ull * F);
   giant_edges = giant_edges > 16384 ? 16384 : giant_edges < kLongRowEdges ? kLongRowEdges : giant_edges;
+  if (int rc = take_long_rows(lr, rows, stream)) return rc;
   if (int rc = collect_long_rows(lr, off, rows, 1u, kLongRowEdges, giant_edges, static_cast<uint32_t>(giant_edges / 4),
                                  stream))
     return rc;
@@ -2340,6 +2833,57 @@ class SideWork {
   SideLane *lane_;
 };
 
+// Destinations that a wavefront of the softmax wave kernels looks at together: it visits those of its class one after the other, so
+// as few as leave the chip its 8,192 wavefronts.  us, 64 / so, fused backward, H = 1 and 4: 60 K rows, 4 M edges 134 / 99, 232 / 123; 169 K,
+// 2.48 M 90 / 84, 145 / 121; from 524,288 rows up 64 (600 K, 3 M forward 115, 16 129).
+uint32_t softmax_rows_per_wave(uint32_t Vd) {
+  constexpr uint32_t kChipWaves = 8192;
+  uint32_t per = kWave;
+  while (per > 8 && Vd / per < kChipWaves) per /= 2;
+  return per;
+}
+
+constexpr uint32_t kFewHubBlocks = 128;  // that look for their hub rows themselves
+// Destinations that a wavefront takes together in a call of few rows (kDenseSet where these are long): 64 / 16 / 4 fused forward
+// 169 K rows, 2.48 M edges H = 1 74 / 66 / 76, 30 K, 1 M 64 / 39 / 35, 200 K, 20 M 235 / 192 / 179.
+uint32_t few_rows_per_wave(uint32_t Vd) {
+  constexpr uint32_t kChipWaves = 8192;
+  uint32_t per = kWave;
+  while (per > 4 && Vd / per < kChipWaves) per /= 2;
+  return per;
+}
+
+template <bool FUSED, bool BWD, bool VEC4>
+int few_softmax(float *out, float *ger, const float *x_or_gy, const float *y, const float *el, const float *er, const uint32_t *co,
+                const uint32_t *ri, uint32_t Vd, uint32_t H, float slope, bool look_for_hubs, hipStream_t stream, const char *who) {
+  LongRows lr;
+  ScratchBlock stats_block;
+  FewHubs hubs{};
+  if (look_for_hubs) {
+    if (int rc = take_long_rows(lr, Vd, stream)) return rc;
+    hubs.blocks = lr.list ? kLongGrid : kFewHubBlocks;
+  }
+  if (lr.list) {
+    NTS_HIP_TRY(stats_block.alloc(static_cast<size_t>(kPieceCap) * 2 * H * sizeof(float), stream));
+    hubs = FewHubs{lr.list, lr.count, lr.hdr, lr.first, lr.pieces, static_cast<float *>(stats_block.ptr), kLongGrid};
+    hipLaunchKernelGGL(few_long_rows_kernel, dim3(1), dim3(kLongBlock), 0, stream, lr.list, lr.count, lr.giant_rows, lr.hdr, lr.first,
+                       lr.pieces, co, Vd, H, kFewPieceValues / H);
+    NTS_LAUNCH_CHECK(who);
+  }
+  const uint32_t set = few_rows_per_wave(Vd);
+  hipLaunchKernelGGL((few_softmax_kernel<FUSED, BWD, VEC4>), dim3(hubs.blocks + ceil_div(Vd, 4 * (set < kDenseSet ? set : kDenseSet))), dim3(256), 0, stream, out,
+                     ger, x_or_gy, y, el, er, co, ri, Vd, H, slope, set, hubs);
+  NTS_LAUNCH_CHECK(who);
+  if (!lr.list) return NTS_OK;
+  hipLaunchKernelGGL((few_giant_apply_kernel<FUSED, BWD, VEC4>), dim3(kLongGrid), dim3(256), 0, stream, out, x_or_gy, y, el, er, ri, H, slope, hubs);
+  if (FUSED && BWD)
+    hipLaunchKernelGGL(giant_softmax_combine_kernel<1>, dim3(kGiantCap / 4), dim3(64), 0, stream, static_cast<float *>(nullptr), ger,
+                       hubs.stats + H, lr.hdr, lr.giant_rows, lr.first, H, 2 * H);
+  NTS_LAUNCH_CHECK(who);
+  NTS_HIP_TRY(stats_block.release());
+  return release_long_rows(lr);
+}
+
 // Edge softmax / fused attention, forward (gy == nullptr) or backward; x / el / er / ri / ger are
 // null where the variant does not use them.
 int softmax_impl(bool backward, bool fused, float *out, float *ger, const float *x_or_gy, const float *y,
@@ -2352,8 +2896,17 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   // also one that a call without a bound would hand to a block because its values are few in all.  A longer segment than
   // stated is still computed, by one wavefront.
   const bool no_hubs = max_degree != 0 && static_cast<uint64_t>(max_degree) * H <= kLongRowValues;
+  const bool one_short_launch = fused && max_degree != 0 && static_cast<uint64_t>(max_degree) * H <= kShortValues;
+  if (pow2 && H <= static_cast<uint32_t>(kShortG) && Vd <= (fused && backward ? kFewRowsFusedBackward : kFewRows) && !one_short_launch) {
+    const bool vec4 = fused && H % 4 == 0 && aligned_to(out, 16) && aligned_to(x_or_gy, 16) && aligned_to(y, 16) && aligned_to(el, 16) &&
+                      aligned_to(er, 16) && aligned_to(ger, 16);
+    auto call = [&](auto f) { return f(out, ger, x_or_gy, y, el, er, co, ri, Vd, H, slope, !no_hubs, stream, who); };
+    if (!fused) return backward ? call(few_softmax<false, true, false>) : call(few_softmax<false, false, false>);
+    if (vec4) return backward ? call(few_softmax<true, true, true>) : call(few_softmax<true, false, true>);
+    return backward ? call(few_softmax<true, true, false>) : call(few_softmax<true, false, false>);
+  }
   if (pow2 && !no_hubs)
-    if (int rc = collect_long_rows(lr, co, Vd, H, kByTotal, 0, kGiantMinPiece, stream)) return rc;
+    if (int rc = take_long_rows(lr, Vd, stream)) return rc;
   const uint32_t max_values = lr.list ? kByTotal : kNoLimit;
   // The block kernels of the hub rows and the kernels of the giant ones' pieces run on the side lane,
   // beside the launches for all other rows below (they write other rows); their scratch is taken
@@ -2363,6 +2916,8 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   if (lr.list) NTS_HIP_TRY(stats_block.alloc((stats_floats + row_floats) * sizeof(float), stream));
   SideWork side(stream, lr.list != nullptr);
   const hipStream_t hub_stream = side.stream();
+  // (listing them too: the launches of the other rows do not need it; 169 K rows, 2.48 M edges, one head 86 -> 76 us)
+  if (int rc = collect_long_rows(lr, co, Vd, H, kByTotal, 0, kGiantMinPiece, hub_stream)) return rc;
   // 16-byte lanes for the segments that do not fit the register paths: whole heads per lane and
   // every array 16-byte aligned (a segment starts at e0 * H floats).
   const uint32_t vec4 = pow2 && H % 4 == 0 && aligned_to(out, 16) && aligned_to(x_or_gy, 16) && aligned_to(y, 16) &&
@@ -2375,6 +2930,7 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   const dim3 short_grid(short_blocks < 16384u ? short_blocks : 16384u);
   const uint32_t wave_blocks = ceil_div(Vd, 4);  // at most one destination per wavefront
   const dim3 grid(wave_blocks < 8192u ? wave_blocks : 8192u);
+  const uint32_t set = softmax_rows_per_wave(Vd);
   if (lr.list) {
     // The hub rows first: their few large blocks take their places on the chip before the launches for
     // all other rows fill it.
@@ -2406,7 +2962,7 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
         hipLaunchKernelGGL(giant_softmax_stats_kernel<false>, pgrid, pblock, 0, hub_stream, stats, out, x_or_gy, el, er, ri,
                            lr.hdr, lr.pieces, H, slope);
       hipLaunchKernelGGL(giant_softmax_combine_kernel<0>, cgrid, cblock, 0, hub_stream, rowstat,
-                         static_cast<float *>(nullptr), stats, lr.hdr, lr.giant_rows, lr.first, H);
+                         static_cast<float *>(nullptr), stats, lr.hdr, lr.giant_rows, lr.first, H, 2 * H);
       if (fused)
         hipLaunchKernelGGL(giant_softmax_apply_kernel<true>, pgrid, pblock, 0, hub_stream, out, x_or_gy, rowstat, lr.hdr,
                            lr.pieces, H);
@@ -2416,12 +2972,12 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
     } else {
       hipLaunchKernelGGL(giant_softmax_dot_kernel, pgrid, pblock, 0, hub_stream, stats, x_or_gy, y, lr.hdr, lr.pieces, H);
       hipLaunchKernelGGL(giant_softmax_combine_kernel<1>, cgrid, cblock, 0, hub_stream, rowstat,
-                         static_cast<float *>(nullptr), stats, lr.hdr, lr.giant_rows, lr.first, H);
+                         static_cast<float *>(nullptr), stats, lr.hdr, lr.giant_rows, lr.first, H, H);
       if (fused) {
         hipLaunchKernelGGL(giant_softmax_bwd_apply_kernel<true>, pgrid, pblock, 0, hub_stream, out, stats, x_or_gy, y, el, er,
                            ri, rowstat, lr.hdr, lr.pieces, H, slope);
         hipLaunchKernelGGL(giant_softmax_combine_kernel<1>, cgrid, cblock, 0, hub_stream, rowstat, ger, stats, lr.hdr,
-                           lr.giant_rows, lr.first, H);
+                           lr.giant_rows, lr.first, H, H);
       } else {
         hipLaunchKernelGGL(giant_softmax_bwd_apply_kernel<false>, pgrid, pblock, 0, hub_stream, out, stats, x_or_gy, y, el, er,
                            ri, rowstat, lr.hdr, lr.pieces, H, slope);
@@ -2429,7 +2985,7 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
     }
     NTS_LAUNCH_CHECK(who);
   }
-  if (use_short && fused && max_degree != 0 && static_cast<uint64_t>(max_degree) * H <= kShortValues) {
+  if (use_short && one_short_launch) {
     // Every segment fits the short class by the caller's word: one launch (which still computes a
     // longer segment, slowly, should there be one).
     if (backward)
@@ -2453,7 +3009,7 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   if (!backward) {
 #define NTS_FWD(FU, P2, PART, LO, HI)                                                                             \
   hipLaunchKernelGGL((edge_softmax_fwd_kernel<FU, P2, PART>), grid, block, 0, stream, out, x_or_gy, el, er, co, ri, \
-                     Vd, H, slope, LO, HI, vec4)
+                     Vd, H, slope, LO, HI, vec4, set)
     if (pow2 && fused) {
       // the register-resident segments, then the longer ones
       NTS_FWD(true, true, 1, min_values, kWaveRegValues);
@@ -2471,7 +3027,7 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   } else {
 #define NTS_BWD(FU, P2, PART, LO, HI)                                                                            \
   hipLaunchKernelGGL((edge_softmax_bwd_kernel<FU, P2, PART>), grid, block, 0, stream, out, ger, x_or_gy, y, el, er, co, \
-                     ri, Vd, H, slope, LO, HI, vec4)
+                     ri, Vd, H, slope, LO, HI, vec4, set)
     if (pow2 && fused) {
       NTS_BWD(true, true, 1, min_values, kWaveRegValues);
       // (a launch of its own for the class above that, held in registers as in the forward pass, measured no

@@ -1,0 +1,90 @@
+"""The softmax operators on few rows, which take one to four launches: segments on both sides of the lines between the groups of
+16 lanes, the wavefronts, the blocks and the pieces (1/2,048 and 1/256 of the call's values, within 1,024 .. 32,768 and 8,192 ..
+131,072), rows on both sides of where hub rows are listed by a launch (16,384) and of where other kernels take over (32,768
+for the fused backward, 262,144), long and short rows on average, arrays on and off 16-byte boundaries.
+
+A segment of n values is summed by chains of at most n / 64 additions whose results are added in trees: off by at most
+(n / 64 + 64) 2^-24 of the sum of its terms' magnitudes.  An exponential is off by |x| 2^-24 of itself (|x| < 32 here:
+2e-6), a quotient and a product by an ulp each."""
+import pytest
+import torch
+
+from neutronbench_amd.abi import call, ptr
+
+pytestmark = pytest.mark.gpu
+
+
+def degrees(total, H, V):
+    """V degrees with about total edges * H values in all, some on either side of every line, three above the last."""
+    line = min(max(total // 2048, 1024), 32768)
+    giant = min(max(total // 256, 8192), 131072)
+    marks = [n // H + d for n in (128, 512, line, giant) for d in (-1, 0, 1)] + [3 * giant // H, 5 * giant // H, 0, 1]
+    marks = marks[:V] if V > len(marks) else [giant // H + 1, 0, 129 // H + 1][:V]
+    deg = torch.zeros(V, dtype=torch.int64)
+    at = torch.randperm(V, generator=torch.Generator().manual_seed(total + H))
+    deg[at[:len(marks)]] = torch.tensor(marks)
+    rest = at[len(marks):]
+    left = max(0, total // H - int(deg.sum()))
+    if len(rest):
+        deg[rest] = left // len(rest)
+        deg[rest[:left % len(rest)]] += 1
+    return deg
+
+
+@pytest.mark.parametrize("V,total,H,shift", [(1, 20000, 1, 0), (3, 20000, 4, 0), (100, 1 << 17, 16, 0), (2047, 1 << 18, 2, 0),
+                                             (2500, 1 << 21, 4, 0), (2500, 1 << 21, 4, 1), (2500, 1 << 20, 8, 0), (16383, 1 << 20, 1, 0),
+                                             (16384, 1 << 20, 1, 0), (16385, 1 << 22, 4, 0), (16385, 1 << 22, 4, 1), (20001, 1 << 23, 8, 0),
+                                             (20001, 1 << 22, 16, 0), (32768, 1 << 20, 4, 0), (32769, 1 << 20, 4, 0),
+                                             (262144, 1 << 21, 1, 0), (262145, 1 << 21, 1, 0), (262143, 1 << 22, 4, 0)])
+def test_softmax_on_few_rows(device, V, total, H, shift):
+    print(f"case V={V} total={total} H={H} shift={shift}", flush=True)
+    slope = 0.2
+    deg = degrees(total, H, V).to(device)
+    E = int(deg.sum())
+    off = torch.cat([deg.new_zeros(1), deg.cumsum(0)])
+    co, own = off.to(torch.int32), torch.repeat_interleave(torch.arange(V, device=device), deg)
+    g = torch.Generator(device=device).manual_seed(H)
+    s = torch.cuda.current_stream().cuda_stream
+
+    def array(rows, fill=None):
+        a = torch.randn(rows * H + shift, generator=g, device=device) if fill is None else torch.full((rows * H + shift,), fill, device=device)
+        return a[shift:].view(rows, H)
+
+    el, er, gy, x = array(V), array(V), array(E), array(E)
+    ri = torch.randint(V, (E,), generator=g, device=device)
+    n = (deg * H).double()[own, None]
+    bound = (n / 64 + 64) * 2.0 ** -24 + 4e-6
+
+    def per_row(v):
+        return torch.zeros(V, H, dtype=torch.float64, device=device).index_add_(0, own, v)
+
+    def near(got, want, size):
+        assert ((got.double() - want).abs() <= bound * size).all()
+
+    pre = el[ri] + er[own]
+    for fused in (True, False):
+        wide = (torch.where(pre > 0, pre, pre * slope) if fused else x).double()
+        top = torch.full((V, H), -torch.inf, dtype=torch.float64, device=device)
+        top.scatter_reduce_(0, own[:, None].expand(E, H), wide, "amax")
+        ex = (wide - top[own]).exp()
+        want = ex / per_row(ex)[own]
+        y, gx, ger = array(E, float("nan")), array(E, float("nan")), array(V, float("nan"))
+        ri32 = ri.to(torch.int32)
+        if fused:
+            call("nts_gat_attention_fwd", ptr(y), ptr(el), ptr(er), ptr(co), ptr(ri32), V, H, slope, s)
+        else:
+            call("nts_edge_softmax_fwd", ptr(y), ptr(x), ptr(co), V, H, s)
+        near(y, want, want)
+        if fused:
+            call("nts_gat_attention_bwd", ptr(gx), ptr(ger), ptr(gy), ptr(y), ptr(el), ptr(er), ptr(co), ptr(ri32), V, H, slope, s)
+        else:
+            call("nts_edge_softmax_bwd", ptr(gx), ptr(gy), ptr(y), ptr(co), V, H, s)
+        ya, ga = y.double(), gy.double()
+        sign = torch.where(pre > 0, 1.0, slope).double() if fused else 1.0
+        size = ya.abs() * (ga.abs() + per_row((ya * ga).abs())[own])
+        wgx = ya * (ga - per_row(ya * ga)[own]) * sign
+        near(gx, wgx, size)
+        if fused:
+            want_er, mag = per_row(wgx), per_row(size)
+            row_bound = (deg * H).double()[:, None] / 64 * 2.0 ** -24 + 64 * 2.0 ** -24 + 4e-6
+            assert ((ger.double() - want_er).abs() <= 2 * row_bound * mag).all()
