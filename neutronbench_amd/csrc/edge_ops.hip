@@ -200,61 +200,6 @@ constexpr uint32_t kByTotal = 0;               // in place of a line: long_segme
 constexpr uint32_t kLongMinVertices = 16384;  // vertex count below which the extra launches are not worth it
 constexpr int kLongBlock = 1024;
 
-// out[r,:] (+)= sum_{k in [off[r], off[r+1])} msg[perm ? perm[k] : k, :], added in k order.
-template <typename V, int G>
-__global__ __launch_bounds__(256) void gather_edge_to_row_kernel(V *__restrict__ out, const V *__restrict__ msg,
-                                                                 const uint32_t *__restrict__ off,
-                                                                 const uint32_t *__restrict__ perm, uint32_t rows,
-                                                                 uint32_t Fv, int accumulate, uint32_t long_limit) {
-  const uint32_t r = (blockIdx.x * blockDim.x + threadIdx.x) / G;
-  if (r >= rows) return;
-  const uint32_t gl = threadIdx.x & (G - 1);
-  const uint32_t e0 = off[r], e1 = off[r + 1];
-  if (e1 - e0 > long_limit) return;
-  constexpr int NF = sizeof(V) / 4;
-  for (uint32_t c = gl; c < Fv; c += G) {
-    float a[NF];
-#pragma unroll
-    for (int t = 0; t < NF; ++t) a[t] = 0.f;
-    // Eight edge rows are loaded before they are added, in order: the loads overlap, the order of
-    // the additions stays the edge order.
-    uint32_t k = e0;
-    for (; k + 8 <= e1; k += 8) {
-      V v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const uint32_t e = perm ? perm[k + u] : k + u;
-        v[u] = msg[static_cast<size_t>(e) * Fv + c];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const float *vf = reinterpret_cast<const float *>(&v[u]);
-#pragma unroll
-        for (int t = 0; t < NF; ++t) a[t] += vf[t];
-      }
-    }
-    for (; k < e1; ++k) {
-      const uint32_t e = perm ? perm[k] : k;
-      const V v = msg[static_cast<size_t>(e) * Fv + c];
-      const float *vf = reinterpret_cast<const float *>(&v);
-#pragma unroll
-      for (int t = 0; t < NF; ++t) a[t] += vf[t];
-    }
-    V *p = out + static_cast<size_t>(r) * Fv + c;
-    if (accumulate) {
-      const V o = *p;
-      const float *of = reinterpret_cast<const float *>(&o);
-#pragma unroll
-      for (int t = 0; t < NF; ++t) a[t] += of[t];
-    }
-    V res;
-    float *rf = reinterpret_cast<float *>(&res);
-#pragma unroll
-    for (int t = 0; t < NF; ++t) rf[t] = a[t];
-    *p = res;
-  }
-}
-
 // What the first blocks of a row launch do beside it when the rows above `long_limit` edges are summed
 // in the same launch: the list of those rows, the piece table of the giant ones, where the pieces' sums
 // go, the column tile of a 256-thread block and how many blocks are set aside (0: none).
@@ -284,37 +229,49 @@ __device__ __forceinline__ float4 vnull<float4>() {
   return make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// Sum of the edge rows [e0, e1) by one block of BLOCK threads, added into dst[0 .. Fv) (V = float, or
+// Sum of the columns [first_col, end_col) of the edge rows [e0, e1) by one block of BLOCK threads, added into dst (V = float, or
 // float4 when rows are 16-byte aligned: a quarter of the load instructions and of the rounds a row
 // takes).  Columns are taken in tiles of `tile` vectors (a power of two <= BLOCK); thread t owns
 // column t % tile of slice t / tile, a slice adds every (BLOCK/tile)-th edge of the range in ascending
-// order (eight loads in flight), and the slices' sums are then added pairwise in a fixed tree.
-template <typename V, int BLOCK>
+// order (a round's loads together), and the slices' sums are then added pairwise in a fixed tree.
+template <typename V, int BLOCK, int U>
 __device__ __forceinline__ void block_sum_edge_rows(V *__restrict__ dst, const V *__restrict__ msg,
                                                     const uint32_t *__restrict__ perm, uint32_t e0, uint32_t e1,
-                                                    uint32_t Fv, uint32_t tile, int accumulate, V *part) {
+                                                    uint32_t Fv, uint32_t first_col, uint32_t end_col, uint32_t tile,
+                                                    int accumulate, V *part) {
   const uint32_t c = threadIdx.x & (tile - 1);
   const uint32_t slice = threadIdx.x / tile;
   const uint32_t n_slices = BLOCK / tile;
-  for (uint32_t cb = 0; cb < Fv; cb += tile) {
+  for (uint32_t cb = first_col; cb < end_col; cb += tile) {
     const uint32_t col = cb + c;
     V a = vnull<V>();
-    if (col < Fv) {
-      uint32_t k = e0 + slice;
-      for (; static_cast<uint64_t>(k) + 7ull * n_slices < e1; k += 8 * n_slices) {
-        V v[8];
+    if (col < end_col && e1 - e0 > slice) {
+      // The edge ids of the next round are requested while the rows of this one are on their way; beyond the range the last edge's.
+      // Through a permutation, 2.48 M edges of 47 floats 704 -> 379 us.  Eight vectors a round took the kernels 98 registers instead of
+      // 62 (30 K rows, 3 M edges F = 128 467, held to 72 with spills 502, four a round 467); narrow rows, whose kernels hold as many anyway,
+      // have room for them.
+      uint32_t k = e0 + slice, left = e1 - k, id[U];
+      auto request_ids = [&] {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const uint32_t kk = k + u * n_slices;
-          const uint32_t e = perm ? perm[kk] : kk;
-          v[u] = msg[static_cast<size_t>(e) * Fv + col];
+        for (int u = 0; u < U; ++u) {
+          const uint32_t kk = k + (u * n_slices < left ? u * n_slices : left - 1);
+          id[u] = perm ? perm[kk] : kk;
+        }
+      };
+      request_ids();
+      while (left) {
+        V v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = msg[static_cast<size_t>(id[u]) * Fv + col];
+        const uint32_t now = left;
+        left = left > U * n_slices ? left - U * n_slices : 0u;
+        if (left) {
+          k += U * n_slices;
+          request_ids();
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) vadd(a, v[u]);
-      }
-      for (; k < e1; k += n_slices) {
-        const uint32_t e = perm ? perm[k] : k;
-        vadd(a, msg[static_cast<size_t>(e) * Fv + col]);
+        for (int u = 0; u < U; ++u)
+          if (u * n_slices < now) vadd(a, v[u]);
       }
     }
     part[threadIdx.x] = a;
@@ -327,7 +284,7 @@ __device__ __forceinline__ void block_sum_edge_rows(V *__restrict__ dst, const V
       }
       __syncthreads();
     }
-    if (slice == 0 && col < Fv) {
+    if (slice == 0 && col < end_col) {
       V total = part[c];
       if (accumulate) vadd(total, dst[col]);
       dst[col] = total;
@@ -336,27 +293,133 @@ __device__ __forceinline__ void block_sum_edge_rows(V *__restrict__ dst, const V
   }
 }
 
+// Calls of fewer than kLongMinVertices rows, whose hub rows no launch lists: the edges of a row above which it is the first
+// blocks' (a row of 1,024 edges and less is one running sum, whoever adds it up), so that there are fewer than kFewLongRows of them.
+// One group or wavefront added a hub row up before, 8 edges a memory latency: contiguous / permuted sums, us, 2 K rows, 100 K edges
+// F = 4 321 / 454 -> 51 / 71, F = 128 1,063 / 1,132 -> 138 / 155; 10 K, 3 M F = 4 960 / 788 -> 52 / 63, F = 47 5,932 / 11,554 -> 645 / 827;
+// 16 K, 1 M F = 128 1,604 / 3,746 -> 190 / 319; without hub rows 16 K, 40 K F = 4 15 / 11 -> 14 / 11, 2.7 K, 13 K F = 128 52 / 53 -> 53 / 52.
+constexpr uint32_t kFewLongRows = 2048;
+constexpr uint32_t kMinHubGroups = 64;
+static_assert(kLongMinVertices <= 256 * kMinHubGroups && kLongMinVertices % 2 == 0, "a row a thread");
+template <typename V, int G>
+constexpr int kHubLoads = sizeof(V) == 16 && G > 8 ? 4 : 8;  // vectors that a thread of a hub block requests together
+template <typename V>
+constexpr uint32_t kHubBytes = 256 * (sizeof(V) + sizeof(uint16_t));  // scratch of a block that looks for them
+__device__ __forceinline__ uint32_t few_long_edges(const uint32_t *__restrict__ off, uint32_t rows) {
+  const uint32_t share = (off[rows] - off[0]) / kFewLongRows;
+  return share < kLongRowEdges ? kLongRowEdges : share;
+}
+template <typename V>
+__device__ __forceinline__ uint32_t long_limit_of(const LongRowWork<V> &lw, uint32_t limit, const uint32_t *__restrict__ off, uint32_t rows) {
+  return lw.blocks && !lw.list ? few_long_edges(off, rows) : limit;
+}
+
 // The first blocks of a row launch take the listed long rows, one 256-thread block per row, and the
 // pieces of the giant ones (their partial sums are combined by a launch of its own afterwards); the
 // rows of the launch proper fill the chip meanwhile.
-template <typename V>
+template <typename V, int U>
 __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out, const V *__restrict__ msg,
                                                             const uint32_t *__restrict__ off,
-                                                            const uint32_t *__restrict__ perm, uint32_t Fv,
-                                                            int accumulate, const LongRowWork<V> &lw) {
-  __shared__ V long_part[256];
-  const uint32_t n_rows = *lw.count;
+                                                            const uint32_t *__restrict__ perm, uint32_t rows, uint32_t Fv,
+                                                            int accumulate, const LongRowWork<V> &lw, void *scratch) {
+  V *part = static_cast<V *>(scratch);  // 256 of them
+  if (!lw.list) {
+    // Few enough rows for these blocks to find the hubs among them: the rows are dealt out to groups of blocks in an order without
+    // pattern (hubs of a generated graph have neighbouring numbers), a row a thread, and the blocks of a group take the column
+    // tiles of the hub rows among its own.  (A list of all hub rows in every block took it 20 us where the offsets were not in its L2.)
+    uint16_t *found = reinterpret_cast<uint16_t *>(part + 256);  // 256 of them
+    __shared__ uint32_t n_found;
+    if (threadIdx.x == 0) n_found = 0;
+    const uint32_t tiles = (Fv + lw.tile - 1) / lw.tile, most = lw.blocks / kMinHubGroups, sharers = tiles < most ? tiles : most;
+    const uint32_t groups = lw.blocks / sharers, group = blockIdx.x / sharers;
+    const uint32_t at = threadIdx.x * groups + group, r = at * 40503u % kLongMinVertices;  // (odd: every row once)
+    uint32_t deg = 0;
+    if (group < groups && at < kLongMinVertices && r < rows) deg = off[r + 1] - off[r];
+    const uint32_t limit = few_long_edges(off, rows);
+    __syncthreads();
+    if (deg > limit) found[atomicAdd(&n_found, 1u)] = static_cast<uint16_t>(r);
+    __syncthreads();
+    const uint32_t n = n_found;
+    for (uint32_t i = 0; i < n; ++i) {
+      const uint32_t row = found[i];
+      for (uint32_t t = blockIdx.x % sharers; t < tiles; t += sharers) {
+        const uint32_t c0 = t * lw.tile, c1 = c0 + lw.tile < Fv ? c0 + lw.tile : Fv;
+        block_sum_edge_rows<V, 256, U>(out + static_cast<size_t>(row) * Fv, msg, perm, off[row], off[row + 1], Fv, c0, c1, lw.tile, accumulate, part);
+      }
+    }
+    return;
+  }
+  const uint32_t n_rows = *lw.count, n_pieces = lw.hdr[1];
   for (uint32_t i = blockIdx.x; i < n_rows; i += lw.blocks) {
     const uint32_t r = lw.list[i];
-    block_sum_edge_rows<V, 256>(out + static_cast<size_t>(r) * Fv, msg, perm, off[r], off[r + 1], Fv, lw.tile,
-                                accumulate, long_part);
+    block_sum_edge_rows<V, 256, U>(out + static_cast<size_t>(r) * Fv, msg, perm, off[r], off[r + 1], Fv, 0, Fv, lw.tile, accumulate, part);
   }
-  const uint32_t n_pieces = lw.hdr[1];
   // the pieces start with the blocks that the rows left idle
   for (uint32_t p = (blockIdx.x + lw.blocks - n_rows % lw.blocks) % lw.blocks; p < n_pieces; p += lw.blocks) {
     const uint4 pc = lw.pieces[p];
-    block_sum_edge_rows<V, 256>(lw.partial + static_cast<size_t>(p) * Fv, msg, perm, pc.z, pc.w, Fv, lw.tile, 0,
-                                long_part);
+    block_sum_edge_rows<V, 256, U>(lw.partial + static_cast<size_t>(p) * Fv, msg, perm, pc.z, pc.w, Fv, 0, Fv, lw.tile, 0, part);
+  }
+}
+
+// out[r,:] (+)= sum_{k in [off[r], off[r+1])} msg[perm ? perm[k] : k, :], added in k order.
+template <typename V, int G>
+__global__ __launch_bounds__(256, (sizeof(V) == 4 ? 8 : 1)) void gather_edge_to_row_kernel(V *__restrict__ out, const V *__restrict__ msg,
+                                                                 const uint32_t *__restrict__ off,
+                                                                 const uint32_t *__restrict__ perm, uint32_t rows,
+                                                                 uint32_t Fv, int accumulate, uint32_t long_limit, LongRowWork<V> lw) {
+  if (blockIdx.x < lw.blocks) {
+    __shared__ V scratch[kHubBytes<V> / sizeof(V)];
+    sum_long_rows_in_this_block<V, sizeof(V) == 16 ? 4 : 8>(out, msg, off, perm, rows, Fv, accumulate, lw, scratch);
+    return;
+  }
+  long_limit = long_limit_of(lw, long_limit, off, rows);
+  const uint32_t r = ((blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / G;
+  if (r >= rows) return;
+  const uint32_t gl = threadIdx.x & (G - 1);
+  const uint32_t e0 = off[r], e1 = off[r + 1];
+  if (e1 - e0 > long_limit) return;
+  constexpr int NF = sizeof(V) / 4;
+  for (uint32_t c = gl; c < Fv; c += G) {
+    float a[NF];
+#pragma unroll
+    for (int t = 0; t < NF; ++t) a[t] = 0.f;
+    // U edge rows are loaded before they are added, in order: the loads overlap, the order of
+    // the additions stays the edge order.
+    constexpr int U = 16;
+    uint32_t k = e0;
+    for (; static_cast<uint64_t>(k) + U <= e1; k += U) {
+      V v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t e = perm ? perm[k + u] : k + u;
+        v[u] = msg[static_cast<size_t>(e) * Fv + c];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float *vf = reinterpret_cast<const float *>(&v[u]);
+#pragma unroll
+        for (int t = 0; t < NF; ++t) a[t] += vf[t];
+      }
+    }
+    for (; k < e1; ++k) {
+      const uint32_t e = perm ? perm[k] : k;
+      const V v = msg[static_cast<size_t>(e) * Fv + c];
+      const float *vf = reinterpret_cast<const float *>(&v);
+#pragma unroll
+      for (int t = 0; t < NF; ++t) a[t] += vf[t];
+    }
+    V *p = out + static_cast<size_t>(r) * Fv + c;
+    if (accumulate) {
+      const V o = *p;
+      const float *of = reinterpret_cast<const float *>(&o);
+#pragma unroll
+      for (int t = 0; t < NF; ++t) a[t] += of[t];
+    }
+    V res;
+    float *rf = reinterpret_cast<float *>(&res);
+#pragma unroll
+    for (int t = 0; t < NF; ++t) rf[t] = a[t];
+    *p = res;
   }
 }
 
@@ -393,16 +456,18 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
                                                                         const uint32_t *__restrict__ off,
                                                                         uint32_t rows, uint32_t Fv, int accumulate,
                                                                         uint32_t long_limit, LongRowWork<V> lw) {
-  if (blockIdx.x < lw.blocks) {
-    sum_long_rows_in_this_block(out, msg, off, static_cast<const uint32_t *>(nullptr), Fv, accumulate, lw);
-    return;
-  }
   constexpr int NF = sizeof(V) / 4;
   constexpr int U = 8;                            // loads per lane and round
+  __shared__ __align__(16) float tiles[4][kWave * U * NF];
+  if (blockIdx.x < lw.blocks) {
+    static_assert(sizeof(tiles) >= kHubBytes<V>, "the hub blocks' scratch");
+    sum_long_rows_in_this_block<V, kHubLoads<V, G>>(out, msg, off, static_cast<const uint32_t *>(nullptr), rows, Fv, accumulate, lw, tiles);
+    return;
+  }
+  long_limit = long_limit_of(lw, long_limit, off, rows);
   constexpr uint32_t kSlots = kWave / G;          // edge rows per load of the wavefront
   constexpr uint32_t kRound = kSlots * U;         // edge rows per round
   constexpr uint32_t kPitch = G * NF;             // floats of an edge row in the tile
-  __shared__ float tiles[4][kWave * U * NF];
   float *tile = tiles[wave_of_block()];
   const uint32_t lane = lane_id();
   const uint32_t col = lane & (G - 1), slot = lane / G;
@@ -538,21 +603,23 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
 template <int GG>  // lanes that share a row
 constexpr uint32_t kFullSet = kWave / GG * 8u < kWave ? kWave / GG * 8u : static_cast<uint32_t>(kWave);
 template <typename V, int G, int S, bool FEW>
-__global__ __launch_bounds__(256) void gather_edge_to_row_balanced_kernel(V *__restrict__ out,
+__global__ __launch_bounds__(256, (sizeof(V) == 4 ? 8 : G <= 8 ? 5 : 1)) void gather_edge_to_row_balanced_kernel(V *__restrict__ out,
                                                                           const V *__restrict__ msg,
                                                                           const uint32_t *__restrict__ off,
                                                                           const uint32_t *__restrict__ perm,
                                                                           uint32_t rows, uint32_t Fv, int accumulate,
                                                                           uint32_t long_limit, uint32_t coop_limit,
                                                                           uint32_t few_rows, LongRowWork<V> lw) {
-  if (blockIdx.x < lw.blocks) {
-    sum_long_rows_in_this_block(out, msg, off, perm, Fv, accumulate, lw);
-    return;
-  }
   constexpr bool kCoop = G <= 8;
   constexpr int kCoopU = sizeof(V) == 16 ? 4 : 8;           // loads per lane and round on the cooperative path
   constexpr uint32_t kCoopFloats = kWave * kCoopU * (sizeof(V) / 4);  // floats of a wavefront's tile
-  __shared__ float coop_tile[kCoop ? 4 : 1][kCoop ? kCoopFloats : 1];
+  __shared__ __align__(16) float coop_tile[kCoop ? 4 : 1][kCoop ? kCoopFloats : kHubBytes<V> / 4];
+  if (blockIdx.x < lw.blocks) {
+    static_assert(sizeof(coop_tile) >= kHubBytes<V>, "the hub blocks' scratch");
+    sum_long_rows_in_this_block<V, kHubLoads<V, G>>(out, msg, off, perm, rows, Fv, accumulate, lw, coop_tile);
+    return;
+  }
+  long_limit = long_limit_of(lw, long_limit, off, rows);
   constexpr int NF = sizeof(V) / 4;
   const uint32_t lane = lane_id();
   constexpr int GG = G * S;  // lanes that share a row
@@ -809,8 +876,9 @@ __device__ __forceinline__ uint64_t giant_segment_values(uint64_t total_values) 
 // The same for a call of few rows (kFewRows), whose launch has blocks of 256 threads for both.
 // The rows, by both sides' times in us, the kernels of many rows / these, edge softmax (H = 1, 4) and attention, forward, backward:
 //   rows, edges     softmax fwd       bwd               attention fwd       bwd
-//   2.7 K, 13 K     7 / 6, 7 / 7      8 / 6, 7 / 6      14 / 7, 18 / 10     11 / 7, 18 / 9
-//   10 K, 3 M       69 / 39, 304 / 129  67 / 40, 307 / 125  327 / 115, 572 / 182  387 / 129, 525 / 180
+//   2.7 K, 13 K     7 / 4, 7 / 5      8 / 5, 7 / 5      14 / 6, 18 / 9      11 / 6, 18 / 9
+//   16 K, 200 K     10 / 8, 20 / 15   9 / 7, 17 / 12    37 / 14, 51 / 29    30 / 13, 38 / 26
+//   10 K, 3 M       69 / 33, 304 / 128  67 / 34, 307 / 120  327 / 116, 572 / 207  387 / 141, 525 / 197
 //   30 K, 1 M       82 / 40, 94 / 39  85 / 40, 96 / 40  88 / 39, 99 / 55    92 / 42, 106 / 67
 //   60 K, 4 M       84 / 43, 84 / 65  86 / 41, 95 / 76  94 / 70, 135 / 113  99 / 88, 125 / 134
 //   169 K, 2.48 M   65 / 48, 70 / 62  66 / 47, 72 / 64  80 / 65, 139 / 109  84 / 86, 118 / 124
@@ -989,7 +1057,7 @@ __global__ __launch_bounds__(kLongBlock) void gather_edge_to_row_long_kernel(
   const uint32_t n_rows = *count;
   for (uint32_t i = blockIdx.x; i < n_rows; i += gridDim.x) {
     const uint32_t r = list[i];
-    block_sum_edge_rows<V, kLongBlock>(out + static_cast<size_t>(r) * Fv, msg, perm, off[r], off[r + 1], Fv, tile,
+    block_sum_edge_rows<V, kLongBlock, sizeof(V) == 16 ? 4 : 8>(out + static_cast<size_t>(r) * Fv, msg, perm, off[r], off[r + 1], Fv, 0, Fv, tile,
                                        accumulate, part);
   }
 }
@@ -1006,7 +1074,7 @@ __global__ __launch_bounds__(kLongBlock) void giant_sum_pieces_kernel(V *__restr
   const uint32_t n_pieces = hdr[1];
   for (uint32_t p = blockIdx.x; p < n_pieces; p += gridDim.x) {
     const uint4 pc = pieces[p];
-    block_sum_edge_rows<V, kLongBlock>(partial + static_cast<size_t>(p) * Fv, msg, perm, pc.z, pc.w, Fv, tile, 0, part);
+    block_sum_edge_rows<V, kLongBlock, sizeof(V) == 16 ? 4 : 8>(partial + static_cast<size_t>(p) * Fv, msg, perm, pc.z, pc.w, Fv, 0, Fv, tile, 0, part);
   }
 }
 
@@ -2196,19 +2264,20 @@ __global__ __launch_bounds__(256) void few_softmax_kernel(float *__restrict__ ou
   if (blockIdx.x < hubs.blocks) {
     __shared__ float red[256 / kWave][kWave];
     if (!hubs.list) {
-      // Few enough rows for every hub block to find its own: a row is the block's that its number hashes to.  (There are fewer
-      // than 2,048 of them: each holds more than a 1/2,048 share of the values.)
-      __shared__ uint32_t found, rows_here[2048];
-      if (threadIdx.x == 0) found = 0;
-      __syncthreads();
+      // Few enough rows for the hub blocks to find their own, a row a thread, dealt out in an order without pattern as in the edge
+      // sums (sum_long_rows_in_this_block).
+      __shared__ uint32_t n_found;
+      __shared__ uint16_t found[256];
+      if (threadIdx.x == 0) n_found = 0;
+      const uint32_t at = threadIdx.x * hubs.blocks + blockIdx.x, r = at * 40503u % kLongMinVertices;  // (odd: every row once)
+      uint32_t deg = 0;
+      if (at < kLongMinVertices && r < Vd) deg = co[r + 1] - co[r];
       const uint64_t limit = few_long_values(static_cast<uint64_t>(co[Vd] - co[0]) * H);
-      each_row_by_block<256>(co, Vd, [&](uint32_t r, uint32_t deg) {
-        if (static_cast<uint64_t>(deg) * H > limit && (r * 2654435761u >> 16) % hubs.blocks == blockIdx.x)
-          if (const uint32_t at = atomicAdd(&found, 1u); at < 2048) rows_here[at] = r;
-      });
       __syncthreads();
-      const uint32_t n = found < 2048 ? found : 2048;
-      for (uint32_t i = 0; i < n; ++i) few_hub_row<FUSED, BWD, VEC4>(out, ger, x_or_gy, y, el, er, co, ri, rows_here[i], H, slope, red);
+      if (static_cast<uint64_t>(deg) * H > limit) found[atomicAdd(&n_found, 1u)] = static_cast<uint16_t>(r);
+      __syncthreads();
+      const uint32_t n = n_found;
+      for (uint32_t i = 0; i < n; ++i) few_hub_row<FUSED, BWD, VEC4>(out, ger, x_or_gy, y, el, er, co, ri, found[i], H, slope, red);
       return;
     }
     const uint32_t n_rows = *hubs.count, n_pieces = hubs.hdr[1];
@@ -2590,6 +2659,11 @@ uint32_t merged_long_blocks() {
   return value;
 }
 
+// The same for calls of fewer than kLongMinVertices rows, which find them themselves; not where rows are so few that each has a
+// block's worth of wavefronts beside it anyway.
+constexpr uint32_t kOwnHubBlocks = 512;
+constexpr uint32_t kMinHubRows = 64;
+
 // The row launch whose first blocks also sum the long rows: one-group rows of a vertex set large enough.
 bool rows_launch_takes_long_rows(uint32_t rows, uint32_t Fv) { return Fv <= 64 && rows >= 4096; }
 
@@ -2606,11 +2680,12 @@ bool stream_contiguous_rows() {
 // the 8,192 wavefronts that the chip holds: whatever the width, 64 rows cost a small vertex set its parallelism and 16
 // cost a large one a wavefront's start-up per four rows' worth of work.  us, 64 / 16 rows a wavefront: 50 K rows, 5 M
 // edges F = 4 191 / 95, F = 128 833 / 599; 169 K, 2.48 M F = 4 88 / 80, F = 32 117 / 108, F = 128 348 / 307; 1 M, 2.5 M F = 4
-// 135 / 168, F = 32 166 / 211, F = 64 224 / 259, F = 128 436 / 439; 2.4 M, 60 M within 3 %.
+// 135 / 168, F = 32 166 / 211, F = 64 224 / 259, F = 128 436 / 439; 2.4 M, 60 M within 3 %.  16 / 8: 30 K, 3 M F = 4 68 / 59, F = 47 264 /
+// 214, 16 K, 1 M F = 4 34 / 24, F = 128 149 / 131; 50 K, 500 K F = 4 45 / 45, F = 128 110 / 112, with four 117.
 uint32_t streamed_rows_per_wave(uint32_t rows) {
   constexpr uint32_t kChipWaves = 8192;
   uint32_t per = kWave;
-  while (per > 16 && rows / per < kChipWaves) per /= 2;
+  while (per > 8 && rows / per < kChipWaves) per /= 2;
   return per;
 }
 
@@ -2672,9 +2747,9 @@ void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_
 #undef NTS_BALANCED
     return;
   }
-#define NTS_GATHER(GG)                                                                                          \
-  hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG>), dim3(ceil_div(static_cast<uint64_t>(rows) * GG, 256)),  \
-                     dim3(256), 0, stream, out, msg, off, perm, rows, Fv, accumulate, limit)
+#define NTS_GATHER(GG)                                                                                             \
+  hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG>), dim3(ceil_div(static_cast<uint64_t>(rows) * GG, 256) + lw.blocks), \
+                     dim3(256), 0, stream, out, msg, off, perm, rows, Fv, accumulate, limit, lw)
   switch (lanes_for(Fv)) {
     case 1: NTS_GATHER(1); break;
     case 2: NTS_GATHER(2); break;
@@ -2712,8 +2787,12 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   // blocks into stream-ordered scratch, then the ordered combine.
   const bool merged = lr.list && rows_launch_takes_long_rows(rows, Fv) && merged_long_blocks() > 0;
   const uint32_t block_threads = merged ? 256u : static_cast<uint32_t>(kLongBlock);
+  // Few rows: the first blocks find the hub rows themselves and take columns of 128 bytes of one each.
+  const uint32_t hub_lanes = v4 ? 8u : 32u;
+  const uint32_t own_hubs = lr.list || rows < kMinHubRows ? 0u : Fv <= hub_lanes ? kOwnHubBlocks / 2 : kOwnHubBlocks;
+  const uint32_t most_lanes = own_hubs ? hub_lanes : block_threads;
   uint32_t tile = 1;
-  while (tile < Fv && tile < block_threads) tile <<= 1;
+  while (tile < Fv && tile < most_lanes) tile <<= 1;
   ScratchBlock partial_block;
   float *partial = nullptr;
   if (lr.list) {
@@ -2722,11 +2801,11 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   }
   if (v4) {
     LongRowWork<float4> lw{lr.list, lr.count, lr.hdr, lr.pieces, reinterpret_cast<float4 *>(partial), tile,
-                           merged ? merged_long_blocks() : 0u};
+                           merged ? merged_long_blocks() : own_hubs};
     launch_gather_rows(reinterpret_cast<float4 *>(out), reinterpret_cast<const float4 *>(msg), off, perm, rows, Fv,
                        accumulate, limit, lw, stream);
   } else {
-    LongRowWork<float> lw{lr.list, lr.count, lr.hdr, lr.pieces, partial, tile, merged ? merged_long_blocks() : 0u};
+    LongRowWork<float> lw{lr.list, lr.count, lr.hdr, lr.pieces, partial, tile, merged ? merged_long_blocks() : own_hubs};
     launch_gather_rows(out, msg, off, perm, rows, Fv, accumulate, limit, lw, stream);
   }
   hipError_t launch_err = hipGetLastError();
@@ -2844,6 +2923,7 @@ uint32_t softmax_rows_per_wave(uint32_t Vd) {
 }
 
 constexpr uint32_t kFewHubBlocks = 128;  // that look for their hub rows themselves
+static_assert(kLongMinVertices <= 256 * kFewHubBlocks, "a row a thread");
 // Destinations that a wavefront takes together in a call of few rows (kDenseSet where these are long): 64 / 16 / 4 fused forward
 // 169 K rows, 2.48 M edges H = 1 74 / 66 / 76, 30 K, 1 M 64 / 39 / 35, 200 K, 20 M 235 / 192 / 179.
 uint32_t few_rows_per_wave(uint32_t Vd) {

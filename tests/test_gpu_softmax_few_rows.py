@@ -56,7 +56,8 @@ def test_softmax_on_few_rows(device, V, total, H, shift):
     bound = (n / 64 + 64) * 2.0 ** -24 + 4e-6
 
     def per_row(v):
-        return torch.zeros(V, H, dtype=torch.float64, device=device).index_add_(0, own, v)
+        total = torch.cat([v.new_zeros(1, H), v.cumsum(0)])
+        return total[off[1:]] - total[off[:-1]]
 
     def near(got, want, size):
         assert ((got.double() - want).abs() <= bound * size).all()
@@ -64,9 +65,7 @@ def test_softmax_on_few_rows(device, V, total, H, shift):
     pre = el[ri] + er[own]
     for fused in (True, False):
         wide = (torch.where(pre > 0, pre, pre * slope) if fused else x).double()
-        top = torch.full((V, H), -torch.inf, dtype=torch.float64, device=device)
-        top.scatter_reduce_(0, own[:, None].expand(E, H), wide, "amax")
-        ex = (wide - top[own]).exp()
+        ex = wide.exp()  # (no score is large enough to need its segment's maximum in 64 bits)
         want = ex / per_row(ex)[own]
         y, gx, ger = array(E, float("nan")), array(E, float("nan")), array(V, float("nan"))
         ri32 = ri.to(torch.int32)
