@@ -361,66 +361,63 @@ __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out,
   }
 }
 
-// out[r,:] (+)= sum_{k in [off[r], off[r+1])} msg[perm ? perm[k] : k, :], added in k order.
-template <typename V, int G>
-__global__ __launch_bounds__(256, (sizeof(V) == 4 ? 8 : 1)) void gather_edge_to_row_kernel(V *__restrict__ out, const V *__restrict__ msg,
+// out[r,:] (+)= sum_{k in [off[r], off[r+1])} msg[perm ? perm[k] : k, :], added in k order: a group of G lanes for every row and
+// every G vectors of it.  The edge rows of a round are requested together and their ids a round ahead, so that a long row is a
+// memory latency per U edges; the last, partial rounds are of eight, whose requests beyond the row are its last edge's again.
+template <typename V, int G, int U>
+__global__ __launch_bounds__(256, (U > 8 ? 4 : 8)) void gather_edge_to_row_kernel(V *__restrict__ out, const V *__restrict__ msg,
                                                                  const uint32_t *__restrict__ off,
                                                                  const uint32_t *__restrict__ perm, uint32_t rows,
-                                                                 uint32_t Fv, int accumulate, uint32_t long_limit, LongRowWork<V> lw) {
+                                                                 uint32_t Fv, int accumulate, uint32_t long_limit, uint32_t tiles,
+                                                                 LongRowWork<V> lw) {
   if (blockIdx.x < lw.blocks) {
     __shared__ V scratch[kHubBytes<V> / sizeof(V)];
-    sum_long_rows_in_this_block<V, sizeof(V) == 16 ? 4 : 8>(out, msg, off, perm, rows, Fv, accumulate, lw, scratch);
+    sum_long_rows_in_this_block<V, sizeof(V) == 16 ? 4 : (U > 8 ? 16 : 8)>(out, msg, off, perm, rows, Fv, accumulate, lw, scratch);
     return;
   }
   long_limit = long_limit_of(lw, long_limit, off, rows);
-  const uint32_t r = ((blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / G;
-  if (r >= rows) return;
-  const uint32_t gl = threadIdx.x & (G - 1);
+  const uint64_t group = (static_cast<uint64_t>(blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / G;
+  if (group >= static_cast<uint64_t>(rows) * tiles) return;
+  const uint32_t r = static_cast<uint32_t>(group / tiles), c = static_cast<uint32_t>(group % tiles) * G + (threadIdx.x & (G - 1));
+  if (c >= Fv) return;
   const uint32_t e0 = off[r], e1 = off[r + 1];
   if (e1 - e0 > long_limit) return;
-  constexpr int NF = sizeof(V) / 4;
-  for (uint32_t c = gl; c < Fv; c += G) {
-    float a[NF];
+  V a = vnull<V>();
+  uint32_t k = e0, left = e1 - e0;
+  if (left >= U) {
+    uint32_t id[U];
+    auto request_ids = [&] {
 #pragma unroll
-    for (int t = 0; t < NF; ++t) a[t] = 0.f;
-    // U edge rows are loaded before they are added, in order: the loads overlap, the order of
-    // the additions stays the edge order.
-    constexpr int U = 16;
-    uint32_t k = e0;
-    for (; static_cast<uint64_t>(k) + U <= e1; k += U) {
+      for (int u = 0; u < U; ++u) id[u] = perm ? perm[k + u] : k + u;
+    };
+    request_ids();
+    do {
       V v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint32_t e = perm ? perm[k + u] : k + u;
-        v[u] = msg[static_cast<size_t>(e) * Fv + c];
-      }
+      for (int u = 0; u < U; ++u) v[u] = msg[static_cast<size_t>(id[u]) * Fv + c];
+      k += U;
+      left -= U;
+      if (left >= U) request_ids();
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float *vf = reinterpret_cast<const float *>(&v[u]);
-#pragma unroll
-        for (int t = 0; t < NF; ++t) a[t] += vf[t];
-      }
-    }
-    for (; k < e1; ++k) {
-      const uint32_t e = perm ? perm[k] : k;
-      const V v = msg[static_cast<size_t>(e) * Fv + c];
-      const float *vf = reinterpret_cast<const float *>(&v);
-#pragma unroll
-      for (int t = 0; t < NF; ++t) a[t] += vf[t];
-    }
-    V *p = out + static_cast<size_t>(r) * Fv + c;
-    if (accumulate) {
-      const V o = *p;
-      const float *of = reinterpret_cast<const float *>(&o);
-#pragma unroll
-      for (int t = 0; t < NF; ++t) a[t] += of[t];
-    }
-    V res;
-    float *rf = reinterpret_cast<float *>(&res);
-#pragma unroll
-    for (int t = 0; t < NF; ++t) rf[t] = a[t];
-    *p = res;
+      for (int u = 0; u < U; ++u) vadd(a, v[u]);
+    } while (left >= U);
   }
+  while (left) {
+    V v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const uint32_t kk = k + (u < left ? u : left - 1);
+      v[u] = msg[static_cast<size_t>(perm ? perm[kk] : kk) * Fv + c];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (u < left) vadd(a, v[u]);
+    k += 8;
+    left = left > 8 ? left - 8 : 0u;
+  }
+  V *p = out + static_cast<size_t>(r) * Fv + c;
+  if (accumulate) vadd(a, *p);
+  *p = a;
 }
 
 // Smallest row r in [0, rows] whose weight before it, (off[r] - off0) + r, is at least x (x at most the
@@ -2662,10 +2659,34 @@ uint32_t merged_long_blocks() {
 // The same for calls of fewer than kLongMinVertices rows, which find them themselves; not where rows are so few that each has a
 // block's worth of wavefronts beside it anyway.
 constexpr uint32_t kOwnHubBlocks = 512;
-constexpr uint32_t kMinHubRows = 64;
 
-// The row launch whose first blocks also sum the long rows: one-group rows of a vertex set large enough.
-bool rows_launch_takes_long_rows(uint32_t rows, uint32_t Fv) { return Fv <= 64 && rows >= 4096; }
+// Whether a group of lanes takes a row of its own and of 64 vectors at most (gather_edge_to_row_kernel), and not wavefronts sets of
+// rows.  us, sets / a row each, contiguous and permuted sums of edge rows:
+//                   contiguous: F = 47, 128    permuted: F = 47, 64, 100, 128, 200
+//   6 K, 12 K         30 / 13, 26 / 15           62 / 13, 64 / 13, 68 / 15, 68 / 16
+//   16 K, 100 K       61 / 33, 55 / 46           231 / 39, 241 / 39, 250 / 55, 244 / 55
+//   16 K, 1 M         202 / 105, 191 / 159       504 / 154, 172 / 166, 304 / 170, 318 / 214
+//   30 K, 3 M         213 / 175, 361 / 348       534 / 221, 298 / 240, 447 / 335, 463 / 366
+//   169 K, 2.48 M     186 / 188, 310 / 319       381 / 229, 258 / 226, 374 / 309, 388 / 343, 639 / 523
+//   400 K, 2 M        187 / 223, 301 / 298       337 / 263, 294 / 214, 391 / 285, 409 / 312
+//   1 M, 8 M          508 / 639, 1,021 / 1,004   943 / 786, 689 / 645, 1,109 / 961, 1,133 / 1,061
+//   1.5 M, 6 M                                   763 / 791, 545 / 568, 888 / 809, 889 / 876
+//   2.4 M, 5 M                                   807 / 978, 508 / 629, 840 / 946, 861 / 976, 1,437 / 1,519
+// so a row each for the permuted sums up to a million rows, for the contiguous ones below 16,384.  Rows of up to eight vectors leave
+// a lane or two a whole row there: 2.9 K, 110 K F = 4 34 / 46 with a row each, sets 15 / 18; but eight permuted vectors 30 K, 3 M 224
+// sets, 164, 169 K 191, 170 (400 K 161, 171; 16 K, 100 K 38, 49).
+constexpr uint32_t kMinHubRows = 64;  // (fewer rows have a block's worth of wavefronts beside each anyway: no hub blocks)
+bool group_takes_a_row(uint32_t rows, uint32_t Fv, bool vectors, bool permuted) {
+  if (rows < kMinHubRows || Fv > kWave) return true;
+  if (Fv <= 8) return permuted && vectors && Fv > 4 && rows >= kLongMinVertices && rows <= 1u << 18;
+  return rows < (permuted ? 1u << 20 : kLongMinVertices);
+}
+// Rows that are few leave the chip idle, and floats spread them over four times as many lanes, each with 32 loads in flight where
+// vectors have room for eight: 2.9 K, 110 K F = 128 42 / 54 -> 35 / 41 us, 16 K, 1 M 193 / 319 -> 159 / 214; from five wavefronts a row on only
+// the fewest rows: F = 300 2.9 K 77 / 87 -> 55 / 65, but 4 K, 2 M 1,320 / 1,755 -> 1,355 / 1,862.
+bool floats_for_few_rows(uint32_t rows, uint32_t F) {
+  return F > 32 && rows < kLongMinVertices && (F <= 256 || static_cast<uint64_t>(rows) * ceil_div(F, kWave) <= 16384);
+}
 
 // NTS_EDGE_SUM_STREAM=0 in the environment: contiguous edge rows take the lane-group kernel like permuted ones.
 bool stream_contiguous_rows() {
@@ -2703,7 +2724,8 @@ uint32_t balanced_rows_per_wave(uint32_t rows, uint32_t set) {
 template <typename V>
 void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_t *perm, uint32_t rows, uint32_t Fv,
                         int accumulate, uint32_t limit, const LongRowWork<V> &lw, hipStream_t stream) {
-  if (rows_launch_takes_long_rows(rows, Fv) && !perm && stream_contiguous_rows()) {
+  const bool row_each = group_takes_a_row(rows, Fv, sizeof(V) == 16, perm != nullptr);
+  if (!row_each && !perm && stream_contiguous_rows()) {
     const uint32_t blocks = ceil_div(rows, 4 * streamed_rows_per_wave(rows));
     const dim3 grid((blocks < 16384u ? blocks : 16384u) + lw.blocks);
 #define NTS_STREAM(GG)                                                                                          \
@@ -2721,7 +2743,7 @@ void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_
 #undef NTS_STREAM
     return;
   }
-  if (rows_launch_takes_long_rows(rows, Fv)) {
+  if (!row_each) {
     // One group covers a row: wavefronts hand their 64 rows out dynamically (strided launch).
 #define NTS_BALANCED(GG, SS)                                                                                    \
   do {                                                                                                          \
@@ -2747,9 +2769,17 @@ void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_
 #undef NTS_BALANCED
     return;
   }
-#define NTS_GATHER(GG)                                                                                             \
-  hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG>), dim3(ceil_div(static_cast<uint64_t>(rows) * GG, 256) + lw.blocks), \
-                     dim3(256), 0, stream, out, msg, off, perm, rows, Fv, accumulate, limit, lw)
+#define NTS_GATHER(GG)                                                                                            \
+  do {                                                                                                            \
+    const uint32_t tiles = ceil_div(Fv, GG);                                                                      \
+    const uint32_t blocks = ceil_div(static_cast<uint64_t>(rows) * tiles * GG, 256) + lw.blocks;                  \
+    if (sizeof(V) == 4 && rows < kLongMinVertices)                                                                \
+      hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG, sizeof(V) == 16 ? 8 : 32>), dim3(blocks), dim3(256), 0, \
+                         stream, out, msg, off, perm, rows, Fv, accumulate, limit, tiles, lw);                    \
+    else                                                                                                          \
+      hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG, 8>), dim3(blocks), dim3(256), 0, stream, out, msg, off, \
+                         perm, rows, Fv, accumulate, limit, tiles, lw);                                           \
+  } while (0)
   switch (lanes_for(Fv)) {
     case 1: NTS_GATHER(1); break;
     case 2: NTS_GATHER(2); break;
@@ -2780,15 +2810,16 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
     return rc;
   const uint32_t limit = lr.list ? kLongRowEdges : kNoLimit;
   // 16-byte vectors for the row kernels and the block kernels alike
-  const bool v4 = F % 4 == 0 && aligned_to(out, 16) && aligned_to(msg, 16);
+  bool v4 = F % 4 == 0 && aligned_to(out, 16) && aligned_to(msg, 16);
+  if (v4 && floats_for_few_rows(rows, F)) v4 = false;
   const uint32_t Fv = v4 ? F / 4 : F;
   // Long rows: in the first blocks of the row launch where that launch has them (256-thread blocks),
   // else in launches of their own after it (1,024-thread blocks).  Giant rows: pieces by separate
   // blocks into stream-ordered scratch, then the ordered combine.
-  const bool merged = lr.list && rows_launch_takes_long_rows(rows, Fv) && merged_long_blocks() > 0;
+  const bool merged = lr.list && merged_long_blocks() > 0;
   const uint32_t block_threads = merged ? 256u : static_cast<uint32_t>(kLongBlock);
   // Few rows: the first blocks find the hub rows themselves and take columns of 128 bytes of one each.
-  const uint32_t hub_lanes = v4 ? 8u : 32u;
+  const uint32_t hub_lanes = v4 ? 8u : F > 32 ? 16u : 32u;
   const uint32_t own_hubs = lr.list || rows < kMinHubRows ? 0u : Fv <= hub_lanes ? kOwnHubBlocks / 2 : kOwnHubBlocks;
   const uint32_t most_lanes = own_hubs ? hub_lanes : block_threads;
   uint32_t tile = 1;

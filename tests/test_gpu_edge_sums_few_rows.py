@@ -1,4 +1,4 @@
-"""Sums of edge rows over few vertex rows (fewer than 16,384), whose hub rows the launch's first blocks find and add up a
+"""Sums of edge rows over few vertex rows, whose hub rows the launch's first blocks find and add up a
 column tile at a time: rows of at most 1,024 edges are the running sum in edge order, bit for bit; longer ones are added by at
 most n / 2 chains in a fixed tree, off by at most n 2^-24 of the sum of the magnitudes."""
 import pytest
@@ -22,9 +22,10 @@ def running_sums(msg, off, rows):
     return out
 
 
-# rows on both sides of 64 (below it no row is a hub), 4,096 (another kernel from there on) and 16,384
-@pytest.mark.parametrize("rows", [1, 63, 64, 4095, 4096, 16383, 16384])
-@pytest.mark.parametrize("F", [1, 4, 32, 47, 128, 260])
+# rows on both sides of 64 (below it no block looks for hub rows) and of 16,384 (from there on a launch lists them); widths of a
+# lane to eight, one of four to eight vectors, 33 floats and more in a wavefront of floats, and several wavefronts of them
+@pytest.mark.parametrize("rows", [1, 63, 64, 4095, 16383, 16384])
+@pytest.mark.parametrize("F", [1, 4, 17, 32, 33, 128, 260])
 @pytest.mark.parametrize("dense", [False, True])
 def test_sums_over_few_rows(device, rows, F, dense):
     print(f"case rows={rows} F={F} dense={dense}", flush=True)
@@ -41,7 +42,7 @@ def test_sums_over_few_rows(device, rows, F, dense):
 
     msg = torch.randn(E, F, generator=g, device=device)
     perm = torch.randperm(E, generator=g, device=device)
-    co, s = off.to(torch.int32), torch.cuda.current_stream().cuda_stream
+    co, ids, s = off.to(torch.int32), perm.to(torch.int32), torch.cuda.current_stream().cuda_stream
     init = torch.randn(rows, F, generator=g, device=device)
     for order in (None, perm):
         terms = msg if order is None else msg[order]
@@ -54,10 +55,29 @@ def test_sums_over_few_rows(device, rows, F, dense):
             if order is None:
                 call("nts_gather_edge_to_dst", ptr(out), ptr(msg), ptr(co), rows, F, accumulate, s)
             else:
-                call("nts_gather_edge_to_src", ptr(out), ptr(msg), ptr(co), ptr(order.to(torch.int32)), rows, F, accumulate, s)
+                call("nts_gather_edge_to_src", ptr(out), ptr(msg), ptr(co), ptr(ids), rows, F, accumulate, s)
             if want is not None:
                 assert torch.equal(out[chains], want + init[chains] if accumulate else want)
             assert torch.equal(out[deg == 0], init[deg == 0] if accumulate else torch.zeros_like(out[deg == 0]))
             full = exact + init.double() if accumulate else exact
             bound = (deg.double()[:, None] + 1) * 2.0 ** -24 * (size + init.double().abs() * accumulate) + 1e-8  # (64-bit prefix sums)
             assert ((out.double() - full).abs() <= bound).all()
+
+
+# a row each up to 2^18 rows of eight vectors and 2^20 wider ones, sets of rows beyond
+@pytest.mark.parametrize("rows,F", [(1 << 18, 32), ((1 << 18) + 1, 32), ((1 << 20) - 1, 33), (1 << 20, 33), ((1 << 20) - 1, 40), (1 << 20, 40)])
+def test_permuted_sums_of_many_rows(device, rows, F):
+    g = torch.Generator(device=device).manual_seed(F)
+    deg = torch.randint(0, 3, (rows,), generator=g, device=device)
+    deg[:4] = torch.tensor([1025, 1024, 40000, 9], device=device)
+    off = torch.cat([deg.new_zeros(1), deg.cumsum(0)])
+    msg = torch.randn(int(off[-1]), F, generator=g, device=device)
+    perm = torch.randperm(msg.shape[0], generator=g, device=device)
+    out = torch.full((rows, F), float("nan"), device=device)
+    ro, ids = off.to(torch.int32), perm.to(torch.int32)  # named: the first temporary's memory would be the second's
+    call("nts_gather_edge_to_src", ptr(out), ptr(msg), ptr(ro), ptr(ids), rows, F, 0, torch.cuda.current_stream().cuda_stream)
+    terms = msg[perm]
+    total = torch.cat([terms.new_zeros(1, F, dtype=torch.float64), terms.double().cumsum(0)])
+    size = torch.cat([terms.new_zeros(1, F, dtype=torch.float64), terms.double().abs().cumsum(0)])
+    want, scale = total[off[1:]] - total[off[:-1]], size[off[1:]] - size[off[:-1]]
+    assert ((out.double() - want).abs() <= (deg.double()[:, None] + 1) * 2.0 ** -24 * scale + 1e-8).all()
