@@ -786,10 +786,46 @@ __global__ __launch_bounds__(256, (grad_waves<G, LH, NJ, VEC>())) void attention
   }
 }
 
+// a[j] = the columns c[j] of n >= 1 consecutive partial rows of stride ld, added one after the other from the first on.  Up to U of
+// them are requested together (a row's sum is a memory latency per round, and the launch lasts as long as its longest row; U = 8 before:
+// 8 K rows, 2 M edges F = 47 19 -> 8 us, F = 300 26 -> 18, 169 K, 2.48 M F = 128 5.2 -> 3.7, 233 K, 50 M with source ranges F = 128 104 ->
+// 74; F = 602, 359 us, is bound by the 1.1 GB that it reads), the last ones eight at a time, whose requests
+// beyond the end are the last row's again.
+template <int J, int U>
+__device__ __forceinline__ void add_partial_rows(const float *__restrict__ src, size_t ld, uint32_t n, const uint32_t (&c)[J], float (&a)[J]) {
+#pragma unroll
+  for (int j = 0; j < J; ++j) a[j] = src[c[j]];
+  uint32_t k = 1;
+  for (; n - k >= U; k += U) {
+    float v[U][J];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < J; ++j) v[u][j] = src[(k + u) * ld + c[j]];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < J; ++j) a[j] += v[u][j];
+  }
+  for (; k < n; k += 8) {
+    float v[8][J];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int j = 0; j < J; ++j) v[u][j] = src[(k + u < n ? k + u : n - 1) * ld + c[j]];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        if (k + u < n) a[j] += v[u][j];
+  }
+}
+template <int J>
+constexpr int kPartialRows = J == 1 ? 32 : J == 2 ? 16 : 8;
+
 // Second stage for split rows: out[row,:] (+)= partial[first,:] + partial[first+1,:] + ... in slot
 // order.  Block (x, y) owns 256 columns (tile y) of split row x; `splits[i]` = (row, first slot,
-// slot count, unused).  Eight slots are loaded at a time and then added one after the other, so the
-// loads overlap while the order of the additions stays fixed.
+// slot count, unused).
 __global__ __launch_bounds__(256) void spmm_reduce_partials_kernel(float *__restrict__ out,
                                                                    const float *__restrict__ partial,
                                                                    const uint4 *__restrict__ splits, uint32_t F,
@@ -797,20 +833,11 @@ __global__ __launch_bounds__(256) void spmm_reduce_partials_kernel(float *__rest
   const uint4 s = splits[blockIdx.x];
   const uint32_t c = blockIdx.y * blockDim.x + threadIdx.x;
   if (c >= F) return;
-  const float *src = partial + static_cast<size_t>(s.y) * ld + c;
-  float a = src[0];
-  uint32_t k = 1;
-  for (; k + 8 <= s.z; k += 8) {
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = src[static_cast<size_t>(k + u) * ld];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) a += v[u];
-  }
-  for (; k < s.z; ++k) a += src[static_cast<size_t>(k) * ld];
+  const uint32_t col[1] = {c};
+  float a[1];
+  add_partial_rows<1, kPartialRows<1>>(partial + static_cast<size_t>(s.y) * ld, ld, s.z, col, a);
   float *dst = out + static_cast<size_t>(s.x) * F + c;
-  if (accumulate) a += *dst;
-  *dst = a;
+  *dst = accumulate ? a[0] + *dst : a[0];
 }
 
 // The same for rows of up to 1,024 columns: one block per split row covers all columns (thread t
@@ -830,34 +857,8 @@ __global__ __launch_bounds__(256) void spmm_reduce_partials_wide_kernel(float *_
     c[j] = threadIdx.x + 256u * j;
     live[j] = c[j] < F;
     if (!live[j]) c[j] = F - 1;  // re-read the last column, never stored
-    a[j] = src[c[j]];
   }
-  uint32_t k = 1;
-  for (; k + 8 <= s.z; k += 8) {
-    float v[8][J];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int j = 0; j < J; ++j) v[u][j] = src[static_cast<size_t>(k + u) * ld + c[j]];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int j = 0; j < J; ++j) a[j] += v[u][j];
-  }
-  for (; k + 2 <= s.z; k += 2) {
-    float v[2][J];
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int j = 0; j < J; ++j) v[u][j] = src[static_cast<size_t>(k + u) * ld + c[j]];
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int j = 0; j < J; ++j) a[j] += v[u][j];
-  }
-  for (; k < s.z; ++k)
-#pragma unroll
-    for (int j = 0; j < J; ++j) a[j] += src[static_cast<size_t>(k) * ld + c[j]];
+  add_partial_rows<J, kPartialRows<J>>(src, ld, s.z, c, a);
   float *dst = out + static_cast<size_t>(s.x) * F;
 #pragma unroll
   for (int j = 0; j < J; ++j)
@@ -1399,20 +1400,11 @@ __global__ __launch_bounds__(256) void auto_reduce_kernel(float *__restrict__ ou
   if (n == 0) return;
   const uint32_t c = blockIdx.y * blockDim.x + threadIdx.x;
   if (c >= F) return;
-  const float *src = partial + static_cast<size_t>(i) * F + c;
-  float a = src[0];
-  uint32_t k = 1;
-  for (; k + 8 <= n; k += 8) {
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = src[static_cast<size_t>(k + u) * F];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) a += v[u];
-  }
-  for (; k < n; ++k) a += src[static_cast<size_t>(k) * F];
+  const uint32_t col[1] = {c};
+  float a[1];
+  add_partial_rows<1, kPartialRows<1>>(partial + static_cast<size_t>(i) * F, F, n, col, a);
   float *dst = out + static_cast<size_t>(r) * F + c;
-  if (accumulate) a += *dst;
-  *dst = a;
+  *dst = accumulate ? a[0] + *dst : a[0];
 }
 
 // The same with one block per work item covering all columns (rows of up to 1,024 columns): whole,
@@ -1437,23 +1429,8 @@ __global__ __launch_bounds__(256) void auto_reduce_wide_kernel(float *__restrict
     c[j] = threadIdx.x + 256u * j;
     live[j] = c[j] < F;
     if (!live[j]) c[j] = F - 1;  // re-read the last column, never stored
-    a[j] = src[c[j]];
   }
-  uint32_t k = 1;
-  for (; k + 8 <= n; k += 8) {
-    float v[8][J];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int j = 0; j < J; ++j) v[u][j] = src[static_cast<size_t>(k + u) * F + c[j]];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int j = 0; j < J; ++j) a[j] += v[u][j];
-  }
-  for (; k < n; ++k)
-#pragma unroll
-    for (int j = 0; j < J; ++j) a[j] += src[static_cast<size_t>(k) * F + c[j]];
+  add_partial_rows<J, kPartialRows<J>>(src, F, n, c, a);
   float *dst = out + static_cast<size_t>(r) * F;
 #pragma unroll
   for (int j = 0; j < J; ++j)
@@ -1543,20 +1520,11 @@ __global__ __launch_bounds__(256) void auto_reduce_listed_kernel(float *__restri
   const uint4 sp = splits[blockIdx.x];
   const uint32_t c = blockIdx.y * blockDim.x + threadIdx.x;
   if (c >= F || sp.z == 0) return;
-  const float *src = partial + static_cast<size_t>(sp.y) * F + c;
-  float a = src[0];
-  uint32_t k = 1;
-  for (; k + 8 <= sp.z; k += 8) {
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = src[static_cast<size_t>(k + u) * F];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) a += v[u];
-  }
-  for (; k < sp.z; ++k) a += src[static_cast<size_t>(k) * F];
+  const uint32_t col[1] = {c};
+  float a[1];
+  add_partial_rows<1, kPartialRows<1>>(partial + static_cast<size_t>(sp.y) * F, F, sp.z, col, a);
   float *dst = out + static_cast<size_t>(sp.x) * F + c;
-  if (accumulate) a += *dst;
-  *dst = a;
+  *dst = accumulate ? a[0] + *dst : a[0];
 }
 
 int launch_spmm_cut_small(const LaunchArgs &a, uint32_t edges, unsigned char *fixed, size_t fixed_cap) {
