@@ -197,6 +197,7 @@ constexpr uint32_t kLongRowValues = 32768;  // the same for softmax segments, in
 constexpr uint32_t kLongRowMinValues = 2048;   // and at least
 constexpr uint64_t kGiantMinValues = 32768;
 constexpr uint32_t kByTotal = 0;               // in place of a line: long_segment_values of the call's values
+constexpr uint32_t kByFewTotal = 1;            // few_long_values of them
 constexpr uint32_t kLongMinVertices = 16384;  // vertex count below which the extra launches are not worth it
 constexpr int kLongBlock = 1024;
 
@@ -882,7 +883,7 @@ __device__ __forceinline__ uint64_t giant_segment_values(uint64_t total_values) 
 //   250 K, 3 M      78 / 61, 95 / 75  82 / 57, 97 / 76  101 / 83, 157 / 140 92 / 105, 141 / 161
 //   200 K, 20 M     102 / 84, 245 / 239  108 / 91, 328 / 316  319 / 180, 492 / 459  418 / 282, 525 / 561
 //   100 K, 40 M     160 / 148, 459 / 485  204 / 185, 629 / 671  495 / 457, 766 / 802  526 / 521, 838 / 930
-// Above, one block takes too long over the offsets (1 M rows 30 us).  The fused backward holds two arrays and the signs of the scores a
+// Above they were not measured.  The fused backward holds two arrays and the signs of the scores a
 // lane, 114 registers for all of its paths together, and loses from some 32 K rows on.
 constexpr uint32_t kFewRows = 1u << 18;
 constexpr uint32_t kFewRowsFusedBackward = 1u << 15;
@@ -901,7 +902,7 @@ __device__ __forceinline__ uint64_t few_giant_values(uint64_t total_values) {
 //      (`count` points here, so that one fill clears all of them).
 // list[0 .. *count) = rows r with (off[r+1] - off[r]) * width > limit that are not listed as giant
 // (any order); giant_rows[0 .. hdr[0]) = rows above giant_limit values and above the share.  limit
-// kByTotal: a softmax call, whose lines lie where its values put them.
+// kByTotal and kByFewTotal: softmax calls, whose lines lie where their values put them.
 __global__ __launch_bounds__(256) void collect_long_rows_kernel(uint32_t *__restrict__ list,
                                                                 uint32_t *__restrict__ count,
                                                                 uint32_t *__restrict__ giant_rows,
@@ -917,6 +918,10 @@ __global__ __launch_bounds__(256) void collect_long_rows_kernel(uint32_t *__rest
     const uint64_t total = static_cast<uint64_t>(off[rows] - off[0]) * width;
     limit = long_segment_values(total);
     giant_limit = giant_segment_values(total);
+  } else if (limit == kByFewTotal) {
+    const uint64_t total = static_cast<uint64_t>(off[rows] - off[0]) * width;
+    limit = static_cast<uint32_t>(few_long_values(total));
+    giant_limit = few_giant_values(total);
   }
   if (n > giant_limit && deg > (off[rows] - off[0]) / kGiantCap) {
     const uint32_t gi = atomicAdd(&hdr[0], 1u);
@@ -1010,12 +1015,15 @@ __device__ __forceinline__ void each_row_by_block(const uint32_t *__restrict__ o
   }
 }
 
-// The lists, their counters and the piece table in one launch of one block, for a softmax call of few rows (kFewRows): a fill, a
-// launch that lists and one that plans are 14 us and as much of the host's time.
+// The lists, their counters and the piece table in one launch of one block, for up to kOneBlockRows rows: a fill, a launch that lists
+// and one that plans are 14 us and as much of the host's time, this one 5 with 20 K rows, but a block reads the offsets of 169 K, from
+// beyond its L2, in some 25 (attention layer of one head of 47, 2.48 M edges 527 -> 541).  limit: as in collect_long_rows_kernel.
+constexpr uint32_t kOneBlockRows = 1u << 16;
 __global__ __launch_bounds__(kLongBlock) void few_long_rows_kernel(uint32_t *__restrict__ list, uint32_t *__restrict__ count,
                                                                    uint32_t *giant_rows, uint32_t *hdr, uint32_t *first,
                                                                    uint4 *__restrict__ pieces, const uint32_t *__restrict__ off,
-                                                                   uint32_t rows, uint32_t width, uint32_t min_piece) {
+                                                                   uint32_t rows, uint32_t width, uint32_t limit_or_total,
+                                                                   uint64_t most, uint32_t min_piece) {
   __shared__ uint32_t n_long, n_giant;
   __shared__ unsigned long long giant_edges;
   if (threadIdx.x == 0) {
@@ -1024,7 +1032,15 @@ __global__ __launch_bounds__(kLongBlock) void few_long_rows_kernel(uint32_t *__r
   }
   __syncthreads();
   const uint32_t edges = off[rows] - off[0];
-  const uint64_t total = static_cast<uint64_t>(edges) * width, limit = few_long_values(total), giant_limit = few_giant_values(total);
+  const uint64_t total = static_cast<uint64_t>(edges) * width;
+  uint64_t limit = limit_or_total, giant_limit = most;
+  if (limit_or_total == kByTotal) {
+    limit = long_segment_values(total);
+    giant_limit = giant_segment_values(total);
+  } else if (limit_or_total == kByFewTotal) {
+    limit = few_long_values(total);
+    giant_limit = few_giant_values(total);
+  }
   auto look = [&](uint32_t r, uint32_t deg) {
     const uint64_t n = static_cast<uint64_t>(deg) * width;
     if (n <= limit) return;
@@ -2023,8 +2039,9 @@ __global__ __launch_bounds__(kLongBlock) void giant_softmax_bwd_apply_kernel(
 //
 // Calls of at most kFewRows destinations, heads a power of two up to kShortG: what the kernels above do in nine to eleven
 // launches on two streams, whose gaps and idle ends are most of the time there (and, below a million values, the host's
-// launching them all of it), in one, or three to four where there are hub rows:
-//   few_long_rows_kernel   lists the hub rows and cuts the giant ones (from kLongMinVertices rows up)
+// launching them all of it), in one, or three to six where there are hub rows:
+//   few_long_rows_kernel   lists the hub rows and cuts the giant ones (from kLongMinVertices rows up; above kOneBlockRows the three
+//                          launches of many rows)
 //   few_softmax_kernel     its first blocks take the listed rows and the pieces' statistics; every other wavefront a set of
 //                          consecutive rows, short segments four at a time, each of the longer ones by the whole wavefront
 //   few_giant_apply_kernel combines the statistics of a piece's row itself and writes the piece
@@ -2611,6 +2628,12 @@ int take_long_rows(LongRows &lr, uint32_t rows, hipStream_t stream) {
 int collect_long_rows(const LongRows &lr, const uint32_t *off, uint32_t rows, uint32_t width, uint32_t limit,
                       uint64_t giant_limit, uint32_t min_piece, hipStream_t stream) {
   if (!lr.list) return NTS_OK;
+  if (rows <= kOneBlockRows) {
+    hipLaunchKernelGGL(few_long_rows_kernel, dim3(1), dim3(kLongBlock), 0, stream, lr.list, lr.count, lr.giant_rows, lr.hdr, lr.first,
+                       lr.pieces, off, rows, width, limit, giant_limit, min_piece);
+    NTS_LAUNCH_CHECK("few_long_rows_kernel");
+    return NTS_OK;
+  }
   if (int rc = nts_memset_zero(lr.hdr, 8 * sizeof(uint32_t), stream)) return rc;  // counters and the ticket
   hipLaunchKernelGGL(collect_long_rows_kernel, dim3(ceil_div(rows, 256)), dim3(256), 0, stream, lr.list, lr.count,
                      lr.giant_rows, lr.hdr, off, rows, width, limit, giant_limit);
@@ -2977,9 +3000,7 @@ int few_softmax(float *out, float *ger, const float *x_or_gy, const float *y, co
   if (lr.list) {
     NTS_HIP_TRY(stats_block.alloc(static_cast<size_t>(kPieceCap) * 2 * H * sizeof(float), stream));
     hubs = FewHubs{lr.list, lr.count, lr.hdr, lr.first, lr.pieces, static_cast<float *>(stats_block.ptr), kLongGrid};
-    hipLaunchKernelGGL(few_long_rows_kernel, dim3(1), dim3(kLongBlock), 0, stream, lr.list, lr.count, lr.giant_rows, lr.hdr, lr.first,
-                       lr.pieces, co, Vd, H, kFewPieceValues / H);
-    NTS_LAUNCH_CHECK(who);
+    if (int rc = collect_long_rows(lr, co, Vd, H, kByFewTotal, 0, kFewPieceValues / H, stream)) return rc;
   }
   const uint32_t set = few_rows_per_wave(Vd);
   hipLaunchKernelGGL((few_softmax_kernel<FUSED, BWD, VEC4>), dim3(hubs.blocks + ceil_div(Vd, 4 * (set < kDenseSet ? set : kDenseSet))), dim3(256), 0, stream, out,
