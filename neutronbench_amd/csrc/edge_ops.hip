@@ -883,10 +883,12 @@ __device__ __forceinline__ uint64_t giant_segment_values(uint64_t total_values) 
 //   250 K, 3 M      78 / 61, 95 / 75  82 / 57, 97 / 76  101 / 83, 157 / 140 92 / 105, 141 / 161
 //   200 K, 20 M     102 / 84, 245 / 239  108 / 91, 328 / 316  319 / 180, 492 / 459  418 / 282, 525 / 561
 //   100 K, 40 M     160 / 148, 459 / 485  204 / 185, 629 / 671  495 / 457, 766 / 802  526 / 521, 838 / 930
-// Above they were not measured.  The fused backward holds two arrays and the signs of the scores a
-// lane, 114 registers for all of its paths together, and loses from some 32 K rows on.
+// (the fused backward's above 32 K rows with the rows listed by one block, which now takes three launches; whole attention layers, both
+// directions, with the backward of many rows / of few: 169 K, 2.48 M one head 513 / 516, 200 K, 20 M two 2,798 / 2,581, 60 K, 4 M four 807 /
+// 803, 250 K, 3 M four 755 / 754; but eight heads 60 K, 10 M 2,306 / 2,408, 50 K, 600 K 344 / 317: that kernel holds two arrays and the
+// signs of the scores a lane, 114 registers for all of its paths together).  More rows were not measured.
 constexpr uint32_t kFewRows = 1u << 18;
-constexpr uint32_t kFewRowsFusedBackward = 1u << 15;
+constexpr uint32_t kFewRowsManyHeads = 1u << 15;
 constexpr uint32_t kFewPieceValues = 4096;
 __device__ __forceinline__ uint64_t few_long_values(uint64_t total_values) {
   const uint64_t v = total_values / 2048;
@@ -3029,7 +3031,7 @@ int softmax_impl(bool backward, bool fused, float *out, float *ger, const float 
   // stated is still computed, by one wavefront.
   const bool no_hubs = max_degree != 0 && static_cast<uint64_t>(max_degree) * H <= kLongRowValues;
   const bool one_short_launch = fused && max_degree != 0 && static_cast<uint64_t>(max_degree) * H <= kShortValues;
-  if (pow2 && H <= static_cast<uint32_t>(kShortG) && Vd <= (fused && backward ? kFewRowsFusedBackward : kFewRows) && !one_short_launch) {
+  if (pow2 && H <= static_cast<uint32_t>(kShortG) && Vd <= (fused && backward && H > 4 ? kFewRowsManyHeads : kFewRows) && !one_short_launch) {
     const bool vec4 = fused && H % 4 == 0 && aligned_to(out, 16) && aligned_to(x_or_gy, 16) && aligned_to(y, 16) && aligned_to(el, 16) &&
                       aligned_to(er, 16) && aligned_to(ger, 16);
     auto call = [&](auto f) { return f(out, ger, x_or_gy, y, el, er, co, ri, Vd, H, slope, !no_hubs, stream, who); };

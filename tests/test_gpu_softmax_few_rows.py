@@ -1,7 +1,7 @@
-"""The softmax operators on few rows, which take one to four launches: segments on both sides of the lines between the groups of
+"""The softmax operators on few rows, which take one to six launches: segments on both sides of the lines between the groups of
 16 lanes, the wavefronts, the blocks and the pieces (1/2,048 and 1/256 of the call's values, within 1,024 .. 32,768 and 8,192 ..
-131,072), rows on both sides of where hub rows are listed by a launch (16,384) and of where other kernels take over (32,768
-for the fused backward, 262,144), long and short rows on average, arrays on and off 16-byte boundaries.
+131,072), rows on both sides of where hub rows are listed by a launch (16,384; by one block up to 65,536) and of where other kernels
+take over (32,768 for the fused backward of more than four heads, 262,144), long and short rows on average, arrays on and off 16-byte boundaries.
 
 A segment of n values is summed by chains of at most n / 64 additions whose results are added in trees: off by at most
 (n / 64 + 64) 2^-24 of the sum of its terms' magnitudes.  An exponential is off by |x| 2^-24 of itself (|x| < 32 here:
@@ -34,7 +34,8 @@ def degrees(total, H, V):
 @pytest.mark.parametrize("V,total,H,shift", [(1, 20000, 1, 0), (3, 20000, 4, 0), (100, 1 << 17, 16, 0), (2047, 1 << 18, 2, 0),
                                              (2500, 1 << 21, 4, 0), (2500, 1 << 21, 4, 1), (2500, 1 << 20, 8, 0), (16383, 1 << 20, 1, 0),
                                              (16384, 1 << 20, 1, 0), (16385, 1 << 22, 4, 0), (16385, 1 << 22, 4, 1), (20001, 1 << 23, 8, 0),
-                                             (20001, 1 << 22, 16, 0), (32768, 1 << 20, 4, 0), (32769, 1 << 20, 4, 0),
+                                             (20001, 1 << 22, 16, 0), (32768, 1 << 20, 8, 0), (32769, 1 << 20, 8, 0), (65536, 1 << 21, 2, 0),
+                                             (65537, 1 << 21, 2, 0), (65537, 1 << 22, 4, 0),
                                              (262144, 1 << 21, 1, 0), (262145, 1 << 21, 1, 0), (262143, 1 << 22, 4, 0)])
 def test_softmax_on_few_rows(device, V, total, H, shift):
     print(f"case V={V} total={total} H={H} shift={shift}", flush=True)
