@@ -294,18 +294,81 @@ __device__ __forceinline__ void block_sum_edge_rows(V *__restrict__ dst, const V
   }
 }
 
+// The same columns (tile vectors from first_col on, at most 32 floats) as one running sum in edge order: the block stages U vectors a
+// thread in LDS while the next ones are on their way, and the threads that each own a float add them up.  some 12 ns an
+// edge, what the additions take one after the other, where a lane group that loads and adds by itself takes 60 to 125.  `staged` holds 256 U vectors.
+template <typename V, int U>
+__device__ __forceinline__ void block_running_sum(V *__restrict__ dst, const V *__restrict__ msg, const uint32_t *__restrict__ perm,
+                                                  uint32_t e0, uint32_t e1, uint32_t Fv, uint32_t first_col, uint32_t end_col, uint32_t tile,
+                                                  int accumulate, V *staged) {
+  constexpr uint32_t NF = sizeof(V) / 4;
+  const uint32_t slice = threadIdx.x / tile, n_slices = 256 / tile, col = first_col + (threadIdx.x & (tile - 1));
+  const uint32_t read_col = col < end_col ? col : end_col - 1;
+  const uint32_t own = threadIdx.x, floats = tile * NF, live_floats = (end_col - first_col) * NF;
+  uint32_t k = e0, left = e1 - e0, id[U];
+  V v[U];
+  auto request_ids = [&] {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t at = u * n_slices + slice, kk = k + (at < left ? at : left - 1);
+      id[u] = perm ? perm[kk] : kk;
+    }
+  };
+  auto request_rows = [&] {
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = msg[static_cast<size_t>(id[u]) * Fv + read_col];
+  };
+  request_ids();
+  request_rows();
+  float a = 0.f;
+  while (left) {
+    const uint32_t now = left < U * n_slices ? left : U * n_slices;
+    __syncthreads();  // the values before these have been added
+#pragma unroll
+    for (int u = 0; u < U; ++u) staged[u * 256 + threadIdx.x] = v[u];
+    __syncthreads();
+    k += now;
+    left -= now;
+    if (left) {
+      request_ids();
+      request_rows();
+    }
+    if (own < floats) {
+      const float *f = reinterpret_cast<const float *>(staged) + own;
+      uint32_t i = 0;
+      for (; i + 16 <= now; i += 16) {
+        float t[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) t[q] = f[(i + q) * floats];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) a += t[q];
+      }
+      for (; i < now; ++i) a += f[i * floats];
+    }
+  }
+  if (own < live_floats) {
+    float *d = reinterpret_cast<float *>(dst + first_col) + own;
+    *d = accumulate ? a + *d : a;
+  }
+  __syncthreads();
+}
+
 // Calls of fewer than kLongMinVertices rows, whose hub rows no launch lists: the edges of a row above which it is the first
-// blocks' (a row of 1,024 edges and less is one running sum, whoever adds it up), so that there are fewer than kFewLongRows of them.
-// One group or wavefront added a hub row up before, 8 edges a memory latency: contiguous / permuted sums, us, 2 K rows, 100 K edges
-// F = 4 321 / 454 -> 51 / 71, F = 128 1,063 / 1,132 -> 138 / 155; 10 K, 3 M F = 4 960 / 788 -> 52 / 63, F = 47 5,932 / 11,554 -> 645 / 827;
-// 16 K, 1 M F = 128 1,604 / 3,746 -> 190 / 319; without hub rows 16 K, 40 K F = 4 15 / 11 -> 14 / 11, 2.7 K, 13 K F = 128 52 / 53 -> 53 / 52.
+// blocks', so that there are fewer than kFewLongRows of them.  Such rows stay one running sum in edge order, whoever adds them up (a
+// sum in slices is three times as fast on dense graphs but 1.6e-6 of itself from what these calls returned before).  A lane group or a
+// wavefront added a hub row up before, 8 or 16 edges a memory latency: contiguous / permuted sums, us, 2.9 K rows, 110 K edges F = 47 842 / 922
+// -> 57 / 62, F = 128 903 / 945 -> 59 / 64; 10 K, 3 M F = 47 5,932 / 11,554 -> 939 / 1,074, F = 128 4,873 / 11,117 -> 1,225 / 1,364; 16 K, 1 M F = 128
+// 1,604 / 3,746 -> 459 / 510; 16 K, 40 K F = 128 67 / 275 -> 33 / 38.  Rows of up to eight vectors, which a wavefront stages by itself, gain where
+// there are few of them (kMaxNarrowHubRows): 4 K, 2 M F = 4 7,269 / 9,055 -> 1,001 / 1,054, but 16 K, 1 M 313 / 268 -> 329 / 351;
+// through a permutation eight vectors do in any case: F = 32 10 K, 3 M 3,768 -> 1,625, 16 K, 1 M 976 -> 615.
+constexpr uint32_t kMaxNarrowHubRows = 4096;
 constexpr uint32_t kFewLongRows = 2048;
 constexpr uint32_t kMinHubGroups = 64;
 static_assert(kLongMinVertices <= 256 * kMinHubGroups && kLongMinVertices % 2 == 0, "a row a thread");
 template <typename V, int G>
 constexpr int kHubLoads = sizeof(V) == 16 && G > 8 ? 4 : 8;  // vectors that a thread of a hub block requests together
-template <typename V>
-constexpr uint32_t kHubBytes = 256 * (sizeof(V) + sizeof(uint16_t));  // scratch of a block that looks for them
+template <typename V, int OWN>
+constexpr uint32_t kHubBytes = 256 * sizeof(V) * (OWN > 1 ? OWN : 1);  // scratch of a block that looks for them
 __device__ __forceinline__ uint32_t few_long_edges(const uint32_t *__restrict__ off, uint32_t rows) {
   const uint32_t share = (off[rows] - off[0]) / kFewLongRows;
   return share < kLongRowEdges ? kLongRowEdges : share;
@@ -318,18 +381,18 @@ __device__ __forceinline__ uint32_t long_limit_of(const LongRowWork<V> &lw, uint
 // The first blocks of a row launch take the listed long rows, one 256-thread block per row, and the
 // pieces of the giant ones (their partial sums are combined by a launch of its own afterwards); the
 // rows of the launch proper fill the chip meanwhile.
-template <typename V, int U>
+template <typename V, int U, int OWN>
 __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out, const V *__restrict__ msg,
                                                             const uint32_t *__restrict__ off,
                                                             const uint32_t *__restrict__ perm, uint32_t rows, uint32_t Fv,
                                                             int accumulate, const LongRowWork<V> &lw, void *scratch) {
-  V *part = static_cast<V *>(scratch);  // 256 of them
-  if (!lw.list) {
+  V *part = static_cast<V *>(scratch);  // 256 of them, 256 OWN without a list
+  if constexpr (OWN > 0) if (!lw.list) {
     // Few enough rows for these blocks to find the hubs among them: the rows are dealt out to groups of blocks in an order without
     // pattern (hubs of a generated graph have neighbouring numbers), a row a thread, and the blocks of a group take the column
     // tiles of the hub rows among its own.  (A list of all hub rows in every block took it 20 us where the offsets were not in its L2.)
-    uint16_t *found = reinterpret_cast<uint16_t *>(part + 256);  // 256 of them
     __shared__ uint32_t n_found;
+    __shared__ uint16_t found[256];
     if (threadIdx.x == 0) n_found = 0;
     const uint32_t tiles = (Fv + lw.tile - 1) / lw.tile, most = lw.blocks / kMinHubGroups, sharers = tiles < most ? tiles : most;
     const uint32_t groups = lw.blocks / sharers, group = blockIdx.x / sharers;
@@ -345,7 +408,7 @@ __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out,
       const uint32_t row = found[i];
       for (uint32_t t = blockIdx.x % sharers; t < tiles; t += sharers) {
         const uint32_t c0 = t * lw.tile, c1 = c0 + lw.tile < Fv ? c0 + lw.tile : Fv;
-        block_sum_edge_rows<V, 256, U>(out + static_cast<size_t>(row) * Fv, msg, perm, off[row], off[row + 1], Fv, c0, c1, lw.tile, accumulate, part);
+        block_running_sum<V, OWN>(out + static_cast<size_t>(row) * Fv, msg, perm, off[row], off[row + 1], Fv, c0, c1, lw.tile, accumulate, part);
       }
     }
     return;
@@ -372,8 +435,9 @@ __global__ __launch_bounds__(256, (U > 8 ? 4 : 8)) void gather_edge_to_row_kerne
                                                                  uint32_t Fv, int accumulate, uint32_t long_limit, uint32_t tiles,
                                                                  LongRowWork<V> lw) {
   if (blockIdx.x < lw.blocks) {
-    __shared__ V scratch[kHubBytes<V> / sizeof(V)];
-    sum_long_rows_in_this_block<V, sizeof(V) == 16 ? 4 : (U > 8 ? 16 : 8)>(out, msg, off, perm, rows, Fv, accumulate, lw, scratch);
+    constexpr int kOwn = sizeof(V) == 16 ? 4 : U > 8 ? 16 : 0;  // (of floats, only the few rows' kernel has rows without a list)
+    __shared__ V scratch[kHubBytes<V, kOwn> / sizeof(V)];
+    sum_long_rows_in_this_block<V, sizeof(V) == 16 ? 4 : 8, kOwn>(out, msg, off, perm, rows, Fv, accumulate, lw, scratch);
     return;
   }
   long_limit = long_limit_of(lw, long_limit, off, rows);
@@ -458,8 +522,8 @@ __global__ __launch_bounds__(256) void gather_edge_to_row_stream_kernel(V *__res
   constexpr int U = 8;                            // loads per lane and round
   __shared__ __align__(16) float tiles[4][kWave * U * NF];
   if (blockIdx.x < lw.blocks) {
-    static_assert(sizeof(tiles) >= kHubBytes<V>, "the hub blocks' scratch");
-    sum_long_rows_in_this_block<V, kHubLoads<V, G>>(out, msg, off, static_cast<const uint32_t *>(nullptr), rows, Fv, accumulate, lw, tiles);
+    static_assert(sizeof(tiles) >= kHubBytes<V, 8>, "the hub blocks' scratch");
+    sum_long_rows_in_this_block<V, kHubLoads<V, G>, G <= 8 ? 8 : 0>(out, msg, off, static_cast<const uint32_t *>(nullptr), rows, Fv, accumulate, lw, tiles);
     return;
   }
   long_limit = long_limit_of(lw, long_limit, off, rows);
@@ -611,10 +675,11 @@ __global__ __launch_bounds__(256, (sizeof(V) == 4 ? 8 : G <= 8 ? 5 : 1)) void ga
   constexpr bool kCoop = G <= 8;
   constexpr int kCoopU = sizeof(V) == 16 ? 4 : 8;           // loads per lane and round on the cooperative path
   constexpr uint32_t kCoopFloats = kWave * kCoopU * (sizeof(V) / 4);  // floats of a wavefront's tile
-  __shared__ __align__(16) float coop_tile[kCoop ? 4 : 1][kCoop ? kCoopFloats : kHubBytes<V> / 4];
+  __shared__ __align__(16) float coop_tile[kCoop ? 4 : 1][kCoop ? kCoopFloats : kHubBytes<V, 0> / 4];
   if (blockIdx.x < lw.blocks) {
-    static_assert(sizeof(coop_tile) >= kHubBytes<V>, "the hub blocks' scratch");
-    sum_long_rows_in_this_block<V, kHubLoads<V, G>>(out, msg, off, perm, rows, Fv, accumulate, lw, coop_tile);
+    constexpr int kOwn = !kCoop ? 0 : sizeof(V) == 16 ? 4 : 8;  // (wider rows come in millions, with a list)
+    static_assert(sizeof(coop_tile) >= kHubBytes<V, kOwn>, "the hub blocks' scratch");
+    sum_long_rows_in_this_block<V, kHubLoads<V, G>, kOwn>(out, msg, off, perm, rows, Fv, accumulate, lw, coop_tile);
     return;
   }
   long_limit = long_limit_of(lw, long_limit, off, rows);
@@ -2690,7 +2755,7 @@ constexpr uint32_t kOwnHubBlocks = 512;
 //                   contiguous: F = 47, 128    permuted: F = 47, 64, 100, 128, 200
 //   6 K, 12 K         30 / 13, 26 / 15           62 / 13, 64 / 13, 68 / 15, 68 / 16
 //   16 K, 100 K       61 / 33, 55 / 46           231 / 39, 241 / 39, 250 / 55, 244 / 55
-//   16 K, 1 M         202 / 105, 191 / 159       504 / 154, 172 / 166, 304 / 170, 318 / 214
+//   16 K, 1 M         202 / 105, 191 / 159       504 / 154, 172 / 166, 304 / 170, 318 / 214 (hub rows in slices)
 //   30 K, 3 M         213 / 175, 361 / 348       534 / 221, 298 / 240, 447 / 335, 463 / 366
 //   169 K, 2.48 M     186 / 188, 310 / 319       381 / 229, 258 / 226, 374 / 309, 388 / 343, 639 / 523
 //   400 K, 2 M        187 / 223, 301 / 298       337 / 263, 294 / 214, 391 / 285, 409 / 312
@@ -2707,7 +2772,7 @@ bool group_takes_a_row(uint32_t rows, uint32_t Fv, bool vectors, bool permuted) 
   return rows < (permuted ? 1u << 20 : kLongMinVertices);
 }
 // Rows that are few leave the chip idle, and floats spread them over four times as many lanes, each with 32 loads in flight where
-// vectors have room for eight: 2.9 K, 110 K F = 128 42 / 54 -> 35 / 41 us, 16 K, 1 M 193 / 319 -> 159 / 214; from five wavefronts a row on only
+// vectors have room for eight (figures with hub rows in slices): 2.9 K, 110 K F = 128 42 / 54 -> 35 / 41 us, 16 K, 1 M 193 / 319 -> 159 / 214; from five wavefronts a row on only
 // the fewest rows: F = 300 2.9 K 77 / 87 -> 55 / 65, but 4 K, 2 M 1,320 / 1,755 -> 1,355 / 1,862.
 bool floats_for_few_rows(uint32_t rows, uint32_t F) {
   return F > 32 && rows < kLongMinVertices && (F <= 256 || static_cast<uint64_t>(rows) * ceil_div(F, kWave) <= 16384);
@@ -2845,7 +2910,8 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   const uint32_t block_threads = merged ? 256u : static_cast<uint32_t>(kLongBlock);
   // Few rows: the first blocks find the hub rows themselves and take columns of 128 bytes of one each.
   const uint32_t hub_lanes = v4 ? 8u : F > 32 ? 16u : 32u;
-  const uint32_t own_hubs = lr.list || rows < kMinHubRows ? 0u : Fv <= hub_lanes ? kOwnHubBlocks / 2 : kOwnHubBlocks;
+  const bool own = !lr.list && rows >= kMinHubRows && (Fv > 8 || (perm && Fv > 4 && v4) || rows < kMaxNarrowHubRows);
+  const uint32_t own_hubs = !own ? 0u : Fv <= hub_lanes ? kOwnHubBlocks / 2 : kOwnHubBlocks;
   const uint32_t most_lanes = own_hubs ? hub_lanes : block_threads;
   uint32_t tile = 1;
   while (tile < Fv && tile < most_lanes) tile <<= 1;
