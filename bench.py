@@ -250,7 +250,7 @@ def main():
     ms_per_step = elapsed * 1e3 / args.steps
     edges_per_s = 4.0 * E / (elapsed / args.steps)
 
-    # Dominant kernel: the F=602 gather (spmm_wave_kernel), launched twice per step: forward over the
+    # Dominant kernel: the F=602 gather, launched twice per step: forward over the
     # CSC and backward over the CSR.  Same algorithmic bytes per launch for both.
     kernel_ms = (per_pass[0] + per_pass[3]) / 2
     algo = algorithmic_bytes(E, V, F_IN)
@@ -267,7 +267,8 @@ def main():
         # `achieved` / `frac` are that traffic over this run's kernel time against the HBM peak.
         "bound": "l2+fabric",
         "kernel": (measured or {}).get("kernel") or
-        ("spmm_wave_kernel<4,3,...> over a padded input copy" if padded else "spmm_wave_kernel<1,10,...>")
+        (("spmm_wave_kernel<4,3,...> over a padded input copy" if not simple else
+          "spmm_group_kernel<true,true,32,...>, column panels of a padded input copy") if padded else "spmm_wave_kernel<1,10,...>")
         + " (F=602 gather, forward and backward launches)",
         "achieved": round(fabric_gbs, 1) if measured else None,
         "peak": HBM_PEAK_GBS,

@@ -2755,7 +2755,8 @@ constexpr uint32_t kOwnHubBlocks = 512;
 //                   contiguous: F = 47, 128    permuted: F = 47, 64, 100, 128, 200
 //   6 K, 12 K         30 / 13, 26 / 15           62 / 13, 64 / 13, 68 / 15, 68 / 16
 //   16 K, 100 K       61 / 33, 55 / 46           231 / 39, 241 / 39, 250 / 55, 244 / 55
-//   16 K, 1 M         202 / 105, 191 / 159       504 / 154, 172 / 166, 304 / 170, 318 / 214 (hub rows in slices)
+//   16 K, 1 M         202 / 105, 191 / 159       504 / 154, 172 / 166, 304 / 170, 318 / 214 (hub rows in slices; as one
+//                     running sum, a row each: 358, 457, permuted 397, 464, 367, 513)
 //   30 K, 3 M         213 / 175, 361 / 348       534 / 221, 298 / 240, 447 / 335, 463 / 366
 //   169 K, 2.48 M     186 / 188, 310 / 319       381 / 229, 258 / 226, 374 / 309, 388 / 343, 639 / 523
 //   400 K, 2 M        187 / 223, 301 / 298       337 / 263, 294 / 214, 391 / 285, 409 / 312
