@@ -292,6 +292,8 @@ int nts_spmm_plan_reserve(nts_spmm_plan_t *plan, uint32_t F);
  * caller must not destroy a plan while a call on it is being made.  A call on a stream that is being
  * captured is recorded without that ordering (no event is waited for or recorded under capture): the
  * caller orders replays of the captured call against eager calls and other streams that use the plan.
+ * It also records where the scratch lies: a later call of the same or a smaller width leaves that in place, one of
+ * a greater width may move it (reserve the greatest width before the capture).
  * `in` must hold all n_index rows the plan was built for: a plan that gathers from a padded copy of
  * the input (see below) copies every row of `in` on each call. */
 int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, const float *w,

@@ -34,6 +34,7 @@
 
 #include "common.hpp"
 #include "edge_sort.hpp"
+#include "plan_scratch.hpp"
 
 // Fixed scratch of nts_spmm_gather_static_scratch, the entry point for callers that must not allocate:
 // each device that loads this library holds one copy of the array until the process ends.  Host code
@@ -2054,6 +2055,17 @@ void parallel_blocks(uint32_t n, Fn fn) {
 
 }  // namespace
 
+namespace {
+struct PlanMemory {
+  using Error = hipError_t;
+  using Block = nts::DeviceBlock;
+  static constexpr hipError_t kSuccess = hipSuccess;
+  static hipError_t retire(nts::DeviceBlock &block) { return nts::retire_blocks({&block}); }
+  static bool out_of_memory(hipError_t err) { return err == hipErrorOutOfMemory; }
+  static void clear_error() { (void)hipGetLastError(); }
+};
+}  // namespace
+
 struct nts_spmm_plan {
   uint32_t rows = 0;
   uint32_t edges = 0;
@@ -2062,17 +2074,14 @@ struct nts_spmm_plan {
   uint32_t n_splits = 0;
   uint32_t n_partials = 0;
   const uint32_t *offsets = nullptr;  // identity check only
-  nts::DeviceBlock items_block, splits_block, sorted_block, ids_block, partial_block, padded_block;
+  nts::DeviceBlock items_block, splits_block, sorted_block, ids_block;
   uint4 *items = nullptr;             // device
   uint4 *splits = nullptr;            // device
   // Scratch shared by every call on this plan: the partial sums of split rows and, for widths whose
   // rows do not start on 16-byte boundaries, a padded copy of the input.  `mu` serialises the host
   // side of the calls (growing the scratch, enqueueing); `done` is recorded after the last kernel of
   // each call, and a call on another stream waits for it before it touches the scratch.
-  float *partial = nullptr;           // device
-  size_t partial_floats = 0;          // its capacity
-  float *in_padded = nullptr;         // device
-  size_t in_padded_floats = 0;
+  nts::PlanScratch<PlanMemory> scratch;
   uint32_t n_index = 0;               // rows of the gathered matrix (0 = not known: no padded copy)
   // At least 1 in 20 edges repeats the gather index of the edge before it: the wave kernel then loads
   // a row once per run of equal indices (and widths off 16-byte boundaries get the padded copy).
@@ -2748,7 +2757,7 @@ int nts_spmm_plan_destroy(nts_spmm_plan_t *plan) {
   { std::lock_guard<std::mutex> lock(plan->mu); }  // a call that is still enqueueing finishes first
   // Work queued on any stream of the plan's device may still read the arrays.
   const hipError_t given = nts::retire_blocks({&plan->items_block, &plan->splits_block, &plan->sorted_block,
-                                               &plan->ids_block, &plan->partial_block, &plan->padded_block});
+                                               &plan->ids_block, plan->scratch.partial_block(), plan->scratch.copy_block()});
   const hipError_t event = plan->done ? hipEventDestroy(plan->done) : hipSuccess;
   delete plan;
   if (given != hipSuccess) return nts::fail_hip(given, "nts_spmm_plan_destroy");
@@ -2797,12 +2806,12 @@ namespace {
 // there have to be 48 edges a gathered row, or 24 where rows are wider than 512 floats (300 floats 300 K rows, 10 M edges 1,082 ->
 // 1,114 us, 1 M, 40 M 4,226 -> 4,275; 500 1 M, 24 M 5,213 -> 5,068, 450 4,664 -> 4,868; 602 2.45 M, 40 M 12,905 -> 14,108).
 // NTS_SPMM_PAD=0 / 1 in the environment forces it off / on.
-uint32_t padded_stride(const nts_spmm_plan *plan, uint32_t F, bool heads) {
+uint32_t padded_stride(const nts_spmm_plan *plan, uint32_t F) {
   static const int forced = [] {
     const char *e = getenv("NTS_SPMM_PAD");
     return e ? (e[0] != '0' ? 1 : 0) : -1;
   }();
-  if (heads || plan->n_index == 0 || F <= 128 || forced == 0) return 0;
+  if (plan->n_index == 0 || F <= 128 || forced == 0) return 0;
   const uint32_t padded = (F + 31) / 32 * 32;
   if (forced == 1 || plan->dup_runs) return F % 4 ? padded : 0u;
   const uint64_t least = F > 512 ? 24 : 48;
@@ -2818,41 +2827,14 @@ bool use_runs(const nts_spmm_plan *plan) {
   return forced < 0 ? plan->dup_runs : forced == 1;
 }
 
-// Grows the plan's scratch for width F and leaves the call's row stride (padded_stride) in *stride: 0 also where the copy
-// has no room yet and there is no memory for it, or `fixed` says that none can be had now (the call gathers from the rows as
-// they are, with the same sums).  Caller holds plan->mu.
-int reserve_locked(nts_spmm_plan *plan, uint32_t F, bool heads, bool fixed, uint32_t *stride) {
-  uint32_t ld = padded_stride(plan, F, heads);
-  // A buffer that grows may still be read by work queued earlier, on any stream.
-  auto grow = [](nts::DeviceBlock &block, float **ptr, size_t *floats, size_t want) -> int {
-    if (want <= *floats) return NTS_OK;
-    *ptr = nullptr;
-    *floats = 0;
-    NTS_HIP_TRY(nts::retire_blocks({&block}));
-    NTS_HIP_TRY(block.take(want * sizeof(float)));
-    *ptr = block.as<float>();
-    *floats = block.bytes / sizeof(float);
-    return NTS_OK;
-  };
-  if (const size_t want = static_cast<size_t>(plan->n_index) * ld; want > plan->in_padded_floats) {
-    if (fixed) {
-      ld = 0;
-    } else if (grow(plan->padded_block, &plan->in_padded, &plan->in_padded_floats, want)) {
-      (void)hipGetLastError();
-      ld = 0;
-    }
-  }
-  const size_t n = plan->n_partials;
-  if (ld && grow(plan->partial_block, &plan->partial, &plan->partial_floats, n * ld)) {
-    // the copy has taken the memory that the partial sums need more
-    (void)hipGetLastError();
-    plan->in_padded = nullptr;
-    plan->in_padded_floats = 0;
-    NTS_HIP_TRY(nts::retire_blocks({&plan->padded_block}));
-    ld = 0;
-  }
-  *stride = ld;
-  return ld ? NTS_OK : grow(plan->partial_block, &plan->partial, &plan->partial_floats, n * F);
+// Makes room in the plan's scratch for a call of width F and leaves the call's row stride (padded_stride) in *stride: 0 where it
+// gathers from the rows as they are, with the same sums (PlanScratch::place).  Caller holds plan->mu.
+int reserve_locked(nts_spmm_plan *plan, uint32_t F, bool heads, bool recorded, uint32_t *stride) {
+  const nts::ScratchNeed need{plan->n_partials, F, padded_stride(plan, F), plan->n_index};
+  size_t ld = 0;
+  NTS_HIP_TRY(plan->scratch.place(need, !heads, recorded, &ld));
+  *stride = static_cast<uint32_t>(ld);
+  return NTS_OK;
 }
 
 // A call on `stream` is about to use the plan's scratch: if the previous call ran on another stream,
@@ -2889,7 +2871,7 @@ int nts_spmm_plan_scratch_info(nts_spmm_plan_t *plan, uint32_t F, size_t *partia
   NTS_TRACE_RANGE("nts_spmm_plan_scratch_info");
   if (!plan) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_scratch_info: null plan");
   if (F == 0) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_scratch_info: F is 0");
-  const uint32_t ld = padded_stride(plan, F, false);
+  const uint32_t ld = padded_stride(plan, F);
   if (partial_bytes) *partial_bytes = static_cast<size_t>(plan->n_partials) * (ld ? ld : F) * sizeof(float);
   if (padded_input_bytes) *padded_input_bytes = ld ? static_cast<size_t>(plan->n_index) * ld * sizeof(float) : 0;
   if (repeated_edges) *repeated_edges = plan->repeated_edges;
@@ -2994,10 +2976,10 @@ int nts_spmm_gather_heads_planned(nts_spmm_plan_t *plan, const float *in, float 
   if (plan->rows == 0) return NTS_OK;
   std::lock_guard<std::mutex> lock(plan->mu);
   uint32_t ld = 0;
-  if (int rc = reserve_locked(plan, F, true, false, &ld)) return rc;
+  if (int rc = reserve_locked(plan, F, true, stream_is_capturing(stream), &ld)) return rc;
   if (int rc = enter_stream(plan, stream)) return rc;
   nts::LaunchArgs a{in,  out,         alpha,         offsets,    indices, 0u, plan->n_items,
-                    F,   plan->items, plan->partial, accumulate, stream};
+                    F,   plan->items, plan->scratch.partial(), accumulate, stream};
   a.heads = nts::HeadArgs{perm, H, Fh};
   a.scheduled_rows = plan->rows;
   a.ranged = plan->ranged;
@@ -3009,7 +2991,7 @@ int nts_spmm_gather_heads_planned(nts_spmm_plan_t *plan, const float *in, float 
   nts::launch_spmm(a);
   NTS_LAUNCH_CHECK("nts_spmm_gather_heads_planned");
   if (plan->n_splits) {
-    nts::launch_reduce_partials(out, plan->partial, plan->splits, plan->n_splits, F, accumulate, stream);
+    nts::launch_reduce_partials(out, plan->scratch.partial(), plan->splits, plan->n_splits, F, accumulate, stream);
     NTS_LAUNCH_CHECK("spmm_reduce_partials_kernel");
   }
   return leave_stream(plan, stream);
@@ -3041,7 +3023,7 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
   if (int rc = reserve_locked(plan, F, false, stream_is_capturing(stream), &ld)) return rc;
   if (int rc = enter_stream(plan, stream)) return rc;
   nts::LaunchArgs a{in,  out,         w,           offsets,       indices,   index_base, plan->n_items,
-                    F,   plan->items, plan->partial, accumulate, stream};
+                    F,   plan->items, plan->scratch.partial(), accumulate, stream};
   if (plan->sorted_idx) {  // the schedule's own copy of the indices, base already subtracted
     a.indices = plan->sorted_idx;
     a.index_base = 0;
@@ -3056,9 +3038,9 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
     const uint64_t vecs = static_cast<uint64_t>(plan->n_index) * (ld / 4);
     const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>((vecs + 255) / 256, 1u << 16));
     hipLaunchKernelGGL(nts::pad_rows_kernel, dim3(blocks), dim3(256), 0, stream,
-                       reinterpret_cast<float4 *>(plan->in_padded), in, plan->n_index, F, ld);
+                       reinterpret_cast<float4 *>(plan->scratch.copy()), in, plan->n_index, F, ld);
     NTS_LAUNCH_CHECK("pad_rows_kernel");
-    a.in = plan->in_padded;
+    a.in = plan->scratch.copy();
     a.in_ld = ld;
     a.partial_ld = ld;
   }
@@ -3067,7 +3049,7 @@ int nts_spmm_gather_planned(nts_spmm_plan_t *plan, const float *in, float *out, 
   NTS_LAUNCH_CHECK("nts_spmm_gather_planned");
   if (plan->ev_start && plan->ev_stop) NTS_HIP_TRY(hipEventRecord(plan->ev_stop, stream));
   if (plan->n_splits) {
-    nts::launch_reduce_partials(out, plan->partial, plan->splits, plan->n_splits, F, accumulate, stream, a.partial_ld);
+    nts::launch_reduce_partials(out, plan->scratch.partial(), plan->splits, plan->n_splits, F, accumulate, stream, a.partial_ld);
     NTS_LAUNCH_CHECK("spmm_reduce_partials_kernel");
   }
   return leave_stream(plan, stream);

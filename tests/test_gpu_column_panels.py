@@ -121,6 +121,32 @@ def test_captured_call_without_room_for_the_copy(device):
             assert torch.equal(out, want)
 
 
+def test_partial_sums_stay_where_a_capture_found_them(device):
+    """Heads of the same width make the room, a capture records it, and an ordinary call that then takes the copy leaves it there."""
+    rows, edges, F = 3001, 150050, 602
+    off, idx = simple_graph(rows, edges, device, True)
+    g = torch.Generator(device=device).manual_seed(2)
+    x, w = torch.randn(rows, F, generator=g, device=device), torch.rand(edges, generator=g, device=device)
+    alpha = torch.rand(edges, 2, generator=g, device=device)
+    plan = SpmmPlan(off, rows, edges, 64, idx, rows, 8)
+    assert plan.info()["partials"] > 0
+    out, other, want = (torch.empty(rows, F, device=device) for _ in range(3))
+    call("nts_spmm_gather_heads_planned", plan.handle, ptr(x), ptr(other), ptr(alpha), 0, ptr(off), ptr(idx), 2, F // 2, 0,
+         torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call("nts_spmm_gather_planned", plan.handle, ptr(x), ptr(out), ptr(w), ptr(off), ptr(idx), 0, F, 0,
+             torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        call("nts_spmm_gather_planned", plan.handle, ptr(x), ptr(want), ptr(w), ptr(off), ptr(idx), 0, F, 0,
+             torch.cuda.current_stream().cuda_stream)
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 def compare(device, plan, off, idx, rows, edges, F, narrow):
     g = torch.Generator(device=device).manual_seed(F)
     x, w = torch.randn(rows, F, generator=g, device=device), torch.rand(edges, generator=g, device=device)
