@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "launch_size.hpp"
 
 namespace nts {
 namespace {
@@ -203,13 +204,15 @@ constexpr int kLongBlock = 1024;
 
 // What the first blocks of a row launch do beside it when the rows above `long_limit` edges are summed
 // in the same launch: the list of those rows, the piece table of the giant ones, where the pieces' sums
-// go, the column tile of a 256-thread block and how many blocks are set aside (0: none).
+// go, the column tile of a 256-thread block, how many blocks are set aside (0: none), and whether hub rows are looked for
+// where there is no list (few_long_edges).
 template <typename V>
 struct LongRowWork {
   const uint32_t *list, *count, *hdr;
   const uint4 *pieces;
   V *partial;
   uint32_t tile, blocks;
+  bool own;
 };
 
 __device__ __forceinline__ void vadd(float &a, const float &b) { a += b; }
@@ -375,7 +378,7 @@ __device__ __forceinline__ uint32_t few_long_edges(const uint32_t *__restrict__ 
 }
 template <typename V>
 __device__ __forceinline__ uint32_t long_limit_of(const LongRowWork<V> &lw, uint32_t limit, const uint32_t *__restrict__ off, uint32_t rows) {
-  return lw.blocks && !lw.list ? few_long_edges(off, rows) : limit;
+  return lw.own ? few_long_edges(off, rows) : limit;
 }
 
 // The first blocks of a row launch take the listed long rows, one 256-thread block per row, and the
@@ -426,14 +429,14 @@ __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out,
 }
 
 // out[r,:] (+)= sum_{k in [off[r], off[r+1])} msg[perm ? perm[k] : k, :], added in k order: a group of G lanes for every row and
-// every G vectors of it.  The edge rows of a round are requested together and their ids a round ahead, so that a long row is a
+// every G vectors of it from first_group on.  The edge rows of a round are requested together and their ids a round ahead, so that a long row is a
 // memory latency per U edges; the last, partial rounds are of eight, whose requests beyond the row are its last edge's again.
 template <typename V, int G, int U>
 __global__ __launch_bounds__(256, (U > 8 ? 4 : 8)) void gather_edge_to_row_kernel(V *__restrict__ out, const V *__restrict__ msg,
                                                                  const uint32_t *__restrict__ off,
                                                                  const uint32_t *__restrict__ perm, uint32_t rows,
                                                                  uint32_t Fv, int accumulate, uint32_t long_limit, uint32_t tiles,
-                                                                 LongRowWork<V> lw) {
+                                                                 uint64_t first_group, LongRowWork<V> lw) {
   if (blockIdx.x < lw.blocks) {
     constexpr int kOwn = sizeof(V) == 16 ? 4 : U > 8 ? 16 : 0;  // (of floats, only the few rows' kernel has rows without a list)
     __shared__ V scratch[kHubBytes<V, kOwn> / sizeof(V)];
@@ -441,7 +444,7 @@ __global__ __launch_bounds__(256, (U > 8 ? 4 : 8)) void gather_edge_to_row_kerne
     return;
   }
   long_limit = long_limit_of(lw, long_limit, off, rows);
-  const uint64_t group = (static_cast<uint64_t>(blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / G;
+  const uint64_t group = first_group + (static_cast<uint64_t>(blockIdx.x - lw.blocks) * blockDim.x + threadIdx.x) / G;
   if (group >= static_cast<uint64_t>(rows) * tiles) return;
   const uint32_t r = static_cast<uint32_t>(group / tiles), c = static_cast<uint32_t>(group % tiles) * G + (threadIdx.x & (G - 1));
   if (c >= Fv) return;
@@ -2860,16 +2863,23 @@ void launch_gather_rows(V *out, const V *msg, const uint32_t *off, const uint32_
 #undef NTS_BALANCED
     return;
   }
+  // One launch up to 2^32 threads; the hub rows are the first one's.
 #define NTS_GATHER(GG)                                                                                            \
   do {                                                                                                            \
     const uint32_t tiles = ceil_div(Fv, GG);                                                                      \
-    const uint32_t blocks = ceil_div(static_cast<uint64_t>(rows) * tiles * GG, 256) + lw.blocks;                  \
-    if (sizeof(V) == 4 && rows < kLongMinVertices)                                                                \
-      hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG, sizeof(V) == 16 ? 8 : 32>), dim3(blocks), dim3(256), 0, \
-                         stream, out, msg, off, perm, rows, Fv, accumulate, limit, tiles, lw);                    \
-    else                                                                                                          \
-      hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG, 8>), dim3(blocks), dim3(256), 0, stream, out, msg, off, \
-                         perm, rows, Fv, accumulate, limit, tiles, lw);                                           \
+    const uint64_t groups = static_cast<uint64_t>(rows) * tiles;                                                  \
+    LongRowWork<V> hubs = lw;                                                                                     \
+    for (uint64_t first = 0; first < groups;) {                                                                   \
+      const uint32_t blocks = blocks_of_groups(groups - first, GG, hubs.blocks);                                  \
+      if (sizeof(V) == 4 && rows < kLongMinVertices)                                                              \
+        hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG, sizeof(V) == 16 ? 8 : 32>), dim3(blocks), dim3(256), 0, \
+                           stream, out, msg, off, perm, rows, Fv, accumulate, limit, tiles, first, hubs);         \
+      else                                                                                                        \
+        hipLaunchKernelGGL((gather_edge_to_row_kernel<V, GG, 8>), dim3(blocks), dim3(256), 0, stream, out, msg, off, \
+                           perm, rows, Fv, accumulate, limit, tiles, first, hubs);                                \
+      first += static_cast<uint64_t>(blocks - hubs.blocks) * (256 / GG);                                          \
+      hubs.blocks = 0;                                                                                            \
+    }                                                                                                             \
   } while (0)
   switch (lanes_for(Fv)) {
     case 1: NTS_GATHER(1); break;
@@ -2924,11 +2934,11 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   }
   if (v4) {
     LongRowWork<float4> lw{lr.list, lr.count, lr.hdr, lr.pieces, reinterpret_cast<float4 *>(partial), tile,
-                           merged ? merged_long_blocks() : own_hubs};
+                           merged ? merged_long_blocks() : own_hubs, own};
     launch_gather_rows(reinterpret_cast<float4 *>(out), reinterpret_cast<const float4 *>(msg), off, perm, rows, Fv,
                        accumulate, limit, lw, stream);
   } else {
-    LongRowWork<float> lw{lr.list, lr.count, lr.hdr, lr.pieces, partial, tile, merged ? merged_long_blocks() : own_hubs};
+    LongRowWork<float> lw{lr.list, lr.count, lr.hdr, lr.pieces, partial, tile, merged ? merged_long_blocks() : own_hubs, own};
     launch_gather_rows(out, msg, off, perm, rows, Fv, accumulate, limit, lw, stream);
   }
   hipError_t launch_err = hipGetLastError();

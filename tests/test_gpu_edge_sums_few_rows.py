@@ -81,3 +81,47 @@ def test_permuted_sums_of_many_rows(device, rows, F):
     size = torch.cat([terms.new_zeros(1, F, dtype=torch.float64), terms.double().abs().cumsum(0)])
     want, scale = total[off[1:]] - total[off[:-1]], size[off[1:]] - size[off[:-1]]
     assert ((out.double() - want).abs() <= (deg.double()[:, None] + 1) * 2.0 ** -24 * scale + 1e-8).all()
+
+
+# 29 groups of 64 columns for every row: 71 M groups, more than a launch has threads for
+@pytest.mark.parametrize("permuted", [False, True])
+def test_sums_of_more_groups_than_a_launch_holds(device, permuted):
+    rows, F, E = 2449029, 1793, 3000
+    assert rows * 29 * 64 >= 1 << 32
+    g = torch.Generator(device=device).manual_seed(3)
+    at = torch.randperm(rows, generator=g, device=device)[:E - 1]
+    at = torch.cat([at, torch.tensor([rows - 1], device=device)]).unique()  # a row each, the last one among them
+    deg = torch.zeros(rows, dtype=torch.int64, device=device)
+    deg[at] = 1
+    off = torch.cat([deg.new_zeros(1), deg.cumsum(0)]).to(torch.int32)
+    msg = torch.randn(at.numel(), F, generator=g, device=device)
+    perm = torch.randperm(at.numel(), generator=g, device=device)
+    ids = perm.to(torch.int32)
+    out = torch.full((rows, F), float("nan"), device=device)
+    s = torch.cuda.current_stream().cuda_stream
+    if permuted:
+        call("nts_gather_edge_to_src", ptr(out), ptr(msg), ptr(off), ptr(ids), rows, F, 0, s)
+    else:
+        call("nts_gather_edge_to_dst", ptr(out), ptr(msg), ptr(off), rows, F, 0, s)
+    assert torch.equal(out[at], msg[perm] if permuted else msg)
+    out[at] = 0
+    assert not out.any()
+
+
+def test_a_hub_row_of_the_second_launch_is_summed_once(device):
+    rows, F, E = 16383, 262209, 1100
+    assert rows * 4098 > 1 << 26  # groups of 64 columns, 2^26 of them to a launch; the last row's are the next one's
+    g = torch.Generator(device=device).manual_seed(4)
+    off = torch.zeros(rows + 1, dtype=torch.int64, device=device)
+    off[rows - 1] = 3
+    off[rows] = E
+    msg = torch.randn(E, F, generator=g, device=device)
+    out = torch.ones(rows, F, device=device)
+    co = off.to(torch.int32)
+    call("nts_gather_edge_to_dst", ptr(out), ptr(msg), ptr(co), rows, F, 1, torch.cuda.current_stream().cuda_stream)
+    for r in (rows - 2, rows - 1):
+        want = torch.zeros(F, device=device)
+        for e in range(int(off[r]), int(off[r + 1])):
+            want += msg[e]
+        assert torch.equal(out[r], want + 1)
+    assert bool((out[:rows - 2] == 1).all())
