@@ -185,10 +185,10 @@ __global__ __launch_bounds__(256) void edge_copy_kernel(V *__restrict__ msg, con
 // Rows with at most `long_limit` edges: a group of G lanes per row (64/G rows per wavefront) adds
 // the row's edge rows in order; where the edge rows of consecutive vertices follow each other in
 // memory (no permutation), a wavefront streams the edges of a run of rows through LDS instead (same
-// sums).  Longer rows (power-law hubs) are listed first and summed by whole
-// blocks -- the first blocks of the same launch where the row launch is the balanced kernel, the
-// block kernels below otherwise -- which spread a row's edges over the slices of the block and add
-// the slices' partial sums in a fixed order.
+// sums).  Longer rows (power-law hubs) are listed first and summed by the first blocks of the same
+// launch, which spread a row's edges over the slices of the block and add
+// the slices' partial sums in a fixed order; calls of fewer than kLongMinVertices rows list none, and their first blocks
+// find the hub rows themselves (few_long_edges).
 
 constexpr uint32_t kNoLimit = 0xFFFFFFFFu;
 constexpr uint32_t kLongRowEdges = 1024;    // edges of a row above which the block kernel takes over
@@ -205,7 +205,7 @@ constexpr int kLongBlock = 1024;
 // What the first blocks of a row launch do beside it when the rows above `long_limit` edges are summed
 // in the same launch: the list of those rows, the piece table of the giant ones, where the pieces' sums
 // go, the column tile of a 256-thread block, how many blocks are set aside (0: none), and whether hub rows are looked for
-// where there is no list (few_long_edges).
+// where there is no list (few_long_edges); how many slices of a listed row a thread adds up.
 template <typename V>
 struct LongRowWork {
   const uint32_t *list, *count, *hdr;
@@ -213,6 +213,7 @@ struct LongRowWork {
   V *partial;
   uint32_t tile, blocks;
   bool own;
+  uint32_t chains;
 };
 
 __device__ __forceinline__ void vadd(float &a, const float &b) { a += b; }
@@ -233,68 +234,70 @@ __device__ __forceinline__ float4 vnull<float4>() {
   return make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// Sum of the columns [first_col, end_col) of the edge rows [e0, e1) by one block of BLOCK threads, added into dst (V = float, or
+// Sum of the columns [first_col, end_col) of the edge rows [e0, e1) by one block of 256 threads, added into dst (V = float, or
 // float4 when rows are 16-byte aligned: a quarter of the load instructions and of the rounds a row
-// takes).  Columns are taken in tiles of `tile` vectors (a power of two <= BLOCK); thread t owns
-// column t % tile of slice t / tile, a slice adds every (BLOCK/tile)-th edge of the range in ascending
-// order (a round's loads together), and the slices' sums are then added pairwise in a fixed tree.
-template <typename V, int BLOCK, int U>
+// takes).  They are at most `tile` vectors (a power of two <= 256); thread t owns
+// column t % tile of C of the C * 256 / tile slices, a slice adds every so many-th edge of the range in ascending
+// order (a round's loads together), and the slices' sums are then added pairwise in a fixed tree, the upper half to the lower.
+template <typename V, int U, int C>
 __device__ __forceinline__ void block_sum_edge_rows(V *__restrict__ dst, const V *__restrict__ msg,
                                                     const uint32_t *__restrict__ perm, uint32_t e0, uint32_t e1,
                                                     uint32_t Fv, uint32_t first_col, uint32_t end_col, uint32_t tile,
                                                     int accumulate, V *part) {
-  const uint32_t c = threadIdx.x & (tile - 1);
-  const uint32_t slice = threadIdx.x / tile;
-  const uint32_t n_slices = BLOCK / tile;
-  for (uint32_t cb = first_col; cb < end_col; cb += tile) {
-    const uint32_t col = cb + c;
-    V a = vnull<V>();
-    if (col < end_col && e1 - e0 > slice) {
-      // The edge ids of the next round are requested while the rows of this one are on their way; beyond the range the last edge's.
-      // Through a permutation, 2.48 M edges of 47 floats 704 -> 379 us.  Eight vectors a round took the kernels 98 registers instead of
-      // 62 (30 K rows, 3 M edges F = 128 467, held to 72 with spills 502, four a round 467); narrow rows, whose kernels hold as many anyway,
-      // have room for them.
-      uint32_t k = e0 + slice, left = e1 - k, id[U];
-      auto request_ids = [&] {
+  const uint32_t slice = threadIdx.x / tile, n_slices = 256 / tile, col = first_col + (threadIdx.x & (tile - 1));
+  static_assert(U % C == 0 && C <= 4, "a round's first load is the first slice's");
+  V a[C];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const uint32_t kk = k + (u * n_slices < left ? u * n_slices : left - 1);
-          id[u] = perm ? perm[kk] : kk;
-        }
-      };
-      request_ids();
-      while (left) {
-        V v[U];
+  for (int j = 0; j < C; ++j) a[j] = vnull<V>();
+  if (col < end_col && e1 - e0 > slice) {
+    // The edge ids of the next round are requested while the rows of this one are on their way; beyond the range the last edge's.
+    // Through a permutation, 2.48 M edges of 47 floats 704 -> 379 us.  Eight vectors a round took the kernels 98 registers instead of
+    // 62 (30 K rows, 3 M edges F = 128 467, held to 72 with spills 502, four a round 467); narrow rows, whose kernels hold as many anyway,
+    // have room for them.
+    uint32_t k = e0 + slice, left = e1 - k, id[U];
+    auto request_ids = [&] {
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = msg[static_cast<size_t>(id[u]) * Fv + col];
-        const uint32_t now = left;
-        left = left > U * n_slices ? left - U * n_slices : 0u;
-        if (left) {
-          k += U * n_slices;
-          request_ids();
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (u * n_slices < now) vadd(a, v[u]);
+      for (int u = 0; u < U; ++u) {
+        const uint32_t kk = k + (u * n_slices < left ? u * n_slices : left - 1);
+        id[u] = perm ? perm[kk] : kk;
       }
-    }
-    part[threadIdx.x] = a;
-    __syncthreads();
-    for (uint32_t stride = n_slices / 2; stride >= 1; stride >>= 1) {
-      if (slice < stride) {
-        V lo = part[threadIdx.x];
-        vadd(lo, part[threadIdx.x + stride * tile]);
-        part[threadIdx.x] = lo;
+    };
+    request_ids();
+    while (left) {
+      V v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = msg[static_cast<size_t>(id[u]) * Fv + col];
+      const uint32_t now = left;
+      left = left > U * n_slices ? left - U * n_slices : 0u;
+      if (left) {
+        k += U * n_slices;
+        request_ids();
       }
-      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (u * n_slices < now) vadd(a[u % C], v[u]);
     }
-    if (slice == 0 && col < end_col) {
-      V total = part[c];
-      if (accumulate) vadd(total, dst[col]);
-      dst[col] = total;
+  }
+#pragma unroll
+  for (int half = C / 2; half >= 1; half /= 2)
+#pragma unroll
+    for (int j = 0; j < half; ++j) vadd(a[j], a[j + half]);
+  part[threadIdx.x] = a[0];
+  __syncthreads();
+  for (uint32_t stride = n_slices / 2; stride >= 1; stride >>= 1) {
+    if (slice < stride) {
+      V lo = part[threadIdx.x];
+      vadd(lo, part[threadIdx.x + stride * tile]);
+      part[threadIdx.x] = lo;
     }
     __syncthreads();
   }
+  if (slice == 0 && col < end_col) {
+    V total = part[threadIdx.x];
+    if (accumulate) vadd(total, dst[col]);
+    dst[col] = total;
+  }
+  __syncthreads();
 }
 
 // The same columns (tile vectors from first_col on, at most 32 floats) as one running sum in edge order: the block stages U vectors a
@@ -384,7 +387,7 @@ __device__ __forceinline__ uint32_t long_limit_of(const LongRowWork<V> &lw, uint
 // The first blocks of a row launch take the listed long rows, one 256-thread block per row, and the
 // pieces of the giant ones (their partial sums are combined by a launch of its own afterwards); the
 // rows of the launch proper fill the chip meanwhile.
-template <typename V, int U, int OWN>
+template <typename V, int U, int OWN, bool WIDE = false>
 __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out, const V *__restrict__ msg,
                                                             const uint32_t *__restrict__ off,
                                                             const uint32_t *__restrict__ perm, uint32_t rows, uint32_t Fv,
@@ -416,15 +419,28 @@ __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out,
     }
     return;
   }
-  const uint32_t n_rows = *lw.count, n_pieces = lw.hdr[1];
-  for (uint32_t i = blockIdx.x; i < n_rows; i += lw.blocks) {
-    const uint32_t r = lw.list[i];
-    block_sum_edge_rows<V, 256, U>(out + static_cast<size_t>(r) * Fv, msg, perm, off[r], off[r + 1], Fv, 0, Fv, lw.tile, accumulate, part);
-  }
-  // the pieces start with the blocks that the rows left idle
-  for (uint32_t p = (blockIdx.x + lw.blocks - n_rows % lw.blocks) % lw.blocks; p < n_pieces; p += lw.blocks) {
-    const uint4 pc = lw.pieces[p];
-    block_sum_edge_rows<V, 256, U>(lw.partial + static_cast<size_t>(p) * Fv, msg, perm, pc.z, pc.w, Fv, 0, Fv, lw.tile, 0, part);
+  // the column tiles of a listed row one after the other, then those of the pieces
+  const uint32_t tiles = (Fv + lw.tile - 1) / lw.tile;
+  const uint64_t n_rows = static_cast<uint64_t>(*lw.count) * tiles, n_all = n_rows + static_cast<uint64_t>(lw.hdr[1]) * tiles;
+  for (uint64_t i = blockIdx.x; i < n_all; i += lw.blocks) {
+    const uint64_t at = (i < n_rows ? i : i - n_rows) / tiles;
+    const uint32_t c0 = static_cast<uint32_t>(i % tiles) * lw.tile, c1 = c0 + lw.tile < Fv ? c0 + lw.tile : Fv;
+    uint32_t e0, e1;
+    V *dst;
+    if (i < n_rows) {
+      const uint32_t r = lw.list[at];
+      e0 = off[r];
+      e1 = off[r + 1];
+      dst = out + static_cast<size_t>(r) * Fv;
+    } else {
+      const uint4 pc = lw.pieces[at];
+      e0 = pc.z;
+      e1 = pc.w;
+      dst = lw.partial + at * Fv;
+    }
+    const int add = i < n_rows && accumulate;
+    if (WIDE && lw.chains == 4) block_sum_edge_rows<V, U, WIDE ? 4 : 1>(dst, msg, perm, e0, e1, Fv, c0, c1, lw.tile, add, part);
+    else block_sum_edge_rows<V, U, 1>(dst, msg, perm, e0, e1, Fv, c0, c1, lw.tile, add, part);
   }
 }
 
@@ -440,7 +456,7 @@ __global__ __launch_bounds__(256, (U > 8 ? 4 : 8)) void gather_edge_to_row_kerne
   if (blockIdx.x < lw.blocks) {
     constexpr int kOwn = sizeof(V) == 16 ? 4 : U > 8 ? 16 : 0;  // (of floats, only the few rows' kernel has rows without a list)
     __shared__ V scratch[kHubBytes<V, kOwn> / sizeof(V)];
-    sum_long_rows_in_this_block<V, sizeof(V) == 16 ? 4 : 8, kOwn>(out, msg, off, perm, rows, Fv, accumulate, lw, scratch);
+    sum_long_rows_in_this_block<V, sizeof(V) == 16 ? 4 : 8, kOwn, G == kWave && U == 8>(out, msg, off, perm, rows, Fv, accumulate, lw, scratch);
     return;
   }
   long_limit = long_limit_of(lw, long_limit, off, rows);
@@ -1128,37 +1144,6 @@ __global__ __launch_bounds__(kLongBlock) void few_long_rows_kernel(uint32_t *__r
   __syncthreads();
   if (threadIdx.x == 0) *count = n_long;
   plan_giant_rows<kLongBlock>(n_giant, giant_edges, hdr, giant_rows, first, pieces, off, min_piece);
-}
-
-// One 1024-thread block per listed long row.
-template <typename V>
-__global__ __launch_bounds__(kLongBlock) void gather_edge_to_row_long_kernel(
-    V *__restrict__ out, const V *__restrict__ msg, const uint32_t *__restrict__ off,
-    const uint32_t *__restrict__ perm, const uint32_t *__restrict__ list, const uint32_t *__restrict__ count,
-    uint32_t Fv, uint32_t tile, int accumulate) {
-  __shared__ V part[kLongBlock];
-  const uint32_t n_rows = *count;
-  for (uint32_t i = blockIdx.x; i < n_rows; i += gridDim.x) {
-    const uint32_t r = list[i];
-    block_sum_edge_rows<V, kLongBlock, sizeof(V) == 16 ? 4 : 8>(out + static_cast<size_t>(r) * Fv, msg, perm, off[r], off[r + 1], Fv, 0, Fv, tile,
-                                       accumulate, part);
-  }
-}
-
-// One block per piece of a giant row: partial[piece, :] = sum of the piece's edge rows.
-template <typename V>
-__global__ __launch_bounds__(kLongBlock) void giant_sum_pieces_kernel(V *__restrict__ partial,
-                                                                      const V *__restrict__ msg,
-                                                                      const uint32_t *__restrict__ perm,
-                                                                      const uint32_t *__restrict__ hdr,
-                                                                      const uint4 *__restrict__ pieces, uint32_t Fv,
-                                                                      uint32_t tile) {
-  __shared__ V part[kLongBlock];
-  const uint32_t n_pieces = hdr[1];
-  for (uint32_t p = blockIdx.x; p < n_pieces; p += gridDim.x) {
-    const uint4 pc = pieces[p];
-    block_sum_edge_rows<V, kLongBlock, sizeof(V) == 16 ? 4 : 8>(partial + static_cast<size_t>(p) * Fv, msg, perm, pc.z, pc.w, Fv, 0, Fv, tile, 0, part);
-  }
 }
 
 // out[row, :] (+)= the row's piece sums, added in piece order.
@@ -2734,20 +2719,8 @@ uint32_t coop_limit() {
   return value;
 }
 
-// Blocks of a row launch set aside for the long rows when they are summed in the same launch: as many
-// threads as the long-row kernels of their own bring (512 blocks of 1,024).
+// Blocks of a row launch set aside for the listed long rows and the pieces of the giant ones.
 constexpr uint32_t kMergedLongBlocks = 2048;
-// NTS_EDGE_SUM_MERGE in the environment: 0 = long rows always in launches of their own; n > 0 = that many
-// blocks of the row launch for them.
-uint32_t merged_long_blocks() {
-  static const uint32_t value = [] {
-    const char *env = getenv("NTS_EDGE_SUM_MERGE");
-    if (!env) return kMergedLongBlocks;
-    const long v = atol(env);
-    return v <= 0 ? 0u : static_cast<uint32_t>(v);
-  }();
-  return value;
-}
 
 // The same for calls of fewer than kLongMinVertices rows, which find them themselves; not where rows are so few that each has a
 // block's worth of wavefronts beside it anyway.
@@ -2914,18 +2887,21 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   bool v4 = F % 4 == 0 && aligned_to(out, 16) && aligned_to(msg, 16);
   if (v4 && floats_for_few_rows(rows, F)) v4 = false;
   const uint32_t Fv = v4 ? F / 4 : F;
-  // Long rows: in the first blocks of the row launch where that launch has them (256-thread blocks),
-  // else in launches of their own after it (1,024-thread blocks).  Giant rows: pieces by separate
-  // blocks into stream-ordered scratch, then the ordered combine.
-  const bool merged = lr.list && merged_long_blocks() > 0;
-  const uint32_t block_threads = merged ? 256u : static_cast<uint32_t>(kLongBlock);
-  // Few rows: the first blocks find the hub rows themselves and take columns of 128 bytes of one each.
+  // Long rows, and giant rows in pieces: in the first blocks of the row launch; the pieces' sums go to stream-ordered scratch and a
+  // launch of its own combines them in order.  Few rows: the first blocks find the hub rows themselves and take columns of 128 bytes of one each.
   const uint32_t hub_lanes = v4 ? 8u : F > 32 ? 16u : 32u;
   const bool own = !lr.list && rows >= kMinHubRows && (Fv > 8 || (perm && Fv > 4 && v4) || rows < kMaxNarrowHubRows);
-  const uint32_t own_hubs = !own ? 0u : Fv <= hub_lanes ? kOwnHubBlocks / 2 : kOwnHubBlocks;
-  const uint32_t most_lanes = own_hubs ? hub_lanes : block_threads;
+  const uint32_t hub_blocks = lr.list ? kMergedLongBlocks : !own ? 0u : Fv <= hub_lanes ? kOwnHubBlocks / 2 : kOwnHubBlocks;
+  const uint32_t most_lanes = own ? hub_lanes : 256u;
   uint32_t tile = 1;
   while (tile < Fv && tile < most_lanes) tile <<= 1;
+  // Listed rows of more than 64 vectors are added by as many slices as 1,024 threads have beside the whole row: eight or four, four of
+  // them a thread; two, of a thread each, beside 128 vectors of a row of up to 512; one above.  With tiles of 256 and a slice a thread a chain of
+  // additions was two to four times as many edges, and rows of 65 to 127 floats were 2.7 times as far from their sums in 64 bits (1.8e-7
+  // instead of 6.7e-8, values in [0, 1), 16.5 K rows, 1 M edges).  us, so / as it is, 30 K rows, 3 M edges F = 65 229 / 218, 127 362 / 342, 257 747 /
+  // 695 (two slices a thread 818), 512 1,217 / 1,220, 169 K, 2.48 M F = 602 1,608 / 1,573; the first of these as four tiles with a slice a thread 277.
+  const uint32_t chains = !own && Fv > kWave && Fv <= 256 ? 4 : 1;
+  if (!own && Fv > 256 && Fv <= 512) tile = 128;
   ScratchBlock partial_block;
   float *partial = nullptr;
   if (lr.list) {
@@ -2934,30 +2910,15 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   }
   if (v4) {
     LongRowWork<float4> lw{lr.list, lr.count, lr.hdr, lr.pieces, reinterpret_cast<float4 *>(partial), tile,
-                           merged ? merged_long_blocks() : own_hubs, own};
+                           hub_blocks, own, chains};
     launch_gather_rows(reinterpret_cast<float4 *>(out), reinterpret_cast<const float4 *>(msg), off, perm, rows, Fv,
                        accumulate, limit, lw, stream);
   } else {
-    LongRowWork<float> lw{lr.list, lr.count, lr.hdr, lr.pieces, partial, tile, merged ? merged_long_blocks() : own_hubs, own};
+    LongRowWork<float> lw{lr.list, lr.count, lr.hdr, lr.pieces, partial, tile, hub_blocks, own, chains};
     launch_gather_rows(out, msg, off, perm, rows, Fv, accumulate, limit, lw, stream);
   }
   hipError_t launch_err = hipGetLastError();
   if (lr.list && launch_err == hipSuccess) {
-    if (!merged) {
-      if (v4) {
-        hipLaunchKernelGGL(gather_edge_to_row_long_kernel<float4>, dim3(kLongGrid), dim3(kLongBlock), 0, stream,
-                           reinterpret_cast<float4 *>(out), reinterpret_cast<const float4 *>(msg), off, perm, lr.list,
-                           lr.count, Fv, tile, accumulate);
-        hipLaunchKernelGGL(giant_sum_pieces_kernel<float4>, dim3(kLongGrid), dim3(kLongBlock), 0, stream,
-                           reinterpret_cast<float4 *>(partial), reinterpret_cast<const float4 *>(msg), perm, lr.hdr,
-                           lr.pieces, Fv, tile);
-      } else {
-        hipLaunchKernelGGL(gather_edge_to_row_long_kernel<float>, dim3(kLongGrid), dim3(kLongBlock), 0, stream, out, msg,
-                           off, perm, lr.list, lr.count, Fv, tile, accumulate);
-        hipLaunchKernelGGL(giant_sum_pieces_kernel<float>, dim3(kLongGrid), dim3(kLongBlock), 0, stream, partial, msg,
-                           perm, lr.hdr, lr.pieces, Fv, tile);
-      }
-    }
     hipLaunchKernelGGL(giant_sum_combine_kernel, dim3(kGiantCap / 4), dim3(256), 0, stream, out, partial, lr.hdr,
                        lr.giant_rows, lr.first, F, accumulate);
     launch_err = hipGetLastError();

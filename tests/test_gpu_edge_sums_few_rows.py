@@ -83,6 +83,50 @@ def test_permuted_sums_of_many_rows(device, rows, F):
     assert ((out.double() - want).abs() <= (deg.double()[:, None] + 1) * 2.0 ** -24 * scale + 1e-8).all()
 
 
+def sliced_sum(terms, slices):
+    """Slice s adds the terms s, s + slices, ... one after the other, the slices' sums are then added pairwise, the upper half to the
+    lower."""
+    n, F = terms.shape
+    terms = torch.cat([terms, terms.new_zeros(-n % slices, F)]).view(-1, slices, F)
+    a = torch.zeros(slices, F, device=terms.device)
+    for t in terms:
+        a = a + t
+    while a.shape[0] > 1:
+        a = a[:a.shape[0] // 2] + a[a.shape[0] // 2:]
+    return a[0]
+
+
+# listed rows of 65 vectors and more: as many slices as 1,024 threads have beside the whole row; whole rows, and pieces of giant ones
+@pytest.mark.parametrize("F", [65, 127, 129, 255, 257, 260, 300, 516, 602, 1025, 1028, 4100])
+def test_chains_of_listed_wide_rows(device, F):
+    rows = 16390
+    g = torch.Generator(device=device).manual_seed(F)
+    deg = torch.randint(0, 3, (rows,), generator=g, device=device)
+    marks = torch.tensor([1025, 1300, 2047, 2500, 4100], device=device)
+    hubs = torch.randperm(rows, generator=g, device=device)[:len(marks)]
+    deg[hubs] = marks
+    off = torch.cat([deg.new_zeros(1), deg.cumsum(0)])
+    msg = torch.rand(int(off[-1]), F, generator=g, device=device)
+    perm = torch.randperm(msg.shape[0], generator=g, device=device)
+    co, ids, s = off.to(torch.int32), perm.to(torch.int32), torch.cuda.current_stream().cuda_stream
+    vectors = F // 4 if F % 4 == 0 else F
+    slices = max(1, 1024 >> (vectors - 1).bit_length())
+    giant = min(16384, max(1024, (1 << 20) // (4 * F)))
+    for order in (None, perm):
+        out = torch.full((rows, F), float("nan"), device=device)
+        if order is None:
+            call("nts_gather_edge_to_dst", ptr(out), ptr(msg), ptr(co), rows, F, 0, s)
+        else:
+            call("nts_gather_edge_to_src", ptr(out), ptr(msg), ptr(co), ptr(ids), rows, F, 0, s)
+        for r in hubs.tolist():
+            terms = msg[off[r]:off[r + 1]] if order is None else msg[order[off[r]:off[r + 1]]]
+            pieces = [terms] if terms.shape[0] <= giant else terms.split(giant // 4)
+            want = torch.zeros(F, device=device)
+            for p in pieces:
+                want = want + sliced_sum(p, slices)
+            assert torch.equal(out[r], want), (r, terms.shape)
+
+
 # 29 groups of 64 columns for every row: 71 M groups, more than a launch has threads for
 @pytest.mark.parametrize("permuted", [False, True])
 def test_sums_of_more_groups_than_a_launch_holds(device, permuted):
