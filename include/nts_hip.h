@@ -263,14 +263,15 @@ int nts_spmm_plan_copy_schedule(const nts_spmm_plan_t *plan, uint32_t *items_out
 int nts_spmm_plan_info(const nts_spmm_plan_t *plan, uint32_t *items, uint32_t *split_rows,
                        uint32_t *partials);
 /* What a call of width F through this plan keeps in the plan's scratch, and what the schedule found:
- * bytes of partial sums, bytes of the padded input copy (0 when the call gathers from `in` itself),
+ * bytes of partial sums, bytes of the padded input copy (0 when the call gathers from `in` itself, also for want of memory),
  * the number of edges that repeat the gather index of the edge before them in their row, and whether
  * calls load a source row once per run of such edges.  Any out-pointer may be NULL. */
 int nts_spmm_plan_scratch_info(nts_spmm_plan_t *plan, uint32_t F, size_t *partial_bytes, size_t *padded_input_bytes,
                                uint64_t *repeated_edges, int *loads_once_per_run);
 /* Grow the plan's scratch (partial sums of split rows; for some schedules and widths also a copy of
  * the input with padded rows, see below) so that a later call of width F allocates
- * nothing. */
+ * nothing.  NTS_OK also where there is no memory for the copy: calls of that width then gather from
+ * `in` itself and do not ask for it, until the next nts_spmm_plan_reserve on the plan does. */
 int nts_spmm_plan_reserve(nts_spmm_plan_t *plan, uint32_t F);
 /* NtsScheduler::GatherByDstFromSrc / GatherBySrcFromDst on a full-graph chunk
  * (core/NtsScheduler.hpp:146-178, 239-271; core/graph.hpp:3432-3478).  `offsets` must be the
@@ -283,7 +284,7 @@ int nts_spmm_plan_reserve(nts_spmm_plan_t *plan, uint32_t F);
  * 128-byte lines (made by the call, in the plan's scratch, n_index * 4 * ceil(F / 32) * 32 bytes), so
  * that the row loads are 16 bytes per lane.  So does a schedule with source ranges and without such runs for rows of 257 to
  * 768 floats that are not whole lines, if it has 48 edges (24 from 513 floats up) for every row of `in`.  A call that finds no
- * memory for the copy, or is captured before nts_spmm_plan_reserve or an earlier call has made room for it, gathers from
+ * memory for the copy (it is asked for once, and again by nts_spmm_plan_reserve), or is captured before nts_spmm_plan_reserve or an earlier call has made room for it, gathers from
  * `in` itself; the sums are the same.
  * Concurrency.  A plan's scratch is shared by all calls on it.  The host side of a call is
  * serialised per plan, and a call on another stream than the previous one first waits, on the

@@ -2827,12 +2827,15 @@ bool use_runs(const nts_spmm_plan *plan) {
   return forced < 0 ? plan->dup_runs : forced == 1;
 }
 
+nts::ScratchNeed scratch_need(const nts_spmm_plan *plan, uint32_t F) {
+  return {plan->n_partials, F, padded_stride(plan, F), plan->n_index};
+}
+
 // Makes room in the plan's scratch for a call of width F and leaves the call's row stride (padded_stride) in *stride: 0 where it
 // gathers from the rows as they are, with the same sums (PlanScratch::place).  Caller holds plan->mu.
 int reserve_locked(nts_spmm_plan *plan, uint32_t F, bool heads, bool recorded, uint32_t *stride) {
-  const nts::ScratchNeed need{plan->n_partials, F, padded_stride(plan, F), plan->n_index};
   size_t ld = 0;
-  NTS_HIP_TRY(plan->scratch.place(need, !heads, recorded, &ld));
+  NTS_HIP_TRY(plan->scratch.place(scratch_need(plan, F), !heads, recorded, &ld));
   *stride = static_cast<uint32_t>(ld);
   return NTS_OK;
 }
@@ -2871,7 +2874,8 @@ int nts_spmm_plan_scratch_info(nts_spmm_plan_t *plan, uint32_t F, size_t *partia
   NTS_TRACE_RANGE("nts_spmm_plan_scratch_info");
   if (!plan) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_scratch_info: null plan");
   if (F == 0) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_scratch_info: F is 0");
-  const uint32_t ld = padded_stride(plan, F);
+  std::lock_guard<std::mutex> lock(plan->mu);
+  const size_t ld = plan->scratch.stride_of(scratch_need(plan, F));
   if (partial_bytes) *partial_bytes = static_cast<size_t>(plan->n_partials) * (ld ? ld : F) * sizeof(float);
   if (padded_input_bytes) *padded_input_bytes = ld ? static_cast<size_t>(plan->n_index) * ld * sizeof(float) : 0;
   if (repeated_edges) *repeated_edges = plan->repeated_edges;
@@ -2884,6 +2888,7 @@ int nts_spmm_plan_reserve(nts_spmm_plan_t *plan, uint32_t F) {
   if (!plan) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_reserve: null plan");
   if (F == 0) return nts::fail(NTS_ERR_INVALID, "nts_spmm_plan_reserve: F is 0");
   std::lock_guard<std::mutex> lock(plan->mu);
+  plan->scratch.ask_again();
   uint32_t ld = 0;
   return reserve_locked(plan, F, false, false, &ld);
 }

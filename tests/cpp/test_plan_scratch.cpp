@@ -4,6 +4,8 @@
 
 #include <stdio.h>
 
+#include <utility>
+
 namespace {
 size_t g_free = 0;
 int g_asked = 0, g_refused = 0, g_retired = 0;
@@ -15,6 +17,7 @@ struct Memory {
   struct Block {
     void *ptr = nullptr;
     size_t bytes = 0;
+    void swap(Block &o) { std::swap(*this, o); }
     int take(size_t want) {
       if (want == 0) return 0;
       ++g_asked;
@@ -108,10 +111,63 @@ int a_widths_partial_sums_stay_where_a_capture_found_them() {
   }
   return 0;
 }
+
+// Memory that was not there is asked for once, and what there is stays.
+int a_refusal_is_remembered() {
+  size_t ld = 9;
+  {  // no room for the copy: one attempt for any number of calls, one more for a reservation
+    fresh(kSlots * 320 + kRows * 320 - 1);
+    Scratch s;
+    for (int i = 0; i < 4; ++i) CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 0 && s.partial() && !s.copy());
+    CHECK(g_asked == 2 && g_refused == 1 && g_retired == 0 && s.stride_of(need(300)) == 0);
+    g_free += 1;
+    CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 0 && g_asked == 2);
+    s.ask_again();
+    CHECK(s.stride_of(need(300)) == 320 && s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 0 && g_refused == 2);  // (3 bytes short)
+    g_free += 4;
+    s.ask_again();
+    CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 320 && s.copy() && s.stride_of(need(300)) == 320);
+  }
+  {  // a wider copy that does not fit leaves the narrower one; narrower ones than refused are still had
+    fresh(kSlots * 640 + kRows * 320 + kRows * 500);
+    Scratch s;
+    CHECK(s.place(need(640), kCopy, kEager, &ld) == 0 && ld == 0);
+    CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 320);
+    const float *at = s.copy();
+    for (int i = 0; i < 3; ++i) CHECK(s.place(need(602), kCopy, kEager, &ld) == 0 && ld == 0 && s.copy() == at);
+    CHECK(g_refused == 1 && g_retired == 0);
+    CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 320 && s.copy() == at && g_refused == 1);
+    CHECK(s.place(need(420), kCopy, kEager, &ld) == 0 && ld == 448 && g_refused == 1 && g_retired == 1);
+  }
+  {  // the partial sums of a wider call need the memory that the copy has
+    fresh(kSlots * 320 + kRows * 320 + kSlots * 320);
+    Scratch s;
+    const nts::ScratchNeed wider{kSlots, 1000, 0, kRows};
+    CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 320);
+    CHECK(s.place(wider, kCopy, kEager, &ld) == 0 && ld == 0 && !s.copy() && s.partial());
+    const int asked = g_asked;
+    for (int i = 0; i < 3; ++i) CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && s.place(wider, kCopy, kEager, &ld) == 0);
+    CHECK(g_asked == asked);  // (the copy's size is known to be too much)
+  }
+  {  // room for the sums as they are and not for those beside a copy
+    fresh(kSlots * 300);
+    Scratch s;
+    for (int i = 0; i < 3; ++i) CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 0 && s.partial());
+    CHECK(g_asked == 2 && g_refused == 1 && g_retired == 0 && s.stride_of(need(300)) == 0);
+  }
+  {  // none for these either: an error, each time
+    fresh(kSlots * 300 - 1);
+    Scratch s;
+    for (int i = 0; i < 2; ++i) CHECK(s.place(need(300), kCopy, kEager, &ld) == 2 && ld == 0 && !s.partial());
+    g_free += 4;
+    CHECK(s.place(need(300), kCopy, kEager, &ld) == 0 && ld == 0 && s.partial());
+  }
+  return 0;
+}
 }  // namespace
 
 int main() {
-  if (a_widths_partial_sums_stay_where_a_capture_found_them()) return 1;
+  if (a_widths_partial_sums_stay_where_a_capture_found_them() || a_refusal_is_remembered()) return 1;
   printf("ok\n");
   return 0;
 }
