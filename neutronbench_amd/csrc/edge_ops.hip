@@ -2728,18 +2728,21 @@ constexpr uint32_t kOwnHubBlocks = 512;
 
 // Whether a group of lanes takes a row of its own and of 64 vectors at most (gather_edge_to_row_kernel), and not wavefronts sets of
 // rows.  us, sets / a row each, contiguous and permuted sums of edge rows:
+//                   contiguous: F = 47, 128, 200      permuted: F = 47, 64, 100, 128, 200
+//   2.9 K, 110 K      56 / 56, 78 / 59, 110 / 87        472 / 62, 150 / 62, 305 / 63, 296 / 63, 564 / 95
+//   6 K, 12 K         17 / 9, 16 / 11, 28 / 10          36 / 10, 36 / 10, 38 / 12, 38 / 12, 41 / 11
+//   16 K, 100 K       54 / 29, 52 / 45, 100 / 46        216 / 34, 178 / 32, 211 / 51, 207 / 51, 250 / 49
+//   16 K, 1 M         303 / 317, 427 / 386, 515 / 576   372 / 346, 462 / 318, 523 / 358, 500 / 426, 584 / 622
+//   10 K, 3 M         881 / 909, 1,667 / 1,349, 2,191 / 2,201   1,098 / 995, 1,776 / 1,156, 1,936 / 1,345, 1,920 / 1,508, 2,410 / 2,429
 //                   contiguous: F = 47, 128    permuted: F = 47, 64, 100, 128, 200
-//   6 K, 12 K         30 / 13, 26 / 15           62 / 13, 64 / 13, 68 / 15, 68 / 16
-//   16 K, 100 K       61 / 33, 55 / 46           231 / 39, 241 / 39, 250 / 55, 244 / 55
-//   16 K, 1 M         202 / 105, 191 / 159       504 / 154, 172 / 166, 304 / 170, 318 / 214 (hub rows in slices; as one
-//                     running sum, a row each: 358, 457, permuted 397, 464, 367, 513)
 //   30 K, 3 M         213 / 175, 361 / 348       534 / 221, 298 / 240, 447 / 335, 463 / 366
 //   169 K, 2.48 M     186 / 188, 310 / 319       381 / 229, 258 / 226, 374 / 309, 388 / 343, 639 / 523
 //   400 K, 2 M        187 / 223, 301 / 298       337 / 263, 294 / 214, 391 / 285, 409 / 312
 //   1 M, 8 M          508 / 639, 1,021 / 1,004   943 / 786, 689 / 645, 1,109 / 961, 1,133 / 1,061
 //   1.5 M, 6 M                                   763 / 791, 545 / 568, 888 / 809, 889 / 876
 //   2.4 M, 5 M                                   807 / 978, 508 / 629, 840 / 946, 861 / 976, 1,437 / 1,519
-// so a row each for the permuted sums up to a million rows, for the contiguous ones below 16,384.  Rows of up to eight vectors leave
+// so a row each for the permuted sums up to a million rows, for the contiguous ones below 16,384 (there hub rows are one running sum on
+// either side, and dense graphs lose up to a tenth at some widths to what sparse ones gain several times).  Rows of up to eight vectors leave
 // a lane or two a whole row there: 2.9 K, 110 K F = 4 34 / 46 with a row each, sets 15 / 18; but eight permuted vectors 30 K, 3 M 224
 // sets, 164, 169 K 191, 170 (400 K 161, 171; 16 K, 100 K 38, 49).
 constexpr uint32_t kMinHubRows = 64;  // (fewer rows have a block's worth of wavefronts beside each anyway: no hub blocks)
@@ -2749,10 +2752,11 @@ bool group_takes_a_row(uint32_t rows, uint32_t Fv, bool vectors, bool permuted) 
   return rows < (permuted ? 1u << 20 : kLongMinVertices);
 }
 // Rows that are few leave the chip idle, and floats spread them over four times as many lanes, each with 32 loads in flight where
-// vectors have room for eight (figures with hub rows in slices): 2.9 K, 110 K F = 128 42 / 54 -> 35 / 41 us, 16 K, 1 M 193 / 319 -> 159 / 214; from five wavefronts a row on only
-// the fewest rows: F = 300 2.9 K 77 / 87 -> 55 / 65, but 4 K, 2 M 1,320 / 1,755 -> 1,355 / 1,862.
+// vectors have room for eight.  us, vectors / floats, contiguous and permuted: F = 64 4 K, 200 K 148 / 102, 159 / 110, 16 K, 1 M 443 / 290, 484 /
+// 318; F = 128 153 / 103, 164 / 111 and 518 / 384, 558 / 426, 6 K, 12 K 9.6 / 10.9, 10.7 / 12.2.  From three wavefronts of floats a row on only
+// where these do not fill the chip twice: F = 200 40 rows, 3 K 26 / 18, 2 K, 8 K 12 / 10, but 16 K, 100 K 46 / 67, 16 K, 1 M 576 / 759.
 bool floats_for_few_rows(uint32_t rows, uint32_t F) {
-  return F > 32 && rows < kLongMinVertices && (F <= 256 || static_cast<uint64_t>(rows) * ceil_div(F, kWave) <= 16384);
+  return F > 32 && rows < kLongMinVertices && (F <= 128 || static_cast<uint64_t>(rows) * ceil_div(F, kWave) <= 16384);
 }
 
 // NTS_EDGE_SUM_STREAM=0 in the environment: contiguous edge rows take the lane-group kernel like permuted ones.
@@ -2888,8 +2892,9 @@ int gather_edge_impl(float *out, const float *msg, const uint32_t *off, const ui
   if (v4 && floats_for_few_rows(rows, F)) v4 = false;
   const uint32_t Fv = v4 ? F / 4 : F;
   // Long rows, and giant rows in pieces: in the first blocks of the row launch; the pieces' sums go to stream-ordered scratch and a
-  // launch of its own combines them in order.  Few rows: the first blocks find the hub rows themselves and take columns of 128 bytes of one each.
-  const uint32_t hub_lanes = v4 ? 8u : F > 32 ? 16u : 32u;
+  // launch of its own combines them in order.  Few rows: the first blocks find the hub rows themselves and take columns of 128 bytes of one each,
+  // of 64 where that leaves a row's blocks a tile each.
+  const uint32_t hub_lanes = v4 ? 8u : F > 32 && F <= 128 ? 16u : 32u;
   const bool own = !lr.list && rows >= kMinHubRows && (Fv > 8 || (perm && Fv > 4 && v4) || rows < kMaxNarrowHubRows);
   const uint32_t hub_blocks = lr.list ? kMergedLongBlocks : !own ? 0u : Fv <= hub_lanes ? kOwnHubBlocks / 2 : kOwnHubBlocks;
   const uint32_t most_lanes = own ? hub_lanes : 256u;

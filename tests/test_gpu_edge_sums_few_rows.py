@@ -23,9 +23,9 @@ def running_sums(msg, off, rows):
 
 
 # rows on both sides of 64 (below it no block looks for hub rows) and of 16,384 (from there on a launch lists them); widths of a
-# lane to eight, one of four to eight vectors, 33 floats and more in a wavefront of floats, and several wavefronts of them
+# lane to eight, one of four to eight vectors, 33 to 128 floats in wavefronts of floats, and wider ones in vectors
 @pytest.mark.parametrize("rows", [1, 63, 64, 4095, 16383, 16384])
-@pytest.mark.parametrize("F", [1, 4, 17, 32, 33, 128, 260])
+@pytest.mark.parametrize("F", [1, 4, 17, 32, 33, 128, 132, 260])
 @pytest.mark.parametrize("dense", [False, True])
 def test_sums_over_few_rows(device, rows, F, dense):
     print(f"case rows={rows} F={F} dense={dense}", flush=True)
@@ -81,6 +81,40 @@ def test_permuted_sums_of_many_rows(device, rows, F):
     size = torch.cat([terms.new_zeros(1, F, dtype=torch.float64), terms.double().abs().cumsum(0)])
     want, scale = total[off[1:]] - total[off[:-1]], size[off[1:]] - size[off[:-1]]
     assert ((out.double() - want).abs() <= (deg.double()[:, None] + 1) * 2.0 ** -24 * scale + 1e-8).all()
+
+
+# above 2.1 M edges the line between hub rows and others is a share of them: 2,100 edges here, with rows on and beside it; all rows,
+# the longest too, are one running sum, whoever adds them up; 4,096 narrow rows and more have no hub blocks
+@pytest.mark.parametrize("rows", [4095, 4096, 16383])
+@pytest.mark.parametrize("F", [4, 32, 40])
+def test_hub_line_of_many_edges(device, rows, F):
+    E, share = 2048 * 2100, 2100
+    marks = torch.tensor([share - 1, share, share + 1, 2 * share, 20001], device=device)
+    g = torch.Generator(device=device).manual_seed(rows + F)
+    at = torch.randperm(rows, generator=g, device=device)
+    hubs, rest = at[:len(marks)], at[len(marks):]
+    left, deg = E - int(marks.sum()), torch.zeros(rows, dtype=torch.int64, device=device)
+    deg[hubs], deg[rest] = marks, left // len(rest)
+    deg[rest[:left % len(rest)]] += 1
+    off = torch.cat([deg.new_zeros(1), deg.cumsum(0)])
+    assert int(off[-1]) // 2048 == share and int(deg[rest].max()) < share - 1
+    msg = torch.randn(E, F, generator=g, device=device)
+    perm = torch.randperm(E, generator=g, device=device)
+    co, ids, s = off.to(torch.int32), perm.to(torch.int32), torch.cuda.current_stream().cuda_stream
+    some = torch.cat([hubs[:-1], rest[:20]])
+    for order in (None, perm):
+        out = torch.full((rows, F), float("nan"), device=device)
+        if order is None:
+            call("nts_gather_edge_to_dst", ptr(out), ptr(msg), ptr(co), rows, F, 0, s)
+        else:
+            call("nts_gather_edge_to_src", ptr(out), ptr(msg), ptr(co), ptr(ids), rows, F, 0, s)
+        terms = msg if order is None else msg[order]
+        assert torch.equal(out[some], running_sums(terms, off, some))
+        assert torch.equal(out[hubs[-1:]], running_sums(terms, off, hubs[-1:]))
+        total = torch.cat([terms.new_zeros(1, F, dtype=torch.float64), terms.double().cumsum(0)])
+        size = torch.cat([terms.new_zeros(1, F, dtype=torch.float64), terms.double().abs().cumsum(0)])
+        want, scale = total[off[1:]] - total[off[:-1]], size[off[1:]] - size[off[:-1]]
+        assert ((out.double() - want).abs() <= (deg.double()[:, None] + 1) * 2.0 ** -24 * scale + 1e-7).all()  # (64-bit prefix sums)
 
 
 def sliced_sum(terms, slices):
