@@ -239,7 +239,8 @@ __device__ __forceinline__ float4 vnull<float4>() {
 // takes).  They are at most `tile` vectors (a power of two <= 256); thread t owns
 // column t % tile of C of the C * 256 / tile slices, a slice adds every so many-th edge of the range in ascending
 // order (a round's loads together), and the slices' sums are then added pairwise in a fixed tree, the upper half to the lower.
-template <typename V, int U, int C>
+// SKIP: nothing is requested beyond the range.
+template <typename V, int U, int C, bool SKIP>
 __device__ __forceinline__ void block_sum_edge_rows(V *__restrict__ dst, const V *__restrict__ msg,
                                                     const uint32_t *__restrict__ perm, uint32_t e0, uint32_t e1,
                                                     uint32_t Fv, uint32_t first_col, uint32_t end_col, uint32_t tile,
@@ -250,7 +251,9 @@ __device__ __forceinline__ void block_sum_edge_rows(V *__restrict__ dst, const V
 #pragma unroll
   for (int j = 0; j < C; ++j) a[j] = vnull<V>();
   if (col < end_col && e1 - e0 > slice) {
-    // The edge ids of the next round are requested while the rows of this one are on their way; beyond the range the last edge's.
+    // The edge ids of the next round are requested while the rows of this one are on their way; beyond the range the last edge's, which
+    // costs rows of a vector or two floats through a permutation, a line of memory a request, more than the rounds without a choice at each load give
+    // (60 K rows, 4 M edges F = 1 109 -> 102 us, F = 4 119 -> 113; but F = 7 171 -> 230, 30 K, 3 M F = 47 230 -> 658).
     // Through a permutation, 2.48 M edges of 47 floats 704 -> 379 us.  Eight vectors a round took the kernels 98 registers instead of
     // 62 (30 K rows, 3 M edges F = 128 467, held to 72 with spills 502, four a round 467); narrow rows, whose kernels hold as many anyway,
     // have room for them.
@@ -258,15 +261,20 @@ __device__ __forceinline__ void block_sum_edge_rows(V *__restrict__ dst, const V
     auto request_ids = [&] {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const uint32_t kk = k + (u * n_slices < left ? u * n_slices : left - 1);
-        id[u] = perm ? perm[kk] : kk;
+        const bool there = u * n_slices < left;
+        const uint32_t kk = k + (there ? u * n_slices : left - 1);
+        if (SKIP) id[u] = 0;
+        if (!SKIP || there) id[u] = perm ? perm[kk] : kk;
       }
     };
     request_ids();
     while (left) {
       V v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = msg[static_cast<size_t>(id[u]) * Fv + col];
+      for (int u = 0; u < U; ++u) {
+        if (SKIP) v[u] = vnull<V>();
+        if (!SKIP || u * n_slices < left) v[u] = msg[static_cast<size_t>(id[u]) * Fv + col];
+      }
       const uint32_t now = left;
       left = left > U * n_slices ? left - U * n_slices : 0u;
       if (left) {
@@ -387,7 +395,7 @@ __device__ __forceinline__ uint32_t long_limit_of(const LongRowWork<V> &lw, uint
 // The first blocks of a row launch take the listed long rows, one 256-thread block per row, and the
 // pieces of the giant ones (their partial sums are combined by a launch of its own afterwards); the
 // rows of the launch proper fill the chip meanwhile.
-template <typename V, int U, int OWN, bool WIDE = false>
+template <typename V, int U, int OWN, bool WIDE = false, bool SKIP = false>
 __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out, const V *__restrict__ msg,
                                                             const uint32_t *__restrict__ off,
                                                             const uint32_t *__restrict__ perm, uint32_t rows, uint32_t Fv,
@@ -439,8 +447,8 @@ __device__ __forceinline__ void sum_long_rows_in_this_block(V *__restrict__ out,
       dst = lw.partial + at * Fv;
     }
     const int add = i < n_rows && accumulate;
-    if (WIDE && lw.chains == 4) block_sum_edge_rows<V, U, WIDE ? 4 : 1>(dst, msg, perm, e0, e1, Fv, c0, c1, lw.tile, add, part);
-    else block_sum_edge_rows<V, U, 1>(dst, msg, perm, e0, e1, Fv, c0, c1, lw.tile, add, part);
+    if (WIDE && lw.chains == 4) block_sum_edge_rows<V, U, WIDE ? 4 : 1, false>(dst, msg, perm, e0, e1, Fv, c0, c1, lw.tile, add, part);
+    else block_sum_edge_rows<V, U, 1, SKIP>(dst, msg, perm, e0, e1, Fv, c0, c1, lw.tile, add, part);
   }
 }
 
@@ -698,7 +706,7 @@ __global__ __launch_bounds__(256, (sizeof(V) == 4 ? 8 : G <= 8 ? 5 : 1)) void ga
   if (blockIdx.x < lw.blocks) {
     constexpr int kOwn = !kCoop ? 0 : sizeof(V) == 16 ? 4 : 8;  // (wider rows come in millions, with a list)
     static_assert(sizeof(coop_tile) >= kHubBytes<V, kOwn>, "the hub blocks' scratch");
-    sum_long_rows_in_this_block<V, kHubLoads<V, G>, kOwn>(out, msg, off, perm, rows, Fv, accumulate, lw, coop_tile);
+    sum_long_rows_in_this_block<V, kHubLoads<V, G>, kOwn, false, G == 1 || (G == 2 && sizeof(V) == 4)>(out, msg, off, perm, rows, Fv, accumulate, lw, coop_tile);
     return;
   }
   long_limit = long_limit_of(lw, long_limit, off, rows);
