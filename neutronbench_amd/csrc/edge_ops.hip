@@ -14,15 +14,7 @@
 namespace nts {
 namespace {
 
-constexpr int kWavesPerBlock = 4;
-
-__device__ __forceinline__ uint32_t wave_item() {
-  return blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
-}
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & (kWave - 1); }
-
-inline dim3 wave_grid(uint32_t items) { return dim3(ceil_div(items ? items : 1, kWavesPerBlock)); }
-inline dim3 wave_block() { return dim3(kWavesPerBlock * kWave); }
 
 // ---- vertex -> edge copies ------------------------------------------------------------------
 //
@@ -964,21 +956,27 @@ __device__ __forceinline__ uint64_t giant_segment_values(uint64_t total_values) 
 }
 
 // The same for a call of few rows (kFewRows), whose launch has blocks of 256 threads for both.
-// The rows, by both sides' times in us, the kernels of many rows / these, edge softmax (H = 1, 4) and attention, forward, backward:
-//   rows, edges     softmax fwd       bwd               attention fwd       bwd
-//   2.7 K, 13 K     7 / 4, 7 / 5      8 / 5, 7 / 5      14 / 6, 18 / 9      11 / 6, 18 / 9
-//   16 K, 200 K     10 / 8, 20 / 15   9 / 7, 17 / 12    37 / 14, 51 / 29    30 / 13, 38 / 26
-//   10 K, 3 M       69 / 33, 304 / 128  67 / 34, 307 / 120  327 / 116, 572 / 207  387 / 141, 525 / 197
-//   30 K, 1 M       82 / 40, 94 / 39  85 / 40, 96 / 40  88 / 39, 99 / 55    92 / 42, 106 / 67
-//   60 K, 4 M       84 / 43, 84 / 65  86 / 41, 95 / 76  94 / 70, 135 / 113  99 / 88, 125 / 134
-//   169 K, 2.48 M   65 / 48, 70 / 62  66 / 47, 72 / 64  80 / 65, 139 / 109  84 / 86, 118 / 124
-//   250 K, 3 M      78 / 61, 95 / 75  82 / 57, 97 / 76  101 / 83, 157 / 140 92 / 105, 141 / 161
-//   200 K, 20 M     102 / 84, 245 / 239  108 / 91, 328 / 316  319 / 180, 492 / 459  418 / 282, 525 / 561
-//   100 K, 40 M     160 / 148, 459 / 485  204 / 185, 629 / 671  495 / 457, 766 / 802  526 / 521, 838 / 930
-// (the fused backward's above 32 K rows with the rows listed by one block, which now takes three launches; whole attention layers, both
-// directions, with the backward of many rows / of few: 169 K, 2.48 M one head 513 / 516, 200 K, 20 M two 2,798 / 2,581, 60 K, 4 M four 807 /
-// 803, 250 K, 3 M four 755 / 754; but eight heads 60 K, 10 M 2,306 / 2,408, 50 K, 600 K 344 / 317: that kernel holds two arrays and the
-// signs of the scores a lane, 114 registers for all of its paths together).  More rows were not measured.
+// The rows, by both sides' times in us, a call after the other, the kernels of many rows / these, for one, four and eight heads:
+//   rows, edges    softmax fwd                  bwd                          attention fwd                bwd (eight heads always of many rows)
+//   16 K, 200 K    78 / 34, 89 / 40, 91 / 40    84 / 34, 91 / 41, 91 / 40    94 / 34, 98 / 41, 97 / 42    96 / 39, 101 / 44
+//   30 K, 1 M      76 / 33, 86 / 43, 84 / 50    79 / 33, 88 / 42, 86 / 53    86 / 38, 94 / 60, 107 / 72   89 / 44, 101 / 69
+//   60 K, 4 M      79 / 43, 87 / 66, 116 / 106  79 / 42, 98 / 76, 176 / 159  92 / 71, 146 / 110, 191 / 164  93 / 85, 140 / 133
+//   60 K, 10 M     84 / 55, 155 / 152, 294 / 300  86 / 57, 198 / 192, 388 / 385  149 / 121, 234 / 197, 513 / 473  140 / 139, 325 / 335
+//   169 K, 2.48 M  90 / 42, 94 / 54, 96 / 71    93 / 38, 94 / 55, 101 / 84   104 / 57, 142 / 100, 186 / 134  108 / 76, 127 / 119
+//   250 K, 3 M     91 / 47, 94 / 59, 97 / 74    94 / 43, 93 / 61, 121 / 101  107 / 67, 157 / 118, 201 / 150  107 / 87, 136 / 139
+//   200 K, 20 M    100 / 80, 257 / 248, 448 / 428  108 / 80, 339 / 322, 648 / 608  329 / 194, 504 / 494, 732 / 712  405 / 305, 543 / 604
+//   100 K, 40 M    166 / 133, 463 / 476         206 / 182, 638 / 666         462 / 398, 782 / 779         483 / 466, 836 / 908
+//   beyond the line:
+//   400 K, 2 M     68 / 49, 71 / 60, 79 / 71    68 / 48, 71 / 54, 84 / 69    92 / 70, 134 / 116, 183 / 146  95 / 100, 127 / 137
+//   500 K, 20 M    98 / 82, 252 / 239, 446 / 453  102 / 78, 320 / 309, 616 / 618  297 / 187, 474 / 468, 826 / 792  368 / 307, 554 / 596
+//   1 M, 8 M       93 / 90, 131 / 126, 251 / 227  82 / 76, 164 / 139, 279 / 263  196 / 176, 264 / 278, 453 / 489  187 / 226, 339 / 420
+// What decides is how many edges a row has, which a call does not say.  Up to the line these kernels take a third to a half of sparse
+// graphs' time off and cost the four-head calls of graphs of hundreds of edges a row 2 to 10 % of an operator (0.6 to 1.5 % of a layer:
+// four heads, both directions, the backward of few / of many rows 100 K, 30 M 4,740 / 4,713, 200 K, 20 M 3,684 / 3,660, 60 K, 10 M 1,828 / 1,772,
+// but 40 K, 1 M 342 / 350, 169 K, 2.48 M 707 / 712).  Sixteen heads 16 K, 1 M 105 / 72, 97 / 77, 159 / 86, 60 K, 4 M 238 / 249, 305 / 308, 372 / 334,
+// 169 K, 2.48 M 171 / 142, 205 / 176, 290 / 203.  Beyond it the fused backward loses and the other three still gain a little; the line is not
+// theirs alone.  The fused backward of more than four heads holds two arrays and the signs of the scores a lane, 114 registers for all of its paths
+// together: above 32 K rows it is even in the operator (60 K, 4 M 256 / 257) and was slower in whole layers (60 K, 10 M 2,306 / 2,408, 50 K, 600 K 344 / 317).
 constexpr uint32_t kFewRows = 1u << 18;
 constexpr uint32_t kFewRowsManyHeads = 1u << 15;
 constexpr uint32_t kFewPieceValues = 4096;
@@ -2697,7 +2695,7 @@ int collect_long_rows(const LongRows &lr, const uint32_t *off, uint32_t rows, ui
     NTS_LAUNCH_CHECK("few_long_rows_kernel");
     return NTS_OK;
   }
-  if (int rc = nts_memset_zero(lr.hdr, 8 * sizeof(uint32_t), stream)) return rc;  // counters and the ticket
+  if (int rc = nts_memset_zero(lr.hdr, 8 * sizeof(uint32_t), stream)) return rc;  // counters
   hipLaunchKernelGGL(collect_long_rows_kernel, dim3(ceil_div(rows, 256)), dim3(256), 0, stream, lr.list, lr.count,
                      lr.giant_rows, lr.hdr, off, rows, width, limit, giant_limit);
   NTS_LAUNCH_CHECK("collect_long_rows_kernel");

@@ -423,9 +423,9 @@ __global__ __launch_bounds__(256, (group_waves<G, HEADS, RUNS>())) void spmm_gro
   using V = typename Vec<VEC>::type;
   static_assert(U <= G, "a step's pairs come from one tile");  // U edges per step: their rows are requested together
   const uint32_t gl = threadIdx.x & (G - 1);
-  // Blocks are dealt out to the eight XCDs in turn.  1 << panel_bits panels (up to eight) alternate and an XCD meets one of
-  // them.  Of other numbers, eight blocks of items are 8 * panels units of work, panel by panel, and XCD x takes the units
-  // x * panels and on: an XCD meets as few panels as can be.  (The alternating panels too by that rule: 169 K rows, 2.48 M edges
+  // Blocks are dealt out to the eight XCDs in turn.  1 << panel_bits panels (two or four; one needs no turns) alternate and an XCD
+  // meets one of them.  Of other numbers, eight blocks of items are 8 * panels units of work, panel by panel, and XCD x takes the units
+  // x * panels and on: an XCD meets two panels, three where there are eleven (641 to 704 floats).  (The alternating panels too by that rule: 169 K rows, 2.48 M edges
   // F = 128 97 -> 100 us.)
   uint32_t panel = 0, block = blockIdx.x;
   if (PANELS) {
@@ -1033,7 +1033,7 @@ void launch_group(const LaunchArgs &a, uint32_t panels = 1) {
   const uint32_t per_block = 256 / G;
   const uint32_t n_list = a.items ? a.n_items : 0u, n_total = a.n_items + (a.items ? a.rows_after_items : 0u);
   int panel_bits = -1;
-  for (uint32_t bits = 0; bits < 4; ++bits)
+  for (uint32_t bits = 0; bits < 3; ++bits)
     if (panels == 1u << bits) panel_bits = static_cast<int>(bits);
   // where panels do not alternate, whole turns of the XCDs (the last ones' surplus blocks leave at once)
   const uint32_t turn = PANELS && panel_bits < 0 ? kXcds : 1u;
@@ -1117,7 +1117,7 @@ int pick_vec(const LaunchArgs &a) {
 }
 
 // Lanes of a column panel (16 or 32, of four floats each: panels of 256 or 512 bytes), or 0 for rows that are not cut into panels.
-// An XCD meets one or two panels of a row only, so that its 4 MB L2 holds a share of the gathered matrix that is as many times
+// An XCD meets one or two panels of a row only (three of eleven), so that its 4 MB L2 holds a share of the gathered matrix that is as many times
 // smaller.  us without / with, panels of whole lines (the last one may be shorter):
 //   rows          169 K, 2.48 M   60 K, 4 M   1 M, 6 M        20 M of 500 K   233 K, 114.8 M simple   2.45 M, 126 M (40 M)
 //   128  2 x 16   111 / 98                                    722 / 690       2,651 / 2,660           5,221 / 5,108
