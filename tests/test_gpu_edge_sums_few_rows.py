@@ -89,7 +89,7 @@ def test_permuted_sums_of_many_rows(device, rows, F):
 @pytest.mark.parametrize("F", [4, 32, 40])
 def test_hub_line_of_many_edges(device, rows, F):
     E, share = 2048 * 2100, 2100
-    marks = torch.tensor([share - 1, share, share + 1, 2 * share, 20001], device=device)
+    marks = torch.tensor([share - 1, share, share + 1, 2 * share, 9001], device=device)
     g = torch.Generator(device=device).manual_seed(rows + F)
     at = torch.randperm(rows, generator=g, device=device)
     hubs, rest = at[:len(marks)], at[len(marks):]
