@@ -95,6 +95,30 @@ def test_panels_that_share_lines(device, rows, edges, F):
     compare(device, SpmmPlan(off, rows, edges, 4096), off, idx, rows, edges, F, 100)
 
 
+# arrays that start at any float: with and without a copy, whole lines and others
+@pytest.mark.parametrize("ranges", [1, 8])
+@pytest.mark.parametrize("lead_in,lead_out", [(1, 0), (0, 1), (2, 3), (3, 2)])
+@pytest.mark.parametrize("F", [128, 300, 384, 500, 512, 602, 640])
+def test_panels_of_arrays_off_16_bytes(device, ranges, lead_in, lead_out, F):
+    rows, edges = 16500, 800000
+    off, idx = simple_graph(rows, edges, device, True)
+    plan = SpmmPlan(off, rows, edges, 64, idx, rows, ranges) if ranges > 1 else SpmmPlan(off, rows, edges, 4096)
+    g = torch.Generator(device=device).manual_seed(F)
+    x, w = torch.randn(rows, F, generator=g, device=device), torch.rand(edges, generator=g, device=device)
+    init = torch.randn(rows, F, generator=g, device=device)
+    s = torch.cuda.current_stream().cuda_stream
+    for accumulate in (0, 1):
+        want = init.clone()
+        call("nts_spmm_gather_planned", plan.handle, ptr(x), ptr(want), ptr(w), ptr(off), ptr(idx), 0, F, accumulate, s)
+        x_at, out_at = torch.empty(rows * F + 4, device=device), torch.full((rows * F + 8,), 7.0, device=device)
+        xs, out = x_at[lead_in:lead_in + rows * F], out_at[lead_out:lead_out + rows * F]
+        xs.copy_(x.view(-1))
+        out.copy_(init.view(-1))
+        call("nts_spmm_gather_planned", plan.handle, ptr(xs), ptr(out), ptr(w), ptr(off), ptr(idx), 0, F, accumulate, s)
+        assert torch.equal(out.view(rows, F), want)
+        assert bool((out_at[:lead_out] == 7).all()) and bool((out_at[lead_out + rows * F:] == 7).all())
+
+
 def test_captured_call_without_room_for_the_copy(device):
     """The capture of a call whose copy has no room yet gathers from the rows as they are; one with room, from the copy."""
     rows, edges, F = 3001, 150050, 602
