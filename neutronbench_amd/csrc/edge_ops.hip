@@ -2735,7 +2735,7 @@ constexpr uint32_t kOwnHubBlocks = 512;
 // Whether a group of lanes takes a row of its own and of 64 vectors at most (gather_edge_to_row_kernel), and not wavefronts sets of
 // rows.  us, sets / a row each, contiguous and permuted sums of edge rows:
 //                   contiguous: F = 47, 128, 200      permuted: F = 47, 64, 100, 128, 200
-//   2.9 K, 110 K      56 / 56, 78 / 59, 110 / 87        472 / 62, 150 / 62, 305 / 63, 296 / 63, 564 / 95
+//   2.9 K, 110 K      56 / 56, 78 / 59, 110 / 69        472 / 62, 150 / 62, 305 / 63, 296 / 63, 564 / 77
 //   6 K, 12 K         17 / 9, 16 / 11, 28 / 10          36 / 10, 36 / 10, 38 / 12, 38 / 12, 41 / 11
 //   16 K, 100 K       54 / 29, 52 / 45, 100 / 46        216 / 34, 178 / 32, 211 / 51, 207 / 51, 250 / 49
 //   16 K, 1 M         303 / 317, 427 / 386, 515 / 576   372 / 346, 462 / 318, 523 / 358, 500 / 426, 584 / 622
